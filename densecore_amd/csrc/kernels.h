@@ -123,7 +123,7 @@ hipError_t launch_dense_lds(const DenseLdsArgs& a, hipStream_t stream, hipEvent_
 // Wavefronts per row tile of the LDS-staged dense kernels for a matrix (pick_waves, as a divisor of eight; 0: none)
 int dense_lds_wpr(int64_t nb, int64_t rowtiles);
 
-// ---- prefill.hip: nine to sixteen rows as ONE activation tile against a streamed Q4_K matrix (skinny16_kernel) ----
+// ---- skinny16.hip: nine to sixteen rows as ONE activation tile against a streamed Q4_K matrix (skinny16_kernel) ----
 struct Skinny16Args {
     const uint8_t* w0 = nullptr;   // tiled Q4_K weights; gate when w1 is set
     const uint8_t* w1 = nullptr;   // up weights: y = silu(w0 x) * (w1 x)
@@ -214,8 +214,8 @@ hipError_t launch_swiglu_quantize_q8k_pmajor(const float* gate, const float* up,
 // y[n][ldy] = P-major activations . tiled weights^T on the int8 matrix cores.  A launch that would leave workgroup
 // slots empty splits K into runs of super-blocks whose sums go to planes of `part` (prefill_part_bytes() bytes, 0 when
 // nothing is split) and are added in order by a second launch.
-// wtype: kTypeQ4K, or kTypeQ5K (a third MFMA chain for the fifth code bits; 64-row workgroups).
-size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n, int wtype);
+// wtype: kTypeQ4K, kTypeQ5K or kTypeQ6K.
+size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n);
 // silu(gate . x) * (up . x) from ONE launch (prefill.hip: the pair form of the GEMM kernel), dense and expert-grouped
 bool prefill_pair_applies(int wtype, int64_t rows, int64_t nb, int64_t n);
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,

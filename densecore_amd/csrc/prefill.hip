@@ -15,7 +15,8 @@
 // thirteen bits, exact as fp16; every product and every partial sum is an integer below 2^24, so the fp32 result
 // is the integer min_dot itself -- the value (float)min_dot that the update needs, with nothing to combine or
 // convert on the vector unit.
-// Nine MFMAs per 16x16 output tile and super-block, no per-sub-block vector work; the fp32 update
+// Nine MFMAs per 16x16 output tile and super-block (Q5_K the same, Q6_K eight: weight_digits.h), no per-sub-block vector
+// work; the fp32 update
 //     acc += yd * (d * dot_scaled - dmin * min_dot)
 // is done once per super-block, as every reference kernel does (three fp32 operations per output, five vector
 // instructions with the digits' shift-add and one conversion; the reference's
@@ -29,273 +30,23 @@
 //   wavefront = 2 weight tiles (32 rows) x the 8 activation tiles; it reads its weight tiles
 //               straight from HBM in MFMA lane order and expands them in registers
 //
-// P-major activations (written by quantize_q8k_pmajor_kernel): [b][mt][4688 B], mt = m / 16:
-//   [j 0..3][kq 0..3][tok 0..15][16 B]   codes: bytes 0..7 = sub-block ga(j), elements 8kq..8kq+7,
-//                                        bytes 8..15 = sub-block gb(j), same elements, with
-//                                        (ga, gb) = (0,2) (1,3) (4,6) (5,7) for j = 0..3 -- the pairs
-//                                        that one 16-byte word of a weight tile holds per nibble half
-//   [tok][32 B] at 4096                  fp16: l_0..l_7, then 128 h_0..128 h_7
-//   [tok] fp32 at 4608                   block scale d
-//   16 zero bytes at 4672                what the lanes of k-groups 2 and 3 feed the min MFMA
+// The activations come in the P-major layout (pmajor.h).
 #include <hip/hip_ext.h>
 
 #include "common.h"
 #include "kernels.h"
 #include "decode_tile.h"
+#include "pmajor.h"
 #include "q8k_block.h"
+#include "weight_digits.h"
 
 namespace mq {
 
 namespace {
 
-constexpr int kPTileBytes = 4688;
-constexpr int kPTileWords = kPTileBytes / 16;  // 293
-constexpr int kPDigitOff = 4096, kPScaleOff = 4608, kPZeroOff = 4672;
 constexpr int kMTilesPerGroup = 8;             // activation tiles (of 16 rows) per workgroup
 constexpr int kMTilesSmall = 2;                // ... of an expert-grouped launch whose experts hold a dozen or two rows
 constexpr int kMTilesMid = 4;                  // ... or three or four dozen
-
-typedef unsigned short v2us __attribute__((ext_vector_type(2)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-// four bytes (each <= 15) times a 3-bit digit, bytewise: two 16-bit products whose bytes do not carry into each
-// other (15 * 7 < 256).  The digit is half H of `digits`, taken for both products (the operand-select bits of the
-// packed multiply: no instruction of its own).
-template <int H>
-__device__ __forceinline__ uint32_t scale_bytes(uint32_t nibbles, uint32_t digits) {
-    const v2us a = __builtin_bit_cast(v2us, nibbles);
-    const v2us d = __builtin_bit_cast(v2us, digits);
-    const v2us dd = H ? v2us{d.y, d.y} : v2us{d.x, d.x};
-    return __builtin_bit_cast(uint32_t, (v2us)(a * dd));
-}
-
-// bytes i and i + 1 of `word` as two 16-bit numbers (one v_perm_b32: selector 0x0c yields a zero byte)
-__device__ __forceinline__ uint32_t digit_pair(uint32_t word, int i) {
-    return __builtin_amdgcn_perm(0u, word, 0x0c000c00u | (uint32_t)i | ((uint32_t)(i + 1) << 16));
-}
-
-struct WTile {
-    v4i b5[4];         // Q5_K only: the fifth code bits times the whole 6-bit scale (16 * scale * bit is their share)
-    v4i hi[4], lo[4];  // B operands of the four chunk pairs, scaled by the high / low scale digit
-    v8h mins;          // B operand of the min MFMA: the eight mins as fp16, in every k-group
-    float d, dmin;
-};
-
-// Q5: the codes are nibble + 16 * bit (bit s of the bytes of qh = fifth bit in sub-block s, core/src/kernels/hwy/hwy_moe_quant.cc:177-200);
-// scale * code = scale * nibble + 16 * (scale * bit), and scale * bit <= 63 is a byte: a third MFMA chain.
-template <bool Q5>
-__device__ __forceinline__ void expand_tile(const v4u seg0, const v4u seg1, const v4u hdr, const v2u qh, int kq, WTile& t) {
-    // 6-bit scales and mins (core/src/kernels/hwy/hwy_moe_quant.cc:90-101), four to a word
-    const uint32_t sc03 = hdr.y & 0x3f3f3f3fu, mn03 = hdr.z & 0x3f3f3f3fu;
-    const uint32_t sc47 = (hdr.w & 0x0f0f0f0fu) | (((hdr.y >> 6) & 0x03030303u) << 4);
-    const uint32_t mn47 = ((hdr.w >> 4) & 0x0f0f0f0fu) | (((hdr.z >> 6) & 0x03030303u) << 4);
-    const uint32_t s1_03 = (sc03 >> 3) & 0x07070707u, s0_03 = sc03 & 0x07070707u;
-    const uint32_t s1_47 = (sc47 >> 3) & 0x07070707u, s0_47 = sc47 & 0x07070707u;
-    const v4u seg[2] = {seg0, seg1};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t s1w = i ? s1_47 : s1_03, s0w = i ? s0_47 : s0_03;
-        // sub-blocks 4i .. 4i+3 are bytes 0..3 of the digit words
-        const uint32_t l0 = seg[i].x & 0x0f0f0f0fu, l1 = seg[i].y & 0x0f0f0f0fu;  // sub-block 4i
-        const uint32_t l2 = seg[i].z & 0x0f0f0f0fu, l3 = seg[i].w & 0x0f0f0f0fu;  // sub-block 4i+2
-        const uint32_t h0 = (seg[i].x >> 4) & 0x0f0f0f0fu, h1 = (seg[i].y >> 4) & 0x0f0f0f0fu;  // 4i+1
-        const uint32_t h2 = (seg[i].z >> 4) & 0x0f0f0f0fu, h3 = (seg[i].w >> 4) & 0x0f0f0f0fu;  // 4i+3
-        // digits of sub-blocks (4i, 4i+1) and (4i+2, 4i+3), two to a word
-        const uint32_t ab1 = digit_pair(s1w, 0), ab0 = digit_pair(s0w, 0);
-        const uint32_t ce1 = digit_pair(s1w, 2), ce0 = digit_pair(s0w, 2);
-        t.hi[2 * i] = v4i{(int)scale_bytes<0>(l0, ab1), (int)scale_bytes<0>(l1, ab1), (int)scale_bytes<0>(l2, ce1),
-                          (int)scale_bytes<0>(l3, ce1)};
-        t.lo[2 * i] = v4i{(int)scale_bytes<0>(l0, ab0), (int)scale_bytes<0>(l1, ab0), (int)scale_bytes<0>(l2, ce0),
-                          (int)scale_bytes<0>(l3, ce0)};
-        t.hi[2 * i + 1] = v4i{(int)scale_bytes<1>(h0, ab1), (int)scale_bytes<1>(h1, ab1), (int)scale_bytes<1>(h2, ce1),
-                              (int)scale_bytes<1>(h3, ce1)};
-        t.lo[2 * i + 1] = v4i{(int)scale_bytes<1>(h0, ab0), (int)scale_bytes<1>(h1, ab0), (int)scale_bytes<1>(h2, ce0),
-                              (int)scale_bytes<1>(h3, ce0)};
-        if constexpr (Q5) {
-            const uint32_t scw = i ? sc47 : sc03;
-            const uint32_t abs_ = digit_pair(scw, 0), ces = digit_pair(scw, 2);  // whole scales of sub-blocks (4i, 4i+1), (4i+2, 4i+3)
-            auto bits = [&](uint32_t word, int sb) { return (word >> sb) & 0x01010101u; };
-            t.b5[2 * i] = v4i{(int)scale_bytes<0>(bits(qh.x, 4 * i), abs_), (int)scale_bytes<0>(bits(qh.y, 4 * i), abs_),
-                              (int)scale_bytes<0>(bits(qh.x, 4 * i + 2), ces), (int)scale_bytes<0>(bits(qh.y, 4 * i + 2), ces)};
-            t.b5[2 * i + 1] = v4i{(int)scale_bytes<1>(bits(qh.x, 4 * i + 1), abs_), (int)scale_bytes<1>(bits(qh.y, 4 * i + 1), abs_),
-                                  (int)scale_bytes<1>(bits(qh.x, 4 * i + 3), ces), (int)scale_bytes<1>(bits(qh.y, 4 * i + 3), ces)};
-        }
-    }
-    // byte -> fp16: 0x6400 | n is 1024 + n; two at a time
-    const v2h bias = {(_Float16)1024.0f, (_Float16)1024.0f};
-    const v2h m01 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64006400u, mn03, 0x05010500u)) - bias;
-    const v2h m23 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64006400u, mn03, 0x05030502u)) - bias;
-    const v2h m45 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64006400u, mn47, 0x05010500u)) - bias;
-    const v2h m67 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64006400u, mn47, 0x05030502u)) - bias;
-    t.mins = v8h{m01.x, m01.y, m23.x, m23.y, m45.x, m45.y, m67.x, m67.y};
-    t.d = half_bits_to_float(hdr.x & 0xffffu);
-    t.dmin = half_bits_to_float(hdr.x >> 16);
-}
-
-// ---- Q6_K on the matrix cores ---------------------------------------------------------------------------------
-// weight = d * scale_g * (code - 32): sixteen signed 8-bit scales per super-block, one per 16 weights, six-bit codes
-// (core/src/llm/matmul/q6_small_batch.h:13-92).  scale * (code - 32) reaches 4096, so both factors are cut in two:
-//     scale + 128 = u = 16 u1 + u0   (u1, u0 in 0..15)          code - 32 = c = 8 c1 + c0   (c0 in 0..7, c1 in -4..3)
-//     sum_g scale_g sum_i c_i q_i = 128 P11 + 16 P10 + 8 P01 + P00 - 128 R,
-//     Pjk = sum_i (u_j c_k)_i q_i,  R = sum_i c_i q_i
-// exactly, in int32: every byte u_j * c_k lies in [-60, 105] and c itself in [-32, 31] (the chain R multiplies
-// 4 c, the tile's own bytes, and enters with -32).  Five chains of four K = 64 MFMAs per 16 x 16 outputs and
-// super-block, no term from the activations' block sums, so the activation tiles are the Q4_K kernel's: the tile
-// keeps each 64-byte run of low / high nibbles as two 32-weight sub-blocks (4 j + z and 4 j + z + 2 for the low and
-// high nibbles of one byte), the pairs the P-major layout puts side by side.
-// u_j * c1 for a signed c1 comes bytewise from the unsigned product with d1 = c1 + 4 = code >> 3:
-//     u c1 = u d1 - 4 u,   ((u d1 | 0x80) - 4 u) ^ 0x80 per byte (u d1 <= 105 < 128, 4 u <= 60: no borrow).
-struct WTile6 {
-    v4i p11[4], p10[4], p01[4], p00[4], r4[4];
-    float d;
-};
-
-__device__ __forceinline__ uint32_t signed_digit_bytes(uint32_t prod, uint32_t four_u) {
-    return ((prod | 0x80808080u) - four_u) ^ 0x80808080u;
-}
-
-__device__ __forceinline__ void expand_tile6(const v4u ql0, const v4u ql1, const v4u qh, const v4u sc, uint32_t dw, int kq, WTile6& t) {
-    const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
-    uint32_t u1w[4], u0w[4], f1w[4], f0w[4];  // digits of the sixteen scales, and four times the digits
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const uint32_t u = scw[w] ^ 0x80808080u;  // scale + 128, bytewise
-        u1w[w] = (u >> 4) & 0x0f0f0f0fu;
-        u0w[w] = u & 0x0f0f0f0fu;
-        f1w[w] = u1w[w] << 2;
-        f0w[w] = u0w[w] << 2;
-    }
-    // weights 128 j + 32 z + l, l = 8 kq .. 8 kq + 7, have scale 8 j + 2 z + (kq >> 1): byte 2 (z & 1) + (kq >> 1) of
-    // scale word 2 j + (z >> 1)
-    const uint32_t sel = (uint32_t)(kq >> 1);
-    const v4u qlw[2] = {ql0, ql1};
-    const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-        for (int zp = 0; zp < 2; ++zp) {  // B operand jj = 2 j + zp: sub-blocks z = zp (dwords 0, 1) and z = zp + 2 (dwords 2, 3)
-            const int jj = 2 * j + zp;
-            const uint32_t k = 2u * (uint32_t)zp + sel;
-            // the two sub-blocks' digits as 16-bit numbers side by side (low half: z = zp, high half: z = zp + 2)
-            const uint32_t pick = 0x0c040c00u + k * 0x00010001u;
-            const uint32_t d1p = __builtin_amdgcn_perm(u1w[2 * j + 1], u1w[2 * j], pick);
-            const uint32_t d0p = __builtin_amdgcn_perm(u0w[2 * j + 1], u0w[2 * j], pick);
-            const uint32_t spread = k * 0x01010101u;  // byte k in all four bytes
-            const uint32_t f1[2] = {__builtin_amdgcn_perm(0u, f1w[2 * j], spread), __builtin_amdgcn_perm(0u, f1w[2 * j + 1], spread)};
-            const uint32_t f0[2] = {__builtin_amdgcn_perm(0u, f0w[2 * j], spread), __builtin_amdgcn_perm(0u, f0w[2 * j + 1], spread)};
-            const uint32_t src[2] = {zp ? qlw[j].z : qlw[j].x, zp ? qlw[j].w : qlw[j].y};
-            uint32_t r4[4], p11[4], p10[4], p01[4], p00[4];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {      // h = 0: z = zp (low nibbles), h = 1: z = zp + 2 (high nibbles)
-                const int z = zp + 2 * h;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {  // the lane's eight weights of the sub-block, four to a word
-                    const uint32_t nib = (h ? src[i] >> 2 : src[i] << 2) & 0x3c3c3c3cu;
-                    const uint32_t hi = qhw[2 * j + i];
-                    const uint32_t top = (z == 3 ? hi : hi << (6 - 2 * z)) & 0xc0c0c0c0u;
-                    const uint32_t b4 = top | nib;              // 4 (code - 32) as signed bytes
-                    const uint32_t code4 = b4 ^ 0x80808080u;    // 4 code
-                    const uint32_t d1 = (code4 >> 5) & 0x07070707u, c0 = (code4 >> 2) & 0x07070707u;
-                    const int o = 2 * h + i;
-                    r4[o] = b4;
-                    if (h == 0) {
-                        p10[o] = scale_bytes<0>(c0, d1p), p00[o] = scale_bytes<0>(c0, d0p);
-                        p11[o] = signed_digit_bytes(scale_bytes<0>(d1, d1p), f1[0]);
-                        p01[o] = signed_digit_bytes(scale_bytes<0>(d1, d0p), f0[0]);
-                    } else {
-                        p10[o] = scale_bytes<1>(c0, d1p), p00[o] = scale_bytes<1>(c0, d0p);
-                        p11[o] = signed_digit_bytes(scale_bytes<1>(d1, d1p), f1[1]);
-                        p01[o] = signed_digit_bytes(scale_bytes<1>(d1, d0p), f0[1]);
-                    }
-                }
-            }
-            t.r4[jj] = v4i{(int)r4[0], (int)r4[1], (int)r4[2], (int)r4[3]};
-            t.p11[jj] = v4i{(int)p11[0], (int)p11[1], (int)p11[2], (int)p11[3]};
-            t.p10[jj] = v4i{(int)p10[0], (int)p10[1], (int)p10[2], (int)p10[3]};
-            t.p01[jj] = v4i{(int)p01[0], (int)p01[1], (int)p01[2], (int)p01[3]};
-            t.p00[jj] = v4i{(int)p00[0], (int)p00[1], (int)p00[2], (int)p00[3]};
-        }
-    }
-    t.d = half_bits_to_float(dw & 0xffffu);
-}
-
-// Q6_K the way compute_tile6 multiplies it (decode_tile.h), for activation tiles of sixteen rows: the B bytes are
-// 4 * (code - 32), a scale per 16 weights.  Word jj = 2 j + zp of a P-major activation tile holds a lane's eight values
-// of sub-block z = zp (bytes 0..7) and of z = zp + 2 (bytes 8..15) of half j, and the k-groups 0, 1 / 2, 3 of a K = 32
-// MFMA over one of those runs are the two 16-weight scale groups of the sub-block: four MFMAs per word, each with the
-// bytes of one group alone (the others' lanes zero), sixteen group sums per (row, token) and super-block, each times
-// its scale in integers -- dot = sum_g scale_g * sum (code - 32) * q8 exactly (core/src/llm/matmul/q6_small_batch.h:56-83),
-// carrying the bytes' factor 4.
-struct WTile6G {
-    long bg[4][4];  // [word jj][(z = zp, first 16), (zp, last 16), (zp + 2, first 16), (zp + 2, last 16)]
-    int sg[4][4];   // their scales
-    float d;
-};
-
-__device__ __forceinline__ long two_words(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); }
-
-__device__ __forceinline__ void expand_tile6g(const v4u ql0, const v4u ql1, const v4u qh, const v4u sc, uint32_t dw, int kq, WTile6G& t) {
-    const uint32_t qlw[2][4] = {{ql0.x, ql0.y, ql0.z, ql0.w}, {ql1.x, ql1.y, ql1.z, ql1.w}};
-    const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
-    const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
-    const uint32_t keep_lo = kq < 2 ? 0xffffffffu : 0u, keep_hi = ~keep_lo;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int zp = 0; zp < 2; ++zp) {
-            const int jj = 2 * j + zp;
-            uint32_t b4[2][2];  // [nibble side h][word i]: 4 * (code - 32) of z = zp + 2 h
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int z = zp + 2 * h;
-                    const uint32_t src = qlw[j][2 * zp + i];
-                    const uint32_t nib = (h ? src >> 2 : src << 2) & 0x3c3c3c3cu;
-                    const uint32_t hi = qhw[2 * j + i];
-                    const uint32_t top = (z == 3 ? hi : hi << (6 - 2 * z)) & 0xc0c0c0c0u;
-                    b4[h][i] = top | nib;
-                }
-            t.bg[jj][0] = two_words(b4[0][0] & keep_lo, b4[0][1] & keep_lo);
-            t.bg[jj][1] = two_words(b4[0][0] & keep_hi, b4[0][1] & keep_hi);
-            t.bg[jj][2] = two_words(b4[1][0] & keep_lo, b4[1][1] & keep_lo);
-            t.bg[jj][3] = two_words(b4[1][0] & keep_hi, b4[1][1] & keep_hi);
-            // group 8 j + 2 z + half: byte 2 (z & 1) + half of scale word 2 j + (z >> 1)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const int z = zp + 2 * h;
-                    t.sg[jj][2 * h + half] = (int)(int8_t)((scw[2 * j + (z >> 1)] >> (8 * (2 * (z & 1) + half))) & 0xffu);
-                }
-        }
-    t.d = half_bits_to_float(dw & 0xffffu);
-}
-
-// one activation tile of sixteen rows (its four words a[]) against the expanded tile: dot[i] += the lane's four
-// (token 4 kq + i, weight row r) sums, times 4
-template <bool kFenced = false>
-__device__ __forceinline__ void mul_tile6g(const v4i (&a)[4], const WTile6G& w, int (&dot)[4]) {
-    const v4i zero = {0, 0, 0, 0};
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-        // kFenced: the scheduler keeps each word's four MFMAs and their sums together instead of sixteen results in
-        // flight (kernels with many accumulators: registers)
-        if (kFenced && jj > 0) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-            const long a8 = gq < 2 ? two_words((uint32_t)a[jj].x, (uint32_t)a[jj].y) : two_words((uint32_t)a[jj].z, (uint32_t)a[jj].w);
-            const v4i pg = __builtin_amdgcn_mfma_i32_16x16x32_i8(a8, w.bg[jj][gq], zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dot[i] += __mul24(pg[i], w.sg[jj][gq]);
-        }
-    }
-}
-
-typedef __attribute__((address_space(1))) const void* global_ptr_t;
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // Requests the activation tiles of super-block b (copy_words 16-byte words, contiguous in HBM) straight
 // into LDS with global_load_lds_dwordx4: lane l of a request writes its 16 bytes at base + 16*l, so a
@@ -323,7 +74,7 @@ __device__ __forceinline__ void request_a_tiles(const uint8_t* __restrict__ src,
 
 // kWTilesPerWave = 2: the 128 x 128 workgroup tile above.  1: 64 weight rows per workgroup, for launches whose
 // 128-row workgroups would leave compute units without their two workgroups (M up to a few hundred).
-// PAIR (two weight tiles per wavefront, Q4_K): the wavefront's two tiles are the SAME row tile of two matrices, gate
+// PAIR (two weight tiles per wavefront): the wavefront's two tiles are the SAME row tile of two matrices, gate
 // (w) and up (w2), and what is stored is silu(gate) * up -- the two fp32 planes a gate launch and an up launch would
 // write, and the pass that reads them back to form the product, never exist (for 2048 rows of a 4096 -> 14336 FFN that
 // is 235 MB written and read).  The same accumulators, the same SiLU function on the same values: the same bits.
@@ -340,7 +91,7 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                                                            const uint8_t* __restrict__ w_shared,
                                                            const uint8_t* __restrict__ w2 = nullptr,
                                                            const uint8_t* __restrict__ w2_shared = nullptr, int silu_mode = 0) {
-    static_assert(!PAIR || (kWTilesPerWave == 2 && WT == kWtQ4), "the pair form is the two-tile Q4_K kernel");
+    static_assert(!PAIR || kWTilesPerWave == 2, "the pair form is the two-tile kernel");
     extern __shared__ __align__(16) uint8_t a_lds[];  // two buffers of MT * kPTileBytes bytes
     constexpr int kBufBytes = MT * kPTileBytes;
     constexpr bool Q5 = WT == kWtQ5, Q6 = WT == kWtQ6;
@@ -433,7 +184,8 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 WTile w1;
-                expand_tile<false>(seg0[t], seg1[t], hdr[t], qh[t], kq, w1);
+                if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, w1);
+                else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, w1);
                 if (b + 1 < b_end) request_w(b + 1, t);  // the raw tile's registers are free again
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
@@ -444,33 +196,40 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                         for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
                         const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
                         const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
-                        const v8h dg = *reinterpret_cast<const v8h*>(at + digit_off);
                         const v4i zero = {0, 0, 0, 0};
                         const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
                         v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.hi[0], zero, 0, 0, 0);
                         v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.lo[0], zero, 0, 0, 0);
-                        const v4f mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, w1.mins, zero_f, 0, 0, 0);
+                        v4i b5 = zero;
+                        if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.b5[0], zero, 0, 0, 0);
+                        v4f mn = zero_f;
+                        if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(at + digit_off), w1.mins, zero_f, 0, 0, 0);
 #pragma unroll
                         for (int j = 1; j < 4; ++j) {
                             hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.hi[j], hi, 0, 0, 0);
                             lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.lo[j], lo, 0, 0, 0);
+                            if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.b5[j], b5, 0, 0, 0);
                         }
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {  // the arithmetic of the two-tiles-at-once form below
-                            const int dot = hi[i] * 8 + lo[i];
-                            const float v = __fmaf_rn(-w1.dmin, mn[i], __fmul_rn(w1.d, (float)dot));
-                            acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                            const int dot = join_digits<WT, MT>(hi[i], lo[i], b5[i]);
+                            if constexpr (Q6) {
+                                acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], w1.d), (float)dot, acc[t][m][i]);
+                            } else {
+                                const float v = __fmaf_rn(-w1.dmin, mn[i], __fmul_rn(w1.d, (float)dot));
+                                acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                            }
                         }
                     }
                 }
             }
             continue;
         }
-        std::conditional_t<Q6, WTile6, WTile> wt[kWTilesPerWave];
+        WTile wt[kWTilesPerWave];
 #pragma unroll
         for (int t = 0; t < kWTilesPerWave; ++t) {
             if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, wt[t]);
-            else expand_tile<Q5>(seg0[t], seg1[t], hdr[t], qh[t], kq, wt[t]);
+            else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, wt[t]);
         }
         if (b + 1 < b_end) {
             request_a_tiles<MT>(a_src + (size_t)(b + 1) * a_stride, a_lds + ((b + 1) & 1) * kBufBytes, copy_words, wave, lane);
@@ -487,67 +246,43 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                 for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
                 const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
                 const v4i zero = {0, 0, 0, 0};
+                const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
                 const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
-                if constexpr (Q6) {
-                    v4i p11[kWTilesPerWave], p10[kWTilesPerWave], p01[kWTilesPerWave], p00[kWTilesPerWave], r4[kWTilesPerWave];
+                v4i hi[kWTilesPerWave], lo[kWTilesPerWave], b5[kWTilesPerWave];
+                v4f mn[kWTilesPerWave];
+                v8h dg;
+                if constexpr (!Q6) dg = *reinterpret_cast<const v8h*>(at + digit_off);
+#pragma unroll
+                for (int t = 0; t < kWTilesPerWave; ++t) {
+                    hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].hi[0], zero, 0, 0, 0);
+                    lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].lo[0], zero, 0, 0, 0);
+                    b5[t] = zero;
+                    if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].b5[0], zero, 0, 0, 0);
+                    if constexpr (!Q6) mn[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, wt[t].mins, zero_f, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 1; j < 4; ++j)
 #pragma unroll
                     for (int t = 0; t < kWTilesPerWave; ++t) {
-                        p11[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].p11[0], zero, 0, 0, 0);
-                        p10[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].p10[0], zero, 0, 0, 0);
-                        p01[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].p01[0], zero, 0, 0, 0);
-                        p00[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].p00[0], zero, 0, 0, 0);
-                        r4[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].r4[0], zero, 0, 0, 0);
+                        hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].hi[j], hi[t], 0, 0, 0);
+                        lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].lo[j], lo[t], 0, 0, 0);
+                        if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].b5[j], b5[t], 0, 0, 0);
                     }
 #pragma unroll
-                    for (int j = 1; j < 4; ++j)
+                for (int t = 0; t < kWTilesPerWave; ++t)
 #pragma unroll
-                        for (int t = 0; t < kWTilesPerWave; ++t) {
-                            p11[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].p11[j], p11[t], 0, 0, 0);
-                            p10[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].p10[j], p10[t], 0, 0, 0);
-                            p01[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].p01[j], p01[t], 0, 0, 0);
-                            p00[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].p00[j], p00[t], 0, 0, 0);
-                            r4[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].r4[j], r4[t], 0, 0, 0);
-                        }
-#pragma unroll
-                    for (int t = 0; t < kWTilesPerWave; ++t)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            // sum_g scale_g sum (code - 32) q8, the integer of the reference's kernel, then its one fused
-                            // multiply-add per block (core/src/llm/matmul/q6_small_batch.h:84-86)
-                            const int isum = p11[t][i] * 128 + p10[t][i] * 16 + p01[t][i] * 8 + p00[t][i] - r4[t][i] * 32;
-                            acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], wt[t].d), (float)isum, acc[t][m][i]);
-                        }
-                } else {
-                    const v8h dg = *reinterpret_cast<const v8h*>(at + digit_off);
-                    const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
-                    v4i hi[kWTilesPerWave], lo[kWTilesPerWave], fb[kWTilesPerWave];
-                    v4f mn[kWTilesPerWave];
-#pragma unroll
-                    for (int t = 0; t < kWTilesPerWave; ++t) {
-                        hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].hi[0], zero, 0, 0, 0);
-                        lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].lo[0], zero, 0, 0, 0);
-                        if (Q5) fb[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].b5[0], zero, 0, 0, 0);
-                        mn[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, wt[t].mins, zero_f, 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int j = 1; j < 4; ++j)
-#pragma unroll
-                        for (int t = 0; t < kWTilesPerWave; ++t) {
-                            hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].hi[j], hi[t], 0, 0, 0);
-                            lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].lo[j], lo[t], 0, 0, 0);
-                            if (Q5) fb[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].b5[j], fb[t], 0, 0, 0);
-                        }
-#pragma unroll
-                    for (int t = 0; t < kWTilesPerWave; ++t)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            int dot = hi[t][i] * 8 + lo[t][i];
-                            if (Q5) dot += fb[t][i] * 16;
+                    for (int i = 0; i < 4; ++i) {
+                        const int dot = join_digits<WT, MT>(hi[t][i], lo[t][i], b5[t][i]);
+                        if constexpr (Q6) {
+                            // the integer of the reference's kernel (times 4, taken out of d), then its one fused multiply-add
+                            // per block (core/src/llm/matmul/q6_small_batch.h:84-86)
+                            acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], wt[t].d), (float)dot, acc[t][m][i]);
+                        } else {
                             // yd * (d * dot - dmin * min_dot): three fp32 operations per output and super-block
                             const float v = __fmaf_rn(-wt[t].dmin, mn[t][i], __fmul_rn(wt[t].d, (float)dot));
                             acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
                         }
-                }
+                    }
             }
         }
     }
@@ -592,309 +327,6 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                 yp += ldy;
             }
             yp += 12 * ldy;
-        }
-    }
-}
-
-// ---- nine to sixteen activation rows against a streamed matrix ------------------------------------------------
-// The decode kernels multiply a weight tile with EIGHT activation rows per MFMA (the sixteen operand rows hold a row's
-// two sub-blocks of a 64-weight chunk side by side, the sub-block scales are applied on the vector unit); from nine rows
-// they take two such token tiles per weight tile: 16 MFMAs and ~147 vector instructions.  This kernel multiplies the
-// same rows as ONE tile of sixteen, the way prefill_gemm_kernel does (scale digits folded into the weight operand, the
-// min term as one fp16 MFMA): 9 MFMAs and ~126 vector instructions per weight tile.  Everything else is
-// dense_lds_kernel's (dense_lds.hip): eight wavefronts, WPR of them per row tile taking the super-blocks h, h + WPR, ...
-// in ascending order, partial sums met in wave order, two register stages of raw weight tiles; the rows' quantized
-// activations -- here P-major tiles -- are staged in LDS once per workgroup while the first weight tiles travel, or,
-// where all super-blocks do not fit LDS (GA: the 14336 columns of an FFN's down projection), requested from global
-// memory a stage ahead, beside the weight tile (six loads, all answered by the L2).  The integers of a (row, token,
-// super-block) are the same and so is the fp32 update, (wd * yd) * dot - (wm * yd) * min_dot added to the running
-// sum: the same bits as dense_lds_kernel and matmul_kernel.
-// WT: Q4_K; Q5_K with a third MFMA chain for the fifth code bits times the whole scale (expand_tile<true>), the decode
-// kernels' integers (scale * (nibble + 16 bit)) and update; Q6_K with the arithmetic of compute_tile6 carried over to
-// tiles of sixteen (expand_tile6g, mul_tile6g above): sixteen K = 32 MFMAs per activation tile and super-block, one per
-// 16-weight scale group, the group sums times their scales in integers, one fused multiply-add per super-block.
-// LDS: [nb][4688] activation tiles (not GA), then the partial sums [8 / WPR][WPR - 1][NMAT][4][64].
-// nb % WPR == 0 (host-checked): every wavefront has nb / WPR stages; FLOW 1: that count is odd (a single run); 0: even, a
-// single run or runs of an even number of stages; 2: even, runs of an odd number of stages.
-struct ATile16 {
-    v4i a[4];   // the four 64-weight chunks of this lane's operand
-    v4f yd;     // the Q8_K scales of rows 4 kq .. 4 kq + 3
-    v8h dg;     // this lane's operand of the min MFMA (fp16 digits of the sub-block sums, or zeros)
-};
-
-// MT: activation tiles of sixteen rows (one, or two for 17 to 32 rows: the weight tile is expanded once for both, 18
-// MFMAs and ~156 vector instructions against the 32 + 294 of two passes over two token tiles of eight each).  With two
-// tiles the partial sums share LDS with the activation tiles (one more barrier before they are written).
-template <int NMAT, int WPR, int FLOW, bool GA, int MT, int WT = kWtQ4>
-__global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
-    constexpr bool ODD = FLOW == 1;  // (FLOW: the shape of the stage loop, below)
-    constexpr int RPW = 8 / WPR;  // row tiles per workgroup
-    constexpr bool Q5 = WT == kWtQ5, Q6 = WT == kWtQ6;
-    constexpr int kStride = tile_stride<WT>();
-    constexpr int kTileLoads = Q6 ? 5 : Q5 ? 4 : 3;  // requests of a weight tile (load_tile, load_tile6)
-    constexpr bool kRedShares = MT > 1 && !GA;  // the partial sums reuse the activation tiles' LDS
-    extern __shared__ __align__(16) uint8_t lds16[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, kq = lane >> 4;
-    const int nb = (int)p.nb;
-    const int64_t rowtiles = (p.rows + 15) >> 4;
-    const int pair = wave / WPR, h = wave % WPR;
-    int64_t rt = (int64_t)blockIdx.x * RPW + pair;
-    const bool dead = rt >= rowtiles;  // past the last row tile: stream the last one again and store nothing
-    if (dead) rt = rowtiles - 1;
-    float* red = reinterpret_cast<float*>(lds16 + ((GA || kRedShares) ? (size_t)0 : (size_t)nb * MT * kPTileBytes));  // (one run when the sums lie behind the tiles)
-
-    const uint8_t* tiles[NMAT];
-    tiles[0] = p.w0 + tile_offset(rt, 0, nb, kStride);
-    if (NMAT == 2) tiles[1] = p.w1 + tile_offset(rt, 0, nb, kStride);
-    const int cnt = nb / WPR;  // stages of this wavefront: super-blocks h, h + WPR, ...
-
-    // lane (r, kq): weight row r of the tile, activation rows 4 kq .. 4 kq + 3 of every activation tile
-    const int digit_off = kq < 2 ? kPDigitOff + r * 32 + kq * 16 : kPZeroOff;
-    auto read_a = [&](ATile16& t, const uint8_t* at) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) t.a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
-        t.yd = *reinterpret_cast<const v4f*>(at + kPScaleOff + kq * 16);
-        if constexpr (!Q6) t.dg = *reinterpret_cast<const v8h*>(at + digit_off);  // (Q6_K has no min term)
-    };
-
-    // ---- the activation tiles ([super-block][tile]) -> LDS: a linear copy, 1 KB per request, the wavefronts taking the
-    // requests in turn.  Rows too long for LDS in one piece come in `ranges` runs of super-blocks, one run at a time:
-    // stage i of every wavefront lies in run i / (cnt / ranges), so the wavefronts change runs together (cnt % ranges == 0,
-    // host-checked).
-    const int sb_per_range = nb / p.ranges, stages_per_range = cnt / p.ranges;
-    auto stage_range = [&](int rg) {
-        const uint32_t base = (uint32_t)(uintptr_t)(lds_ptr_t)lds16;
-        const int words = sb_per_range * MT * kPTileWords;
-        const uint8_t* src = p.ap + (size_t)rg * (size_t)words * 16;
-        for (int c = wave; c * 64 < words; c += 8) {
-            const int first = c * 64;
-            if (first + lane < words) {
-                const uint8_t* g = src + (size_t)(first + lane) * 16;
-                const uint32_t dst = base + (uint32_t)first * 16u;
-                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(dst) : "memory", "m0");
-            }
-        }
-    };
-    if constexpr (!GA) stage_range(0);
-
-    typename TileOf<WT>::Regs ring_t[2][NMAT];
-    ATile16 ring_a[GA ? 2 : 1][GA ? MT : 1];
-    auto issue = [&](auto st_c, int i) {  // only ever called for a stage that exists
-        constexpr int st = decltype(st_c)::value;
-        const int b = h + i * WPR;
-        if constexpr (GA) {  // ahead of the tiles: they are needed first
-#pragma unroll
-            for (int t = 0; t < MT; ++t) read_a(ring_a[st][t], p.ap + ((size_t)b * MT + t) * kPTileBytes);
-        }
-#pragma unroll
-        for (int m = 0; m < NMAT; ++m) load_tile_wt<WT>(ring_t[st][m], tiles[m] + (size_t)b * kStride, lane);
-    };
-
-    float acc[NMAT][MT][4];
-#pragma unroll
-    for (int m = 0; m < NMAT; ++m)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[m][t][i] = 0.0f;
-
-    int b_range0 = 0;  // first super-block of the run in LDS
-    auto consume = [&](auto st_c, int i) {
-        constexpr int st = decltype(st_c)::value;
-        const int b = h + i * WPR;
-        const v4i zero = {0, 0, 0, 0};
-        const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int m = 0; m < NMAT; ++m) {
-            // three and four tiles: the second matrix reads the activation tiles from LDS again instead of keeping the first
-            // one's copies in registers (they would not fit)
-            if (MT > 2 && m > 0) asm volatile("" ::: "memory");
-            if constexpr (Q6) {
-                const TileRegs6& tr = ring_t[st][m];
-                WTile6G w6;
-                expand_tile6g(tr.ql0, tr.ql1, tr.qh, tr.sc, tr.d, kq, w6);
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    if (MT > 2 && t > 0) asm volatile("" ::: "memory");  // a tile's LDS reads stay behind the tile before (registers)
-                    ATile16 from_lds;
-                    if constexpr (!GA) read_a(from_lds, lds16 + ((size_t)(b - b_range0) * MT + t) * kPTileBytes);
-                    const ATile16& at = GA ? ring_a[GA ? st : 0][GA ? t : 0] : from_lds;
-                    const float ydv[4] = {at.yd.x, at.yd.y, at.yd.z, at.yd.w};
-                    int dot[4] = {0, 0, 0, 0};
-                    mul_tile6g<(MT > 2)>(at.a, w6, dot);
-#pragma unroll
-                    for (int i2 = 0; i2 < 4; ++i2) {  // compute_tile6's update
-                        const int isum = dot[i2] >> 2;  // the B bytes carried a factor 4
-                        acc[m][t][i2] = __fmaf_rn(__fmul_rn(ydv[i2], w6.d), (float)isum, acc[m][t][i2]);
-                    }
-                }
-            } else {
-            WTile wt;
-            expand_tile<Q5>(ring_t[st][m].q0, ring_t[st][m].q1, ring_t[st][m].hdr, Q5 ? ring_t[st][m].qh : v2u{0u, 0u}, kq, wt);
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                ATile16 from_lds;
-                if constexpr (!GA) read_a(from_lds, lds16 + ((size_t)(b - b_range0) * MT + t) * kPTileBytes);
-                const ATile16& at = GA ? ring_a[GA ? st : 0][GA ? t : 0] : from_lds;
-                const float ydv[4] = {at.yd.x, at.yd.y, at.yd.z, at.yd.w};
-                v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[0], wt.hi[0], zero, 0, 0, 0);
-                v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[0], wt.lo[0], zero, 0, 0, 0);
-                v4i fb = zero;  // Q5_K: the fifth code bits times the whole scale
-                if constexpr (Q5) fb = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[0], wt.b5[0], zero, 0, 0, 0);
-                const v4f mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(at.dg, wt.mins, zero_f, 0, 0, 0);
-#pragma unroll
-                for (int j = 1; j < 4; ++j) {
-                    hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[j], wt.hi[j], hi, 0, 0, 0);
-                    lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[j], wt.lo[j], lo, 0, 0, 0);
-                    if constexpr (Q5) fb = __builtin_amdgcn_mfma_i32_16x16x64_i8(at.a[j], wt.b5[j], fb, 0, 0, 0);
-                }
-#pragma unroll
-                for (int i2 = 0; i2 < 4; ++i2) {  // compute_tile's update (decode_tile.h); mn[i2] is the integer min_dot, exactly
-                    int dot = hi[i2] * 8 + lo[i2];
-                    if constexpr (Q5) dot += fb[i2] * 16;
-                    const float d = __fmul_rn(wt.d, ydv[i2]);
-                    const float dm = __fmul_rn(wt.dmin, ydv[i2]);
-                    const float term = __fsub_rn(__fmul_rn(d, (float)dot), __fmul_rn(dm, mn[i2]));
-                    acc[m][t][i2] = __fadd_rn(acc[m][t][i2], term);
-                }
-            }
-            }
-        }
-    };
-
-    // Two register stages, one in flight while the other is multiplied; written out for an even and for an odd number
-    // of stages (an odd run is one stage followed by an even run with the stages' roles swapped), so that no request
-    // is ever made for a stage that does not exist.
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    const bool single = ODD && cnt == 1;  // wave-uniform
-    issue(S0{}, 0);
-    asm volatile("" ::: "memory");  // requests stay in stage order
-    if (!single) {
-        issue(S1{}, 1);
-        asm volatile("" ::: "memory");
-    }
-    if constexpr (!GA) {
-        // the LDS-direct copies are older than the tile requests: they have landed once at most those are outstanding
-        if (single) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NMAT * kTileLoads) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * NMAT * kTileLoads) : "memory");
-        __builtin_amdgcn_s_barrier();  // no fence: a fence would wait for the outstanding weight tiles as well
-        asm volatile("" ::: "memory");
-    }
-    if constexpr (ODD) {
-        consume(S0{}, 0);
-        if (!single) {
-            issue(S0{}, 2);  // cnt >= 3
-            asm volatile("" ::: "memory");
-            int i = 1;
-            for (; i + 2 < cnt; i += 2) {
-                consume(S1{}, i);
-                issue(S1{}, i + 2);
-                asm volatile("" ::: "memory");
-                consume(S0{}, i + 1);
-                issue(S0{}, i + 3);
-                asm volatile("" ::: "memory");
-            }
-            consume(S1{}, i);
-            consume(S0{}, i + 1);
-        }
-    } else {
-        // The next run of super-blocks replaces the one in LDS once every wavefront has multiplied its last stage of it
-        // (the weight tiles of the next run's first two stages are already on their way: they do not depend on LDS).
-        if constexpr (FLOW == 0) {
-            // A single run, or runs of an even number of stages: run by run, the change of runs between two inner loops
-            // (a conditional change inside the pipelined loop, as below, costs the Q6_K forms their registers: 256 and
-            // spills against 120-130).  The last pair of stages of the launch is peeled off: no request past the end.
-            const int runs = GA ? 1 : p.ranges;
-            int i = 0;
-            for (int rg = 0; rg < runs; ++rg) {
-                if (rg > 0) {  // wave-uniform, the same in every wavefront
-                    __syncthreads();
-                    stage_range(rg);
-                    b_range0 = rg * sb_per_range;
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's share of the copy (and its two stages of weight tiles)
-                    __syncthreads();
-                }
-                const int i_stop = (rg + 1) * (cnt / runs) - (rg == runs - 1 ? 2 : 0);
-                for (; i < i_stop; i += 2) {
-                    consume(S0{}, i);
-                    issue(S0{}, i + 2);
-                    asm volatile("" ::: "memory");
-                    consume(S1{}, i + 1);
-                    issue(S1{}, i + 3);
-                    asm volatile("" ::: "memory");
-                }
-            }
-            consume(S0{}, i);
-            consume(S1{}, i + 1);
-        } else {
-            // FLOW == 2: runs of an odd number of stages begin at either stage of a pair
-            auto next_range = [&](int i) {
-                if (GA || p.ranges == 1 || i == 0 || i % stages_per_range) return;  // wave-uniform, the same i in every wavefront
-                __syncthreads();
-                const int rg = i / stages_per_range;
-                stage_range(rg);
-                b_range0 = rg * sb_per_range;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's share of the copy (and its two stages of weight tiles)
-                __syncthreads();
-            };
-            int i = 0;
-            for (; i + 2 < cnt; i += 2) {
-                next_range(i);
-                consume(S0{}, i);
-                issue(S0{}, i + 2);
-                asm volatile("" ::: "memory");
-                next_range(i + 1);
-                consume(S1{}, i + 1);
-                issue(S1{}, i + 3);
-                asm volatile("" ::: "memory");
-            }
-            next_range(i);
-            consume(S0{}, i);
-            next_range(i + 1);
-            consume(S1{}, i + 1);
-        }
-    }
-
-    // ---- the WPR wavefronts of a row tile meet in wave order; the first one stores ----
-    if (WPR > 1) {
-        if (kRedShares) __syncthreads();  // every wavefront has read its last activation tile
-        if (h > 0) {
-#pragma unroll
-            for (int m = 0; m < NMAT; ++m)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        red[(((((pair * (WPR - 1) + (h - 1)) * NMAT + m) * MT + t) * 4 + i) * 64) + lane] = acc[m][t][i];
-        }
-        __syncthreads();
-    }
-    if (h == 0 && !dead) {
-        for (int wv = 1; wv < WPR; ++wv) {
-#pragma unroll
-            for (int m = 0; m < NMAT; ++m)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        acc[m][t][i] = __fadd_rn(acc[m][t][i], red[(((((pair * (WPR - 1) + (wv - 1)) * NMAT + m) * MT + t) * 4 + i) * 64) + lane]);
-        }
-        const int64_t row = rt * 16 + r;
-        if (row < p.rows) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int tok = 16 * t + 4 * kq + i;
-                    if (tok < p.n) {
-                        float v = acc[0][t][i];
-                        if (NMAT == 2) v = silu_mul(v, acc[NMAT - 1][t][i], p.silu_mode);
-                        p.y[(size_t)tok * (size_t)p.ldy + (size_t)row] = v;
-                    }
-                }
         }
     }
 }
@@ -1039,7 +471,7 @@ PrefillShape prefill_shape(int64_t rows, int64_t nb, int64_t n, bool one_tile_pe
     // two workgroups fit a compute unit: while the 128-row workgroups would not even give every unit one, 64-row
     // ones fill the chip better (14336 rows on 256 units: up to M = 256; 52 -> 40 us at M = 128, 55 -> 51 at 256,
     // and 76 -> 79, 78 -> 91 at M = 384, 512, where the wide ones stay)
-    ps.narrow = one_tile_per_wave || ((rowtiles + 7) / 8) * (int64_t)ps.groups <= (int64_t)compute_units();  // Q5_K, Q6_K: their operand sets only fit the registers of 64-row workgroups
+    ps.narrow = one_tile_per_wave || ((rowtiles + 7) / 8) * (int64_t)ps.groups <= (int64_t)compute_units();  // (the pair form: a wavefront's two tiles are one row tile of two matrices)
     ps.row_wgs = (unsigned)(ps.narrow ? (rowtiles + 3) / 4 : (rowtiles + 7) / 8);
     const int64_t wgs = (int64_t)ps.row_wgs * ps.groups;
     int splits = (int)(2 * (int64_t)compute_units() / (wgs > 0 ? wgs : 1));
@@ -1214,54 +646,62 @@ int moe_gemm_item_tiles(int64_t entries, int64_t groups) {
     return entries <= 30 * groups ? kMTilesSmall : entries <= 160 * groups ? kMTilesMid : kMTilesPerGroup;
 }
 
+namespace {
+// Two activation buffers are more than the default 64 KB of dynamic LDS: raised once for every form that stages eight tiles.
+hipError_t raise_gemm_lds() {
+    static bool raised = false;
+    if (raised) return hipSuccess;
+#define MQ_FORM(KW, WT_, PAIR_) reinterpret_cast<const void*>(&prefill_gemm_kernel<KW, WT_, PAIR_>)
+    for (const void* k : {MQ_FORM(1, kWtQ4, false), MQ_FORM(2, kWtQ4, false), MQ_FORM(2, kWtQ4, true), MQ_FORM(1, kWtQ5, false), MQ_FORM(2, kWtQ5, false),
+                          MQ_FORM(2, kWtQ5, true), MQ_FORM(1, kWtQ6, false), MQ_FORM(2, kWtQ6, false), MQ_FORM(2, kWtQ6, true)}) {
+        hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
+        if (e != hipSuccess) return e;
+    }
+#undef MQ_FORM
+    raised = true;
+    return hipSuccess;
+}
+bool gemm_type(int wtype) { return wtype == kTypeQ4K || wtype == kTypeQ5K || wtype == kTypeQ6K; }
+// GO(form constant) for the weight type of a launch
+#define MQ_BY_TYPE(wtype, GO)              \
+    do {                                   \
+        if ((wtype) == kTypeQ6K) GO(kWtQ6); \
+        else if ((wtype) == kTypeQ5K) GO(kWtQ5); \
+        else GO(kWtQ4);                    \
+    } while (0)
+}  // namespace
+
 hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expert_bytes, const uint8_t* w_shared, int64_t rows,
                                        int64_t nb, const uint8_t* ap, int64_t entries, int64_t groups_max, const int32_t* plan,
                                        bool scatter, float* y, int64_t ldy, hipStream_t stream, int mt) {
-    if (wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K) return hipErrorInvalidValue;
+    if (!gemm_type(wtype)) return hipErrorInvalidValue;
     if (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup) return hipErrorInvalidValue;
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = moe_gemm_tiles_max(entries, groups_max);
     const int64_t items = moe_gemm_items_max(entries, groups_max);
     if (rowtiles == 0 || items == 0) return hipSuccess;
     if (items > 65535) return hipErrorInvalidValue;
-    static bool raised = false;
-    if (!raised) {
-        for (const void* k : {reinterpret_cast<const void*>(&prefill_gemm_kernel<1>), reinterpret_cast<const void*>(&prefill_gemm_kernel<2>),
-                              reinterpret_cast<const void*>(&prefill_gemm_kernel<1, kWtQ5>), reinterpret_cast<const void*>(&prefill_gemm_kernel<1, kWtQ6>)}) {
-            hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
-            if (e != hipSuccess) return e;
-        }
-        raised = true;
-    }
+    if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
     const int32_t* out_row = scatter ? plan + 4 + 3 * items + 16 * m_tiles : nullptr;
     const dim3 narrow((unsigned)((rowtiles + 3) / 4), (unsigned)items), wide((unsigned)((rowtiles + 7) / 8), (unsigned)items);
 #define MQ_GROUPED(KW, WT_, MT_, GRID)                                                                                             \
     MQ_LAUNCH((prefill_gemm_kernel<KW, WT_, false, MT_>), GRID, dim3(256), 2 * MT_ * kPTileBytes, stream, w, rowtiles, rows, nb, ap, \
               m_tiles, m_tiles * 16, y, ldy, (int)nb, (int64_t)0, plan, expert_bytes, out_row, w_shared, (const uint8_t*)nullptr,  \
               (const uint8_t*)nullptr, 0)
-    if (mt == kMTilesSmall) {  // one weight tile per wavefront: few registers, several workgroups to a compute unit
-        if (wtype == kTypeQ6K) MQ_GROUPED(1, kWtQ6, kMTilesSmall, narrow);
-        else if (wtype == kTypeQ5K) MQ_GROUPED(1, kWtQ5, kMTilesSmall, narrow);
-        else MQ_GROUPED(1, kWtQ4, kMTilesSmall, narrow);
-    } else if (mt == kMTilesMid) {
-        if (wtype == kTypeQ6K) MQ_GROUPED(1, kWtQ6, kMTilesMid, narrow);
-        else if (wtype == kTypeQ5K) MQ_GROUPED(1, kWtQ5, kMTilesMid, narrow);
-        else MQ_GROUPED(1, kWtQ4, kMTilesMid, narrow);
-    } else if (wtype == kTypeQ6K) {
-        MQ_GROUPED(1, kWtQ6, kMTilesPerGroup, narrow);
-    } else if (wtype == kTypeQ5K) {
-        MQ_GROUPED(1, kWtQ5, kMTilesPerGroup, narrow);
-    } else {
-        MQ_GROUPED(2, kWtQ4, kMTilesPerGroup, wide);
-    }
+    // two and four tiles: one weight tile per wavefront -- few registers, several workgroups to a compute unit
+#define MQ_GO(WT_)                                                    \
+    if (mt == kMTilesSmall) MQ_GROUPED(1, WT_, kMTilesSmall, narrow); \
+    else if (mt == kMTilesMid) MQ_GROUPED(1, WT_, kMTilesMid, narrow); \
+    else MQ_GROUPED(2, WT_, kMTilesPerGroup, wide)
+    MQ_BY_TYPE(wtype, MQ_GO);
+#undef MQ_GO
 #undef MQ_GROUPED
     return hipGetLastError();
 }
 
 // The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear), so it
-// applies where the two single launches would not split K either; Q4_K only (the other types' operand sets fill the
-// registers with one tile per wavefront).
+// applies where the two single launches would not split K either.
 bool prefill_pair_applies(int wtype, int64_t rows, int64_t nb, int64_t n) {
-    if (wtype != kTypeQ4K) return false;
+    if (!gemm_type(wtype)) return false;
     return prefill_shape(rows, nb, n, true).splits == 1;
 }
 
@@ -1272,16 +712,13 @@ hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int 
     if (!prefill_pair_applies(wtype, rows, nb, n)) return hipErrorInvalidValue;
     const PrefillShape ps = prefill_shape(rows, nb, n, true);
     if (ps.groups > 65535u) return hipErrorInvalidValue;
-    static bool raised = false;
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<2, kWtQ4, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
-    MQ_LAUNCH((prefill_gemm_kernel<2, kWtQ4, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream,
-              gate, rowtiles, rows, nb, ap, m_tiles, n, h, ldh, (int)nb, (int64_t)0, (const int32_t*)nullptr, (int64_t)0,
-              (const int32_t*)nullptr, (const uint8_t*)nullptr, up, (const uint8_t*)nullptr, silu_mode);
+    if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
+#define MQ_GO(WT_)                                                                                                                        \
+    MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, \
+              gate, rowtiles, rows, nb, ap, m_tiles, n, h, ldh, (int)nb, (int64_t)0, (const int32_t*)nullptr, (int64_t)0,               \
+              (const int32_t*)nullptr, (const uint8_t*)nullptr, up, (const uint8_t*)nullptr, silu_mode)
+    MQ_BY_TYPE(wtype, MQ_GO);
+#undef MQ_GO
     return hipGetLastError();
 }
 
@@ -1290,36 +727,29 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
                                             const uint8_t* gate_shared, const uint8_t* up_shared, int64_t rows, int64_t nb,
                                             const uint8_t* ap, int64_t entries, int64_t groups_max, const int32_t* plan, bool scatter,
                                             int silu_mode, float* h, int64_t ldh, hipStream_t stream, int mt) {
-    if (wtype != kTypeQ4K || (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup)) return hipErrorInvalidValue;
+    if (!gemm_type(wtype) || (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup)) return hipErrorInvalidValue;
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = moe_gemm_tiles_max(entries, groups_max);
     const int64_t items = moe_gemm_items_max(entries, groups_max);
     if (rowtiles == 0 || items == 0) return hipSuccess;
     if (items > 65535) return hipErrorInvalidValue;
-    static bool raised = false;
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<2, kWtQ4, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
     const int32_t* out_row = scatter ? plan + 4 + 3 * items + 16 * m_tiles : nullptr;
     const dim3 grid((unsigned)((rowtiles + 3) / 4), (unsigned)items);
-    if (mt == kMTilesSmall)
-        MQ_LAUNCH((prefill_gemm_kernel<2, kWtQ4, true, kMTilesSmall>), grid, dim3(256), 2 * kMTilesSmall * kPTileBytes, stream, gate, rowtiles,
-                  rows, nb, ap, m_tiles, m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared,
-                  silu_mode);
-    else if (mt == kMTilesMid)
-        MQ_LAUNCH((prefill_gemm_kernel<2, kWtQ4, true, kMTilesMid>), grid, dim3(256), 2 * kMTilesMid * kPTileBytes, stream, gate, rowtiles,
-                  rows, nb, ap, m_tiles, m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared,
-                  silu_mode);
-    else
-        MQ_LAUNCH((prefill_gemm_kernel<2, kWtQ4, true>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, gate, rowtiles, rows, nb,
-                  ap, m_tiles, m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared, silu_mode);
+#define MQ_GROUPED(WT_, MT_)                                                                                                                \
+    MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true, MT_>), grid, dim3(256), 2 * MT_ * kPTileBytes, stream, gate, rowtiles, rows, nb, ap, m_tiles, \
+              m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared, silu_mode)
+#define MQ_GO(WT_)                                           \
+    if (mt == kMTilesSmall) MQ_GROUPED(WT_, kMTilesSmall);   \
+    else if (mt == kMTilesMid) MQ_GROUPED(WT_, kMTilesMid);  \
+    else MQ_GROUPED(WT_, kMTilesPerGroup)
+    MQ_BY_TYPE(wtype, MQ_GO);
+#undef MQ_GO
+#undef MQ_GROUPED
     return hipGetLastError();
 }
 
-size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n, int wtype) {
-    const PrefillShape ps = prefill_shape(rows, nb, n, wtype != kTypeQ4K);
+size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n) {
+    const PrefillShape ps = prefill_shape(rows, nb, n);
     return ps.splits > 1 ? (size_t)ps.splits * (size_t)n * (size_t)rows * sizeof(float) : 0;
 }
 
@@ -1357,41 +787,25 @@ hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_
                                int64_t ldy, float* part, hipStream_t stream) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
     if (rowtiles == 0 || m_tiles == 0) return hipSuccess;
-    if (wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K) return hipErrorInvalidValue;
-    const PrefillShape ps = prefill_shape(rows, nb, n, wtype != kTypeQ4K);
+    if (!gemm_type(wtype)) return hipErrorInvalidValue;
+    const PrefillShape ps = prefill_shape(rows, nb, n);
     if (ps.groups > 65535u) return hipErrorInvalidValue;
     if (ps.splits > 1 && !part) return hipErrorInvalidValue;
-    static bool raised = false;  // two activation buffers: more than the default 64 KB of dynamic LDS
-    if (!raised) {
-        for (const void* k : {reinterpret_cast<const void*>(&prefill_gemm_kernel<1>), reinterpret_cast<const void*>(&prefill_gemm_kernel<2>),
-                              reinterpret_cast<const void*>(&prefill_gemm_kernel<1, kWtQ5>), reinterpret_cast<const void*>(&prefill_gemm_kernel<1, kWtQ6>)}) {
-            hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
-            if (e != hipSuccess) return e;
-        }
-        raised = true;
-    }
+    if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
     const bool split = ps.splits > 1;
     float* out = split ? part : y;
     const int64_t ld = split ? rows : ldy;
     const int64_t stride = split ? n * rows : 0;
     const dim3 grid(ps.row_wgs, ps.groups, (unsigned)ps.splits);
-    if (wtype == kTypeQ6K) {
-        MQ_LAUNCH((prefill_gemm_kernel<1, kWtQ6>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb,
-                           ap, m_tiles, n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr,
-                           (const uint8_t*)nullptr);
-    } else if (wtype == kTypeQ5K) {
-        MQ_LAUNCH((prefill_gemm_kernel<1, kWtQ5>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb,
-                           ap, m_tiles, n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr,
-                           (const uint8_t*)nullptr);
-    } else if (ps.narrow) {
-        MQ_LAUNCH(prefill_gemm_kernel<1>, grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb,
-                           ap, m_tiles, n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr,
-                           (const uint8_t*)nullptr);
-    } else {
-        MQ_LAUNCH(prefill_gemm_kernel<2>, grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb,
-                           ap, m_tiles, n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr,
-                           (const uint8_t*)nullptr);
-    }
+#define MQ_DENSE(KW, WT_)                                                                                                                 \
+    MQ_LAUNCH((prefill_gemm_kernel<KW, WT_>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb, ap, m_tiles, \
+              n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr, (const uint8_t*)nullptr)
+#define MQ_GO(WT_)                       \
+    if (ps.narrow) MQ_DENSE(1, WT_);     \
+    else MQ_DENSE(2, WT_)
+    MQ_BY_TYPE(wtype, MQ_GO);
+#undef MQ_GO
+#undef MQ_DENSE
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (split) {
         const int64_t units = n * (rows >> 2);
@@ -1399,149 +813,6 @@ hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_
                            rows, y, ldy);
     }
     return hipGetLastError();
-}
-
-// ---- skinny16 -------------------------------------------------------------------------------------------------
-namespace {
-
-constexpr size_t kSkinnyLdsMax = 160 * 1024;
-
-size_t skinny16_red_bytes(int nmat, int wpr, int mt) { return (size_t)(8 / wpr) * (wpr - 1) * nmat * mt * 4 * 64 * sizeof(float); }
-// LDS of the form with the rows' tiles in LDS, `ranges` runs of super-blocks one after the other: with one tile of
-// sixteen the partial sums lie behind the tiles, with more they share the tiles' bytes
-size_t skinny16_lds_bytes(int nmat, int wpr, int64_t nb, int mt, int ranges) {
-    const size_t tiles = (size_t)(nb / ranges) * mt * kPTileBytes, red = skinny16_red_bytes(nmat, wpr, mt);
-    return mt > 1 ? (tiles > red ? tiles : red) : tiles + red;
-}
-// Runs of super-blocks the rows' tiles need to pass through LDS (1, 2 or 4; every wavefront must have a whole number
-// of stages per run), or 0: they do not fit that way.
-int skinny16_ranges(int nmat, int wpr, int64_t nb, int mt) {
-    for (int ranges = 1; ranges <= 4; ranges *= 2) {
-        if (ranges > 1 && (mt == 1 || nb % ((int64_t)wpr * ranges))) break;
-        if (skinny16_lds_bytes(nmat, wpr, nb, mt, ranges) <= kSkinnyLdsMax) return ranges;
-    }
-    return 0;
-}
-
-template <int NMAT, int WPR, int FLOW, bool GA, int MT, int WT>
-hipError_t launch_skinny16_one(const Skinny16Args& a, int ranges, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    const int64_t rowtiles = (a.rows + 15) / 16;
-    const size_t lds = GA ? skinny16_red_bytes(NMAT, WPR, MT) : skinny16_lds_bytes(NMAT, WPR, a.nb, MT, ranges);
-    auto* kernel = &skinny16_kernel<NMAT, WPR, FLOW, GA, MT, WT>;
-    static bool raised = false;  // per instantiation; the attribute belongs to the function, not to a launch
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSkinnyLdsMax);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
-    Skinny16Args b = a;
-    b.ranges = GA ? 1 : ranges;
-    constexpr int RPW = 8 / WPR;
-    const dim3 grid((unsigned)((rowtiles + RPW - 1) / RPW));
-    if (start && stop) hipExtLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, start, stop, 0, b);
-    else MQ_LAUNCH(kernel, grid, dim3(512), lds, stream, b);
-    return hipGetLastError();
-}
-
-// MT <= 2: the rows' tiles in LDS (in runs if need be), else from global memory a stage ahead; three and four tiles only
-// from LDS (read a stage ahead they do not fit the registers), an even number of stages per wavefront.
-template <int NMAT, int WPR, int MT, int WT>
-hipError_t launch_skinny16_form(const Skinny16Args& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    const bool odd = ((a.nb / WPR) & 1) != 0;
-    const int ranges = odd ? (skinny16_lds_bytes(NMAT, WPR, a.nb, MT, 1) <= kSkinnyLdsMax ? 1 : 0) : skinny16_ranges(NMAT, WPR, a.nb, MT);
-    // (the forms left out below spill registers -- skinny16_applies knows them)
-    if constexpr (WT == kWtQ6 && NMAT == 2 && WPR == 1) {
-        return hipErrorInvalidValue;
-    } else if constexpr (MT <= 2) {
-        const bool ga = ranges != 1;  // (two tiles could also come in runs; read a stage ahead they cost no barrier)
-        if constexpr (WT != kWtQ4 && NMAT == 2 && MT == 2) {  // two tiles of a Q5_K or Q6_K pair: not read a stage ahead
-            if (ga) return hipErrorInvalidValue;
-            if (odd) return launch_skinny16_one<NMAT, WPR, 1, false, MT, WT>(a, 1, stream, start, stop);
-            return launch_skinny16_one<NMAT, WPR, 0, false, MT, WT>(a, 1, stream, start, stop);
-        } else {
-            if (odd) return ga ? launch_skinny16_one<NMAT, WPR, 1, true, MT, WT>(a, 1, stream, start, stop) : launch_skinny16_one<NMAT, WPR, 1, false, MT, WT>(a, 1, stream, start, stop);
-            return ga ? launch_skinny16_one<NMAT, WPR, 0, true, MT, WT>(a, 1, stream, start, stop) : launch_skinny16_one<NMAT, WPR, 0, false, MT, WT>(a, 1, stream, start, stop);
-        }
-    } else if constexpr (WPR == 1 || (NMAT == 2 && MT == 4 && WPR == 8)) {
-        return hipErrorInvalidValue;
-    } else {
-        if (ranges == 0) return hipErrorInvalidValue;
-        if (odd) return launch_skinny16_one<NMAT, WPR, 1, false, MT, WT>(a, 1, stream, start, stop);  // (an odd stage count: one run only)
-        if ((((a.nb / WPR) / ranges) & 1) == 0) return launch_skinny16_one<NMAT, WPR, 0, false, MT, WT>(a, ranges, stream, start, stop);
-        if constexpr (WT == kWtQ6 || (WT == kWtQ5 && NMAT == 2 && MT == 4)) return hipErrorInvalidValue;  // (runs of an odd stage count)
-        else return launch_skinny16_one<NMAT, WPR, 2, false, MT, WT>(a, ranges, stream, start, stop);
-    }
-}
-
-template <int NMAT, int MT, int WT>
-hipError_t launch_skinny16_wpr(const Skinny16Args& a, int wpr, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    switch (wpr) {
-        case 1: return launch_skinny16_form<NMAT, 1, MT, WT>(a, stream, start, stop);
-        case 2: return launch_skinny16_form<NMAT, 2, MT, WT>(a, stream, start, stop);
-        case 4: return launch_skinny16_form<NMAT, 4, MT, WT>(a, stream, start, stop);
-        case 8: return launch_skinny16_form<NMAT, 8, MT, WT>(a, stream, start, stop);
-    }
-    return hipErrorInvalidValue;
-}
-
-template <int NMAT>
-hipError_t launch_skinny16_tiles(const Skinny16Args& a, int wpr, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    const int mt = (int)((a.n + 15) / 16);
-    if (a.wtype == kTypeQ5K) {
-        if (mt == 1) return launch_skinny16_wpr<NMAT, 1, kWtQ5>(a, wpr, stream, start, stop);
-        if (mt == 2) return launch_skinny16_wpr<NMAT, 2, kWtQ5>(a, wpr, stream, start, stop);
-        if (mt == 3) return launch_skinny16_wpr<NMAT, 3, kWtQ5>(a, wpr, stream, start, stop);
-        if (mt == 4) return launch_skinny16_wpr<NMAT, 4, kWtQ5>(a, wpr, stream, start, stop);
-        return hipErrorInvalidValue;
-    }
-    if (a.wtype == kTypeQ6K) {
-        if (mt == 1) return launch_skinny16_wpr<NMAT, 1, kWtQ6>(a, wpr, stream, start, stop);
-        if (mt == 2) return launch_skinny16_wpr<NMAT, 2, kWtQ6>(a, wpr, stream, start, stop);
-        if (mt == 3) return launch_skinny16_wpr<NMAT, 3, kWtQ6>(a, wpr, stream, start, stop);
-        if (mt == 4) return launch_skinny16_wpr<NMAT, 4, kWtQ6>(a, wpr, stream, start, stop);
-        return hipErrorInvalidValue;
-    }
-    switch (mt) {
-        case 1: return launch_skinny16_wpr<NMAT, 1, kWtQ4>(a, wpr, stream, start, stop);
-        case 2: return launch_skinny16_wpr<NMAT, 2, kWtQ4>(a, wpr, stream, start, stop);
-        case 3: return launch_skinny16_wpr<NMAT, 3, kWtQ4>(a, wpr, stream, start, stop);
-        case 4: return launch_skinny16_wpr<NMAT, 4, kWtQ4>(a, wpr, stream, start, stop);
-    }
-    return hipErrorInvalidValue;
-}
-
-}  // namespace
-
-// Whether a product of n rows (nine to 64) runs on skinny16_kernel: the wave split of the other decode kernels must be
-// one of its own (a divisor of eight that divides the super-blocks of a row), and the form must be built
-// (launch_skinny16_form returns an error for the others: those whose registers spill).
-//   One and two tiles (up to 32 rows): always; the two tiles of a Q5_K or Q6_K gate/up pair only where they fit LDS in
-//   one run; a Q6_K pair not with one wavefront per row tile.
-//   Three and four tiles: not with one wavefront per row tile (more than 1,024 row tiles: the GEMM is faster from 33
-//   rows -- 128256 x 4096 at 33 / 64 rows: 93 / 108 us against 102 / 126); the tiles must pass through LDS in at most four
-//   runs of whole stages (in one run where a wavefront's stage count is odd); a pair of four tiles not with eight
-//   wavefronts per row tile; in runs of an odd number of stages no Q6_K form and no Q5_K pair of four tiles.
-bool skinny16_applies(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n, int wtype) {
-    const int wpr = dense_lds_wpr(nb, rowtiles);
-    if (!wpr || nb % wpr || n < 1 || n > 64 || (wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K)) return false;
-    const int nmat = swiglu ? 2 : 1, mt = (int)((n + 15) / 16);
-    if (wtype == kTypeQ6K && swiglu && wpr == 1) return false;
-    if (mt <= 2) return !(wtype != kTypeQ4K && swiglu && mt == 2) || skinny16_lds_bytes(2, wpr, nb, 2, 1) <= kSkinnyLdsMax;
-    if (wpr == 1 || (swiglu && mt == 4 && wpr == 8)) return false;
-    if ((nb / wpr) & 1) return skinny16_lds_bytes(nmat, wpr, nb, mt, 1) <= kSkinnyLdsMax;  // an odd stage count: the tiles in one run
-    const int ranges = skinny16_ranges(nmat, wpr, nb, mt);
-    if (!ranges) return false;
-    const bool odd_runs = (((nb / wpr) / ranges) & 1) != 0;
-    return !odd_runs || !(wtype == kTypeQ6K || (wtype == kTypeQ5K && swiglu && mt == 4));
-}
-
-hipError_t launch_skinny16(const Skinny16Args& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    if (a.rows <= 0 || a.nb <= 0 || a.n < 1 || a.n > 64 || !a.y || !a.w0 || !a.ap) return hipErrorInvalidValue;
-    const int64_t rowtiles = (a.rows + 15) / 16;
-    if (!skinny16_applies(a.nb, rowtiles, a.w1 != nullptr, a.n, a.wtype)) return hipErrorInvalidValue;
-    const int wpr = dense_lds_wpr(a.nb, rowtiles);
-    if (a.w1) return launch_skinny16_tiles<2>(a, wpr, stream, start, stop);
-    return launch_skinny16_tiles<1>(a, wpr, stream, start, stop);
 }
 
 }  // namespace mq
