@@ -90,7 +90,8 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                                                            int64_t expert_bytes, const int32_t* __restrict__ out_rows,
                                                            const uint8_t* __restrict__ w_shared,
                                                            const uint8_t* __restrict__ w2 = nullptr,
-                                                           const uint8_t* __restrict__ w2_shared = nullptr, int silu_mode = 0) {
+                                                           const uint8_t* __restrict__ w2_shared = nullptr, int silu_mode = 0,
+                                                           int tiles_per_wg = MT) {
     static_assert(!PAIR || kWTilesPerWave == 2, "the pair form is the two-tile kernel");
     extern __shared__ __align__(16) uint8_t a_lds[];  // two buffers of MT * kPTileBytes bytes
     constexpr int kBufBytes = MT * kPTileBytes;
@@ -99,10 +100,10 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
-    // Dense: workgroup column blockIdx.y takes the activation tiles 8 y .. 8 y + 7.  Expert-grouped (plan != null): it
-    // takes item blockIdx.y of the plan -- an expert's weights and a run of up to eight tiles of that expert's rows.
-    int64_t mt0 = (int64_t)blockIdx.y * MT;
-    int mt_count = (int)(m_tiles - mt0 < MT ? m_tiles - mt0 : MT);
+    // Dense: workgroup column blockIdx.y takes the next tiles_per_wg (<= MT) activation tiles.  Expert-grouped (plan != null):
+    // it takes item blockIdx.y of the plan -- an expert's weights and a run of up to eight tiles of that expert's rows.
+    int64_t mt0 = (int64_t)blockIdx.y * tiles_per_wg;
+    int mt_count = (int)(m_tiles - mt0 < tiles_per_wg ? m_tiles - mt0 : tiles_per_wg);
     if (plan) {
         const int item = blockIdx.y;
         if (item >= plan[0]) return;  // the whole workgroup, before any barrier
@@ -454,32 +455,54 @@ __global__ void __launch_bounds__(256) prefill_sum_planes_kernel(const float* __
     dst[0] = acc.x, dst[1] = acc.y, dst[2] = acc.z, dst[3] = acc.w;
 }
 
-// Workgroup shape and K split of a launch: 64-row workgroups while the 128-row ones would not give every compute
-// unit one; K in `splits` runs of super-blocks while the launch would still leave workgroup slots empty (a
-// workgroup walks its super-blocks one after the other, 2.2 us each: 4096 rows x 14336 columns at M = 128 are 64
-// workgroups of 56 super-blocks, 115 us; in eight runs 37 us with the launch that adds the planes; at M = 256
-// 119 -> 56 us in four runs, at M = 512 128 -> 100 us in two; 14336 x 4096 at M = 128: 40 -> 35 us in two).
+// Shape of a launch: 128- or 64-row workgroups, the activation tiles dealt evenly over `groups` workgroup columns of
+// tiles_per_wg <= 8, K in `splits` runs of super-blocks (planes of partial sums that a second launch adds in order).  A compute
+// unit holds two workgroups, and a workgroup walks its super-blocks one after the other, so what counts is the length of a
+// workgroup times the rounds of 2 x compute_units() of them.  Time of a workgroup and super-block, us, by its tiles t, measured
+// over 4096 x 14336, 14336 x 4096, 6144 x 4096 at 50 to 2048 rows (two workgroups on a unit | one alone):
+//     128 rows  0.4 + 0.52 t | 0.6 + 0.27 t        64 rows  0.35 + 0.28 t | 0.55 + 0.16 t
+// (and no less than the streaming of the weights: 2.0 and 1.1 us with two workgroups on every unit).
+// The shape with the smallest estimate is taken.  Against the fixed order it replaces (64-row workgroups up to one per compute
+// unit, tiles in eights, K split only to fill the slots), with its quantizer and planes: 4096 x 14336 at 130 / 391 / 700 / 1200 rows
+// 46 / 84 / 145 / 245 -> 37 / 75 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 70 / 109, 2048 x 2048 at 777
+// 27.6 -> 23.8.
 struct PrefillShape {
-    bool narrow;
-    int splits, sb_split;
-    unsigned row_wgs, groups;
+    bool narrow = false;
+    int splits = 1, sb_split = 1, tiles_per_wg = 1;
+    unsigned row_wgs = 1, groups = 1;
+    float us = 1e30f;  // the estimate
 };
-PrefillShape prefill_shape(int64_t rows, int64_t nb, int64_t n, bool one_tile_per_wave = false) {
+// PAIR form: a row tile of both matrices per wavefront (the 128-row body), no K split (SiLU is not linear); one workgroup alone
+// 0.9 + 0.32 t.  From 25 activation tiles on it keeps them in eights with the short column last, whose workgroups fill the last
+// round (14336 x 4096, tiles to a workgroup 8 / 7 / 5: 122 / 121 / 132 us at 391 rows, 310 / 320 / 359 at 1200).
+PrefillShape prefill_shape(int64_t rows, int64_t nb, int64_t n, bool pair = false) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
-    PrefillShape ps;
-    ps.groups = (unsigned)((m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup);
-    // two workgroups fit a compute unit: while the 128-row workgroups would not even give every unit one, 64-row
-    // ones fill the chip better (14336 rows on 256 units: up to M = 256; 52 -> 40 us at M = 128, 55 -> 51 at 256,
-    // and 76 -> 79, 78 -> 91 at M = 384, 512, where the wide ones stay)
-    ps.narrow = one_tile_per_wave || ((rowtiles + 7) / 8) * (int64_t)ps.groups <= (int64_t)compute_units();  // (the pair form: a wavefront's two tiles are one row tile of two matrices)
-    ps.row_wgs = (unsigned)(ps.narrow ? (rowtiles + 3) / 4 : (rowtiles + 7) / 8);
-    const int64_t wgs = (int64_t)ps.row_wgs * ps.groups;
-    int splits = (int)(2 * (int64_t)compute_units() / (wgs > 0 ? wgs : 1));
-    if (splits > nb / 4) splits = (int)(nb / 4);  // at least four super-blocks per run
-    if (splits < 1 || (rows & 3)) splits = 1;
-    ps.sb_split = (int)((nb + splits - 1) / splits);
-    ps.splits = (int)((nb + ps.sb_split - 1) / ps.sb_split);  // every run holds a super-block
-    return ps;
+    const int64_t units = compute_units();
+    const int64_t min_groups = (m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup, max_groups = pair && m_tiles >= 25 ? min_groups : min_groups + 4;
+    const int max_splits = pair || (rows & 3) ? 1 : (int)(nb / 4 < 16 ? nb / 4 : 16);  // at least four super-blocks per run
+    PrefillShape best;
+    for (int narrow = 0; narrow < (pair ? 1 : 2); ++narrow) {
+        const int64_t row_wgs = (pair || narrow) ? (rowtiles + 3) / 4 : (rowtiles + 7) / 8;
+        for (int64_t want = min_groups; want <= max_groups; ++want) {
+            const int64_t t = pair && m_tiles >= 25 ? kMTilesPerGroup : (m_tiles + want - 1) / want, groups = (m_tiles + t - 1) / t;
+            float two = narrow ? 0.35f + 0.28f * t : 0.4f + 0.52f * t;
+            const float one = pair ? 0.9f + 0.32f * t : narrow ? 0.55f + 0.16f * t : 0.6f + 0.27f * t, stream = narrow ? 1.1f : 2.0f;
+            if (two < stream) two = stream;
+            for (int sp = 1; sp == 1 || sp <= max_splits; ++sp) {
+                const int64_t sb = (nb + sp - 1) / sp, splits = (nb + sb - 1) / sb;  // every run holds a super-block
+                if (splits != sp) continue;
+                const int64_t wgs = row_wgs * groups * splits, rest = wgs % (2 * units);
+                float us = (float)sb * ((float)(wgs / (2 * units)) * two + (rest == 0 ? 0.0f : rest <= units ? one : two));
+                if (splits > 1) us += 3.0f + (float)(2 * splits) * (float)(n * rows) * (4.0f / 8e6f);  // planes: a launch, written and read
+                if (us < best.us) {
+                    best.narrow = narrow != 0, best.splits = (int)splits, best.sb_split = (int)sb, best.tiles_per_wg = (int)t;
+                    best.row_wgs = (unsigned)row_wgs, best.groups = (unsigned)groups, best.us = us;
+                }
+                if (wgs > 4 * units) break;  // already two rounds and more: further runs only add planes
+            }
+        }
+    }
+    return best;
 }
 
 // ---- expert-grouped GEMM: the plan ------------------------------------------------------------------------
@@ -686,7 +709,7 @@ hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expe
 #define MQ_GROUPED(KW, WT_, MT_, GRID)                                                                                             \
     MQ_LAUNCH((prefill_gemm_kernel<KW, WT_, false, MT_>), GRID, dim3(256), 2 * MT_ * kPTileBytes, stream, w, rowtiles, rows, nb, ap, \
               m_tiles, m_tiles * 16, y, ldy, (int)nb, (int64_t)0, plan, expert_bytes, out_row, w_shared, (const uint8_t*)nullptr,  \
-              (const uint8_t*)nullptr, 0)
+              (const uint8_t*)nullptr, 0, MT_)
     // two and four tiles: one weight tile per wavefront -- few registers, several workgroups to a compute unit
 #define MQ_GO(WT_)                                                    \
     if (mt == kMTilesSmall) MQ_GROUPED(1, WT_, kMTilesSmall, narrow); \
@@ -698,11 +721,11 @@ hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expe
     return hipGetLastError();
 }
 
-// The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear), so it
-// applies where the two single launches would not split K either.
+// The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear): where the
+// launch is small enough for that to matter, two launches with K in runs and the SwiGLU pass over their planes are faster.
 bool prefill_pair_applies(int wtype, int64_t rows, int64_t nb, int64_t n) {
     if (!gemm_type(wtype)) return false;
-    return prefill_shape(rows, nb, n, true).splits == 1;
+    return prefill_shape(rows, nb, n, true).us <= 2.0f * prefill_shape(rows, nb, n).us + 3.0f + (float)(n * rows) * (12.0f / 4e6f);
 }
 
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,
@@ -716,7 +739,7 @@ hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int 
 #define MQ_GO(WT_)                                                                                                                        \
     MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, \
               gate, rowtiles, rows, nb, ap, m_tiles, n, h, ldh, (int)nb, (int64_t)0, (const int32_t*)nullptr, (int64_t)0,               \
-              (const int32_t*)nullptr, (const uint8_t*)nullptr, up, (const uint8_t*)nullptr, silu_mode)
+              (const int32_t*)nullptr, (const uint8_t*)nullptr, up, (const uint8_t*)nullptr, silu_mode, ps.tiles_per_wg)
     MQ_BY_TYPE(wtype, MQ_GO);
 #undef MQ_GO
     return hipGetLastError();
@@ -737,7 +760,7 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
     const dim3 grid((unsigned)((rowtiles + 3) / 4), (unsigned)items);
 #define MQ_GROUPED(WT_, MT_)                                                                                                                \
     MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true, MT_>), grid, dim3(256), 2 * MT_ * kPTileBytes, stream, gate, rowtiles, rows, nb, ap, m_tiles, \
-              m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared, silu_mode)
+              m_tiles * 16, h, ldh, (int)nb, (int64_t)0, plan, expert_bytes, out_row, gate_shared, up, up_shared, silu_mode, MT_)
 #define MQ_GO(WT_)                                           \
     if (mt == kMTilesSmall) MQ_GROUPED(WT_, kMTilesSmall);   \
     else if (mt == kMTilesMid) MQ_GROUPED(WT_, kMTilesMid);  \
@@ -799,7 +822,8 @@ hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_
     const dim3 grid(ps.row_wgs, ps.groups, (unsigned)ps.splits);
 #define MQ_DENSE(KW, WT_)                                                                                                                 \
     MQ_LAUNCH((prefill_gemm_kernel<KW, WT_>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb, ap, m_tiles, \
-              n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr, (const uint8_t*)nullptr)
+              n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr, (const uint8_t*)nullptr, \
+              (const uint8_t*)nullptr, (const uint8_t*)nullptr, 0, ps.tiles_per_wg)
 #define MQ_GO(WT_)                       \
     if (ps.narrow) MQ_DENSE(1, WT_);     \
     else MQ_DENSE(2, WT_)
