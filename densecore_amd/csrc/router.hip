@@ -122,41 +122,10 @@ __global__ void __launch_bounds__(64) weights_from_ids_kernel(const float* __res
     for (int k = 0; k < top_k; ++k) weights[(size_t)tok * top_k + k] = __fdiv_rn(l[k], den);
 }
 
-// Counting sort of the (token, k) pairs by expert, by one workgroup.  Pairs keep their natural
-// (token, k) order inside an expert, which is the (expert, token, k) order of
-// core/src/llm/moe/native.cpp:1726-1730.  Experts nobody selected produce no group.
-// ids may live in LDS or in global memory; count[] is n_experts ints of LDS.
-// token_mask (LDS, n_experts * (mask_words | 1) + 1 words, or null): one bit per (expert, token).  A pair's place inside
-// its group is the number of earlier pairs of the same expert; when no token names an expert twice (always so for
-// routed ids) that is the number of earlier tokens whose bit is set -- a population count instead of a scan over
-// all earlier pairs.  A repeated (expert, token) raises the word after the masks and the scan is used.
-__device__ __forceinline__ void group_entries(const int32_t* ids, int n_entries, int top_k, int n_experts,
-                                              int32_t* count, int32_t* __restrict__ group_expert,
-                                              int32_t* __restrict__ group_begin, int32_t* __restrict__ n_groups,
-                                              int32_t* __restrict__ entry_token, int32_t* __restrict__ entry_k,
-                                              uint32_t* token_mask = nullptr, int mask_words = 0, int part = 0, int parts = 1,
-                                              uint16_t* mask_prefix = nullptr) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    // an expert's mask words are an odd number of words apart: the lanes of a wavefront (consecutive pairs, different
-    // experts) walk their experts' words side by side, and an even stride puts them all on one LDS bank (225 us
-    // against 20 for the grouping of 2048 tokens)
-    const int mask_stride = mask_words | 1;
-    for (int e = tid; e < n_experts; e += nt) count[e] = 0;
-    if (token_mask)
-        for (int w = tid; w <= n_experts * mask_stride; w += nt) token_mask[w] = 0u;
-    __syncthreads();
-    for (int i = tid; i < n_entries; i += nt) {
-        const int e = ids[i];
-        if (e >= 0 && e < n_experts) {
-            atomicAdd(&count[e], 1);
-            if (token_mask) {
-                const int t = i / top_k;
-                const uint32_t bit = 1u << (t & 31);
-                if (atomicOr(&token_mask[e * mask_stride + (t >> 5)], bit) & bit) token_mask[n_experts * mask_stride] = 1u;
-            }
-        }
-    }
-    __syncthreads();
+// count[] (pairs per expert) -> each expert's first entry; part 0 writes the group lists.  Barriers are the caller's.
+__device__ __forceinline__ void scan_groups(int32_t* count, int n_experts, int part, int32_t* __restrict__ group_expert,
+                                            int32_t* __restrict__ group_begin, int32_t* __restrict__ n_groups) {
+    const int tid = threadIdx.x;
     if (tid < 64) {  // wave 0: exclusive scan over the experts, lane l covers a run of consecutive experts
         const int per = (n_experts + 63) / 64;
         const int e0 = tid * per;
@@ -201,23 +170,45 @@ __device__ __forceinline__ void group_entries(const int32_t* ids, int n_entries,
             *n_groups = groups;
         }
     }
+}
+
+// Counting sort of the (token, k) pairs by expert, by one workgroup.  Pairs keep their natural
+// (token, k) order inside an expert, which is the (expert, token, k) order of
+// core/src/llm/moe/native.cpp:1726-1730.  Experts nobody selected produce no group.
+// ids may live in LDS or in global memory; count[] is n_experts ints of LDS.
+// token_mask (LDS, n_experts * (mask_words | 1) + 1 words, or null): one bit per (expert, token).  A pair's place inside
+// its group is the number of earlier pairs of the same expert; when no token names an expert twice (always so for
+// routed ids) that is the number of earlier tokens whose bit is set -- a population count instead of a scan over
+// all earlier pairs.  A repeated (expert, token) raises the word after the masks and the scan is used.
+__device__ __forceinline__ void group_entries(const int32_t* ids, int n_entries, int top_k, int n_experts,
+                                              int32_t* count, int32_t* __restrict__ group_expert,
+                                              int32_t* __restrict__ group_begin, int32_t* __restrict__ n_groups,
+                                              int32_t* __restrict__ entry_token, int32_t* __restrict__ entry_k,
+                                              uint32_t* token_mask = nullptr, int mask_words = 0, int part = 0, int parts = 1) {
+    const int tid = threadIdx.x, nt = blockDim.x;
+    // an expert's mask words are an odd number of words apart: the lanes of a wavefront (consecutive pairs, different
+    // experts) walk their experts' words side by side, and an even stride puts them all on one LDS bank (225 us
+    // against 20 for the grouping of 2048 tokens)
+    const int mask_stride = mask_words | 1;
+    for (int e = tid; e < n_experts; e += nt) count[e] = 0;
+    if (token_mask)
+        for (int w = tid; w <= n_experts * mask_stride; w += nt) token_mask[w] = 0u;
     __syncthreads();
-    const bool by_mask = token_mask && token_mask[n_experts * mask_stride] == 0u;
-    // mask_prefix (LDS, n_experts * mask_stride 16-bit words, or null; at most 65535 tokens): the number of set bits in an
-    // expert's mask words before word w, so that a pair's place costs one look-up and one population count instead of a
-    // walk over all the expert's earlier words (half of them on average: at 2048 tokens 32 LDS reads per pair)
-    if (by_mask && mask_prefix) {
-        for (int e = tid; e < n_experts; e += nt) {
-            const uint32_t* m = token_mask + e * mask_stride;
-            uint16_t* pre = mask_prefix + e * mask_stride;
-            int run = 0;
-            for (int w = 0; w < mask_words; ++w) {
-                pre[w] = (uint16_t)run;
-                run += __popc(m[w]);
+    for (int i = tid; i < n_entries; i += nt) {
+        const int e = ids[i];
+        if (e >= 0 && e < n_experts) {
+            atomicAdd(&count[e], 1);
+            if (token_mask) {
+                const int t = i / top_k;
+                const uint32_t bit = 1u << (t & 31);
+                if (atomicOr(&token_mask[e * mask_stride + (t >> 5)], bit) & bit) token_mask[n_experts * mask_stride] = 1u;
             }
         }
-        __syncthreads();
     }
+    __syncthreads();
+    scan_groups(count, n_experts, part, group_expert, group_begin, n_groups);
+    __syncthreads();
+    const bool by_mask = token_mask && token_mask[n_experts * mask_stride] == 0u;
     // several workgroups (parts > 1) all build the counts and masks, each places its share of the pairs
     for (int i = part * nt + tid; i < n_entries; i += parts * nt) {
         const int e = ids[i];
@@ -227,9 +218,7 @@ __device__ __forceinline__ void group_entries(const int32_t* ids, int n_entries,
         if (by_mask) {
             const int t = i / top_k;
             const uint32_t* m = token_mask + e * mask_stride;
-            if (mask_prefix) rank = mask_prefix[e * mask_stride + (t >> 5)];
-            else
-                for (int w = 0; w < (t >> 5); ++w) rank += __popc(m[w]);
+            for (int w = 0; w < (t >> 5); ++w) rank += __popc(m[w]);
             rank += __popc(m[t >> 5] & ((1u << (t & 31)) - 1u));
             j = i;  // nothing left to scan
         }
@@ -247,6 +236,83 @@ __device__ __forceinline__ void group_entries(const int32_t* ids, int n_entries,
     }
 }
 
+// The same sort for prefill widths, by `parts` workgroups of 1024 threads that each build the masks and place their share of the
+// pairs.  Bound by its serial steps -- a read of the ids, one LDS atomic per pair, the scan, the placing --, so those are what it is
+// made of: the ids of eight rounds are requested together while the masks are cleared, the counts come out of the masks
+// (no counter per pair), and four lanes share an expert's words.  mask_prefix (n_experts * (mask_words | 1) 16-bit words;
+// at most 65535 tokens): the set bits in an expert's words before word w, which makes a pair's place one look-up and one population
+// count.  False, and nothing placed, if a token names an expert twice.  256 experts, 5600 / 12000 pairs: 8.3 / 13.7 -> 7.0 / 10.7 us
+// against a counter and an id read per pair and round, and a lane per expert's words.
+__device__ __forceinline__ bool group_entries_masked(const int32_t* __restrict__ ids, int32_t* ids_s, int n_entries, int top_k,
+                                                     int n_experts, int32_t* count, int32_t* __restrict__ group_expert,
+                                                     int32_t* __restrict__ group_begin, int32_t* __restrict__ n_groups,
+                                                     int32_t* __restrict__ entry_token, int32_t* __restrict__ entry_k,
+                                                     uint32_t* token_mask, int mask_words, int part, int parts, uint16_t* mask_prefix) {
+    constexpr int kRounds = 8;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int mask_stride = mask_words | 1;
+    int v[kRounds];
+    auto request = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int i = base + u * nt + tid;
+            v[u] = ids[i < n_entries ? i : n_entries - 1];
+        }
+    };
+    request(0);
+    for (int w = tid; w <= n_experts * mask_stride; w += nt) token_mask[w] = 0u;
+    __syncthreads();
+    for (int base = 0; base < n_entries; base += kRounds * nt) {
+        if (base > 0) request(base);
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int i = base + u * nt + tid, e = v[u];
+            if (i >= n_entries) continue;
+            if (ids_s) ids_s[i] = e;
+            if (e >= 0 && e < n_experts) {
+                const uint32_t t = (uint32_t)i / (uint32_t)top_k, bit = 1u << (t & 31);
+                if (atomicOr(&token_mask[e * mask_stride + (int)(t >> 5)], bit) & bit) token_mask[n_experts * mask_stride] = 1u;
+            }
+        }
+    }
+    __syncthreads();
+    if (token_mask[n_experts * mask_stride] != 0u) return false;  // the whole workgroup
+    const int per = (mask_words + 3) >> 2;  // words per lane
+    for (int e = tid >> 2; e < n_experts; e += nt >> 2) {
+        const uint32_t* m = token_mask + e * mask_stride;
+        uint16_t* pre = mask_prefix + e * mask_stride;
+        const int w0 = (tid & 3) * per, w1 = w0 + per < mask_words ? w0 + per : mask_words;
+        int own = 0;
+        for (int w = w0; w < w1; ++w) own += __popc(m[w]);
+        int run = own;  // inclusive over the expert's four lanes
+#pragma unroll
+        for (int d = 1; d < 4; d <<= 1) {
+            const int o = __shfl_up(run, d, 4);
+            if ((tid & 3) >= d) run += o;
+        }
+        if ((tid & 3) == 3) count[e] = run;
+        run -= own;
+        for (int w = w0; w < w1; ++w) {
+            pre[w] = (uint16_t)run;
+            run += __popc(m[w]);
+        }
+    }
+    __syncthreads();
+    scan_groups(count, n_experts, part, group_expert, group_begin, n_groups);
+    __syncthreads();
+    const int32_t* src = ids_s ? ids_s : ids;
+    for (int i = part * nt + tid; i < n_entries; i += parts * nt) {
+        const int e = src[i];
+        if (e < 0 || e >= n_experts) continue;
+        const uint32_t t = (uint32_t)i / (uint32_t)top_k;
+        const int at = e * mask_stride + (int)(t >> 5);
+        const int pos = count[e] + mask_prefix[at] + __popc(token_mask[at] & ((1u << (t & 31)) - 1u));
+        entry_token[pos] = (int)t;
+        entry_k[pos] = i - (int)t * top_k;
+    }
+    return true;
+}
+
 __global__ void __launch_bounds__(1024) build_groups_kernel(const int32_t* __restrict__ ids, int n_entries,
                                                             int top_k, int n_experts, int use_lds, int mask_words, int with_prefix,
                                                             int32_t* __restrict__ group_expert,
@@ -257,15 +323,22 @@ __global__ void __launch_bounds__(1024) build_groups_kernel(const int32_t* __res
     extern __shared__ int32_t sh[];  // [n_experts] counts -> offsets, [n_entries] ids when they fit, then the token masks
     int32_t* count = sh;
     const int32_t* src = ids;
-    if (use_lds) {
-        int32_t* ids_s = sh + n_experts;
+    int32_t* ids_s = use_lds ? sh + n_experts : nullptr;
+    uint32_t* masks = mask_words ? reinterpret_cast<uint32_t*>(sh + n_experts + (use_lds ? n_entries : 0)) : nullptr;
+    if (with_prefix) {
+        uint16_t* prefix = reinterpret_cast<uint16_t*>(masks + n_experts * (mask_words | 1) + 1);
+        if (group_entries_masked(ids, ids_s, n_entries, top_k, n_experts, count, group_expert, group_begin, n_groups, entry_token, entry_k,
+                                 masks, mask_words, (int)blockIdx.x, (int)gridDim.x, prefix))
+            return;
+        __syncthreads();
+        masks = nullptr;  // a repeated (token, expert): by scanning
+        if (use_lds) src = ids_s;
+    } else if (use_lds) {
         for (int i = threadIdx.x; i < n_entries; i += blockDim.x) ids_s[i] = ids[i];
         src = ids_s;  // the barrier inside group_entries orders these stores
     }
-    uint32_t* masks = mask_words ? reinterpret_cast<uint32_t*>(sh + n_experts + (use_lds ? n_entries : 0)) : nullptr;
-    uint16_t* prefix = with_prefix ? reinterpret_cast<uint16_t*>(masks + n_experts * (mask_words | 1) + 1) : nullptr;
     group_entries(src, n_entries, top_k, n_experts, count, group_expert, group_begin, n_groups, entry_token, entry_k, masks, mask_words,
-                  (int)blockIdx.x, (int)gridDim.x, prefix);
+                  (int)blockIdx.x, (int)gridDim.x);
 }
 
 // Router and grouping in one launch (decode widths): a workgroup per token routes it; the last
@@ -521,9 +594,9 @@ hipError_t launch_build_groups(const int32_t* ids, int64_t n, int top_k, int64_t
     int mask_words = n <= 4096 ? (int)((n + 31) / 32) : 0;
     if (lds + ((size_t)n_experts * (mask_words | 1) + 1) * 4 > 150 * 1024) mask_words = 0;
     if (mask_words) lds += ((size_t)n_experts * (mask_words | 1) + 1) * 4;
-    // from 512 tokens the prefix counts of the masks join them (where they fit), ahead of the ids
+    // the prefix counts of the masks join them (where they fit), ahead of the ids
     const size_t prefix_bytes = ((size_t)n_experts * (mask_words | 1) * 2 + 3) & ~(size_t)3;
-    const int with_prefix = mask_words >= 16 && lds + prefix_bytes <= 150 * 1024;
+    const int with_prefix = mask_words > 0 && lds + prefix_bytes <= 150 * 1024;
     if (with_prefix) lds += prefix_bytes;
     const int use_lds = lds + (size_t)entries * 4 <= 150 * 1024;
     if (use_lds) lds += (size_t)entries * 4;
@@ -536,9 +609,9 @@ hipError_t launch_build_groups(const int32_t* ids, int64_t n, int top_k, int64_t
             raised = true;
         }
     }
-    // placing a pair is a population count over its expert's mask words and two scattered stores: beyond a few thousand
-    // pairs several workgroups share that part (each repeats the cheap counting): 43 -> 16 us at 16384 pairs
-    const unsigned parts = entries >= 3072 ? 8u : 1u;
+    // Placing a pair is two look-ups and two scattered stores: a workgroup per 1024 pairs, up to sixteen, shares that part (each
+    // repeats the cheap counting): one workgroup alone took 43 us for 16384 pairs.
+    const unsigned parts = entries >= 1024 ? (unsigned)((entries + 1023) / 1024 < 16 ? (entries + 1023) / 1024 : 16) : 1u;
     MQ_LAUNCH(build_groups_kernel, dim3(parts), dim3(threads), lds, stream, ids, (int)entries, top_k,
                        (int)n_experts, use_lds, mask_words, with_prefix, group_expert, group_begin, n_groups, entry_token, entry_k);
     return hipGetLastError();
@@ -553,7 +626,9 @@ hipError_t launch_route_and_group(const float* logits, int64_t n_experts, int64_
     // one bit per (expert, token) for the grouping (see launch_build_groups)
     const int mask_words = n <= 4096 ? (int)((n + 31) / 32) : 0;
     const size_t lds_group = (size_t)n_experts * 4 + (size_t)n * top_k * 4 + (mask_words ? ((size_t)n_experts * (mask_words | 1) + 1) * 4 : 0);
-    if (lds_group > 60 * 1024 || n * top_k >= 3072) {  // prefill widths: route, then group over several workgroups, quantize on its own
+    // Prefill widths: route, then group over several workgroups, quantize on its own.  With nothing to quantize from 1536 pairs on: the
+    // one launch groups in its last workgroup, 14.1 us at 1600 pairs against 4.6 + 5.2 for the two (11.0 against 4.5 + 5.1 at 1040).
+    if (lds_group > 60 * 1024 || n * top_k >= (qx ? 3072 : 1536)) {
         hipError_t e = launch_route_topk(logits, n_experts, n, top_k, mode, ids, weights, stream);
         if (e != hipSuccess) return e;
         e = launch_build_groups(ids, n, top_k, n_experts, group_expert, group_begin, n_groups, entry_token, entry_k,
