@@ -17,12 +17,15 @@ SILU_EXACT, SILU_FAST, SILU_FAST_FMA = 0, 1, 2
 ROUTE_FUSED, ROUTE_FLOOR, ROUTE_FLOOR_FINITE = 0, 1, 2
 
 
-def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# Handles go to the library as plain integers (every entry point declares its pointer arguments): on a call of a few microseconds
+# the Stream object that torch.cuda.current_stream() builds and a c_void_p per pointer are a quarter of the host's time, which is
+# what such calls are bound by (2048 x 2048, one row, back to back: 9.4 -> 7.05 us; a product of 16 us 13.9).
+def _stream() -> int:
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def _ptr(t: torch.Tensor) -> C.c_void_p:
-    return C.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def _f32(x: torch.Tensor) -> torch.Tensor:
