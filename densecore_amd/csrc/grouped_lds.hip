@@ -264,12 +264,8 @@ template <int NMAT, int WT>
 hipError_t launch_wt(const MatmulArgs& a, dim3 grid, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
     auto* kernel = &grouped_lds_kernel<NMAT, WT>;
     const size_t lds = lds_bytes(a.nb);
-    static bool raised = false;  // per instantiation; the attribute belongs to the function, not to a launch
-    if (!raised && lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    // at most 56.5 KB (14 super-blocks: grouped_lds_applies), inside the 64 KB that need no attribute; asking for all 160 KB is
+    // refused here, the kernel has a static word as well
     if (start && stop) hipExtLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, start, stop, 0, a);
     else MQ_LAUNCH(kernel, grid, dim3(512), lds, stream, a);
     return hipGetLastError();
@@ -284,7 +280,6 @@ bool grouped_lds_applies(const MatmulArgs& a) {
     if (!g_enabled || !a.grouped || a.dbg_dot || a.xf) return false;
     if (a.out_aq && (a.rows & 255)) return false;
     if (a.nb & 1) return false;           // the stage loop runs in pairs
-    if (!a.swiglu && (a.nb & 1)) return false;  // one matrix: the stage loop runs over pairs of super-blocks
     if (a.swiglu && a.wtype != kTypeQ4K) return false;  // fused Q5_K / Q6_K tiles do not fit four wavefronts per SIMD
     return lds_bytes(a.nb) <= 64 * 1024;       // two workgroups per compute unit keep their rows side by side
 }

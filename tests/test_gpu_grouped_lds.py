@@ -128,3 +128,23 @@ def test_mul_mat_id_same_bits(env, x_slots_full, cols, rows, n_exp, top_k, n):
         _, ids = route(torch, n, n_exp, top_k, 9320 + wtype)
         want, got = both_ways(env, lambda: [ops.mul_mat_id(W, x, ids)])
         same_bits(want, got, f"mul_mat_id type {wtype}")
+
+
+@pytest.mark.parametrize("hidden,inter,n_exp,top_k,n", [(3072, 256, 128, 2, 134), (3584, 256, 128, 2, 134), (3584, 512, 128, 8, 12), (4096, 256, 128, 2, 134)])
+def test_rows_of_twelve_and_fourteen_super_blocks(env, hidden, inter, n_exp, top_k, n):
+    """The longest rows that the gathering kernel stages (48.5 and 56.5 KB of LDS; sixteen super-blocks go to the other kernel):
+    gate/up, single products of the three types and the whole layer."""
+    torch, _lib, ops = env
+    seed = synth.tensor_seed("gl-long", hidden, inter, n)
+    G, U = (ops.Q4KWeight.synthetic(seed + i, inter, hidden, n_exp) for i in (1, 2))
+    D = ops.Q4KWeight.synthetic(seed + 3, hidden, inter, n_exp, ggml_type=13)
+    x = torch.from_numpy(synth.normal_f32(seed + 4, (n, hidden))).cuda()
+    logits, ids = route(torch, n, n_exp, top_k, seed + 5)
+    same_bits(*both_ways(env, lambda: [ops.moe_gateup_swiglu(G, U, x, ids, 2)]), "gate/up")
+    same_bits(*both_ways(env, lambda: [ops.moe_layer(G, U, D, x, logits, top_k, silu=ops.SILU_FAST)[0]]), "layer")
+    for wtype in (12, 13, 14):
+        W = ops.Q4KWeight.synthetic(seed + 6 + wtype, inter, hidden, n_exp, ggml_type=wtype)
+        same_bits(*both_ways(env, lambda: [ops.mul_mat_id(W, x, ids)]), f"mul_mat_id type {wtype}")
+        W.free()
+    for w in (G, U, D):
+        w.free()
