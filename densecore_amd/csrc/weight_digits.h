@@ -60,7 +60,9 @@ __device__ __forceinline__ void expand_tile(const v4u seg0, const v4u seg1, cons
     const v4u seg[2] = {seg0, seg1};
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const uint32_t scw = i ? sc47 : sc03;
+        // (the digits ahead of the codes: formed behind them, the GEMM's schedule is 0.4 % slower -- gate/up pair of 14336 x 4096 at
+        // 2048 rows 510.8 against 508.5 us)
+        const uint32_t scw = i ? sc47 : sc03, s1w = (scw >> 3) & 0x07070707u, s0w = scw & 0x07070707u;
         // sub-blocks 4i .. 4i+3 are bytes 0..3 of the scale word
         const uint32_t l0 = seg[i].x & 0x0f0f0f0fu, l1 = seg[i].y & 0x0f0f0f0fu;  // sub-block 4i
         const uint32_t l2 = seg[i].z & 0x0f0f0f0fu, l3 = seg[i].w & 0x0f0f0f0fu;  // sub-block 4i+2
@@ -83,7 +85,6 @@ __device__ __forceinline__ void expand_tile(const v4u seg0, const v4u seg1, cons
             t.hi[2 * i + 1] = v4i{hi[4], hi[5], hi[6], hi[7]}, t.lo[2 * i + 1] = v4i{lo[4], lo[5], lo[6], lo[7]};
         } else {
             // digits of sub-blocks (4i, 4i+1) and (4i+2, 4i+3), two to a word
-            const uint32_t s1w = (scw >> 3) & 0x07070707u, s0w = scw & 0x07070707u;
             const uint32_t ab1 = digit_pair(s1w, 0), ab0 = digit_pair(s0w, 0);
             const uint32_t ce1 = digit_pair(s1w, 2), ce0 = digit_pair(s0w, 2);
             t.hi[2 * i] = v4i{(int)scale_bytes<0>(l0, ab1), (int)scale_bytes<0>(l1, ab1), (int)scale_bytes<0>(l2, ce1),
