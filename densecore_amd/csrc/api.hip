@@ -65,6 +65,7 @@ bool g_graph_seen = false;
 std::vector<void*> g_retired;
 
 int hip_fail(hipError_t e, const char* what) {
+    (void)hipGetLastError();  // reported here: the next launch's check must not find it again
     return fail(MQ_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 

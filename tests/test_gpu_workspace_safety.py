@@ -122,3 +122,16 @@ def test_skeleton_mode_launches_nothing_that_computes_and_restores(env):
     torch.cuda.synchronize()
     assert torch.equal(out, want)
     w.free()
+
+
+def test_a_refused_allocation_does_not_fail_the_next_call(env):
+    """A HIP error belongs to the call that met it: the launch checks of later calls do not report it again."""
+    import ctypes as C
+    torch, _lib, ops = env
+    W = ops.Q4KWeight.synthetic(91, 512, 1024)
+    x = torch.randn((3, 1024), device="cuda")
+    want = ops.mul_mat(W, x)
+    ptr = C.c_void_p()
+    assert _lib.lib().mq_device_malloc(C.byref(ptr), 1 << 50) != 0 and not ptr.value
+    assert torch.equal(ops.mul_mat(W, x), want)
+    W.free()
