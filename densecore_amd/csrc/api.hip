@@ -596,16 +596,21 @@ static bool gemvn_fused_pays(const mq_weight* w, int64_t n) {
 // its own that emits Q8_K for the LDS-staged product: 36.0 / 36.2 us at two rows, 43.9 / 42.4 at three, 48.6 / 45.7 at four.
 constexpr int64_t kNormFusedMaxRows = 2;
 
+// A product of rows that are in the P-major layout already
+static int gemm_quantized_locked(const mq_weight* w, const uint8_t* ap, int64_t n, float* y_dev, int64_t ldy, hipStream_t s) {
+    const GemmShape shape = gemm_shape(w->type, w->rows, w->nb, n);
+    const size_t part_bytes = gemm_part_bytes(shape, w->rows, n);
+    if (part_bytes) MQ_HIP(g.kpart.reserve(part_bytes));
+    MQ_HIP(launch_prefill_gemm(w->data, w->type, w->rows, w->nb, ap, n, y_dev, ldy, part_bytes ? (float*)g.kpart.ptr : nullptr, shape, s));
+    return MQ_OK;
+}
+
 static int gemm_locked(const mq_weight* w, const float* x_dev, int64_t n, int64_t ldx, float* y_dev, int64_t ldy,
                        hipStream_t s) {
     if (n == 0) return MQ_OK;
     MQ_HIP(g.ap.reserve(pmajor_bytes(n, w->nb)));
     MQ_HIP(launch_quantize_q8k_pmajor(x_dev, n, ldx, w->cols, (uint8_t*)g.ap.ptr, s));
-    const size_t part_bytes = prefill_part_bytes(w->rows, w->nb, n);
-    if (part_bytes) MQ_HIP(g.kpart.reserve(part_bytes));
-    MQ_HIP(launch_prefill_gemm(w->data, w->type, w->rows, w->nb, (const uint8_t*)g.ap.ptr, n, y_dev, ldy,
-                               part_bytes ? (float*)g.kpart.ptr : nullptr, s));
-    return MQ_OK;
+    return gemm_quantized_locked(w, (const uint8_t*)g.ap.ptr, n, y_dev, ldy, s);
 }
 
 // Wide FFN on the matrix-core GEMM: gate and up products into the two halves of g.mid2, their SwiGLU formed by the
@@ -615,26 +620,20 @@ static int ffn_wide_locked(const mq_weight* gate, const mq_weight* up, const mq_
     const int64_t inter = gate->rows;
     MQ_HIP(g.ap.reserve(pmajor_bytes(n, gate->nb)));
     MQ_HIP(launch_quantize_q8k_pmajor(x_dev, n, ldx, gate->cols, (uint8_t*)g.ap.ptr, s));
-    if (g_gemm_pair && gate->type == up->type && prefill_pair_applies(gate->type, inter, gate->nb, n)) {
+    GemmShape pair;
+    if (g_gemm_pair && gate->type == up->type && gemm_pair_shape(gate->type, inter, gate->nb, n, &pair)) {
         // gate and up in one launch that stores silu(gate) * up: no fp32 planes, no pass that reads them back
-        MQ_HIP(launch_prefill_gemm_pair(gate->data, up->data, gate->type, inter, gate->nb, (const uint8_t*)g.ap.ptr, n, silu_mode, h_dev, ldh, s));
+        MQ_HIP(launch_prefill_gemm_pair(gate->data, up->data, gate->type, inter, gate->nb, (const uint8_t*)g.ap.ptr, n, silu_mode, h_dev, ldh, pair, s));
         if (!down) return MQ_OK;
         MQ_HIP(g.ap2.reserve(pmajor_bytes(n, down->nb)));
         MQ_HIP(launch_quantize_q8k_pmajor(h_dev, n, ldh, inter, (uint8_t*)g.ap2.ptr, s));
-        const size_t part2 = prefill_part_bytes(down->rows, down->nb, n);
-        if (part2) MQ_HIP(g.kpart.reserve(part2));
-        MQ_HIP(launch_prefill_gemm(down->data, down->type, down->rows, down->nb, (const uint8_t*)g.ap2.ptr, n, y_dev, ldy,
-                                   part2 ? (float*)g.kpart.ptr : nullptr, s));
-        return MQ_OK;
+        return gemm_quantized_locked(down, (const uint8_t*)g.ap2.ptr, n, y_dev, ldy, s);
     }
     MQ_HIP(g.mid2.reserve(2 * (size_t)n * (size_t)inter * sizeof(float)));
     float* gbuf = (float*)g.mid2.ptr;
     float* ubuf = gbuf + (size_t)n * (size_t)inter;
-    const size_t part_bytes = prefill_part_bytes(inter, gate->nb, n);
-    if (part_bytes) MQ_HIP(g.kpart.reserve(part_bytes));
-    float* part = part_bytes ? (float*)g.kpart.ptr : nullptr;
-    MQ_HIP(launch_prefill_gemm(gate->data, gate->type, inter, gate->nb, (const uint8_t*)g.ap.ptr, n, gbuf, inter, part, s));
-    MQ_HIP(launch_prefill_gemm(up->data, up->type, inter, up->nb, (const uint8_t*)g.ap.ptr, n, ubuf, inter, part, s));
+    if (const int rc = gemm_quantized_locked(gate, (const uint8_t*)g.ap.ptr, n, gbuf, inter, s); rc != MQ_OK) return rc;
+    if (const int rc = gemm_quantized_locked(up, (const uint8_t*)g.ap.ptr, n, ubuf, inter, s); rc != MQ_OK) return rc;
     if (!down && inter % kQK) {  // SwiGLU rows that do not divide into super-blocks: nothing to quantize them for
         MQ_HIP(launch_silu_mul(gbuf, ubuf, n, inter, inter, inter, h_dev, ldh, silu_mode, s));
         return MQ_OK;
@@ -646,11 +645,7 @@ static int ffn_wide_locked(const mq_weight* gate, const mq_weight* up, const mq_
     }
     MQ_HIP(g.ap2.reserve(pmajor_bytes(n, down->nb)));
     MQ_HIP(launch_swiglu_quantize_q8k_pmajor(gbuf, ubuf, n, inter, inter, silu_mode, h_dev, ldh, (uint8_t*)g.ap2.ptr, s));
-    const size_t part2 = prefill_part_bytes(down->rows, down->nb, n);
-    if (part2) MQ_HIP(g.kpart.reserve(part2));
-    MQ_HIP(launch_prefill_gemm(down->data, down->type, down->rows, down->nb, (const uint8_t*)g.ap2.ptr, n, y_dev, ldy,
-                               part2 ? (float*)g.kpart.ptr : nullptr, s));
-    return MQ_OK;
+    return gemm_quantized_locked(down, (const uint8_t*)g.ap2.ptr, n, y_dev, ldy, s);
 }
 
 // Q8_0 weights: the activations are quantized to Q8_0 as well (codes into g.aq in the A-major order, fp16 scales
@@ -2089,6 +2084,18 @@ int mq_debug_set_dense_lds(int on) {
     g_skinny16 = (on & 0x1000) ? 0 : 1;      // bit 12: nine to 64 rows stay on the kernels with token tiles of eight (or the GEMM)
     g_dense_xf_rows = ((on >> 4) & 0xf) ? ((on >> 4) & 0xf) - 1 : kDenseXfRowsDefault;  // bits 4..7, experiments: widest product that quantizes its rows itself, plus one (0: the default)
     return before;
+}
+
+int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out) {
+    if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !shape_out)
+        return fail(MQ_ERR_INVALID, "mq_debug_gemm_shape: bad type, size or pointer");
+    GemmShape s;
+    bool taken = true;
+    if (pair) taken = gemm_pair_shape(wtype, rows, cols / kQK, n, &s);
+    else s = gemm_shape(wtype, rows, cols / kQK, n);
+    shape_out[0] = s.narrow, shape_out[1] = s.splits, shape_out[2] = s.sb_split, shape_out[3] = s.tiles_per_wg;
+    shape_out[4] = (int)s.row_wgs, shape_out[5] = (int)s.groups, shape_out[6] = taken, shape_out[7] = (int)(1000.0f * s.us);
+    return MQ_OK;
 }
 
 int mq_debug_set_skeleton(int on) {

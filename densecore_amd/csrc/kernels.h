@@ -211,21 +211,29 @@ hipError_t launch_quantize_q8k_pmajor(const float* x, int64_t n, int64_t ldx, in
 // The same for the rows silu(gate) * up (both [n][ldx]); h_out (may be null) receives them as fp32 [n][ldh] as well.
 hipError_t launch_swiglu_quantize_q8k_pmajor(const float* gate, const float* up, int64_t n, int64_t ldx, int64_t k,
                                              int silu_mode, float* h_out, int64_t ldh, uint8_t* ap, hipStream_t stream);
-// y[n][ldy] = P-major activations . tiled weights^T on the int8 matrix cores.  A launch that would leave workgroup
-// slots empty splits K into runs of super-blocks whose sums go to planes of `part` (prefill_part_bytes() bytes, 0 when
-// nothing is split) and are added in order by a second launch.
+// y[n][ldy] = P-major activations . tiled weights^T on the int8 matrix cores, in the launch shape that gemm_shape chooses for
+// the product: 64- or 128-row workgroups of tiles_per_wg activation tiles, K whole or in `splits` runs of sb_split
+// super-blocks whose sums go to planes of `part` (gemm_part_bytes() bytes, 0 with K whole) and are added in order by a second launch.
 // wtype: kTypeQ4K, kTypeQ5K or kTypeQ6K.
-size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n);
-// silu(gate . x) * (up . x) from ONE launch (prefill.hip: the pair form of the GEMM kernel), dense and expert-grouped
-bool prefill_pair_applies(int wtype, int64_t rows, int64_t nb, int64_t n);
+struct GemmShape {
+    bool narrow = false;  // 64 rows
+    int splits = 1, sb_split = 1, tiles_per_wg = 1;
+    unsigned row_wgs = 1, groups = 1;
+    float us = 0.0f;  // its estimate
+};
+GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n);
+size_t gemm_part_bytes(const GemmShape& shape, int64_t rows, int64_t n);
+hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
+                               int64_t ldy, float* part, const GemmShape& shape, hipStream_t stream);
+// silu(gate . x) * (up . x) from ONE launch (prefill.hip: the pair form of the GEMM kernel), dense and expert-grouped.
+// gemm_pair_shape: false where two products and a SwiGLU pass are the better choice.
+bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* shape);
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,
-                                    int64_t n, int silu_mode, float* h, int64_t ldh, hipStream_t stream);
+                                    int64_t n, int silu_mode, float* h, int64_t ldh, const GemmShape& shape, hipStream_t stream);
 hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t expert_bytes,
                                             const uint8_t* gate_shared, const uint8_t* up_shared, int64_t rows, int64_t nb,
                                             const uint8_t* ap, int64_t entries, int64_t groups_max, const int32_t* plan, bool scatter,
                                             int silu_mode, float* h, int64_t ldh, hipStream_t stream, int mt = 8);
-hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
-                               int64_t ldy, float* part, hipStream_t stream);
 
 // Expert-grouped form of the GEMM (a MoE block at prefill widths): a plan lays the routed entries out in 16-row tiles
 // per expert (moe_gemm_plan_ints() int32 of workspace; sizes from the upper bounds entries = n * top_k and groups_max),

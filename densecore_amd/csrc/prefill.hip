@@ -466,21 +466,16 @@ __global__ void __launch_bounds__(256) prefill_sum_planes_kernel(const float* __
 // unit, tiles in eights, K split only to fill the slots), with its quantizer and planes: 4096 x 14336 at 130 / 391 / 700 / 1200 rows
 // 46 / 84 / 145 / 245 -> 37 / 75 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 70 / 109, 2048 x 2048 at 777
 // 27.6 -> 23.8.
-struct PrefillShape {
-    bool narrow = false;
-    int splits = 1, sb_split = 1, tiles_per_wg = 1;
-    unsigned row_wgs = 1, groups = 1;
-    float us = 1e30f;  // the estimate
-};
 // PAIR form: a row tile of both matrices per wavefront (the 128-row body), no K split (SiLU is not linear); one workgroup alone
 // 0.9 + 0.32 t.  From 25 activation tiles on it keeps them in eights with the short column last, whose workgroups fill the last
 // round (14336 x 4096, tiles to a workgroup 8 / 7 / 5: 122 / 121 / 132 us at 391 rows, 310 / 320 / 359 at 1200).
-PrefillShape prefill_shape(int64_t rows, int64_t nb, int64_t n, bool pair = false) {
+GemmShape choose_shape(int64_t rows, int64_t nb, int64_t n, bool pair = false) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
     const int64_t units = compute_units();
     const int64_t min_groups = (m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup, max_groups = pair && m_tiles >= 25 ? min_groups : min_groups + 4;
     const int max_splits = pair || (rows & 3) ? 1 : (int)(nb / 4 < 16 ? nb / 4 : 16);  // at least four super-blocks per run
-    PrefillShape best;
+    GemmShape best;
+    best.us = 1e30f;
     for (int narrow = 0; narrow < (pair ? 1 : 2); ++narrow) {
         const int64_t row_wgs = (pair || narrow) ? (rowtiles + 3) / 4 : (rowtiles + 7) / 8;
         for (int64_t want = min_groups; want <= max_groups; ++want) {
@@ -721,20 +716,24 @@ hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expe
     return hipGetLastError();
 }
 
+GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n) {
+    (void)wtype;
+    return choose_shape(rows, nb, n);
+}
+
 // The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear): where the
 // launch is small enough for that to matter, two launches with K in runs and the SwiGLU pass over their planes are faster.
-bool prefill_pair_applies(int wtype, int64_t rows, int64_t nb, int64_t n) {
-    if (!gemm_type(wtype)) return false;
-    return prefill_shape(rows, nb, n, true).us <= 2.0f * prefill_shape(rows, nb, n).us + 3.0f + (float)(n * rows) * (12.0f / 4e6f);
+bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* shape) {
+    if (!gemm_type(wtype) || rows <= 0 || n <= 0) return false;
+    *shape = choose_shape(rows, nb, n, true);
+    return shape->us <= 2.0f * gemm_shape(wtype, rows, nb, n).us + 3.0f + (float)(n * rows) * (12.0f / 4e6f);
 }
 
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,
-                                    int64_t n, int silu_mode, float* h, int64_t ldh, hipStream_t stream) {
+                                    int64_t n, int silu_mode, float* h, int64_t ldh, const GemmShape& ps, hipStream_t stream) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
     if (rowtiles == 0 || m_tiles == 0) return hipSuccess;
-    if (!prefill_pair_applies(wtype, rows, nb, n)) return hipErrorInvalidValue;
-    const PrefillShape ps = prefill_shape(rows, nb, n, true);
-    if (ps.groups > 65535u) return hipErrorInvalidValue;
+    if (!gemm_type(wtype) || ps.splits != 1 || ps.groups > 65535u) return hipErrorInvalidValue;
     if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
 #define MQ_GO(WT_)                                                                                                                        \
     MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, \
@@ -771,8 +770,7 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
     return hipGetLastError();
 }
 
-size_t prefill_part_bytes(int64_t rows, int64_t nb, int64_t n) {
-    const PrefillShape ps = prefill_shape(rows, nb, n);
+size_t gemm_part_bytes(const GemmShape& ps, int64_t rows, int64_t n) {
     return ps.splits > 1 ? (size_t)ps.splits * (size_t)n * (size_t)rows * sizeof(float) : 0;
 }
 
@@ -807,11 +805,10 @@ hipError_t launch_swiglu_quantize_q8k_pmajor(const float* gate, const float* up,
 }
 
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
-                               int64_t ldy, float* part, hipStream_t stream) {
+                               int64_t ldy, float* part, const GemmShape& ps, hipStream_t stream) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
     if (rowtiles == 0 || m_tiles == 0) return hipSuccess;
     if (!gemm_type(wtype)) return hipErrorInvalidValue;
-    const PrefillShape ps = prefill_shape(rows, nb, n);
     if (ps.groups > 65535u) return hipErrorInvalidValue;
     if (ps.splits > 1 && !part) return hipErrorInvalidValue;
     if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;

@@ -67,6 +67,11 @@ int mq_census_read(int kind, double* avg_us, double* min_us, double* max_us, int
  * previous setting of bit 0.  No counterpart in the reference. */
 int mq_debug_set_dense_lds(int on);
 
+/* Launch shape that the matrix-core GEMM takes for a product of n rows (pair != 0: for gate and up in one launch), for a 256-unit
+ * device before mq_init.  shape_out: 64-row workgroups (1) or 128-row ones (0), runs of K, super-blocks per run, activation tiles per
+ * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns. */
+int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);
+
 /* Measurement instrument: while on != 0 every compute and routing launch of the library is replaced by a kernel with
  * an empty body and the same grid, block and LDS size (weight set-up and launches that carry timing events are
  * not).  A graph captured in this state has the launches of the real one and none of their work: its replay time
