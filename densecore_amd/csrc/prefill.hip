@@ -455,49 +455,120 @@ __global__ void __launch_bounds__(256) prefill_sum_planes_kernel(const float* __
     dst[0] = acc.x, dst[1] = acc.y, dst[2] = acc.z, dst[3] = acc.w;
 }
 
-// Shape of a launch: 128- or 64-row workgroups, the activation tiles dealt evenly over `groups` workgroup columns of
-// tiles_per_wg <= 8, K in `splits` runs of super-blocks (planes of partial sums that a second launch adds in order).  A compute
-// unit holds two workgroups, and a workgroup walks its super-blocks one after the other, so what counts is the length of a
-// workgroup times the rounds of 2 x compute_units() of them.  Time of a workgroup and super-block, us, by its tiles t, measured
-// over 4096 x 14336, 14336 x 4096, 6144 x 4096 at 50 to 2048 rows (two workgroups on a unit | one alone):
-//     128 rows  0.4 + 0.52 t | 0.6 + 0.27 t        64 rows  0.35 + 0.28 t | 0.55 + 0.16 t
-// (and no less than the streaming of the weights: 2.0 and 1.1 us with two workgroups on every unit).
-// The shape with the smallest estimate is taken.  Against the fixed order it replaces (64-row workgroups up to one per compute
-// unit, tiles in eights, K split only to fill the slots), with its quantizer and planes: 4096 x 14336 at 130 / 391 / 700 / 1200 rows
-// 46 / 84 / 145 / 245 -> 37 / 75 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 70 / 109, 2048 x 2048 at 777
-// 27.6 -> 23.8.
-// PAIR form: a row tile of both matrices per wavefront (the 128-row body), no K split (SiLU is not linear); one workgroup alone
-// 0.9 + 0.32 t.  From 25 activation tiles on it keeps them in eights with the short column last, whose workgroups fill the last
-// round (14336 x 4096, tiles to a workgroup 8 / 7 / 5: 122 / 121 / 132 us at 391 rows, 310 / 320 / 359 at 1200).
-GemmShape choose_shape(int64_t rows, int64_t nb, int64_t n, bool pair = false) {
-    const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
-    const int64_t units = compute_units();
-    const int64_t min_groups = (m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup, max_groups = pair && m_tiles >= 25 ? min_groups : min_groups + 4;
-    const int max_splits = pair || (rows & 3) ? 1 : (int)(nb / 4 < 16 ? nb / 4 : 16);  // at least four super-blocks per run
-    GemmShape best;
-    best.us = 1e30f;
-    for (int narrow = 0; narrow < (pair ? 1 : 2); ++narrow) {
-        const int64_t row_wgs = (pair || narrow) ? (rowtiles + 3) / 4 : (rowtiles + 7) / 8;
-        for (int64_t want = min_groups; want <= max_groups; ++want) {
-            const int64_t t = pair && m_tiles >= 25 ? kMTilesPerGroup : (m_tiles + want - 1) / want, groups = (m_tiles + t - 1) / t;
-            float two = narrow ? 0.35f + 0.28f * t : 0.4f + 0.52f * t;
-            const float one = pair ? 0.9f + 0.32f * t : narrow ? 0.55f + 0.16f * t : 0.6f + 0.27f * t, stream = narrow ? 1.1f : 2.0f;
-            if (two < stream) two = stream;
-            for (int sp = 1; sp == 1 || sp <= max_splits; ++sp) {
-                const int64_t sb = (nb + sp - 1) / sp, splits = (nb + sb - 1) / sb;  // every run holds a super-block
-                if (splits != sp) continue;
-                const int64_t wgs = row_wgs * groups * splits, rest = wgs % (2 * units);
-                float us = (float)sb * ((float)(wgs / (2 * units)) * two + (rest == 0 ? 0.0f : rest <= units ? one : two));
-                if (splits > 1) us += 3.0f + (float)(2 * splits) * (float)(n * rows) * (4.0f / 8e6f);  // planes: a launch, written and read
-                if (us < best.us) {
-                    best.narrow = narrow != 0, best.splits = (int)splits, best.sb_split = (int)sb, best.tiles_per_wg = (int)t;
-                    best.row_wgs = (unsigned)row_wgs, best.groups = (unsigned)groups, best.us = us;
+// Shape of a launch: 128- or 64-row workgroups, the activation tiles in `groups` workgroup columns of tiles_per_wg <= 8, K in
+// `splits` runs of super-blocks (planes of partial sums that a second launch adds in order).  A compute unit holds two workgroups,
+// and a workgroup walks its super-blocks one after the other, so what counts is how long a workgroup takes and how the workgroups
+// fill the 2 x compute_units() slots.  Pace: us a workgroup takes for t activation tiles and sb super-blocks,
+//     two on a unit  sb (sb2 + tile2 t) + fix2 + store t        one alone  sb (sb1 + tile1 t) + fix1 + store t
+// (fix, store: first tiles, last stores), what all units busy cost on top (load: per tile of a round of slots), and the rounds:
+// r workgroups left after a full round take tail0 + tail1 r / slots of one (the rounds do not start together), and a workgroup
+// beside a shorter one is held up for `beside` of their common time.  Least-squares fits over every shape of 8,700 dense products
+// and 3,300 gate/up pairs (512 to 16,384 rows, 4 to 56 super-blocks, 48 to 2048 tokens; residuals 3 to 5 %), 128-row | 64-row | pair:
+struct Pace {
+    float sb2, tile2, sb1, tile1, fix2, store, fix1, load, tail0, tail1, beside;
+};
+enum { kWide, kNarrow, kPairForm };
+constexpr Pace kPace[3][3] = {
+    {{0.880f, 0.222f, 0.530f, 0.190f, 0.78f, 0.118f, 0.65f, 0.151f, 0.337f, 0.733f, 0.415f},   // Q4_K
+     {0.500f, 0.134f, 0.334f, 0.145f, 0.38f, 0.000f, 0.00f, 0.085f, 0.574f, 0.465f, 0.002f},
+     {0.919f, 0.314f, 0.591f, 0.239f, 3.93f, 0.000f, 2.39f, 0.064f, 0.454f, 0.558f, 0.483f}},
+    {{1.609f, 0.220f, 0.916f, 0.181f, 0.53f, 0.078f, 0.71f, 0.160f, 0.271f, 0.757f, 0.767f},   // Q5_K: 16-bit products cost the expansion
+     {0.825f, 0.133f, 0.459f, 0.153f, 0.01f, 0.000f, 0.00f, 0.093f, 0.490f, 0.555f, 0.272f},
+     {1.763f, 0.327f, 1.109f, 0.231f, 2.87f, 0.000f, 1.13f, 0.024f, 0.382f, 0.663f, 0.717f}},
+    {{1.610f, 0.194f, 0.941f, 0.159f, 0.73f, 0.063f, 0.85f, 0.161f, 0.268f, 0.759f, 0.690f},   // Q6_K: no min MFMA
+     {0.874f, 0.111f, 0.476f, 0.121f, 0.13f, 0.000f, 0.00f, 0.083f, 0.396f, 0.635f, 0.580f},
+     {1.782f, 0.290f, 1.119f, 0.209f, 3.32f, 0.000f, 1.25f, 0.039f, 0.394f, 0.677f, 0.723f}}};
+
+GemmShape shape_of(int form, int64_t rows, int64_t nb, int64_t m_tiles, int64_t t, int64_t splits) {
+    const int64_t rowtiles = (rows + 15) / 16;
+    GemmShape s;
+    s.narrow = form == kNarrow, s.tiles_per_wg = (int)t;
+    s.row_wgs = (unsigned)(form == kWide ? (rowtiles + 7) / 8 : (rowtiles + 3) / 4), s.groups = (unsigned)((m_tiles + t - 1) / t);
+    s.sb_split = (int)((nb + splits - 1) / splits);
+    s.splits = (int)((nb + s.sb_split - 1) / s.sb_split);  // every run holds a super-block
+    return s;
+}
+
+// us of a launch, its planes included
+float shape_us(const Pace& p, const GemmShape& s, int64_t rows, int64_t m_tiles, int64_t n) {
+    const int64_t units = compute_units(), slots = 2 * units;
+    const int64_t t = s.tiles_per_wg, t_last = m_tiles - (int64_t)(s.groups - 1) * t, column = (int64_t)s.row_wgs * s.splits;
+    const float sb = (float)s.sb_split;
+    auto two = [&](int64_t k) { return sb * (p.sb2 + p.tile2 * (float)k) + p.fix2 + p.store * (float)k; };
+    auto one = [&](int64_t k) {
+        const float v = sb * (p.sb1 + p.tile1 * (float)k) + p.fix1 + p.store * (float)k;
+        return v < two(k) ? v : two(k);
+    };
+    auto last_round = [&](int64_t r, bool first, int64_t k) {  // r < slots workgroups of k tiles
+        if (r == 0) return 0.0f;
+        if (first) return r <= units ? one(k) : two(k);
+        const float part = p.tail0 + p.tail1 * (float)r / (float)slots;
+        return two(k) * (part < 1.2f ? part : 1.2f);
+    };
+    float us;
+    if (t_last == t || s.groups == 1 || s.splits > 1) {
+        const int64_t wgs = column * s.groups, full = wgs / slots;
+        us = (float)full * two(t) + last_round(wgs % slots, full == 0, t);
+    } else {  // the short column comes last and fills what the last round leaves
+        const int64_t wgs = column * (s.groups - 1), full = wgs / slots, r = wgs % slots, spare = slots - r;
+        us = (float)full * two(t);
+        const float shorter = two(t_last);
+        if (r == 0) {
+            us += (float)(column / slots) * shorter + last_round(column % slots, full + column / slots == 0, t_last);
+        } else if (column <= spare) {
+            if (full > 0) us += last_round(r + column, false, t);
+            else if (r > units) us += two(t);
+            else us += one(t) + (r + column > units ? (two(t) - one(t)) * p.beside * (shorter < two(t) ? shorter / two(t) : 1.0f) : 0.0f);
+        } else {
+            const float chain = (float)((column + spare - 1) / spare) * shorter;
+            int64_t beside = (int64_t)(two(t) / shorter);
+            beside = (beside < 1 ? 1 : beside) * spare;
+            const int64_t left = column > beside ? column - beside : 0;
+            const float after = two(t) + (float)(left / slots) * shorter + last_round(left % slots, false, t_last);
+            const float tail = chain < after ? chain : after;
+            us += tail > two(t) ? tail : two(t);
+        }
+    }
+    us += p.load * sb * (float)(column * m_tiles) / (float)slots;
+    if (s.splits > 1) us += 2.8f + 0.064f * 8e-6f * (float)s.splits * (float)(n * rows);  // a launch, the planes written and read
+    return us;
+}
+
+// The plain shape -- 64-row workgroups up to one 128-row workgroup per unit, tiles in eights, K in as many runs as fill the slots --
+// unless the estimate gives another one at least 6 % less (its own error).  Best of every shape / plain / estimate alone / with the
+// 6 %, mean over the fitted Q4_K products: 1 / 1.12 / 1.010 / 1.012; slower than plain by over 3 %: 3 % / 0.5 % of them, at most 1.16 / 1.13.
+// 4096 x 14336 at 130 / 391 / 700 / 1200 rows against the plain shape, with quantizer and planes: 46 / 84 / 145 / 245 ->
+// 37 / 75 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 70 / 109.
+GemmShape choose_shape(const Pace* pace, bool pair, int64_t rows, int64_t nb, int64_t n) {
+    const int64_t units = compute_units(), m_tiles = (n + 15) / 16, rowtiles = (rows + 15) / 16;
+    const int64_t most = m_tiles < kMTilesPerGroup ? m_tiles : kMTilesPerGroup, min_groups = (m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup;
+    const int64_t max_splits = pair || (rows & 3) ? 1 : (nb / 4 < 1 ? 1 : nb / 4 < 16 ? nb / 4 : 16);  // at least four super-blocks per run
+    const int plain_form = pair ? kPairForm : (rowtiles + 7) / 8 * min_groups <= units ? kNarrow : kWide;
+    GemmShape plain = shape_of(plain_form, rows, nb, m_tiles, most, 1);
+    const int64_t fill = 2 * units / ((int64_t)plain.row_wgs * plain.groups), runs = fill < nb / 4 ? fill : nb / 4;
+    if (!pair && !(rows & 3) && runs > 1) plain = shape_of(plain_form, rows, nb, m_tiles, most, runs);
+    plain.us = shape_us(pace[plain_form], plain, rows, m_tiles, n);
+    GemmShape best = plain;
+    for (int form = pair ? kPairForm : kWide; form <= (pair ? kPairForm : kNarrow); ++form) {
+        const Pace& p = pace[form];
+        int64_t before = 0;
+        for (int64_t want = min_groups; want < min_groups + 6; ++want) {
+            const int64_t t = want < min_groups + 5 ? (m_tiles + want - 1) / want : most;  // dealt evenly; in eights with a short column
+            if (t == before) continue;
+            before = t;
+            GemmShape s = shape_of(form, rows, nb, m_tiles, t, 1);
+            for (int sp = 1; sp <= max_splits; ++sp) {
+                s.sb_split = ((int)nb + sp - 1) / sp, s.splits = ((int)nb + s.sb_split - 1) / s.sb_split;
+                // (no longer than the best so far even as workgroups alone; a count that leaves no empty run)
+                if ((float)s.sb_split * (p.sb1 + p.tile1 * (float)t) < best.us && s.splits == sp) {
+                    s.us = shape_us(p, s, rows, m_tiles, n);
+                    if (s.us < best.us) best = s;
                 }
-                if (wgs > 4 * units) break;  // already two rounds and more: further runs only add planes
+                if ((int64_t)s.row_wgs * s.groups * sp > 4 * units) break;  // two rounds and more: further runs only add planes
             }
         }
     }
-    return best;
+    return best.us <= 0.94f * plain.us ? best : plain;
 }
 
 // ---- expert-grouped GEMM: the plan ------------------------------------------------------------------------
@@ -679,6 +750,7 @@ hipError_t raise_gemm_lds() {
     raised = true;
     return hipSuccess;
 }
+int pace_of(int wtype) { return wtype == kTypeQ6K ? 2 : wtype == kTypeQ5K ? 1 : 0; }
 bool gemm_type(int wtype) { return wtype == kTypeQ4K || wtype == kTypeQ5K || wtype == kTypeQ6K; }
 // GO(form constant) for the weight type of a launch
 #define MQ_BY_TYPE(wtype, GO)              \
@@ -716,17 +788,17 @@ hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expe
     return hipGetLastError();
 }
 
-GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n) {
-    (void)wtype;
-    return choose_shape(rows, nb, n);
-}
+GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n) { return choose_shape(kPace[pace_of(wtype)], false, rows, nb, n); }
 
-// The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear): where the
-// launch is small enough for that to matter, two launches with K in runs and the SwiGLU pass over their planes are faster.
+// The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear): for a few rows of
+// a long K two launches with K in runs and the SwiGLU pass over their planes are faster, by up to half (1 to 4 % of the fitted
+// pairs); taken where the estimate, with 8 us of quantizer on both sides, says so by 6 % (then never slower by more than 5 %).
 bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* shape) {
     if (!gemm_type(wtype) || rows <= 0 || n <= 0) return false;
-    *shape = choose_shape(rows, nb, n, true);
-    return shape->us <= 2.0f * gemm_shape(wtype, rows, nb, n).us + 3.0f + (float)(n * rows) * (12.0f / 4e6f);
+    *shape = choose_shape(kPace[pace_of(wtype)], true, rows, nb, n);
+    const float out = 1e-6f * (float)(n * rows), one_launch = shape->us + 0.25f * out;
+    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 9.0f + 3.3f * out;
+    return two_launches + 8.0f >= 0.94f * (one_launch + 8.0f);
 }
 
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,
