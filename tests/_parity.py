@@ -25,5 +25,15 @@ def assert_fp32_parity(got: np.ndarray, ref: np.ndarray, mag: np.ndarray, what: 
     return float(np.max(err[ok] / np.abs(ref[ok]))) if ok.any() else 0.0
 
 
+def gemm_shape(wtype: int, rows: int, cols: int, n: int, pair: int = 0) -> dict:
+    """The launch shape that the matrix-core GEMM chooses for a product (include/mi355_q4k_debug.h)."""
+    import ctypes as C
+
+    from densecore_amd import _lib
+    out = (C.c_int * 8)()
+    assert _lib.load().mq_debug_gemm_shape(wtype, rows, cols, n, pair, out) == 0
+    return dict(zip(("narrow", "runs", "sb_run", "tiles", "row_wgs", "columns", "taken", "ns"), out))
+
+
 def oracle_all_orders(w: np.ndarray, cols: int, q8: np.ndarray):
     return {name: orc.mul_mat_q4k_q8k(w, cols, q8, order) for name, order in orc.ORDERS.items()}

@@ -1,19 +1,12 @@
 """The launch shape that the matrix-core GEMM chooses (no GPU needed: the rule is host arithmetic, for 256 compute units before a
 device is opened): every shape covers its product, and products where two shapes were measured get the faster one."""
-import ctypes as C
 import random
 
 import pytest
 
-from densecore_amd import _lib
+from tests._parity import gemm_shape as shape
 
 Q4, Q5, Q6 = 12, 13, 14
-
-
-def shape(wtype, rows, cols, n, pair=0):
-    out = (C.c_int * 8)()
-    assert _lib.load().mq_debug_gemm_shape(wtype, rows, cols, n, pair, out) == 0
-    return dict(zip(("narrow", "runs", "sb_run", "tiles", "row_wgs", "columns", "taken", "ns"), out))
 
 
 def test_every_shape_covers_its_product():

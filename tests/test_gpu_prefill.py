@@ -8,7 +8,7 @@ import pytest
 
 from densecore_amd import synth
 from oracle import binding as orc
-from tests._parity import assert_fp32_parity
+from tests._parity import assert_fp32_parity, gemm_shape
 
 pytestmark = pytest.mark.gpu
 
@@ -108,12 +108,13 @@ def test_gemm_agrees_with_decode_kernel_and_dispatch(ops):
     W.free()
 
 
-@pytest.mark.parametrize("rows,cols,n", [(64, 4096, 50), (48, 14336, 130), (272, 2048, 33), (4096, 14336, 48)])
+@pytest.mark.parametrize("rows,cols,n", [(64, 4096, 50), (48, 14336, 130), (272, 2048, 200), (4096, 14336, 48)])
 def test_gemm_with_k_in_runs_matches_oracle_and_decode_kernel(ops, rows, cols, n):
     """Few weight rows and a long K: the launch splits K into runs of super-blocks whose sums are added in order by
-    a second launch (64 x 4096: four runs; 48 x 14336: fourteen; 272 x 2048: two; 4096 x 14336 at 48 rows: eight).
+    a second launch (64 x 4096: four runs; 48 x 14336: fourteen; 272 x 2048 at 200 rows: two; 4096 x 14336 at 48 rows: eight).
     Against the oracle on a sample of weight rows, and against the decode kernel on all of them."""
     import torch
+    assert gemm_shape(12, rows, cols, n)["runs"] == {64: 4, 48: 14, 272: 2, 4096: 8}[rows]
     w = synth.q4k_matrix(synth.tensor_seed("pf-split", rows, cols), rows, cols)
     x = synth.normal_f32(synth.tensor_seed("pf-split-x", n, cols), (n, cols))
     W = ops.Q4KWeight.from_ggml(w, cols)
@@ -137,6 +138,7 @@ def test_gemm_integer_sums_are_exact_with_k_in_runs(ops):
     columns: four runs of four super-blocks): every partial sum is an integer below 2^24, so the planes add exactly."""
     rows, cols, n = 32, 4096, 20
     nb = cols // 256
+    assert gemm_shape(12, rows, cols, n)["runs"] == 4
     w = synth.q4k_matrix(synth.tensor_seed("pf-int-split", rows), rows, cols).reshape(rows, nb, 144).copy()
     w[:, :, 0:2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
     w[:, :, 2:4] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)

@@ -151,7 +151,7 @@ def test_ffn_all_q5k(ops):
 @pytest.mark.parametrize("n", [1, 4, 16, 40, 300])
 def test_moe_with_q5k_down_experts(ops, n):
     """Routed layer with Q4_K gate/up and Q5_K down experts plus a shared expert of the same types (300 tokens: a
-    hundred rows per expert, every product on the expert-grouped matrix-core GEMM, the Q5_K ones with its third chain)."""
+    hundred rows per expert, every product on the expert-grouped matrix-core GEMM)."""
     E, H, I, K = 12, 1024, 512, 4
     ge = np.stack([synth.q4k_matrix(synth.tensor_seed("moe5-g", e), I, H) for e in range(E)])
     ue = np.stack([synth.q4k_matrix(synth.tensor_seed("moe5-u", e), I, H) for e in range(E)])
@@ -212,8 +212,8 @@ def test_q5k_rejections(ops):
 # ----------------------------------------------------------------------------- matrix-core GEMM (prefill widths)
 @pytest.mark.parametrize("rows,cols,n", [(96, 768, 64), (80, 4096, 50), (272, 2048, 130)])
 def test_q5k_gemm_matches_oracle_and_decode_kernel(ops, rows, cols, n):
-    """Prefill widths of Q5_K: the int8 matrix-core GEMM with a third MFMA chain for the fifth code bits (the second
-    shape splits K into runs).  Against the oracle, against 16-row passes of the decode kernel, and through mq_mul_mat_q4k."""
+    """Prefill widths of Q5_K: the int8 matrix-core GEMM with scale * code cut in two byte digits (the second and third
+    shapes split K into runs).  Against the oracle, against 16-row passes of the decode kernel, and through mq_mul_mat_q4k."""
     import torch
     w_np = synth.q5k_matrix(synth.tensor_seed("pf5-w", rows, cols), rows, cols)
     x = synth.normal_f32(synth.tensor_seed("pf5-x", rows, cols, n), (n, cols))

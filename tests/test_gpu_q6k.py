@@ -174,8 +174,8 @@ def test_q6k_rejections(ops):
 # ----------------------------------------------------------------------------- matrix-core GEMM (prefill widths)
 @pytest.mark.parametrize("rows,cols,n", [(96, 768, 64), (80, 4096, 50), (272, 2048, 130), (1000, 1024, 300)])
 def test_q6k_gemm_matches_oracle_and_decode_kernel(ops, rows, cols, n):
-    """48 rows and more of Q6_K: the int8 matrix-core GEMM with both factors of scale * (code - 32) cut in two digits
-    (five MFMA chains; the second shape splits K into runs, the last has a ragged last row tile).  Against the oracle,
+    """48 rows and more of Q6_K: the int8 matrix-core GEMM with 4 * scale * (code - 32) cut in a high and a signed low byte
+    (two MFMA chains; the second and third shapes split K into runs, the last has a ragged last row tile).  Against the oracle,
     against 16-row passes of the decode kernel, and through mq_mul_mat_q4k."""
     import torch
     w_np = synth.q6k_matrix(synth.tensor_seed("pf6-w", rows, cols), rows, cols)
@@ -193,7 +193,7 @@ def test_q6k_gemm_matches_oracle_and_decode_kernel(ops, rows, cols, n):
 
 def test_q6k_gemm_integer_sums_are_exact(ops):
     """d = 1 and integer activations with a +-127 in every block: the output equals the sum of the oracle's integers,
-    so one wrong unit in any of the five chains, in any digit of any scale or code, changes it."""
+    so one wrong unit in either chain, in either digit of any product, changes it."""
     rows, cols, n = 48, 768, 70
     nb = cols // 256
     w = synth.q6k_matrix(synth.tensor_seed("pf6-int", rows), rows, cols).reshape(rows, nb, 210).copy()
@@ -216,10 +216,12 @@ def test_q6k_gemm_integer_sums_are_exact(ops):
     W.free()
 
 
-@pytest.mark.parametrize("scale,code", [(-128, 0), (-128, 63), (127, 0), (127, 63), (-1, 31), (15, 40), (16, 24), (-16, 7)])
+@pytest.mark.parametrize("scale,code", [(-128, 0), (-128, 63), (127, 0), (127, 63), (-1, 31), (15, 40), (16, 24), (-16, 7),
+                                        (1, 63), (-1, 1), (1, 0), (-1, 0), (2, 48), (-3, 43), (127, 1), (-127, 63)])
 def test_q6k_gemm_extreme_blocks(ops, scale, code):
-    """One scale and one code everywhere -- the corners of both digit pairs (scale + 128 = 0, 255, 143, 144, 112;
-    code = 0, 63 and both sides of the digit boundaries) -- with activations at +-full scale."""
+    """One scale and one code everywhere -- the largest products of either sign, and products 4 * scale * (code - 32) whose low
+    digit is its least (128 modulo 256) or its largest multiple of four (124), both signs, small and large -- with
+    activations at +-full scale."""
     rows, cols, n = 32, 512, 48
     w_np = np.zeros((rows, cols // 256 * 210), np.uint8)
     blocks = w_np.reshape(rows, -1, 210)

@@ -328,8 +328,8 @@ def test_shared_activation_handle_up_to_64_rows(env):
     acts.free(), W.free(), U.free()
 
 
-# ---- Q5_K and Q6_K: one and two tiles of sixteen (Q5_K: a third MFMA chain for the fifth code bits; Q6_K: sixteen
-# K = 32 MFMAs, one per 16-weight scale group, as the passes of eight multiply it) ----
+# ---- Q5_K and Q6_K: one and two tiles of sixteen (Q5_K: a third MFMA chain for the fifth code bits; Q6_K: two
+# chains over the byte digits of 4 * scale * (code - 32)) ----
 
 @pytest.mark.parametrize("wtype", [13, 14])
 @pytest.mark.parametrize("rows,cols", SHAPES)

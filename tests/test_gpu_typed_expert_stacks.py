@@ -2,7 +2,7 @@
 
 The loader admits Q4_K and Q5_K gate/up stacks and Q4_K / Q5_K / Q6_K / Q8_0 down stacks
 (core/src/llm/moe/native.cpp:4611-4620); a Q4_K_M file usually carries Q5_K or Q6_K down experts.  Here gate/up are
-Q5_K (their own kernel instantiations: the fifth code bit in the decode tile, a third MFMA chain in the GEMM) and the
+Q5_K (their own kernel instantiations: the fifth code bit in the decode tile, byte digits of scale * code in the GEMM) and the
 down stack Q5_K or Q6_K, at hidden 2048, 256 experts + 1 shared, intermediate 512, top-8:
 
   n = 1, 4, 8   token-major launches (moe_gateup_token / _slots, moe_down_token / _rows)
@@ -190,7 +190,7 @@ def expected_q5k(w, cols, x):
 def test_q5k_gateup_stacks_integer_sums_are_exact(n):
     """Q5_K gate / up stacks through mq_mul_mat_id_q4k, the gate/up node and the layer's own gate/up launch: products
     exact by construction, the polynomial SiLU a fixed fp32 sequence, so the hidden rows are compared bit for bit.
-    384 tokens over 12 experts: the expert-grouped GEMM with its third MFMA chain (the fp32 update there is fused,
+    384 tokens over 12 experts: the expert-grouped GEMM with its byte digits (the fp32 update there is fused,
     still exact on these operands)."""
     import torch
     from densecore_amd import ops

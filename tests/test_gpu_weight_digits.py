@@ -5,7 +5,7 @@ import pytest
 
 from densecore_amd import synth
 from oracle import binding as orc
-from tests._parity import assert_fp32_parity
+from tests._parity import assert_fp32_parity, gemm_shape
 
 pytestmark = pytest.mark.gpu
 Q5, Q6 = synth.GGML_TYPE_Q5_K, synth.GGML_TYPE_Q6_K
@@ -26,11 +26,12 @@ def cu(a):
 
 @pytest.mark.parametrize("wtype", [Q5, Q6])
 def test_wide_workgroups_match_the_oracle(ops, wtype):
-    """265 row tiles and 69 activation tiles: more 128-row workgroups than compute units, the last of each side ragged.
+    """563 row tiles and 44 activation tiles: more 128-row workgroups than compute units, the last of each side ragged.
     Tokens of the first and the last activation tile against the oracle, all of them against the decode kernels
     (summation order only: the bound of assert_fp32_parity)."""
     import torch
-    rows, cols, n = 4232, 768, 1090
+    rows, cols, n = 9000, 1024, 700
+    assert gemm_shape(wtype, rows, cols, n)["narrow"] == 0
     make, product, dequant = ((synth.q5k_matrix, orc.mul_mat_q5k_q8k, orc.q5k_dot_dequant_f64) if wtype == Q5 else
                               (synth.q6k_matrix, orc.mul_mat_q6k_q8k, orc.q6k_dot_dequant_f64))
     w = make(synth.tensor_seed("wd-w", wtype), rows, cols)
@@ -84,3 +85,27 @@ def test_items_and_pair_of_the_moe_block_give_the_same_bits(ops, wtype):
         assert np.array_equal(y.view(np.uint32), out[0].view(np.uint32))
     for w in (ge, ue, de):
         w.free()
+
+
+@pytest.mark.parametrize("scale,code", [(63, 31), (63, 0), (1, 31), (63, 2), (32, 4), (48, 8), (18, 21), (25, 5)])
+def test_q5k_gemm_corners_of_the_byte_digits(ops, scale, code):
+    """One scale and one code everywhere: the products scale * code = 1953, 0, 31 and those either side of a carry into the high
+    byte (126 and 128, 378 and 384, 125), activations at +-full scale."""
+    rows, cols, n = 32, 512, 70
+    w_np = np.zeros((rows, cols // 256 * 176), np.uint8)
+    blocks = w_np.reshape(rows, -1, 176)
+    blocks[:, :, 0:2] = np.array([0.01], np.float16).view(np.uint8)
+    blocks[:, :, 4:8] = scale | (scale >> 4) << 6   # scales 0..3, and the top bits of scales 4..7
+    blocks[:, :, 12:16] = scale & 15                # mins stay zero
+    blocks[:, :, 16:48] = 255 * (code >> 4)
+    blocks[:, :, 48:176] = (code & 15) * 17
+    x = np.ones((n, cols), np.float32)
+    x[1::2] *= -1.0
+    x[2, ::2] *= -1.0
+    q8 = orc.quantize_rows_q8k(x)
+    ds, md = orc.q5k_matrix_block_sums(w_np, cols, q8)
+    assert np.all(np.abs(ds[:, 0]) == 127 * 256 * scale * code) and not md.any()
+    W = ops.Q4KWeight.from_ggml(w_np, cols, Q5)
+    got = ops.gemm(W, cu(x)).cpu().numpy()
+    assert_fp32_parity(got, orc.mul_mat_q5k_q8k(w_np, cols, q8), orc.q5k_dot_dequant_f64(w_np, cols, q8, magnitude=True), "Q5_K corners")
+    W.free()
