@@ -460,24 +460,25 @@ __global__ void __launch_bounds__(256) prefill_sum_planes_kernel(const float* __
 // and a workgroup walks its super-blocks one after the other, so what counts is how long a workgroup takes and how the workgroups
 // fill the 2 x compute_units() slots.  Pace: us a workgroup takes for t activation tiles and sb super-blocks,
 //     two on a unit  sb (sb2 + tile2 t) + fix2 + store t        one alone  sb (sb1 + tile1 t) + fix1 + store t
-// (fix, store: first tiles, last stores), what all units busy cost on top (load: per tile of a round of slots), and the rounds:
-// r workgroups left after a full round take tail0 + tail1 r / slots of one (the rounds do not start together), and a workgroup
-// beside a shorter one is held up for `beside` of their common time.  Least-squares fits over every shape of 8,700 dense products
-// and 3,300 gate/up pairs (512 to 16,384 rows, 4 to 56 super-blocks, 48 to 2048 tokens; residuals 3 to 5 %), 128-row | 64-row | pair:
+// (fix, store: first tiles, last stores); load: what every unit being busy costs on top, per tile of a round of slots; the workgroups
+// that a full round leaves take later1 / later2 of that (up to one per unit / more: the rounds do not end at one time); a
+// workgroup beside one of x of its length is held up by x^3 of the difference (half as long: an eighth, since the short ones pile up
+// on units of their own first).  Least-squares fits over every shape of 8,650 dense products and 3,270 gate/up pairs (512 to 16,384
+// rows, 4 to 56 super-blocks, 48 to 2048 tokens; residuals 4 and 2.5 %), 128 rows | 64 rows | pair:
 struct Pace {
-    float sb2, tile2, sb1, tile1, fix2, store, fix1, load, tail0, tail1, beside;
+    float sb2, tile2, sb1, tile1, fix2, store, fix1, load, later1, later2;
 };
 enum { kWide, kNarrow, kPairForm };
 constexpr Pace kPace[3][3] = {
-    {{0.880f, 0.222f, 0.530f, 0.190f, 0.78f, 0.118f, 0.65f, 0.151f, 0.337f, 0.733f, 0.415f},   // Q4_K
-     {0.500f, 0.134f, 0.334f, 0.145f, 0.38f, 0.000f, 0.00f, 0.085f, 0.574f, 0.465f, 0.002f},
-     {0.919f, 0.314f, 0.591f, 0.239f, 3.93f, 0.000f, 2.39f, 0.064f, 0.454f, 0.558f, 0.483f}},
-    {{1.609f, 0.220f, 0.916f, 0.181f, 0.53f, 0.078f, 0.71f, 0.160f, 0.271f, 0.757f, 0.767f},   // Q5_K: 16-bit products cost the expansion
-     {0.825f, 0.133f, 0.459f, 0.153f, 0.01f, 0.000f, 0.00f, 0.093f, 0.490f, 0.555f, 0.272f},
-     {1.763f, 0.327f, 1.109f, 0.231f, 2.87f, 0.000f, 1.13f, 0.024f, 0.382f, 0.663f, 0.717f}},
-    {{1.610f, 0.194f, 0.941f, 0.159f, 0.73f, 0.063f, 0.85f, 0.161f, 0.268f, 0.759f, 0.690f},   // Q6_K: no min MFMA
-     {0.874f, 0.111f, 0.476f, 0.121f, 0.13f, 0.000f, 0.00f, 0.083f, 0.396f, 0.635f, 0.580f},
-     {1.782f, 0.290f, 1.119f, 0.209f, 3.32f, 0.000f, 1.25f, 0.039f, 0.394f, 0.677f, 0.723f}}};
+    {{0.870f, 0.267f, 0.505f, 0.213f, 1.07f, 0.020f, 0.81f, 0.112f, 0.815f, 0.973f},   // Q4_K
+     {0.511f, 0.143f, 0.353f, 0.143f, 0.38f, 0.000f, 0.00f, 0.075f, 0.917f, 1.011f},
+     {0.901f, 0.332f, 0.579f, 0.242f, 3.85f, 0.000f, 2.50f, 0.044f, 0.893f, 1.030f}},
+    {{1.565f, 0.263f, 0.898f, 0.198f, 1.20f, 0.024f, 0.92f, 0.138f, 0.768f, 0.941f},   // Q5_K: 16-bit products cost the expansion
+     {0.823f, 0.148f, 0.487f, 0.153f, 0.34f, 0.002f, 0.00f, 0.080f, 0.893f, 1.004f},
+     {1.721f, 0.323f, 1.050f, 0.233f, 2.85f, 0.000f, 0.93f, 0.037f, 0.891f, 1.015f}},
+    {{1.626f, 0.230f, 0.956f, 0.177f, 1.19f, 0.021f, 0.70f, 0.129f, 0.763f, 0.938f},   // Q6_K: no min MFMA
+     {0.897f, 0.121f, 0.480f, 0.122f, 0.28f, 0.000f, 0.00f, 0.071f, 0.868f, 0.988f},
+     {1.759f, 0.285f, 1.061f, 0.211f, 3.10f, 0.000f, 0.95f, 0.051f, 0.916f, 1.029f}}};
 
 GemmShape shape_of(int form, int64_t rows, int64_t nb, int64_t m_tiles, int64_t t, int64_t splits) {
     const int64_t rowtiles = (rows + 15) / 16;
@@ -490,55 +491,62 @@ GemmShape shape_of(int form, int64_t rows, int64_t nb, int64_t m_tiles, int64_t 
 }
 
 // us of a launch, its planes included
-float shape_us(const Pace& p, const GemmShape& s, int64_t rows, int64_t m_tiles, int64_t n) {
+float shape_us(const Pace& p, const GemmShape& s, int64_t rows, int64_t nb, int64_t m_tiles, int64_t n) {
     const int64_t units = compute_units(), slots = 2 * units;
-    const int64_t t = s.tiles_per_wg, t_last = m_tiles - (int64_t)(s.groups - 1) * t, column = (int64_t)s.row_wgs * s.splits;
-    const float sb = (float)s.sb_split;
-    auto two = [&](int64_t k) { return sb * (p.sb2 + p.tile2 * (float)k) + p.fix2 + p.store * (float)k; };
-    auto one = [&](int64_t k) {
-        const float v = sb * (p.sb1 + p.tile1 * (float)k) + p.fix1 + p.store * (float)k;
-        return v < two(k) ? v : two(k);
+    const double per_slot = 1.0 / (double)slots;
+    auto rounds = [&](int64_t x) { return (int64_t)(((double)x + 0.5) * per_slot); };  // x / slots without a division
+    const int64_t t = s.tiles_per_wg, sb = s.sb_split, wgs = (int64_t)s.row_wgs * s.groups * s.splits;
+    auto two = [&](int64_t b, int64_t k) { return (float)b * (p.sb2 + p.tile2 * (float)k) + p.fix2 + p.store * (float)k; };
+    auto one = [&](int64_t b, int64_t k) {
+        const float v = (float)b * (p.sb1 + p.tile1 * (float)k) + p.fix1 + p.store * (float)k, w = two(b, k);
+        return v < w ? v : w;
     };
-    auto last_round = [&](int64_t r, bool first, int64_t k) {  // r < slots workgroups of k tiles
+    auto rest = [&](int64_t r, bool later, int64_t b, int64_t k) {  // r < slots workgroups that a full round leaves, or the only ones
         if (r == 0) return 0.0f;
-        if (first) return r <= units ? one(k) : two(k);
-        const float part = p.tail0 + p.tail1 * (float)r / (float)slots;
-        return two(k) * (part < 1.2f ? part : 1.2f);
+        return r <= units ? (later ? p.later1 : 1.0f) * one(b, k) : (later ? p.later2 : 1.0f) * two(b, k);
     };
-    float us;
-    if (t_last == t || s.groups == 1 || s.splits > 1) {
-        const int64_t wgs = column * s.groups, full = wgs / slots;
-        us = (float)full * two(t) + last_round(wgs % slots, full == 0, t);
-    } else {  // the short column comes last and fills what the last round leaves
-        const int64_t wgs = column * (s.groups - 1), full = wgs / slots, r = wgs % slots, spare = slots - r;
-        us = (float)full * two(t);
-        const float shorter = two(t_last);
-        if (r == 0) {
-            us += (float)(column / slots) * shorter + last_round(column % slots, full + column / slots == 0, t_last);
-        } else if (column <= spare) {
-            if (full > 0) us += last_round(r + column, false, t);
-            else if (r > units) us += two(t);
-            else us += one(t) + (r + column > units ? (two(t) - one(t)) * p.beside * (shorter < two(t) ? shorter / two(t) : 1.0f) : 0.0f);
+    // dispatched last, and shorter: the last run of an uneven K split, else the last column
+    const int64_t b_last = s.splits > 1 ? nb - (s.splits - 1) * sb : sb, t_last = s.splits > 1 ? t : m_tiles - (int64_t)(s.groups - 1) * t;
+    const int64_t shorter = wgs > (int64_t)s.row_wgs && (b_last < sb || t_last < t) ? (int64_t)s.row_wgs * (s.splits > 1 ? s.groups : 1) : 0;
+    const int64_t full = rounds(wgs - shorter), r = wgs - shorter - full * slots, spare = slots - r;
+    const float l2 = two(sb, t);
+    float us = (float)full * l2;
+    if (shorter == 0) {
+        us += rest(r, full > 0, sb, t);
+    } else if (r == 0) {
+        const int64_t more = rounds(shorter);
+        us += (float)more * two(b_last, t_last) + rest(shorter - more * slots, true, b_last, t_last);
+    } else {
+        const float s2 = two(b_last, t_last);
+        if (shorter <= spare) {
+            const float l1 = one(sb, t), s1 = one(b_last, t_last);
+            const float x = s2 < l2 ? s2 / l2 : 1.0f;
+            float tail = r > units ? l2 : r + shorter > units ? l1 + (l2 - l1) * x * x * x : l1;
+            if (full > 0) tail *= r > units ? p.later2 : p.later1;
+            us += tail > s1 ? tail : s1;
         } else {
-            const float chain = (float)((column + spare - 1) / spare) * shorter;
-            int64_t beside = (int64_t)(two(t) / shorter);
+            const float chain = (float)((shorter + spare - 1) / spare) * s2;
+            int64_t beside = (int64_t)(l2 / s2);
             beside = (beside < 1 ? 1 : beside) * spare;
-            const int64_t left = column > beside ? column - beside : 0;
-            const float after = two(t) + (float)(left / slots) * shorter + last_round(left % slots, false, t_last);
+            const int64_t left = shorter > beside ? shorter - beside : 0;
+            const int64_t more = rounds(left);
+            const float after = l2 + (float)more * s2 + rest(left - more * slots, true, b_last, t_last);
             const float tail = chain < after ? chain : after;
-            us += tail > two(t) ? tail : two(t);
+            us += tail > l2 ? tail : l2;
         }
     }
-    us += p.load * sb * (float)(column * m_tiles) / (float)slots;
-    if (s.splits > 1) us += 2.8f + 0.064f * 8e-6f * (float)s.splits * (float)(n * rows);  // a launch, the planes written and read
+    us += p.load * (float)(sb * s.splits) * (float)((int64_t)s.row_wgs * m_tiles) / (float)slots;
+    if (s.splits > 1) us += 2.8f + 0.55e-6f * (float)s.splits * (float)(n * rows);  // a launch, the planes written and read
     return us;
 }
 
 // The plain shape -- 64-row workgroups up to one 128-row workgroup per unit, tiles in eights, K in as many runs as fill the slots --
-// unless the estimate gives another one at least 6 % less (its own error).  Best of every shape / plain / estimate alone / with the
-// 6 %, mean over the fitted Q4_K products: 1 / 1.12 / 1.010 / 1.012; slower than plain by over 3 %: 3 % / 0.5 % of them, at most 1.16 / 1.13.
+// unless the estimate of another one is less by kLess.  Over the fitted products Q4_K / Q5_K / Q6_K the chosen shape takes 1.007 /
+// 1.010 / 1.009 of the fastest one's time (pairs 1.003 / 1.002 / 1.003), the plain shape 1.115 / 1.094 / 1.080 (pairs 1.16 / 1.12 /
+// 1.11); the choice is over 5 % slower than plain on 0.2 / 0.5 / 1.2 % of the products, 0.4 / 1.0 / 1.4 % at a kLess of 0.98.
 // 4096 x 14336 at 130 / 391 / 700 / 1200 rows against the plain shape, with quantizer and planes: 46 / 84 / 145 / 245 ->
-// 37 / 75 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 70 / 109.
+// 37 / 70 / 119 / 203 us, 14336 x 4096 at 130 / 391 / 700 39 / 74 / 116 -> 31 / 67 / 109.
+constexpr float kLess = 0.97f, kLessPair = 0.95f;
 GemmShape choose_shape(const Pace* pace, bool pair, int64_t rows, int64_t nb, int64_t n) {
     const int64_t units = compute_units(), m_tiles = (n + 15) / 16, rowtiles = (rows + 15) / 16;
     const int64_t most = m_tiles < kMTilesPerGroup ? m_tiles : kMTilesPerGroup, min_groups = (m_tiles + kMTilesPerGroup - 1) / kMTilesPerGroup;
@@ -547,7 +555,7 @@ GemmShape choose_shape(const Pace* pace, bool pair, int64_t rows, int64_t nb, in
     GemmShape plain = shape_of(plain_form, rows, nb, m_tiles, most, 1);
     const int64_t fill = 2 * units / ((int64_t)plain.row_wgs * plain.groups), runs = fill < nb / 4 ? fill : nb / 4;
     if (!pair && !(rows & 3) && runs > 1) plain = shape_of(plain_form, rows, nb, m_tiles, most, runs);
-    plain.us = shape_us(pace[plain_form], plain, rows, m_tiles, n);
+    plain.us = shape_us(pace[plain_form], plain, rows, nb, m_tiles, n);
     GemmShape best = plain;
     for (int form = pair ? kPairForm : kWide; form <= (pair ? kPairForm : kNarrow); ++form) {
         const Pace& p = pace[form];
@@ -561,14 +569,14 @@ GemmShape choose_shape(const Pace* pace, bool pair, int64_t rows, int64_t nb, in
                 s.sb_split = ((int)nb + sp - 1) / sp, s.splits = ((int)nb + s.sb_split - 1) / s.sb_split;
                 // (no longer than the best so far even as workgroups alone; a count that leaves no empty run)
                 if ((float)s.sb_split * (p.sb1 + p.tile1 * (float)t) < best.us && s.splits == sp) {
-                    s.us = shape_us(p, s, rows, m_tiles, n);
+                    s.us = shape_us(p, s, rows, nb, m_tiles, n);
                     if (s.us < best.us) best = s;
                 }
                 if ((int64_t)s.row_wgs * s.groups * sp > 4 * units) break;  // two rounds and more: further runs only add planes
             }
         }
     }
-    return best.us <= 0.94f * plain.us ? best : plain;
+    return best.us <= (pair ? kLessPair : kLess) * plain.us ? best : plain;
 }
 
 // ---- expert-grouped GEMM: the plan ------------------------------------------------------------------------
@@ -797,7 +805,7 @@ bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* 
     if (!gemm_type(wtype) || rows <= 0 || n <= 0) return false;
     *shape = choose_shape(kPace[pace_of(wtype)], true, rows, nb, n);
     const float out = 1e-6f * (float)(n * rows), one_launch = shape->us + 0.25f * out;
-    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 9.0f + 3.3f * out;
+    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 8.5f + 3.15f * out;
     return two_launches + 8.0f >= 0.94f * (one_launch + 8.0f);
 }
 

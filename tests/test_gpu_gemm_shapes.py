@@ -32,10 +32,10 @@ MAKE = {12: (synth.q4k_matrix, lambda *a: orc.mul_mat_q4k_q8k(*a, orc.ORDER_SCAL
     (2050, 4096, 260, (1, 1, 16, 3, 6)),     # 64 rows, ragged rows, 17 tiles dealt in threes
     (9000, 512, 400, (1, 1, 2, 8, 4)),       # a short K, in eights with a last column of one tile
     (14336, 1024, 512, (0, 1, 4, 8, 4)),     # 128 rows
-    (9000, 1024, 700, (0, 1, 4, None, None)),  # 128 rows, ragged rows and a short last column
-    (4096, 14336, 130, (0, 8, 7, 5, 2)),     # 128 rows with K in runs, nine tiles as 5 + 4
-    (4096, 14336, 260, (0, 5, 12, 6, 3)),    # ... 56 super-blocks as 12 + 12 + 12 + 12 + 8
-    (4096, 14336, 391, (0, 4, 14, 7, 4))])   # ... 25 tiles as 7 + 7 + 7 + 4
+    (13000, 1024, 505, (0, 1, 4, 7, 5)),     # 128 rows, ragged rows, 32 tiles as 7 + 7 + 7 + 7 + 4
+    (4096, 14336, 130, {14: (1, 4, 14, 5, 2), 0: (0, 8, 7, 5, 2)}),  # K in runs over 128 rows (Q6_K: 64), nine tiles as 5 + 4
+    (4096, 14336, 330, {13: (0, 8, 7, 7, 3), 14: (1, 5, 12, 7, 3), 0: (0, 5, 12, 7, 3)}),  # ... 56 super-blocks as 12 x 4 + 8
+    (4096, 14336, 391, (0, 4, 14, 7, 4))])   # ... 25 tiles as 7 + 7 + 7 + 4, all three types over 128 rows
 def test_gemm_shape(ops, wtype, rows, cols, n, form):
     import torch
     make, product, magnitude = MAKE[wtype]
@@ -43,8 +43,9 @@ def test_gemm_shape(ops, wtype, rows, cols, n, form):
     x = synth.normal_f32(synth.tensor_seed("gs-x", n, cols), (n, cols))
     W = ops.Q4KWeight.from_ggml(w, cols, wtype)
     s = gemm_shape(wtype, rows, cols, n)
-    for name, want in zip(("narrow", "runs", "sb_run", "tiles", "columns"), form):
-        assert want is None or s[name] == want, s
+    if isinstance(form, dict):
+        form = form.get(wtype, form[0])
+    assert tuple(s[name] for name in ("narrow", "runs", "sb_run", "tiles", "columns")) == form, s
     xd = torch.from_numpy(x).cuda()
     yp = torch.full((n, rows + 8), 7.0, device="cuda")  # a padded output keeps its padding
     ops.gemm(W, xd, out=yp[:, :rows])
@@ -59,7 +60,7 @@ def test_gemm_shape(ops, wtype, rows, cols, n, form):
     W.free()
 
 
-@pytest.mark.parametrize("rows,n,tiles", [(2064, 65, 1), (2064, 129, 2), (2064, 144, 2), (2064, 393, 4), (5648, 391, 5), (2064, 700, 7), (11008, 200, 8), (11008, 330, 8)])
+@pytest.mark.parametrize("rows,n,tiles", [(2064, 65, 1), (2064, 129, 2), (2064, 144, 2), (2064, 393, 4), (5648, 391, 5), (11008, 330, 5), (2064, 700, 7), (11008, 200, 8), (14336, 330, 8)])
 def test_pair_launch_columns(ops, rows, n, tiles):
     """Gate and up in one launch: tiles dealt evenly, and in eights with a short last column (thirteen as 8 + 5, 21 as 8 + 8 + 5).
     No K runs at 1024 columns, so the two launches and the SwiGLU pass give the same bits."""

@@ -26,11 +26,11 @@ def cu(a):
 
 @pytest.mark.parametrize("wtype", [Q5, Q6])
 def test_wide_workgroups_match_the_oracle(ops, wtype):
-    """563 row tiles and 44 activation tiles: more 128-row workgroups than compute units, the last of each side ragged.
+    """813 row tiles and 32 activation tiles: more 128-row workgroups than compute units, the last of each side ragged.
     Tokens of the first and the last activation tile against the oracle, all of them against the decode kernels
     (summation order only: the bound of assert_fp32_parity)."""
     import torch
-    rows, cols, n = 9000, 1024, 700
+    rows, cols, n = 13000, 1024, 505
     assert gemm_shape(wtype, rows, cols, n)["narrow"] == 0
     make, product, dequant = ((synth.q5k_matrix, orc.mul_mat_q5k_q8k, orc.q5k_dot_dequant_f64) if wtype == Q5 else
                               (synth.q6k_matrix, orc.mul_mat_q6k_q8k, orc.q6k_dot_dequant_f64))
