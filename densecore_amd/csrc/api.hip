@@ -191,7 +191,7 @@ bool dense_lds_quantizes(const mq_weight* w, const float* x, int64_t n, int64_t 
            dense_lds_applies(w->nb, w->rowtiles, n, swiglu, w->type);
 }
 
-// Nine to 64 rows of a Q4_K matrix: one to four activation tiles of sixteen rows per weight tile
+// Nine to 64 rows of a Q4_K, Q5_K or Q6_K matrix: one to four activation tiles of sixteen rows per weight tile
 // (skinny16_kernel, the same bits as the token tiles of eight of the other decode kernels); mq_debug_set_dense_lds
 // bit 12 turns it off.  kSkinnyMaxRows: beyond it the matrix-core GEMM (large matrices) or the 16-row passes of the
 // decode kernels take over.
@@ -575,8 +575,9 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // at 47; 4096 x 4096: 17.4 against 14.1 us at 17 rows, 17.9 against 14.6 at 47).  Q4_K products of up to 32 rows go to
 // skinny16_kernel ahead of both (skinny16_takes: gate/up of a 4096 -> 14336 FFN 41 -> 22 us at 17 to 32 rows,
 // 4096 x 4096 11.5 -> 9.5 us).  The 17-row rule holds for Q5_K and Q6_K matrices of that many weights as well (4096 x
-// 14336: Q5_K 28.7 / 30.7 / 42.5 us in 16-row passes against 22.3 / 22.6 / 25.3 on the GEMM at 17 / 32 / 47 rows, Q6_K 30.7 /
-// 33.2 / 46.3 against 28.2 / 28.5 / 32.3; 4096 x 4096 stays: 12.1 against 14.1 us at 17 rows, 16.8 against 15.9 at 47).
+// 14336 in 16-row passes at 17 / 32 / 47 rows: Q5_K 28.7 / 30.7 / 42.5 us, Q6_K 30.7 / 33.2 / 46.3; on the GEMM with two chains of
+// byte digits 21.7 / 21.8 / 23.9 and 21.8 / 21.9 / 23.9, where skinny16_kernel takes up to 32 rows first, in 18.5 to 19.1).
+// For 4096 x 4096 only Q6_K at 33 to 47 rows still gets here: 15.6 / 15.9 us in passes at 33 / 47 rows, 14.1 / 14.3 on the GEMM.
 constexpr int64_t kPrefillMinRows = 48;
 constexpr int64_t kPrefillMinRowsLarge = 17;
 constexpr int64_t kPrefillLargeBytes = 24ll << 20;
@@ -1546,7 +1547,7 @@ int mq_acts_quantize(mq_acts* a, const float* x_dev, int64_t n, int64_t ldx, voi
     a->tile16 = false;
     if (n == 0) return MQ_OK;
     MQ_HIP(launch_quantize_q8k(x_dev, n, ldx, a->cols, nullptr, 0, (uint8_t*)a->aq, (float*)a->ad, (hipStream_t)stream));
-    // nine to 64 rows: their tiles of sixteen as well, for the Q4_K products that take them (skinny16_takes)
+    // nine to 64 rows: their tiles of sixteen as well, for the products that take them (skinny16_takes)
     a->tile16 = n > 8 && n <= kSkinnyMaxRows && a->ap;
     if (a->tile16) MQ_HIP(launch_quantize_q8k_pmajor(x_dev, n, ldx, a->cols, (uint8_t*)a->ap, (hipStream_t)stream));
     return MQ_OK;

@@ -36,7 +36,7 @@ struct MatmulArgs {
     size_t expert_bytes = 0;       // tiled bytes per expert (grouped mode)
     const uint8_t* aq = nullptr;   // A-major activations
     const float* ad = nullptr;
-    // dense mode, nine to sixteen rows of a Q4_K matrix: the rows as one P-major tile per super-block instead (skinny16_kernel)
+    // dense mode, nine to 64 rows: the rows as one to four P-major tiles per super-block instead (skinny16_kernel)
     const uint8_t* ap = nullptr;
     // dense mode, n == 1: the activation row as fp32 instead; every wavefront quantizes the super-blocks it
     // multiplies (same codes and scales as the stand-alone quantizer, so the same result)
@@ -123,9 +123,9 @@ hipError_t launch_dense_lds(const DenseLdsArgs& a, hipStream_t stream, hipEvent_
 // Wavefronts per row tile of the LDS-staged dense kernels for a matrix (pick_waves, as a divisor of eight; 0: none)
 int dense_lds_wpr(int64_t nb, int64_t rowtiles);
 
-// ---- skinny16.hip: nine to sixteen rows as ONE activation tile against a streamed Q4_K matrix (skinny16_kernel) ----
+// ---- skinny16.hip: nine to 64 rows as one to four activation tiles against a streamed matrix (skinny16_kernel) ----
 struct Skinny16Args {
-    const uint8_t* w0 = nullptr;   // tiled Q4_K weights; gate when w1 is set
+    const uint8_t* w0 = nullptr;   // tiled weights; gate when w1 is set
     const uint8_t* w1 = nullptr;   // up weights: y = silu(w0 x) * (w1 x)
     int64_t rows = 0, nb = 0;
     const uint8_t* ap = nullptr;   // the rows' P-major tiles: [nb][tiles][4688], tiles = ceil(n / 16) (launch_quantize_q8k_pmajor)
@@ -133,7 +133,7 @@ struct Skinny16Args {
     float* y = nullptr;
     int64_t ldy = 0;
     int silu_mode = 0;
-    int wtype = kTypeQ4K;          // kTypeQ4K, or kTypeQ5K / kTypeQ6K (one and two tiles)
+    int wtype = kTypeQ4K;          // kTypeQ4K, kTypeQ5K or kTypeQ6K
     int ranges = 1;                // set by the launcher: runs of super-blocks the tiles pass through LDS in
 };
 bool skinny16_applies(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n, int wtype = kTypeQ4K);
@@ -243,7 +243,7 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
 int64_t moe_gemm_tiles_max(int64_t entries, int64_t groups_max);
 int64_t moe_gemm_items_max(int64_t entries, int64_t groups_max);
 size_t moe_gemm_plan_ints(int64_t entries, int64_t groups_max);
-// activation tiles per item (2 or 8) of an expert-grouped launch over `entries` rows in `groups` groups: the plan and
+// activation tiles per item (2, 4 or 8) of an expert-grouped launch over `entries` rows in `groups` groups: the plan and
 // every launch that reads it take the same value
 int moe_gemm_item_tiles(int64_t entries, int64_t groups);
 hipError_t launch_moe_gemm_plan(const int32_t* n_groups, const int32_t* group_expert, const int32_t* group_begin,

@@ -23,7 +23,6 @@ typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 

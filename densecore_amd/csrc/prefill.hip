@@ -23,11 +23,11 @@
 // grouping (d*yd) * dot_scaled - (dmin*yd) * min_dot takes four, and the update is what the kernel's vector unit is
 // busy with: 308 against 325 us at M = 2048; the two groupings differ in the last bits only).
 //
-//   grid      = (ceil(rowtiles / 8), ceil(m_tiles / 8)); workgroup = 4 wavefronts
-//   workgroup = 128 weight rows x 128 activation rows; per super-block the 128 activation rows (37 KB
-//               in the P-major layout below) are staged in LDS, double-buffered and requested one
-//               super-block ahead with LDS-direct loads
-//   wavefront = 2 weight tiles (32 rows) x the 8 activation tiles; it reads its weight tiles
+//   grid      = (row_wgs, groups, splits) of the shape that choose_shape takes; workgroup = 4 wavefronts
+//   workgroup = 128 or 64 weight rows x up to 128 activation rows (tiles_per_wg tiles) x all super-blocks or a run of them;
+//               per super-block the activation rows (up to 37 KB in the P-major layout) are staged in LDS, double-buffered
+//               and requested one super-block ahead with LDS-direct loads
+//   wavefront = 2 weight tiles (32 rows; 64-row workgroups: 1) x the activation tiles; it reads its weight tiles
 //               straight from HBM in MFMA lane order and expands them in registers
 //
 // The activations come in the P-major layout (pmajor.h).
@@ -738,7 +738,8 @@ int moe_gemm_item_tiles(int64_t entries, int64_t groups) {
     // item larger than its expert's rows holds accumulators and LDS for tiles that do not exist, and a compute unit
     // then holds fewer workgroups.  MoE block of 256 + 1 experts, top-8, 2048 x 512, items of 2 / 4 / 8 tiles: 162 / 172 /
     // 209 us at 384 tokens (13 rows per expert), 173 / 181 / 219 at 512, 195 / 203 / 239 at 768, 236 / 224 / 260 at 1024
-    // (36 rows), 315 / 276 / 311 at 1536, 385 / 356 / 364 at 2048 (72 rows), 686 / 612 / 615 at 4096.
+    // (36 rows), 315 / 276 / 311 at 1536, 385 / 356 / 364 at 2048 (72 rows), 686 / 612 / 615 at 4096.  Swept on Q4_K; the other types take
+    // the same items.
     if (groups <= 0) return kMTilesPerGroup;
     return entries <= 30 * groups ? kMTilesSmall : entries <= 160 * groups ? kMTilesMid : kMTilesPerGroup;
 }

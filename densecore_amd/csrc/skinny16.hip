@@ -11,7 +11,7 @@ namespace mq {
 
 namespace {
 
-// ---- nine to sixteen activation rows against a streamed matrix ------------------------------------------------
+// ---- nine to 64 activation rows against a streamed matrix ------------------------------------------------
 // The decode kernels multiply a weight tile with EIGHT activation rows per MFMA (the sixteen operand rows hold a row's
 // two sub-blocks of a 64-weight chunk side by side, the sub-block scales are applied on the vector unit); from nine rows
 // they take two such token tiles per weight tile: 16 MFMAs and ~147 vector instructions.  This kernel multiplies the
@@ -37,7 +37,7 @@ struct ATile16 {
     v8h dg;     // this lane's operand of the min MFMA (fp16 digits of the sub-block sums, or zeros)
 };
 
-// MT: activation tiles of sixteen rows (one, or two for 17 to 32 rows: the weight tile is expanded once for both, 18
+// MT: activation tiles of sixteen rows (one to four, e.g. two for 17 to 32 rows: the weight tile is expanded once for both, 18
 // MFMAs and ~156 vector instructions against the 32 + 294 of two passes over two token tiles of eight each).  With two
 // tiles the partial sums share LDS with the activation tiles (one more barrier before they are written).
 template <int NMAT, int WPR, int FLOW, bool GA, int MT, int WT = kWtQ4>
@@ -343,12 +343,16 @@ hipError_t launch_skinny16_one(const Skinny16Args& a, int ranges, hipStream_t st
 }
 
 // MT <= 2: the rows' tiles in LDS (in runs if need be), else from global memory a stage ahead; three and four tiles only
-// from LDS (read a stage ahead they do not fit the registers), an even number of stages per wavefront.
+// from LDS (read a stage ahead they do not fit the registers).  Left out for their registers (256 and four to twelve
+// spilled): pairs of four tiles with eight wavefronts per row tile, Q5_K and Q6_K pairs of two tiles read a stage ahead.  Not
+// built although they would fit (106 to 240 registers, nothing spilled; not timed): Q6_K in runs of an odd number of stages and
+// Q6_K pairs with one wavefront per row tile, which spilled while Q6_K multiplied by scale groups, and the Q5_K pair of four
+// tiles in runs of an odd number of stages.
 template <int NMAT, int WPR, int MT, int WT>
 hipError_t launch_skinny16_form(const Skinny16Args& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
     const bool odd = ((a.nb / WPR) & 1) != 0;
     const int ranges = odd ? (skinny16_lds_bytes(NMAT, WPR, a.nb, MT, 1) <= kSkinnyLdsMax ? 1 : 0) : skinny16_ranges(NMAT, WPR, a.nb, MT);
-    // (the forms left out below spill registers -- skinny16_applies knows them)
+    // (skinny16_applies knows the forms that are not built)
     if constexpr (WT == kWtQ6 && NMAT == 2 && WPR == 1) {
         return hipErrorInvalidValue;
     } else if constexpr (MT <= 2) {
@@ -413,7 +417,7 @@ hipError_t launch_skinny16_tiles(const Skinny16Args& a, int wpr, hipStream_t str
 
 // Whether a product of n rows (nine to 64) runs on skinny16_kernel: the wave split of the other decode kernels must be
 // one of its own (a divisor of eight that divides the super-blocks of a row), and the form must be built
-// (launch_skinny16_form returns an error for the others: those whose registers spill).
+// (launch_skinny16_form returns an error for the others).
 //   One and two tiles (up to 32 rows): always; the two tiles of a Q5_K or Q6_K gate/up pair only where they fit LDS in
 //   one run; a Q6_K pair not with one wavefront per row tile.
 //   Three and four tiles: not with one wavefront per row tile (more than 1,024 row tiles: the GEMM is faster from 33
