@@ -622,7 +622,7 @@ static int ffn_wide_locked(const mq_weight* gate, const mq_weight* up, const mq_
     MQ_HIP(g.ap.reserve(pmajor_bytes(n, gate->nb)));
     MQ_HIP(launch_quantize_q8k_pmajor(x_dev, n, ldx, gate->cols, (uint8_t*)g.ap.ptr, s));
     GemmShape pair;
-    if (g_gemm_pair && gate->type == up->type && gemm_pair_shape(gate->type, inter, gate->nb, n, &pair)) {
+    if (g_gemm_pair && gate->type == up->type && gemm_pair_shape(gate->type, inter, gate->nb, n, down != nullptr, &pair)) {
         // gate and up in one launch that stores silu(gate) * up: no fp32 planes, no pass that reads them back
         MQ_HIP(launch_prefill_gemm_pair(gate->data, up->data, gate->type, inter, gate->nb, (const uint8_t*)g.ap.ptr, n, silu_mode, h_dev, ldh, pair, s));
         if (!down) return MQ_OK;
@@ -2092,7 +2092,7 @@ int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
         return fail(MQ_ERR_INVALID, "mq_debug_gemm_shape: bad type, size or pointer");
     GemmShape s;
     bool taken = true;
-    if (pair) taken = gemm_pair_shape(wtype, rows, cols / kQK, n, &s);
+    if (pair) taken = gemm_pair_shape(wtype, rows, cols / kQK, n, pair == 2, &s);
     else s = gemm_shape(wtype, rows, cols / kQK, n);
     shape_out[0] = s.narrow, shape_out[1] = s.splits, shape_out[2] = s.sb_split, shape_out[3] = s.tiles_per_wg;
     shape_out[4] = (int)s.row_wgs, shape_out[5] = (int)s.groups, shape_out[6] = taken, shape_out[7] = (int)(1000.0f * s.us);

@@ -226,8 +226,9 @@ size_t gemm_part_bytes(const GemmShape& shape, int64_t rows, int64_t n);
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
                                int64_t ldy, float* part, const GemmShape& shape, hipStream_t stream);
 // silu(gate . x) * (up . x) from ONE launch (prefill.hip: the pair form of the GEMM kernel), dense and expert-grouped.
-// gemm_pair_shape: false where two products and a SwiGLU pass are the better choice.
-bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* shape);
+// gemm_pair_shape: false where two products and a SwiGLU pass are the better choice (then_quantized: that pass also quantizes its rows
+// for a down product, which the pair launch leaves to a launch of its own).
+bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, bool then_quantized, GemmShape* shape);
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,
                                     int64_t n, int silu_mode, float* h, int64_t ldh, const GemmShape& shape, hipStream_t stream);
 hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t expert_bytes,

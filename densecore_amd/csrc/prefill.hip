@@ -802,12 +802,15 @@ GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n) { return ch
 // The pair form: h[tok][row] = silu(gate[row] . x[tok]) * (up[row] . x[tok]).  It has no K split (SiLU is not linear): for a few rows of
 // a long K two launches with K in runs and the SwiGLU pass over their planes are faster, by up to half (1 to 4 % of the fitted
 // pairs); taken where the estimate, with 8 us of quantizer on both sides, says so by 6 % (then never slower by more than 5 %).
-bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, GemmShape* shape) {
+// In an FFN (then_quantized) the SwiGLU pass of two launches is the down product's quantizer, which the pair form adds: 4 us and
+// more, compared as it is.  Of 7,650 random FFNs (17 to 1200 rows) the pair lost over 2 % on 89 without that, up to 9 % (Q5_K
+// 4608 -> 10496 at 17 rows 61.0 against 56.0 us); with it the choice does on 15 of 7,490, at most 7 %.
+bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, bool then_quantized, GemmShape* shape) {
     if (!gemm_type(wtype) || rows <= 0 || n <= 0) return false;
     *shape = choose_shape(kPace[pace_of(wtype)], true, rows, nb, n);
-    const float out = 1e-6f * (float)(n * rows), one_launch = shape->us + 0.25f * out;
-    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 8.5f + 3.15f * out;
-    return two_launches + 8.0f >= 0.94f * (one_launch + 8.0f);
+    const float out = 1e-6f * (float)(n * rows), one_launch = shape->us + 0.25f * out + 8.0f;
+    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 8.5f + 3.15f * out + 8.0f;
+    return two_launches >= (then_quantized ? one_launch + 4.0f + 0.82f * out : 0.94f * one_launch);
 }
 
 hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int wtype, int64_t rows, int64_t nb, const uint8_t* ap,

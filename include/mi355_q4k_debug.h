@@ -67,7 +67,7 @@ int mq_census_read(int kind, double* avg_us, double* min_us, double* max_us, int
  * previous setting of bit 0.  No counterpart in the reference. */
 int mq_debug_set_dense_lds(int on);
 
-/* Launch shape that the matrix-core GEMM takes for a product of n rows (pair != 0: for gate and up in one launch), for a 256-unit
+/* Launch shape that the matrix-core GEMM takes for a product of n rows (pair 1: for gate and up in one launch, 2: ahead of a down product), for a 256-unit
  * device before mq_init.  shape_out: 64-row workgroups (1) or 128-row ones (0), runs of K, super-blocks per run, activation tiles per
  * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns. */
 int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);

@@ -61,6 +61,13 @@ def test_one_more_row_changes_little(rows, cols):
         before = now
 
 
+@pytest.mark.parametrize("wtype,rows,cols,n", [(Q5, 10496, 4608, 17), (Q5, 9472, 4608, 68), (Q6, 8960, 4352, 101), (Q5, 10752, 5120, 29)])
+def test_an_ffn_counts_the_quantizer_that_the_pair_adds(wtype, rows, cols, n):
+    """Whole FFN with two launches | with the pair launch: 56.0 | 61.0, 70.5 | 76.2, 80.0 | 86.2, 57.3 | 62.2 us."""
+    assert shape(wtype, rows, cols, n, 2)["taken"] == 0
+    assert shape(wtype, rows, cols, 700, 2)["taken"] == 1
+
+
 @pytest.mark.parametrize("wtype,n", [(Q4, 42), (Q5, 38), (Q5, 134), (Q6, 97), (Q6, 139)])
 def test_few_rows_of_a_long_k_take_two_launches(wtype, n):
     """Gate and up of 4096 x 14336: two launches with K in runs against the one that cannot split it, 44.0 | 62.3, 48.6 | 89.4,
