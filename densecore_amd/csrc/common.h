@@ -165,6 +165,26 @@ constexpr uint64_t kScaleStream = 0x5CA1E5CA1E5CA1E5ull;
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// LDS-direct copies: lane l of the wavefront copies kBytes (4 or 16) from its address -- one per lane, or a scalar base and the lane's
+// offset -- to lds + kBytes * l, lds being the wave-uniform LDS byte address in M0.  The instruction offset stays 0 (the hardware adds it
+// to the global address as well).  Written as inline assembly on purpose: the compiler then does not know that LDS is written, and so
+// does not make every later LDS read wait for these requests; the kernels wait for them themselves, with vmcnt and a barrier.  The s_nop
+// is the wait state that the hardware needs between a write of M0 and an LDS-direct load and that the compiler cannot put into a
+// statement of ours: without it a request may go to the address of the request before it.
+template <int kBytes>
+__device__ __forceinline__ void lds_direct(const void* lane_src, uint32_t lds) {
+    static_assert(kBytes == 4 || kBytes == 16, "a dword or four");
+    if constexpr (kBytes == 16) asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_src), "s"(lds) : "memory", "m0");
+    else asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(lane_src), "s"(lds) : "memory", "m0");
+}
+template <int kBytes>
+__device__ __forceinline__ void lds_direct(const uint8_t* base, uint32_t lane_off, uint32_t lds) {
+    static_assert(kBytes == 4 || kBytes == 16, "a dword or four");
+    if constexpr (kBytes == 16) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
+}
 
 __device__ __forceinline__ float half_bits_to_float(uint32_t h16) {
     return __half2float(__ushort_as_half((unsigned short)h16));

@@ -28,8 +28,6 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
 // four bytes (each <= 15) times a 3-bit digit, bytewise: two 16-bit products whose bytes do not carry into each
 // other (15 * 7 < 256).  The digit is half H of `digits`, taken for both products (the operand-select bits of the
 // packed multiply: no instruction of its own).
@@ -56,26 +54,22 @@ __device__ __forceinline__ v8h mins_to_half(uint32_t mn03, uint32_t mn47) {
     return v8h{m01.x, m01.y, m23.x, m23.y, m45.x, m45.y, m67.x, m67.y};
 }
 
-// The four wavefronts of a workgroup request activation tiles (copy_words 16-byte words, contiguous in HBM) straight
-// into LDS with global_load_lds_dwordx4: lane l of a request writes its 16 bytes at base + 16*l, so a
-// run of 64-word requests is a linear copy that never touches a register.  The instruction offset must
-// stay 0 (the hardware adds it to the global address as well).
+// The four wavefronts of a workgroup request activation tiles (copy_words 16-byte words, contiguous in HBM) straight into LDS
+// (lds_direct, common.h): a run of 64-word requests is a linear copy that never touches a register.  The requests fill the buffer that
+// is not being read; the kernel waits for them, with vmcnt(0) and a barrier, before it is.
 __device__ __forceinline__ void request_a_tiles(const uint8_t* __restrict__ src, uint8_t* buf, int copy_words, int wave,
                                                 int lane) {
     // The address is a scalar base and the lane's 16 l: 22 registers less than an address per lane and request, which the compiler kept
-    // over the whole loop.  Written as inline assembly on purpose: the compiler then does not know that LDS is written, and so does
-    // not make every later LDS read wait for these requests (they fill the OTHER buffer).  The kernel waits
-    // for them itself, with vmcnt(0) and a barrier, before the buffer is read.  M0 (the LDS base of the request)
-    // is used by nothing else in this kernel.
+    // over the whole loop.
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)buf;
     const uint32_t lane_off = (uint32_t)lane * 16u;
     const int full = copy_words >> 6;  // whole requests; everything but the lane's offset is scalar work
     const uint8_t* g = src + (size_t)wave * 1024;
     uint32_t dst = lds_base + (uint32_t)wave * 1024u;
     for (int q = wave; q < full; q += 4, g += 4096, dst += 4096)
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(g), "s"(dst) : "memory", "m0");
+        lds_direct<16>(g, lane_off, dst);
     if ((full & 3) == wave && lane < (copy_words & 63))  // the rest of the last tile, at the request behind this wavefront's last one
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(g), "s"(dst) : "memory", "m0");
+        lds_direct<16>(g, lane_off, dst);
 }
 #endif
 

@@ -62,7 +62,7 @@ __device__ __forceinline__ void request_a_tiles_by_lane(const uint8_t* __restric
         if (first + lane < copy_words) {
             const uint8_t* g = src + (size_t)(first + lane) * 16;
             const uint32_t dst = lds_base + (uint32_t)first * 16u;  // wave-uniform; lane l lands at dst + 16*l
-            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(dst) : "memory", "m0");
+            lds_direct<16>(g, dst);
         }
     }
 }
@@ -95,9 +95,9 @@ __device__ __forceinline__ void request_a_rows(const GatherOffsets<MT>& off, con
         const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr_t)buf + (uint32_t)t * kPTileBytes;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off.code[i]), "s"(plane + j * 64), "s"(dst + j * 1024) : "memory", "m0");
-        if (lane < 32) asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off.digit[i]), "s"(plane), "s"(dst + kPDigitOff) : "memory", "m0");
-        if (lane < 16) asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(off.scale[i]), "s"(plane), "s"(dst + kPScaleOff) : "memory", "m0");
+            lds_direct<16>(plane + j * 64, off.code[i], dst + j * 1024);
+        if (lane < 32) lds_direct<16>(plane, off.digit[i], dst + kPDigitOff);
+        if (lane < 16) lds_direct<4>(plane, off.scale[i], dst + kPScaleOff);
     }
 }
 

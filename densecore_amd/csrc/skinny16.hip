@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
             if (first + lane < words) {
                 const uint8_t* g = src + (size_t)(first + lane) * 16;
                 const uint32_t dst = base + (uint32_t)first * 16u;
-                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(dst) : "memory", "m0");
+                lds_direct<16>(g, dst);
             }
         }
     };
