@@ -148,6 +148,7 @@ struct State {
     Buffer route;         // ids / weights / groups / entries
     Buffer stage_in, stage_out;  // host-pointer entry points
     PinnedBuffer pin_in, pin_out;
+    size_t hidden_rows = 0;  // floats at the head of mid that are the SwiGLU rows of the last layer or FFN call (0: it keeps none, or they are overwritten)
     // the stream of the last call that used the workspaces above, and an event to order the next stream behind it
     bool have_last_stream = false;
     hipStream_t last_stream = nullptr;
@@ -415,6 +416,7 @@ int mq_shutdown(void) {
     for (Buffer* b : {&g.aq, &g.ad, &g.ap, &g.ap2, &g.mid, &g.mid2, &g.kpart, &g.plan, &g.aq2, &g.ad2, &g.part, &g.counters, &g.route, &g.stage_in, &g.stage_out}) b->release();
     g.pin_in.release();
     g.pin_out.release();
+    g.hidden_rows = 0;
     if (g.order_event) (void)hipEventDestroy(g.order_event);
     g.order_event = nullptr;
     g.have_last_stream = false;
@@ -974,6 +976,7 @@ int mq_rmsnorm_mul_mat_q4k(const mq_weight* w, const float* x_dev, const float* 
     if (tiles16 || path == kGemm) {
         // ... and prefill widths: the normalised rows as fp32, then the matrix-core GEMM (its quantizer reads them)
         MQ_HIP(g.mid.reserve((size_t)n * (size_t)w->cols * sizeof(float)));
+        g.hidden_rows = 0;
         MQ_HIP(launch_add_rmsnorm(x_dev, delta_dev, weight_dev, n, w->cols, eps, sum_out_dev, (float*)g.mid.ptr, nullptr, nullptr, s));
         if (!tiles16) return gemm_locked(w, (const float*)g.mid.ptr, n, w->cols, y_dev, ldy, s);
         if (int rc = quantize_into_tile16((const float*)g.mid.ptr, n, w->cols, w->cols, s)) return rc;
@@ -1087,10 +1090,12 @@ int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weigh
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    g.hidden_rows = 0;
     const DensePath gate_path = dense_path(gate, n, true), down_path = dense_path(down, n, false);
     if (gate_path == kGemm) {  // wide: the matrix-core GEMM for gate and up, and for down unless another kernel takes less
         MQ_HIP(g.mid.reserve((size_t)n * (size_t)inter * sizeof(float)));
         const int rc = ffn_wide_locked(gate, up, down_path == kGemm ? down : nullptr, x_dev, n, hidden, silu_mode, (float*)g.mid.ptr, inter, y_dev, hidden, s);
+        if (rc == MQ_OK) g.hidden_rows = (size_t)n * (size_t)inter;
         return rc != MQ_OK || down_path == kGemm ? rc : ffn_down_locked(down, n, false, y_dev, down_path, s);
     }
     // One row: both quantizers run inside the products (two launches instead of four, the same bits).
@@ -1124,6 +1129,7 @@ int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weigh
     a.swiglu = 1;
     a.silu_mode = silu_mode;
     MQ_HIP(census_launch(a, s));
+    g.hidden_rows = (size_t)n * (size_t)inter;
     return ffn_down_locked(down, n, one_row, y_dev, down_path, s);
 }
 
@@ -1867,6 +1873,8 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
     Entry entry(s);
     if (entry.rc) return entry.rc;
     const int slots = K + (sh.gate ? 1 : 0);  // hidden / partial rows per token
+    const size_t hidden_rows = (size_t)n * (size_t)slots * (size_t)inter;
+    g.hidden_rows = 0;
     RouteWs r;
     if (int rc = carve_route(n, K, E, r)) return rc;
     // ids and weights go straight to the caller's buffers when it wants them
@@ -1875,7 +1883,7 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
     if (n <= kDirectPairsMaxTokens && E <= kDecoderMaxExperts && token_major_down(L->down_exps, n, slots)) {
         // few tokens: two launches -- gate/up with the router and the input quantizer inside (moe_gateup.hip), down
         // with the hidden-row quantizer and the combine inside (moe_down.hip)
-        MQ_HIP(g.mid.reserve((size_t)n * slots * (size_t)inter * sizeof(float)));
+        MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
         MoeGateupTokenArgs a;
         a.gate = L->gate_exps->data, a.up = L->up_exps->data, a.expert_bytes = L->gate_exps->expert_bytes;
         if (sh.gate) a.sh_gate = sh.gate->data, a.sh_up = sh.up->data;
@@ -1886,6 +1894,7 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         a.waves = moe_gateup_token_waves(L->gate_exps->nb, inter, n, slots, L->gate_exps->type);
         a.x = x_dev, a.logits = logits_dev, a.hidden = (float*)g.mid.ptr, a.ids_out = ids, a.weights_out = wts;
         MQ_HIP(launch_moe_gateup_token(a, s));
+        g.hidden_rows = hidden_rows;
         return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, false, n, K, slots, r, ids, wts, L->sh_gate_inp_dev,
                             x_dev, y_dev, s);
     }
@@ -1917,10 +1926,11 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         if (g_gemm_pair && L->gate_exps->type == L->up_exps->type) {
             // gate and up in ONE launch whose epilogue stores silu(gate) * up (the shared expert's rows with its own SiLU form)
             if (!moe_gemm_takes(L->down_exps)) {  // fp32 rows at their (token, slot) places for the down stack's own kernel
-                MQ_HIP(g.mid.reserve((size_t)n * slots * (size_t)inter * sizeof(float)));
+                MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
                 MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
                                                         L->gate_exps->nb, (const uint8_t*)g.ap.ptr, n, entries, G, plan, true, L->silu_mode,
                                                         (float*)g.mid.ptr, inter, s, mt));
+                g.hidden_rows = hidden_rows;
                 return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, false, n, K, slots, r, ids, wts, L->sh_gate_inp_dev, x_dev, y_dev, s);
             }
             MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
@@ -1941,9 +1951,10 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
             // a down stack of a type the GEMM does not take: the SwiGLU rows leave the quantizer as fp32 at their
             // (token, slot) places as well, and the expert-grouped decode launches take them from there (their own
             // quantizer -- Q8_K, or Q8_0 for Q8_0 experts -- and the same combine)
-            MQ_HIP(g.mid.reserve((size_t)n * slots * (size_t)inter * sizeof(float)));
+            MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
             MQ_HIP(launch_quantize_q8k_pmajor_grouped(gbuf, ubuf, true, L->silu_mode, inter, inter, entries, G, plan, (uint8_t*)g.ap2.ptr,
                                                       (float*)g.mid.ptr, inter, s));
+            g.hidden_rows = hidden_rows;
             return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, false, n, K, slots, r, ids, wts, L->sh_gate_inp_dev, x_dev, y_dev, s);
         }
         MQ_HIP(launch_quantize_q8k_pmajor_grouped(gbuf, ubuf, true, L->silu_mode, inter, inter, entries, G, plan, (uint8_t*)g.ap2.ptr, nullptr, 0, s));
@@ -1960,11 +1971,12 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
                                   n > kDirectPairsMaxTokens, x_dev, hidden, hidden, (uint8_t*)g.aq.ptr, (float*)g.ad.ptr, s));
     // few tokens: nearly every (token, slot) pair has an expert of its own, so the pairs are the groups
     if (n <= kDirectPairsMaxTokens) r.direct_ids = ids;
-    MQ_HIP(g.mid.reserve((size_t)n * slots * (size_t)inter * sizeof(float)));
+    MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
     // the hidden rows leave gate/up in Q8_K, unless the token-major down launch quantizes what it reads itself
     const bool quantize_in_gateup = !token_major_down(L->down_exps, n, slots) && L->down_exps->type != kTypeQ80;
     if (int rc = run_moe_gateup(L->gate_exps, L->up_exps, sh, n, K, slots, L->silu_mode, r, (float*)g.mid.ptr, quantize_in_gateup, s))
         return rc;
+    g.hidden_rows = hidden_rows;
     return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, quantize_in_gateup, n, K, slots, r, ids, wts, L->sh_gate_inp_dev,
                         x_dev, y_dev, s);
 }
@@ -2139,7 +2151,10 @@ int mq_debug_moe_hidden(float* hidden_out_dev, size_t count, void* stream) {
     if (!hidden_out_dev) return fail(MQ_ERR_INVALID, "mq_debug_moe_hidden: null output");
     Entry entry((hipStream_t)stream);
     if (entry.rc) return entry.rc;
-    if (count * sizeof(float) > g.mid.cap) return fail(MQ_ERR_INVALID, "mq_debug_moe_hidden: the intermediate buffer holds %zu bytes", g.mid.cap);
+    if (count > g.hidden_rows) {
+        if (g.hidden_rows) return fail(MQ_ERR_INVALID, "mq_debug_moe_hidden: the last call left %zu floats", g.hidden_rows);
+        return fail(MQ_ERR_STATE, "mq_debug_moe_hidden: the SwiGLU rows of the last call are not there (no call yet, overwritten, or left in the expert-grouped GEMM's tiles)");
+    }
     MQ_HIP(hipMemcpyAsync(hidden_out_dev, g.mid.ptr, count * sizeof(float), hipMemcpyDeviceToDevice, (hipStream_t)stream));
     return MQ_OK;
 }

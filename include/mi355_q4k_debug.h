@@ -34,7 +34,10 @@ int mq_debug_moe_groups(const float* logits_dev, const int32_t* ids_dev, int64_t
 
 /* The fp32 intermediate the last mq_moe_layer_q4k / mq_ffn_swiglu_q4k call on this stream left in the library's
  * workspace, copied out: for the MoE layer the hidden rows silu(gate . x) * (up . x) as [n][top_k (+1 with a shared
- * expert)][inter], for the dense FFN [n][inter].  `count` floats.  A ...ForTest hook like mq_debug_block_sums. */
+ * expert)][inter], for the dense FFN [n][inter].  `count` floats, no more than that call left (MQ_ERR_INVALID).
+ * MQ_ERR_STATE where the rows are not there: no such call yet, a later product used the workspace, or the layer took the
+ * expert-grouped GEMM, which forms them in its tiles' order.  Replays of a captured call do not count as calls.  A ...ForTest hook like
+ * mq_debug_block_sums. */
 int mq_debug_moe_hidden(float* hidden_out_dev, size_t count, void* stream);
 /* Device addresses of a decoder handle's exchange buffers after a step (the LAST layer's values): qkv [n][qkv_rows],
  * o [n][hidden], logits [n][n_experts], hidden rows [n][top_k (+1)][inter], MoE output y [n][hidden].  Any may be NULL. */
