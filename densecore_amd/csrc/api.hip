@@ -586,7 +586,12 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of up
 // to four super-blocks never leave them below 48 (that equality is tested there); a pair's GEMM is not estimated closely enough at
 // these widths (0.6 to 1.6 of its time) to leave them for.
+// Up to kDecodeRows rows the GEMM is never taken: a row's bits are those of the row alone there, and the products that cannot take it
+// (mq_mul_mat_q4k_noalloc, whose scratch holds no planes of partial sums) return them as well.  It would be for one product in a
+// hundred, 11008 columns and more in few row tiles.
 enum DensePath { kPasses, kSixteens, kGemm };
+constexpr int64_t kDecodeRows = 16;
+static_assert(kNoAllocMaxRows <= kDecodeRows, "the product without allocations has no GEMM");
 constexpr int64_t kPrefillMinRows = 48;
 constexpr int64_t kPrefillMinRowsLarge = 17;
 constexpr int64_t kPrefillLargeBytes = 24ll << 20;
@@ -621,7 +626,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         us[kSixteens] = c.sixteens[0] + stages(pick_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
     }
     const float decode = us[kSixteens] < us[kPasses] ? us[kSixteens] : us[kPasses];
-    if (plain == kGemm || (!swiglu && nb > 4 && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
+    if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > 4 && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
         GemmShape shape;
         float gemm;
         if (swiglu && gemm_pair_shape(type, rows, nb, n, false, &shape)) {
@@ -2211,6 +2216,15 @@ int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
     else s = gemm_shape(wtype, rows, cols / kQK, n);
     shape_out[0] = s.narrow, shape_out[1] = s.splits, shape_out[2] = s.sb_split, shape_out[3] = s.tiles_per_wg;
     shape_out[4] = (int)s.row_wgs, shape_out[5] = (int)s.groups, shape_out[6] = taken, shape_out[7] = (int)(1000.0f * s.us);
+    return MQ_OK;
+}
+
+int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out) {
+    if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !path_out)
+        return fail(MQ_ERR_INVALID, "mq_debug_dense_path: bad type, size or pointer");
+    path_out[0] = dense_path_of(wtype, rows, cols / kQK, n, pair != 0);
+    path_out[1] = dense_waves(cols / kQK, (rows + 15) / 16);
+    path_out[2] = skinny16_applies(cols / kQK, (rows + 15) / 16, pair != 0, n, wtype) ? skinny16_wpr(cols / kQK, (rows + 15) / 16) : 0;
     return MQ_OK;
 }
 

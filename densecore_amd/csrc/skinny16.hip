@@ -416,7 +416,7 @@ hipError_t launch_skinny16_tiles(const Skinny16Args& a, int wpr, hipStream_t str
 }  // namespace
 
 // Wavefronts per row tile: a divisor of eight that divides the super-blocks of a row (0: none)
-static int skinny16_wpr(int64_t nb, int64_t rowtiles) {
+int skinny16_wpr(int64_t nb, int64_t rowtiles) {
     const int w = pick_waves(nb, rowtiles);
     return (w == 1 || w == 2 || w == 4 || w == 8) ? w : 0;
 }

@@ -75,6 +75,11 @@ int mq_debug_set_dense_lds(int on);
  * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns. */
 int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);
 
+/* Kernels that a dense product of n rows (pair != 0: gate and up in one call) runs on, for a 256-unit device before mq_init.  path_out:
+ * 0 passes of eight or sixteen rows, 1 tiles of sixteen, 2 the matrix-core GEMM; wavefronts per row tile of the passes, and of the
+ * tiles of sixteen (0: not built for this product). */
+int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out);
+
 /* Measurement instrument: while on != 0 every compute and routing launch of the library is replaced by a kernel with
  * an empty body and the same grid, block and LDS size (weight set-up and launches that carry timing events are
  * not).  A graph captured in this state has the launches of the real one and none of their work: its replay time

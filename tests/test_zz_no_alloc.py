@@ -41,6 +41,19 @@ def test_two_calls_in_a_row_equal_the_allocating_entry_point(env, wtype, rows, c
         assert np.array_equal(want.view(np.uint32), got.view(np.uint32)), f"n={n}: outputs differ"
 
 
+@pytest.mark.parametrize("wtype", [12, 13, 14])
+@pytest.mark.parametrize("rows,cols", [(5120, 11008), (14336, 11008), (8704, 9472), (2048, 5632)])
+def test_rows_of_uneven_super_blocks_equal_the_allocating_entry_point(env, wtype, rows, cols):
+    """Long rows that no useful wavefront count divides, where other kernels take a product from nine or seventeen rows on."""
+    torch, _lib, ops = env
+    W = ops.Q4KWeight.synthetic(synth.tensor_seed("noalloc-u", wtype, rows, cols), rows, cols, ggml_type=wtype)
+    x = torch.from_numpy(synth.normal_f32(synth.tensor_seed("noalloc-ux", rows, cols), (16, cols))).cuda()
+    for n in (8, 9, 16):
+        want, got = _both(env, W, x[:n])
+        assert np.array_equal(want.view(np.uint32), got.view(np.uint32)), f"n={n}: outputs differ"
+    W.free()
+
+
 def test_smaller_matrix_after_larger_one(env):
     """A 16384-column product fills the whole scratch; a 256-column one after it reads only its own corner."""
     torch, _lib, ops = env
