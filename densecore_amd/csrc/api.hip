@@ -574,15 +574,15 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // Which kernel a dense product of n rows (swiglu: gate and up) runs on: passes of the decode kernels, tiles of sixteen
 // (skinny16_kernel) or the matrix-core GEMM.  Up to eight rows the first, beyond 64 the last.  Between them the plain rule -- tiles of
 // sixteen where they are built, else the GEMM from 48 rows, from 17 for matrices of 24 MB and more -- unless an estimate says that
-// another one takes less than kPathLess of its time: split by a count that divides the super-blocks, tiles of sixteen of 43
-// super-blocks are one wavefront's 43 stages (4096 rows at 32: 57 us, 18.5 on the GEMM), and 33 rows are three passes (15966 x 1792
-// 29.9 us, 14.2 on the GEMM).
+// another one takes less than kPathLess of its time: 33 rows are three passes (4096 x 11008, whose tiles do not fit LDS: 58 us, 19 on the
+// GEMM).
 //   st: stages of a wavefront times rounds of workgroups; tiles: (n + 15) / 16; mb: megabytes as Q4_K; us:
 //   passes  c0 + tiles (c1 + c2 st + c3 mb)    sixteens  c0 + st (c1 + c2 tiles + c3 tiles if read from global memory or in runs) + c4 mb
 //   GEMM    c0 + c1 times its shape's estimate
 // Least squares over 2,080 products (512 to 128,256 rows, 4 to 56 super-blocks, 9 to 64 tokens, three types) and 1,088 pairs, all three
 // timed: the choice takes 0.936 (pairs 0.968) of the plain rule's time, 0.62 (0.53) where it differs, and nowhere more; 1.018 (1.024) of
-// the fastest one's.  It stays at
+// the fastest one's -- with tiles of sixteen split by counts that divide a row's super-blocks only; since they split like the passes (the
+// estimate reads the same stages), 300 products of uneven splits take 0.82 of the time they took, 2 % of them over 1.05 of it.  The line is at
 // three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of up
 // to four super-blocks never leave them below 48 (that equality is tested there); a pair's GEMM is not estimated closely enough at
 // these widths (0.6 to 1.6 of its time) to leave them for.
@@ -623,7 +623,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
     float us[3] = {c.passes[0] + tiles * (c.passes[1] + c.passes[2] * stages(dense_waves(nb, rowtiles)) + c.passes[3] * mb), 1e30f, 1e30f};
     if (sixteens) {
         const float far = skinny16_one_run(nb, rowtiles, swiglu, n) ? 0.0f : c.sixteens[3];
-        us[kSixteens] = c.sixteens[0] + stages(pick_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
+        us[kSixteens] = c.sixteens[0] + stages(dense_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
     }
     const float decode = us[kSixteens] < us[kPasses] ? us[kSixteens] : us[kPasses];
     if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > 4 && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
@@ -2224,7 +2224,7 @@ int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
         return fail(MQ_ERR_INVALID, "mq_debug_dense_path: bad type, size or pointer");
     path_out[0] = dense_path_of(wtype, rows, cols / kQK, n, pair != 0);
     path_out[1] = dense_waves(cols / kQK, (rows + 15) / 16);
-    path_out[2] = skinny16_applies(cols / kQK, (rows + 15) / 16, pair != 0, n, wtype) ? skinny16_wpr(cols / kQK, (rows + 15) / 16) : 0;
+    path_out[2] = skinny16_applies(cols / kQK, (rows + 15) / 16, pair != 0, n, wtype) ? dense_lds_wpr(cols / kQK, (rows + 15) / 16) : 0;
     return MQ_OK;
 }
 

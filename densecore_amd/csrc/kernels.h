@@ -139,7 +139,6 @@ struct Skinny16Args {
     int ranges = 1;                // set by the launcher: runs of super-blocks the tiles pass through LDS in
 };
 bool skinny16_applies(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n, int wtype = kTypeQ4K);
-int skinny16_wpr(int64_t nb, int64_t rowtiles);  // wavefronts per row tile (0: not a split it is built for)
 bool skinny16_one_run(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n);  // the rows' tiles fit LDS at once (else read from global memory or in runs)
 hipError_t launch_skinny16(const Skinny16Args& a, hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 

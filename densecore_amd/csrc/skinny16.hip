@@ -29,13 +29,19 @@ namespace {
 // per activation tile in place of sixteen over the bytes of one scale group each with the group sums scaled on the vector
 // unit: an FFN of 4096 -> 14336 -> 4096 all Q6_K at 30 rows 56.3 -> 48.7 us, with a Q6_K down projection at 40 rows 56.8 -> 50.6.
 // LDS: [nb][4688] activation tiles (not GA), then the partial sums [8 / WPR][WPR - 1][NMAT][4][64].
-// nb % WPR == 0 (host-checked): every wavefront has nb / WPR stages; FLOW 1: that count is odd (a single run); 0: even, a
-// single run or runs of an even number of stages; 2: even, runs of an odd number of stages.
+// Every wavefront has ceil(nb / WPR) stages; FLOW 1: that count is odd (a single run); 0: even, a single run or runs of an even number
+// of stages; 2: even, runs of an odd number of stages.  Where nb % WPR != 0 (a single run; the split that dense_waves gives all decode
+// kernels for the matrix) the last stage of the wavefronts from nb % WPR on does not exist: they request the last super-block once
+// more, another wavefront's at that time, and multiply nothing.  Against a count that divides: 2048 x 5632 at 16 rows (eight wavefronts
+// for two) 12.2 -> 8.2 us, 4096 x 11008 at 32 rows (eight for one) 57 -> 15.3.
 struct ATile16 {
     v4i a[4];   // the four 64-weight chunks of this lane's operand
     v4f yd;     // the Q8_K scales of rows 4 kq .. 4 kq + 3
     v8h dg;     // this lane's operand of the min MFMA (fp16 digits of the sub-block sums, or zeros)
 };
+
+// (a pair of two tiles read from global memory would spill 46 registers)
+constexpr bool skinny16_uneven(int nmat, int wpr, bool ga, int mt) { return wpr > 1 && !(ga && nmat == 2 && mt == 2); }
 
 // MT: activation tiles of sixteen rows (one to four, e.g. two for 17 to 32 rows: the weight tile is expanded once for both, 18
 // MFMAs and ~156 vector instructions against the 32 + 294 of two passes over two token tiles of eight each).  With two
@@ -47,6 +53,7 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
     constexpr bool Q5 = WT == kWtQ5, Q6 = WT == kWtQ6;
     constexpr int kStride = tile_stride<WT>();
     constexpr int kTileLoads = Q6 ? 5 : Q5 ? 4 : 3;  // requests of a weight tile (load_tile, load_tile6)
+    constexpr bool kUneven = skinny16_uneven(NMAT, WPR, GA, MT);
     constexpr bool kRedShares = MT > 1 && !GA;  // the partial sums reuse the activation tiles' LDS
     extern __shared__ __align__(16) uint8_t lds16[];
     const int lane = threadIdx.x & 63;
@@ -63,7 +70,8 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
     const uint8_t* tiles[NMAT];
     tiles[0] = p.w0 + tile_offset(rt, 0, nb, kStride);
     if (NMAT == 2) tiles[1] = p.w1 + tile_offset(rt, 0, nb, kStride);
-    const int cnt = nb / WPR;  // stages of this wavefront: super-blocks h, h + WPR, ...
+    const int cnt = kUneven ? (nb + WPR - 1) / WPR : nb / WPR;  // stages: super-blocks h, h + WPR, ...
+    const bool last_exists = !kUneven || h + (cnt - 1) * WPR < nb;  // wave-uniform
 
     // lane (r, kq): weight row r of the tile, activation rows 4 kq .. 4 kq + 3 of every activation tile
     const int digit_off = kq < 2 ? kPDigitOff + r * 32 + kq * 16 : kPZeroOff;
@@ -96,9 +104,9 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
 
     typename TileOf<WT>::Regs ring_t[2][NMAT];
     ATile16 ring_a[GA ? 2 : 1][GA ? MT : 1];
-    auto issue = [&](auto st_c, int i) {  // only ever called for a stage that exists
+    auto issue = [&](auto st_c, int i, auto last_c) {  // i < cnt; last_c: i may be cnt - 1 (looking at every request costs Q6_K 2 % and more)
         constexpr int st = decltype(st_c)::value;
-        const int b = h + i * WPR;
+        const int b = decltype(last_c)::value && kUneven && h + i * WPR >= nb ? nb - 1 : h + i * WPR;
         if constexpr (GA) {  // ahead of the tiles: they are needed first
 #pragma unroll
             for (int t = 0; t < MT; ++t) read_a(ring_a[st][t], p.ap + ((size_t)b * MT + t) * kPTileBytes);
@@ -169,11 +177,13 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
     // is ever made for a stage that does not exist.
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
+    constexpr std::false_type kMore{};
+    constexpr std::true_type kLast{};
     const bool single = ODD && cnt == 1;  // wave-uniform
-    issue(S0{}, 0);
+    issue(S0{}, 0, kMore);
     asm volatile("" ::: "memory");  // requests stay in stage order
     if (!single) {
-        issue(S1{}, 1);
+        issue(S1{}, 1, kLast);
         asm volatile("" ::: "memory");
     }
     if constexpr (!GA) {
@@ -186,19 +196,22 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
     if constexpr (ODD) {
         consume(S0{}, 0);
         if (!single) {
-            issue(S0{}, 2);  // cnt >= 3
+            issue(S0{}, 2, kLast);  // cnt >= 3
             asm volatile("" ::: "memory");
             int i = 1;
-            for (; i + 2 < cnt; i += 2) {
+            auto two_stages = [&](auto last_c) {
                 consume(S1{}, i);
-                issue(S1{}, i + 2);
+                issue(S1{}, i + 2, kMore);
                 asm volatile("" ::: "memory");
                 consume(S0{}, i + 1);
-                issue(S0{}, i + 3);
+                issue(S0{}, i + 3, last_c);
                 asm volatile("" ::: "memory");
-            }
+                i += 2;
+            };
+            while (i + (kUneven ? 4 : 2) < cnt) two_stages(kMore);
+            if (kUneven && i + 2 < cnt) two_stages(kLast);
             consume(S1{}, i);
-            consume(S0{}, i + 1);
+            if (last_exists) consume(S0{}, i + 1);
         }
     } else {
         // The next run of super-blocks replaces the one in LDS once every wavefront has multiplied its last stage of it
@@ -209,6 +222,15 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
             // spills against 120-130).  The last pair of stages of the launch is peeled off: no request past the end.
             const int runs = GA ? 1 : p.ranges;
             int i = 0;
+            auto two_stages = [&](auto last_c) {
+                consume(S0{}, i);
+                issue(S0{}, i + 2, kMore);
+                asm volatile("" ::: "memory");
+                consume(S1{}, i + 1);
+                issue(S1{}, i + 3, last_c);
+                asm volatile("" ::: "memory");
+                i += 2;
+            };
             for (int rg = 0; rg < runs; ++rg) {
                 if (rg > 0) {  // wave-uniform, the same in every wavefront
                     __syncthreads();
@@ -217,18 +239,12 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's share of the copy (and its two stages of weight tiles)
                     __syncthreads();
                 }
-                const int i_stop = (rg + 1) * (cnt / runs) - (rg == runs - 1 ? 2 : 0);
-                for (; i < i_stop; i += 2) {
-                    consume(S0{}, i);
-                    issue(S0{}, i + 2);
-                    asm volatile("" ::: "memory");
-                    consume(S1{}, i + 1);
-                    issue(S1{}, i + 3);
-                    asm volatile("" ::: "memory");
-                }
+                const int i_stop = (rg + 1) * (cnt / runs) - (rg == runs - 1 ? (kUneven ? 4 : 2) : 0);
+                while (i < i_stop) two_stages(kMore);
             }
+            if (kUneven && i + 2 < cnt) two_stages(kLast);
             consume(S0{}, i);
-            consume(S1{}, i + 1);
+            if (last_exists) consume(S1{}, i + 1);
         } else {
             // FLOW == 2: runs of an odd number of stages begin at either stage of a pair
             auto next_range = [&](int i) {
@@ -244,11 +260,11 @@ __global__ void __launch_bounds__(512) skinny16_kernel(const Skinny16Args p) {
             for (; i + 2 < cnt; i += 2) {
                 next_range(i);
                 consume(S0{}, i);
-                issue(S0{}, i + 2);
+                issue(S0{}, i + 2, kMore);
                 asm volatile("" ::: "memory");
                 next_range(i + 1);
                 consume(S1{}, i + 1);
-                issue(S1{}, i + 3);
+                issue(S1{}, i + 3, kMore);
                 asm volatile("" ::: "memory");
             }
             next_range(i);
@@ -350,7 +366,7 @@ hipError_t launch_skinny16_one(const Skinny16Args& a, int ranges, hipStream_t st
 // tiles in runs of an odd number of stages.
 template <int NMAT, int WPR, int MT, int WT>
 hipError_t launch_skinny16_form(const Skinny16Args& a, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
-    const bool odd = ((a.nb / WPR) & 1) != 0;
+    const bool odd = (((a.nb + WPR - 1) / WPR) & 1) != 0;
     const int ranges = odd ? (skinny16_lds_bytes(NMAT, WPR, a.nb, MT, 1) <= kSkinnyLdsMax ? 1 : 0) : skinny16_ranges(NMAT, WPR, a.nb, MT);
     // (skinny16_applies knows the forms that are not built)
     if constexpr (WT == kWtQ6 && NMAT == 2 && WPR == 1) {
@@ -370,7 +386,7 @@ hipError_t launch_skinny16_form(const Skinny16Args& a, hipStream_t stream, hipEv
     } else {
         if (ranges == 0) return hipErrorInvalidValue;
         if (odd) return launch_skinny16_one<NMAT, WPR, 1, false, MT, WT>(a, 1, stream, start, stop);  // (an odd stage count: one run only)
-        if ((((a.nb / WPR) / ranges) & 1) == 0) return launch_skinny16_one<NMAT, WPR, 0, false, MT, WT>(a, ranges, stream, start, stop);
+        if (((((a.nb + WPR - 1) / WPR) / ranges) & 1) == 0) return launch_skinny16_one<NMAT, WPR, 0, false, MT, WT>(a, ranges, stream, start, stop);
         if constexpr (WT == kWtQ6 || (WT == kWtQ5 && NMAT == 2 && MT == 4)) return hipErrorInvalidValue;  // (runs of an odd stage count)
         else return launch_skinny16_one<NMAT, WPR, 2, false, MT, WT>(a, ranges, stream, start, stop);
     }
@@ -415,29 +431,24 @@ hipError_t launch_skinny16_tiles(const Skinny16Args& a, int wpr, hipStream_t str
 
 }  // namespace
 
-// Wavefronts per row tile: a divisor of eight that divides the super-blocks of a row (0: none)
-int skinny16_wpr(int64_t nb, int64_t rowtiles) {
-    const int w = pick_waves(nb, rowtiles);
-    return (w == 1 || w == 2 || w == 4 || w == 8) ? w : 0;
-}
-
 // Whether a product of n rows (nine to 64) runs on skinny16_kernel: the wave split of the other decode kernels must be
-// one of its own (a divisor of eight that divides the super-blocks of a row), and the form must be built
+// one of its own (a divisor of eight), and the form must be built
 // (launch_skinny16_form returns an error for the others).
 //   One and two tiles (up to 32 rows): always; the two tiles of a Q5_K or Q6_K gate/up pair only where they fit LDS in
 //   one run; a Q6_K pair not with one wavefront per row tile.
 //   Three and four tiles: not with one wavefront per row tile (more than 1,024 row tiles: the GEMM is faster from 33
 //   rows -- 128256 x 4096 at 33 / 64 rows: 93 / 108 us against 102 / 126); the tiles must pass through LDS in at most four
-//   runs of whole stages (in one run where a wavefront's stage count is odd); a pair of four tiles not with eight
+//   runs of whole stages (in one run where a wavefront's stage count is odd or the split uneven); a pair of four tiles not with eight
 //   wavefronts per row tile; in runs of an odd number of stages no Q6_K form and no Q5_K pair of four tiles.
 bool skinny16_applies(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n, int wtype) {
-    const int wpr = skinny16_wpr(nb, rowtiles);
+    const int wpr = dense_lds_wpr(nb, rowtiles);
     if (!wpr || n < 1 || n > 64 || (wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K)) return false;
     const int nmat = swiglu ? 2 : 1, mt = (int)((n + 15) / 16);
     if (wtype == kTypeQ6K && swiglu && wpr == 1) return false;
+    if (nb % wpr && !skinny16_uneven(nmat, wpr, skinny16_lds_bytes(nmat, wpr, nb, mt, 1) > kSkinnyLdsMax, mt)) return false;
     if (mt <= 2) return !(wtype != kTypeQ4K && swiglu && mt == 2) || skinny16_lds_bytes(2, wpr, nb, 2, 1) <= kSkinnyLdsMax;
     if (wpr == 1 || (swiglu && mt == 4 && wpr == 8)) return false;
-    if ((nb / wpr) & 1) return skinny16_lds_bytes(nmat, wpr, nb, mt, 1) <= kSkinnyLdsMax;  // an odd stage count: the tiles in one run
+    if (nb % wpr || ((nb / wpr) & 1)) return skinny16_lds_bytes(nmat, wpr, nb, mt, 1) <= kSkinnyLdsMax;  // an uneven split, an odd stage count: the tiles in one run
     const int ranges = skinny16_ranges(nmat, wpr, nb, mt);
     if (!ranges) return false;
     const bool odd_runs = (((nb / wpr) / ranges) & 1) != 0;
@@ -445,7 +456,7 @@ bool skinny16_applies(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n, int 
 }
 
 bool skinny16_one_run(int64_t nb, int64_t rowtiles, bool swiglu, int64_t n) {
-    const int wpr = skinny16_wpr(nb, rowtiles);
+    const int wpr = dense_lds_wpr(nb, rowtiles);
     return wpr && skinny16_lds_bytes(swiglu ? 2 : 1, wpr, nb, (int)((n + 15) / 16), 1) <= kSkinnyLdsMax;
 }
 
@@ -453,7 +464,7 @@ hipError_t launch_skinny16(const Skinny16Args& a, hipStream_t stream, hipEvent_t
     if (a.rows <= 0 || a.nb <= 0 || a.n < 1 || a.n > 64 || !a.y || !a.w0 || !a.ap) return hipErrorInvalidValue;
     const int64_t rowtiles = (a.rows + 15) / 16;
     if (!skinny16_applies(a.nb, rowtiles, a.w1 != nullptr, a.n, a.wtype)) return hipErrorInvalidValue;
-    const int wpr = skinny16_wpr(a.nb, rowtiles);
+    const int wpr = dense_lds_wpr(a.nb, rowtiles);
     if (a.w1) return launch_skinny16_tiles<2>(a, wpr, stream, start, stop);
     return launch_skinny16_tiles<1>(a, wpr, stream, start, stop);
 }

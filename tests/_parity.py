@@ -35,5 +35,18 @@ def gemm_shape(wtype: int, rows: int, cols: int, n: int, pair: int = 0) -> dict:
     return dict(zip(("narrow", "runs", "sb_run", "tiles", "row_wgs", "columns", "taken", "ns"), out))
 
 
+PASSES, SIXTEENS, GEMM = 0, 1, 2
+
+
+def dense_path(wtype: int, rows: int, nb: int, n: int, pair: int = 0) -> tuple:
+    """Kernel of a dense product, wavefronts per row tile of the passes and of the tiles of sixteen (include/mi355_q4k_debug.h)."""
+    import ctypes as C
+
+    from densecore_amd import _lib
+    out = (C.c_int * 3)()
+    assert _lib.load().mq_debug_dense_path(wtype, rows, 256 * nb, n, pair, out) == 0
+    return tuple(out)
+
+
 def oracle_all_orders(w: np.ndarray, cols: int, q8: np.ndarray):
     return {name: orc.mul_mat_q4k_q8k(w, cols, q8, order) for name, order in orc.ORDERS.items()}

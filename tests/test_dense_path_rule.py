@@ -1,16 +1,7 @@
 """Which kernel a dense product takes (no GPU needed: the rule is host arithmetic, for 256 compute units before a device is opened)."""
-import ctypes as C
 import random
 
-from densecore_amd import _lib
-
-PASSES, SIXTEENS, GEMM = 0, 1, 2
-
-
-def dense_path(wtype, rows, nb, n, pair=0):
-    out = (C.c_int * 3)()
-    assert _lib.load().mq_debug_dense_path(wtype, rows, 256 * nb, n, pair, out) == 0
-    return tuple(out)
+from tests._parity import PASSES, SIXTEENS, GEMM, dense_path
 
 
 def products(count, seed):
@@ -26,3 +17,10 @@ def test_up_to_sixteen_rows_stay_on_the_decode_kernels():
             path, _, sixteens = dense_path(wtype, rows, nb, n, pair)
             assert path == PASSES or (path == SIXTEENS and sixteens), (wtype, rows, nb, n, pair)
         assert dense_path(wtype, rows, nb, 65, pair)[0] == GEMM
+
+
+def test_tiles_of_sixteen_split_a_row_like_the_passes():
+    for wtype, rows, nb, pair in products(20000, 6):
+        for n in (9, 16, 17, 33, 64):
+            path, passes, sixteens = dense_path(wtype, rows, nb, n, pair)
+            assert sixteens in (0, passes) and (path != SIXTEENS or sixteens), (wtype, rows, nb, n, pair)
