@@ -582,7 +582,7 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // Least squares over 2,080 products (512 to 128,256 rows, 4 to 56 super-blocks, 9 to 64 tokens, three types) and 1,088 pairs, all three
 // timed: the choice takes 0.936 (pairs 0.968) of the plain rule's time, 0.62 (0.53) where it differs, and nowhere more; 1.018 (1.024) of
 // the fastest one's -- with tiles of sixteen split by counts that divide a row's super-blocks only; since they split like the passes (the
-// estimate reads the same stages), 300 products of uneven splits take 0.82 of the time they took, 2 % of them over 1.05 of it.  The line is at
+// estimate reads the same stages), 300 products of uneven splits take 0.82 of the time they took, 3 % of them over 1.05 of it.  The line is at
 // three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of up
 // to four super-blocks never leave them below 48 (that equality is tested there); a pair's GEMM is not estimated closely enough at
 // these widths (0.6 to 1.6 of its time) to leave them for.
@@ -1684,7 +1684,9 @@ static int acts_matmul(const mq_weight* w0, const mq_weight* w1, const mq_acts* 
     m.w1 = w1 ? w1->data : nullptr;
     m.rows = w0->rows;
     m.nb = w0->nb;
-    if (a->tile16 && skinny16_takes(w0, a->n, swiglu != 0)) {
+    // The decode kernel that the one-shot product takes.  Where that is the GEMM (from 17 rows), tiles of sixteen if they are built: a
+    // handle's products reserve no planes of partial sums, and are the same bits whichever call filled the handle.
+    if (a->tile16 && skinny16_takes(w0, a->n, swiglu != 0) && dense_path(w0, a->n, swiglu != 0) != kPasses) {
         m.ap = (const uint8_t*)a->ap;
     } else {
         m.aq = (const uint8_t*)a->aq;
