@@ -263,10 +263,14 @@ __global__ void __launch_bounds__(256) quantize_q80_tiles_kernel(const float* __
 
 // A workgroup of four wavefronts: four row tiles x MT activation tiles, the activation tiles of a super-block staged in LDS (double
 // buffer, LDS-direct copies a super-block ahead), each wavefront's weight tile in registers, the next one on its way.  One K = 32 MFMA
-// forms the sums of a block for sixteen rows of either side; each takes three vector instructions per output, which is what bounds it
-// (96 beside eight MFMAs per tile; twelve LDS reads).  The launch of eight-row passes walks all rows
-// in one workgroup per row tile: us, passes | this: 8075 x 13312 at 32 / 128 / 500 / 1100 rows 97 / 396 / 1561 / 3438 | 39 / 130 / 213 / 443
-// (533 TOP/s), 920 x 6912 26 / 92 / 369 / 811 | 21 / 23 / 29 / 48.
+// forms the sums of a block for sixteen rows of either side; each takes three vector instructions per output, and one more joins a
+// super-block's sum, which is what bounds it (100 beside eight MFMAs per tile; twelve LDS reads).  A row's sum is two chains, over
+// the even and the odd super-blocks, of chains of eight blocks: against double, the same operands, its error is 0.35 to 0.95 of that of
+// the passes of eight, which split a row over one to eight wavefronts (40 products of 2048 to 14336 columns; 4096 columns on eight
+// wavefronts 0.82e-7 against 0.92e-7, 14336 1.16e-7 against 1.46e-7).  One chain over the row was 1.5 % faster and had up to 2.6 times
+// that error.  The launch of eight-row passes walks all rows
+// in one workgroup per row tile: us, passes | this: 8075 x 13312 at 32 / 128 / 500 / 1100 rows 97 / 396 / 1561 / 3438 | 40 / 136 / 206 / 437
+// (541 TOP/s), 920 x 6912 26 / 92 / 369 / 811 | 22 / 23 / 27 / 43.
 template <int MT>
 __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restrict__ w, int64_t rowtiles, int64_t rows, int nb, const uint8_t* __restrict__ ap,
                                                           int64_t m_tiles, int64_t n, float* __restrict__ y, int64_t ldy) {
@@ -277,11 +281,11 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
     const int mt_count = (int)(m_tiles - mt0 < MT ? m_tiles - mt0 : MT);
     const int64_t rt = (int64_t)blockIdx.x * 4 + wave;  // row tiles past the end: the last one again, not stored
     const uint8_t* tile = w + tile_offset(rt < rowtiles ? rt : rowtiles - 1, 0, nb, kTile80Bytes);
-    float acc[MT][4];
+    float even[MT][4], odd[MT][4];  // sums over the even and the odd super-blocks
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[m][i] = 0.0f;
+        for (int i = 0; i < 4; ++i) even[m][i] = odd[m][i] = 0.0f;
     Tile80 next;
     auto request = [&](int b) {
         request_a_tiles(ap + ((size_t)b * (size_t)m_tiles + (size_t)mt0) * kQ80ATileBytes, a_lds[b & 1], mt_count * kQ80ATileWords, wave, lane);
@@ -290,7 +294,7 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
         next.sc = load16(tile + (size_t)b * kTile80Bytes + kTile80SOff + r * 16);
     };
     request(0);
-    for (int b = 0; b < nb; ++b) {
+    auto step = [&](int b, float (&sum)[MT][4]) {
         __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xF << 8));  // vmcnt(0): what this thread asked for has landed ...
         __syncthreads();                                          // ... and everybody else's; the other buffer is free
         const Tile80 cur = next;
@@ -301,6 +305,7 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
         for (int m = 0; m < MT; ++m) {
             if (m < mt_count) {  // uniform over the workgroup
                 const uint8_t* at = a_lds[b & 1] + m * kQ80ATileBytes;
+                float part[4];  // the super-block's sum
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     typedef long v2l __attribute__((ext_vector_type(2)));
@@ -313,12 +318,23 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
                         const float4 dy = *reinterpret_cast<const float4*>(at + 4096 + (k * 16 + kq * 4) * 4);
                         const float dyv[4] = {dy.x, dy.y, dy.z, dy.w};
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[m][i] = __fmaf_rn(__fmul_rn(dx[k], dyv[i]), (float)s[i], acc[m][i]);
+                        for (int i = 0; i < 4; ++i) {
+                            const float d = __fmul_rn(dx[k], dyv[i]);
+                            part[i] = k == 0 ? __fmul_rn(d, (float)s[i]) : __fmaf_rn(d, (float)s[i], part[i]);
+                        }
                     }
                 }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[m][i] = __fadd_rn(sum[m][i], part[i]);
             }
         }
+    };
+    int b = 0;
+    for (; b + 1 < nb; b += 2) {
+        step(b, even);
+        step(b + 1, odd);
     }
+    if (b < nb) step(b, even);
     const int64_t row = rt * 16 + r;
     if (rt >= rowtiles || row >= rows) return;
 #pragma unroll
@@ -326,7 +342,7 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int64_t tok = (mt0 + m) * 16 + kq * 4 + i;
-            if (tok < n) y[tok * ldy + row] = acc[m][i];
+            if (tok < n) y[tok * ldy + row] = __fadd_rn(even[m][i], odd[m][i]);
         }
 }
 

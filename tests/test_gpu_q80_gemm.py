@@ -42,3 +42,30 @@ def test_many_rows_match_the_oracle(rows, cols, n):
     assert_fp32_parity(y, orc.mul_mat_q80_q80(w_np, cols, q, orc.ORDER_HWY), mag, f"q80 gemm {rows}x{cols} n={n}")
     assert_fp32_parity(y, orc.q80_dot_dequant_f64(w_np, cols, q), mag, "q80 gemm vs double")
     w.free()
+
+
+# the passes of eight split these rows over eight (4096, 14336 columns), five and four wavefronts; 14336 columns on more than one tile
+# of rows, whose passes walk a row in one wavefront
+@pytest.mark.parametrize("rows,cols,n", [(640, 4096, 40), (640, 14336, 40), (640, 5120, 64), (4200, 13312, 32), (8300, 14336, 16)])
+def test_rounding_error_is_no_larger_than_that_of_eight_rows_at_a_time(rows, cols, n):
+    """Both against the same quantized operands in double: the GEMM adds up super-blocks, the even and the odd ones apart, so that it does
+    not lose to the passes' wavefronts (a plain chain over the row has up to 2.6 times their error)."""
+    import torch
+    from densecore_amd import ops
+    w_np = synth.q80_matrix(synth.tensor_seed("mm80e-w", rows, cols), rows, cols)
+    x = synth.normal_f32(synth.tensor_seed("mm80e-x", rows, cols, n), (n, cols))
+    blk = w_np.reshape(rows, cols // 32, 34)
+    scale = torch.from_numpy(blk[:, :, :2].copy().view(np.float16).astype(np.float64)).cuda()
+    codes = torch.from_numpy(blk[:, :, 2:].copy().view(np.int8)).cuda().double()
+    wd = (codes * scale).reshape(rows, cols)
+    xb = x.reshape(n, cols // 32, 32)  # the quantizer of the library, in its own fp32 steps
+    amax = np.abs(xb).max(-1, keepdims=True)
+    xq = np.rint(xb * np.divide(np.float32(127), amax, where=amax != 0, out=np.zeros_like(amax)))
+    xd = torch.from_numpy((xq.astype(np.float64) * (amax / np.float32(127)).astype(np.float16).astype(np.float64)).reshape(n, cols)).cuda()
+    want = (xd @ wd.T.contiguous())
+    w, xg = ops.Q4KWeight.from_ggml(w_np, cols, Q80), torch.from_numpy(x).cuda()
+    error = lambda y: ((y.double() - want).norm() / want.norm()).item()
+    gemm, passes = error(ops.mul_mat(w, xg)), error(torch.cat([ops.mul_mat(w, xg[i:i + 8]) for i in range(0, n, 8)]))
+    assert passes < 1e-6  # the operands above are the library's
+    assert gemm <= passes, (gemm, passes)
+    w.free()
