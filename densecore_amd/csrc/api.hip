@@ -742,26 +742,32 @@ static int ffn_down_locked(const mq_weight* down, int64_t n, bool one_row, float
 
 // Q8_0 weights: the activations are quantized to Q8_0 as well (codes into g.aq in the A-major order, fp16 scales
 // into g.ad), then one launch; many rows: into tiles of sixteen for a GEMM (q8_0.hip).
-// The launch walks the rows in passes of eight with a workgroup per row tile; the GEMM's four row tiles to a workgroup leave units idle
-// for a narrow matrix of few rows.  us, passes | GEMM: 13611 x 4096 at 9 / 17 / 64 rows 28 / 41 / 116 | 17 / 21 / 42, 2339 x 11520 at
-// 17 / 32 rows 31 / 41 | 32 / 32, 155 x 5632 at 9 / 32 rows 17 / 29 | 23 / 18; two million products and less are one launch's cost either way.
-// Over 30 shapes x 15 row counts the line takes 0.43 of the passes' time.
-// Long rows whose super-blocks the passes split well, on units that hold one workgroup, stay with them a little longer: 1041 x 12288 at
-// 25 / 32 rows 31.9 / 32.5 | 33.4 / 33.5 (14336 columns: 39.2 / 40.2 | 38.2 / 38.4), 3328 x 11264 at 17 / 24 rows 29.3 / 30.3 | 30.8 / 31.3.
+// Between the two by estimated time, us:
+//   passes  5.1 + ceil(n / 8) (0.75 + 0.26 (w - 1) + rounds (0.31 nb / w + 0.05 nb) + 0.115 MB), w wavefronts per row tile
+//   GEMM    6.8 + 0.51 nb + 1.18 nb x activation tiles per workgroup x rounds after the first + 0.07 MB
+// A pass waits for nb / w stages of a wavefront whatever the units that it leaves idle; the GEMM's four row tiles to a workgroup leave
+// more of them idle, but its time does not grow with the rows until they fill the units.  Least squares over 84 shapes (32 to 32,000
+// rows, 1 to 63 super-blocks) at 9 to 33 rows.  At 18 row counts from 9 to 96 of each the choice takes 0.565 of the passes' time and 1.008
+// of the faster one's; it is over 3 % behind the passes on 1 %, at most 8 % (1836 x 10752 at 17 rows 30.1 -> 32.5 us).  On 58 shapes that
+// were not fitted: 0.575 of the passes' time, 0.7 % over 3 % behind, at most 9 % (263 x 9984 at 17 rows 26.9 -> 29.2).  us, passes | GEMM:
+// 13611 x 4096 at 9 / 17 / 64 rows 28 / 41 / 116 | 17 / 21 / 42, 1041 x 12288 at 17 / 25 / 33 rows 31.6 / 40.0 / 49.6 | 36.0 / 36.0 / 36.6,
+// 155 x 5632 at 9 / 17 rows 16.3 / 22.6 | 17.7 / 18.2.  Two million products and less are the cost of two launches either way and stay
+// with the passes, as do up to eight rows, whose bits are those of the row alone.
 constexpr int64_t kQ80GemmMaxRows = 16 * 65535, kQ80GemmMinProducts = 1 << 21;
-static bool q80_gemm_applies(const mq_weight* w, int64_t n) {
-    if (n > kQ80GemmMaxRows || w->nb > 65535 || w->rows * w->cols * n < kQ80GemmMinProducts) return false;
-    const int64_t units = compute_units();
-    if (w->rowtiles >= 2 * units) return n >= 9;
-    const int waves = pick_waves(w->nb, w->rowtiles);
-    if (4 * w->rowtiles >= 3 * units) return n >= (w->rowtiles <= units && waves == 4 && w->nb > 40 ? 25 : 17);
-    return n >= (3 * w->rowtiles <= units && waves == 8 && w->nb >= 48 && w->nb < 56 ? 33 : 25);
+static bool q80_gemm_applies(int64_t rows, int64_t nb, int64_t n) {
+    if (n <= 8 || n > kQ80GemmMaxRows || nb > 65535 || rows * nb * kQK * n < kQ80GemmMinProducts) return false;
+    const int64_t rowtiles = (rows + 15) / 16, units = compute_units(), w = pick_waves(nb, rowtiles), mt = q80_gemm_tiles(rows, n);
+    const float k = (float)nb, mb = 272e-6f * (float)rows * k, rounds = (float)((rowtiles * w + 8 * units - 1) / (8 * units));
+    const float load = (float)((rowtiles + 3) / 4 * (((n + 15) / 16 + mt - 1) / mt)) / (float)(2 * units);
+    const float passes = 5.1f + (float)((n + 7) / 8) * (0.75f + 0.26f * (float)(w - 1) + rounds * (0.31f * k / (float)w + 0.05f * k) + 0.115f * mb);
+    const float gemm = 6.8f + 0.51f * k + (load > 1.0f ? 1.18f * k * (float)mt * (load - 1.0f) : 0.0f) + 0.07f * mb;
+    return gemm < 0.97f * passes;
 }
 static int mul_mat_q80_locked(const mq_weight* w, const float* x_dev, int64_t n, int64_t ldx, float* y_dev, int64_t ldy,
                               int32_t* dbg_sum, hipStream_t s) {
     if ((ldx & 3) || (reinterpret_cast<uintptr_t>(x_dev) & 15u))
         return fail(MQ_ERR_INVALID, "Q8_0 product: activation rows must be 16-byte aligned (ldx %% 4 == 0)");
-    if (!dbg_sum && q80_gemm_applies(w, n)) {
+    if (!dbg_sum && q80_gemm_applies(w->rows, w->nb, n)) {
         MQ_HIP(g.ap.reserve(q80_tiles_bytes(n, w->nb)));
         MQ_HIP(launch_q80_gemm(w->data, w->rows, w->nb, x_dev, n, ldx, (uint8_t*)g.ap.ptr, y_dev, ldy, s));
         return MQ_OK;
@@ -2222,11 +2228,19 @@ int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
 }
 
 int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out) {
-    if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !path_out)
+    const bool q80 = wtype == kTypeQ80 && !pair;
+    if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K && !q80) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !path_out)
         return fail(MQ_ERR_INVALID, "mq_debug_dense_path: bad type, size or pointer");
-    path_out[0] = dense_path_of(wtype, rows, cols / kQK, n, pair != 0);
-    path_out[1] = dense_waves(cols / kQK, (rows + 15) / 16);
-    path_out[2] = skinny16_applies(cols / kQK, (rows + 15) / 16, pair != 0, n, wtype) ? dense_lds_wpr(cols / kQK, (rows + 15) / 16) : 0;
+    const int64_t nb = cols / kQK, rowtiles = (rows + 15) / 16;
+    if (q80) {
+        path_out[0] = q80_gemm_applies(rows, nb, n) ? kGemm : kPasses;
+        path_out[1] = pick_waves(nb, rowtiles);
+        path_out[2] = q80_gemm_tiles(rows, n);
+        return MQ_OK;
+    }
+    path_out[0] = dense_path_of(wtype, rows, nb, n, pair != 0);
+    path_out[1] = dense_waves(nb, rowtiles);
+    path_out[2] = skinny16_applies(nb, rowtiles, pair != 0, n, wtype) ? dense_lds_wpr(nb, rowtiles) : 0;
     return MQ_OK;
 }
 

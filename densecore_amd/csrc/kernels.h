@@ -178,6 +178,7 @@ size_t q80_scale_bytes(int64_t n, int64_t nb);
 hipError_t launch_quantize_q80(const float* x, int64_t n, int64_t ldx, int64_t cols, uint8_t* aq, uint16_t* ah, hipStream_t stream);
 // Dense Q8_0 product of many rows: quantizer into tiles of sixteen rows (q80_tiles_bytes(n, nb) bytes at ap), then the GEMM.
 size_t q80_tiles_bytes(int64_t n, int64_t nb);
+int q80_gemm_tiles(int64_t rows, int64_t n);  // activation tiles that a workgroup takes: 1, 2 or 4
 hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy,
                            hipStream_t stream);
 hipError_t launch_q80_matmul(const Q80MatmulArgs& a, hipStream_t stream);

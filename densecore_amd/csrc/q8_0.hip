@@ -348,6 +348,12 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
 
 }  // namespace
 
+// Activation tiles to a workgroup: as many as leave two workgroups for every unit
+int q80_gemm_tiles(int64_t rows, int64_t n) {
+    const int64_t row_wgs = ((rows + 15) / 16 + 3) / 4, m_tiles = (n + 15) / 16, enough = 2 * (int64_t)compute_units();
+    return row_wgs * ((m_tiles + 3) / 4) >= enough ? 4 : row_wgs * ((m_tiles + 1) / 2) >= enough ? 2 : 1;
+}
+
 size_t q80_tiles_bytes(int64_t n, int64_t nb) { return (size_t)((n + 15) / 16) * (size_t)nb * kQ80ATileBytes; }
 
 hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy, hipStream_t stream) {
@@ -356,13 +362,12 @@ hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const flo
     if (nb > 65535 || m_tiles > 65535 || (ldx & 3) || (reinterpret_cast<uintptr_t>(x) & 15u)) return hipErrorInvalidValue;
     MQ_LAUNCH(quantize_q80_tiles_kernel, dim3((unsigned)m_tiles, (unsigned)nb), dim3(256), 0, stream, x, n, ldx, m_tiles, ap);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    // as many activation tiles to a workgroup as leave two workgroups for every unit
-    const int64_t enough = 2 * (int64_t)compute_units();
+    const int tiles = q80_gemm_tiles(rows, n);
 #define MQ_Q80(MT)                                                                                                                     \
     MQ_LAUNCH(q80_gemm_kernel<MT>, dim3((unsigned)row_wgs, (unsigned)((m_tiles + MT - 1) / MT)), dim3(256), 0, stream, w, rowtiles, rows, (int)nb, \
               (const uint8_t*)ap, m_tiles, n, y, ldy)
-    if (row_wgs * ((m_tiles + 3) / 4) >= enough) MQ_Q80(4);
-    else if (row_wgs * ((m_tiles + 1) / 2) >= enough) MQ_Q80(2);
+    if (tiles == 4) MQ_Q80(4);
+    else if (tiles == 2) MQ_Q80(2);
     else MQ_Q80(1);
 #undef MQ_Q80
     return hipGetLastError();

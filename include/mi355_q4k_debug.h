@@ -77,7 +77,8 @@ int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
 
 /* Kernels that a dense product of n rows (pair != 0: gate and up in one call) runs on, for a 256-unit device before mq_init.  path_out:
  * 0 passes of eight or sixteen rows, 1 tiles of sixteen, 2 the matrix-core GEMM; wavefronts per row tile of the passes, and of the
- * tiles of sixteen (0: not built for this product). */
+ * tiles of sixteen (0: not built for this product).  Q8_0 (pair == 0): 0 or 2; wavefronts per row tile of the passes; activation tiles
+ * per workgroup of the GEMM. */
 int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out);
 
 /* Measurement instrument: while on != 0 every compute and routing launch of the library is replaced by a kernel with

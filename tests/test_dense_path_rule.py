@@ -24,3 +24,22 @@ def test_tiles_of_sixteen_split_a_row_like_the_passes():
         for n in (9, 16, 17, 33, 64):
             path, passes, sixteens = dense_path(wtype, rows, nb, n, pair)
             assert sixteens in (0, passes) and (path != SIXTEENS or sixteens), (wtype, rows, nb, n, pair)
+
+
+def test_q80_rule_has_no_single_widths():
+    """The row count from which the GEMM takes a Q8_0 product, over row lengths that the passes split over one wavefront count (eight, and
+    four of more than 128 row tiles): longer rows keep it waiting, none of them alone."""
+    def first(rows, nb):
+        return next(n for n in range(1, 100) if dense_path(8, rows, nb, n)[0] == GEMM)
+    for rows in (200, 700, 1041, 2000, 3328, 4096, 5000, 9000):
+        for lengths in (range(8, 72, 8), range(36, 68, 8)):
+            firsts = [first(rows, nb) for nb in lengths]
+            assert firsts == sorted(firsts) and firsts[0] > 8, (rows, list(lengths), firsts)
+
+
+def test_q80_up_to_eight_rows_are_passes_and_many_are_not():
+    rng = random.Random(7)
+    for _ in range(20000):
+        rows, nb, n = int(2 ** rng.uniform(4, 17)), rng.randint(1, 64), rng.randint(1, 8)
+        assert dense_path(8, rows, nb, n)[0] == PASSES, (rows, nb, n)
+        assert dense_path(8, rows, nb, 64)[0] == (GEMM if rows * nb * 256 * 64 >= 1 << 21 else PASSES), (rows, nb)
