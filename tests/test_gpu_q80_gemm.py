@@ -7,25 +7,31 @@ import pytest
 
 from densecore_amd import synth
 from oracle import binding as orc
-from tests._parity import assert_fp32_parity
+from tests._parity import GEMM, assert_fp32_parity, dense_path
 
 pytestmark = pytest.mark.gpu
 Q80 = synth.GGML_TYPE_Q8_0
 
 
-# one, two and four activation tiles to a workgroup, a part of the last one; whole and ragged row tiles; one and several super-blocks;
-# the smallest row count of each range of matrix rows
-@pytest.mark.parametrize("rows,cols,n", [(600, 256, 25), (1000, 2048, 31), (1003, 1792, 33), (3072, 512, 17), (8192, 256, 9), (8200, 512, 63), (8192, 256, 64),
-                                         (16500, 256, 129), (40, 1024, 512), (2048, 768, 1030)])
-def test_many_rows_match_eight_at_a_time(rows, cols, n):
+# one, two and four activation tiles to a workgroup, whole and partial last ones; whole and ragged row tiles; one and several super-blocks
+@pytest.mark.parametrize("rows,cols,n,tiles", [(600, 256, 25, 1), (1000, 2048, 31, 1), (1003, 1792, 33, 1), (3072, 512, 17, 1), (8192, 256, 9, 1),
+                                               (8200, 512, 63, 1), (8192, 256, 64, 1), (40, 1024, 512, 1), (16500, 512, 33, 2), (16500, 768, 48, 2),
+                                               (16400, 512, 64, 2), (16500, 256, 129, 4), (2048, 768, 1030, 4)])
+def test_many_rows_match_eight_at_a_time(rows, cols, n, tiles):
     import torch
-    from densecore_amd import ops
+    from densecore_amd import _lib, ops
+    path, _, mt = dense_path(Q80, rows, cols // 256, n)
+    assert (path, mt) == (GEMM, tiles)
     w = ops.Q4KWeight.synthetic(rows + n, rows, cols, 1, Q80)
     x = torch.randn(n, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
     want = torch.cat([ops.mul_mat(w, x[i:i + 8]) for i in range(0, n, 8)])
     got = ops.mul_mat(w, x)
     assert (got - want).abs().max().item() <= 1e-5 * want.abs().max().item()
-    assert torch.equal(got, ops.mul_mat(w, x.contiguous()))
+    apart = torch.full((n, cols + 20), float("nan"), device="cuda")  # rows 4 * 5 floats apart, not numbers between them
+    apart[:, :cols] = x
+    again = torch.empty_like(got)
+    _lib.check(_lib.lib().mq_mul_mat_q4k(w._h, apart.data_ptr(), n, cols + 20, again.data_ptr(), rows, torch.cuda.current_stream().cuda_stream), "mq_mul_mat_q4k")
+    assert torch.equal(got, again)
     w.free()
 
 
