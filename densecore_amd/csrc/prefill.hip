@@ -729,10 +729,13 @@ __global__ void __launch_bounds__(1024) moe_gemm_plan_kernel(const int32_t* __re
                                                              int groups_max, int sh_tokens, int sh_slot, int sh_silu_mode,
                                                              int32_t* __restrict__ plan, int32_t* __restrict__ row_src,
                                                              int32_t* __restrict__ out_row, int mt, int plan_wgs, GroupedRows rows) {
-    if ((int)blockIdx.x >= plan_wgs) {  // sixteen rows of a super-block, one per wavefront
-        const uint32_t per_block = (uint32_t)((rows.n + 15) / 16), q = blockIdx.x - (uint32_t)plan_wgs, b = q / per_block;
-        const int64_t row = (int64_t)(q - b * per_block) * 16 + (threadIdx.x >> 6);
-        if (row < rows.n) quantize_prow(rows, row, b, threadIdx.x & 63);
+    if ((int)blockIdx.x >= plan_wgs) {  // sixteen rows of a super-block, one per wavefront, and again as many workgroups further
+        const uint32_t per_block = (uint32_t)((rows.n + 15) / 16), runs = per_block * (uint32_t)rows.nb;  // < 2^31: host-checked
+        for (uint32_t q = blockIdx.x - (uint32_t)plan_wgs; q < runs; q += gridDim.x - (uint32_t)plan_wgs) {
+            const uint32_t b = q / per_block;
+            const int64_t row = (int64_t)(q - b * per_block) * 16 + (threadIdx.x >> 6);
+            if (row < rows.n) quantize_prow(rows, row, b, threadIdx.x & 63);
+        }
         return;
     }
     extern __shared__ int32_t plan_sh[];  // begin[g], tile0[g], item0[g]: groups_max + 2 each
@@ -832,8 +835,11 @@ size_t moe_gemm_plan_ints(int64_t entries, int64_t groups_max) {
 hipError_t launch_moe_gemm_plan(const int32_t* n_groups, const int32_t* group_expert, const int32_t* group_begin,
                                 const int32_t* entry_token, const int32_t* entry_k, int slots, bool src_per_slot, int64_t entries,
                                 int64_t groups_max, int64_t sh_tokens, int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt, const GroupedRows& rows) {
-    const int64_t quant_wgs = rows.x ? (rows.n + 15) / 16 * rows.nb : 0;
-    if (quant_wgs >= ((int64_t)1 << 31) - 64 || (rows.x && (rows.nb > 65535 || rows.n >= (int64_t)1 << 31)) || groups_max > 4097 || (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup)) return hipErrorInvalidValue;
+    // (a grid holds fewer than 2^32 threads, four million workgroups of 1024: beyond kQuantWgs a workgroup takes several runs of rows)
+    constexpr int64_t kQuantWgs = 1 << 16;
+    const int64_t quant_runs = rows.x ? (rows.n + 15) / 16 * rows.nb : 0, quant_wgs = quant_runs < kQuantWgs ? quant_runs : kQuantWgs;
+    if (quant_runs >= (int64_t)1 << 31 || (rows.x && (rows.nb > 65535 || rows.n >= (int64_t)1 << 31))) return hipErrorInvalidValue;
+    if (groups_max > 4097 || (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup)) return hipErrorInvalidValue;
     int32_t* row_src = plan + 4 + 3 * moe_gemm_items_max(entries, groups_max);
     int32_t* out_row = row_src + 16 * moe_gemm_tiles_max(entries, groups_max);
     const int64_t rows_max = 16 * moe_gemm_tiles_max(entries, groups_max);

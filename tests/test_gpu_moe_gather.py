@@ -83,3 +83,17 @@ def test_few_experts_below_the_prefill_widths_match_eight_tokens_at_a_time(exper
         assert (d - dw).abs().max().item() <= 1e-5 * dw.abs().max().item(), n
     for t in (G, U, D) + (tuple(sh[:3]) if sh else ()):
         t.free()
+
+
+def test_more_runs_of_rows_than_workgroups_quantize_them():
+    """256 tiles of rows x 260 super-blocks are more than the launch has workgroups for: the second run of a workgroup, against halves that need none."""
+    import torch
+    from densecore_amd import ops
+    experts, n, cols = 8, 4090, 260 * 256
+    w = ops.Q4KWeight.synthetic(53, 16, cols, experts)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn((n, cols), device="cuda", generator=gen)
+    ids = torch.randint(0, experts, (n, 1), device="cuda", generator=gen, dtype=torch.int32)
+    want = torch.cat([ops.mul_mat_id(w, x[i:i + 2045], ids[i:i + 2045]) for i in (0, 2045)])
+    assert torch.equal(ops.mul_mat_id(w, x, ids), want)
+    w.free()
