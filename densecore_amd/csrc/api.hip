@@ -583,10 +583,9 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // timed: the choice takes 0.936 (pairs 0.968) of the plain rule's time, 0.62 (0.53) where it differs, and nowhere more; 1.018 (1.024) of
 // the fastest one's -- with tiles of sixteen split by counts that divide a row's super-blocks only; since they split like the passes (the
 // estimate reads the same stages), 300 products of uneven splits take 0.82 of the time they took, 3 % of them over 1.05 of it.  The line is at
-// three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of one
-// to three super-blocks, which were not fitted, gain where the estimate leaves: 33 to 47 rows, three types, 0.21 to 0.62 of the time
-// (30000 x 512 Q4_K at 33 rows 25.2 -> 9.8 us, 6000 x 256 Q6_K 42.4 -> 9.6); four super-blocks 0.42 to 0.77.  A pair's GEMM is not
-// estimated closely enough at these widths (0.6 to 1.6 of its time) to leave the decode kernels for.
+// three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of up
+// to four super-blocks never leave them below 48 (that equality is tested there); a pair's GEMM is not estimated closely enough at
+// these widths (0.6 to 1.6 of its time) to leave them for.
 // Up to kDecodeRows rows the GEMM is never taken: a row's bits are those of the row alone there, and the products that cannot take it
 // (mq_mul_mat_q4k_noalloc, whose scratch holds no planes of partial sums) return them as well.  It would be for one product in a
 // hundred, 11008 columns and more in few row tiles.
@@ -627,7 +626,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         us[kSixteens] = c.sixteens[0] + stages(dense_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
     }
     const float decode = us[kSixteens] < us[kPasses] ? us[kSixteens] : us[kPasses];
-    if (plain == kGemm || (n > kDecodeRows && !swiglu && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
+    if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > 4 && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
         GemmShape shape;
         float gemm;
         if (swiglu && gemm_pair_shape(type, rows, nb, n, false, &shape)) {

@@ -26,12 +26,6 @@ def test_tiles_of_sixteen_split_a_row_like_the_passes():
             assert sixteens in (0, passes) and (path != SIXTEENS or sixteens), (wtype, rows, nb, n, pair)
 
 
-def test_short_rows_follow_the_estimate_like_long_ones():
-    for wtype in (12, 13, 14):
-        for nb in range(2, 9):
-            assert [dense_path(wtype, 30000, nb, n)[0] for n in (33, 40, 47)] == [GEMM] * 3, (wtype, nb)
-
-
 def test_q80_rule_has_no_single_widths():
     """The row count from which the GEMM takes a Q8_0 product, over row lengths that the passes split over one wavefront count (eight, and
     four of more than 128 row tiles): longer rows keep it waiting, none of them alone."""

@@ -3,8 +3,6 @@ would walk alone, rows a little beyond a pass of sixteen.  Against the same rows
 to the oracle elsewhere): the same integers, fp32 sums in another order, one fp32 rounding per super-block and product term."""
 import pytest
 
-from tests._parity import GEMM, dense_path
-
 pytestmark = pytest.mark.gpu
 
 
@@ -24,21 +22,6 @@ def test_products_match_their_rows_eight_at_a_time(wtype, rows, nb):
         got = ops.mul_mat(w, x[:n])
         # nb <= 53 roundings of 2^-24 on either side, each at most the largest partial sum (a few times the largest result)
         assert (got - want[:n]).abs().max().item() <= 1e-5 * want.abs().max().item(), n
-    w.free()
-
-
-# rows of one to four super-blocks, whole and ragged row tiles
-@pytest.mark.parametrize("rows,nb,wtype", [(33, 1, 14), (80003, 1, 12), (6000, 1, 13), (16403, 2, 12), (30000, 2, 14), (20001, 3, 13), (16400, 4, 12), (25000, 4, 14)])
-def test_short_rows_match_their_rows_eight_at_a_time(rows, nb, wtype):
-    import torch
-    from densecore_amd import ops
-    w = ops.Q4KWeight.synthetic(rows * 64 + nb, rows, 256 * nb, 1, wtype)
-    x = torch.randn((48, 256 * nb), device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows))
-    want = pieces(torch, lambda t: ops.mul_mat(w, t), x)
-    for n in (32, 33, 40, 47, 48):
-        assert n not in (33, 40, 47) or dense_path(wtype, rows, nb, n)[0] == GEMM
-        got = ops.mul_mat(w, x[:n])
-        assert (got - want[:n]).abs().max().item() <= 1e-5 * want.abs().max().item(), n  # (as above)
     w.free()
 
 
