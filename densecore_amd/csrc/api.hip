@@ -193,8 +193,7 @@ bool dense_lds_quantizes(const mq_weight* w, const float* x, int64_t n, int64_t 
 
 // Nine to 64 rows of a Q4_K, Q5_K or Q6_K matrix: one to four activation tiles of sixteen rows per weight tile
 // (skinny16_kernel, the same bits as the token tiles of eight of the other decode kernels); mq_debug_set_dense_lds
-// bit 12 turns it off.  kSkinnyMaxRows: beyond it the matrix-core GEMM (large matrices) or the 16-row passes of the
-// decode kernels take over.
+// bit 12 turns it off.  kSkinnyMaxRows: beyond it the matrix-core GEMM takes over (handles: the passes of the decode kernels).
 int g_skinny16 = 1;
 constexpr int64_t kSkinnyMaxRows = 64;
 bool skinny16_takes(const mq_weight* w, int64_t n, bool swiglu) {
@@ -583,9 +582,10 @@ static int matmul_from_ws(const mq_weight* w, int64_t n, float* y, int64_t ldy, 
 // timed: the choice takes 0.936 (pairs 0.968) of the plain rule's time, 0.62 (0.53) where it differs, and nowhere more; 1.018 (1.024) of
 // the fastest one's -- with tiles of sixteen split by counts that divide a row's super-blocks only; since they split like the passes (the
 // estimate reads the same stages), 300 products of uneven splits take 0.82 of the time they took, 3 % of them over 1.05 of it.  The line is at
-// three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Rows of up
-// to four super-blocks never leave them below 48 (that equality is tested there); a pair's GEMM is not estimated closely enough at
-// these widths (0.6 to 1.6 of its time) to leave them for.
+// three quarters because a row's bits are those of the row alone on the decode kernels: worth leaving for a real gain only.  Below 48
+// rows matrices that the plain rule keeps there never leave them for the GEMM where rows have up to four super-blocks, by promise
+// (mi355_q4k.h): 33 to 47 rows are three passes there, up to four times the GEMM's time from 6,000 weight rows on (30000 x 512 Q4_K at
+// 33 rows 25.2 against 9.8 us).  Nor do pairs, whose GEMM is not estimated closely enough at these widths (0.6 to 1.6 of its time).
 // Up to kDecodeRows rows the GEMM is never taken: a row's bits are those of the row alone there, and the products that cannot take it
 // (mq_mul_mat_q4k_noalloc, whose scratch holds no planes of partial sums) return them as well.  It would be for one product in a
 // hundred, 11008 columns and more in few row tiles.
@@ -606,6 +606,7 @@ constexpr PathCost kPathCost[2][3] = {
      {{7.63f, 1.57f, 1.123f, 0.156f}, {9.86f, 0.574f, 0.730f, 0.258f, 0.030f}, {13.07f, 0.559f}},
      {{7.89f, 2.00f, 1.378f, 0.342f}, {10.17f, 0.498f, 0.562f, 0.000f, 0.146f}, {10.23f, 0.899f}}}};
 constexpr float kPathLess = 0.77f;
+constexpr int64_t kDecodeShortBlocks = 4;
 static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bool swiglu) {
     if ((type != kTypeQ4K && type != kTypeQ5K && type != kTypeQ6K) || n <= 8) return kPasses;
     if (n > kSkinnyMaxRows) return kGemm;
@@ -626,7 +627,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         us[kSixteens] = c.sixteens[0] + stages(dense_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
     }
     const float decode = us[kSixteens] < us[kPasses] ? us[kSixteens] : us[kPasses];
-    if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > 4 && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
+    if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > kDecodeShortBlocks && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
         GemmShape shape;
         float gemm;
         if (swiglu && gemm_pair_shape(type, rows, nb, n, false, &shape)) {
@@ -1833,7 +1834,8 @@ int decoder_grid(size_t lds_bytes, int* n_workgroups, long long* spin_ticks) {
 
 // The expert-grouped GEMM pays from six routed rows per expert on average (its workgroups multiply 16-row tiles, two,
 // four or eight of an expert at a time): 256 experts, top-8, 2048 x 512: 152 against 153 us per block at 192 tokens, 158
-// against 186 at 256, 164 against 217 at 320 -- and 141 against 119 at 128, where the decode kernels' 8-row groups stay.
+// against 186 at 256, 164 against 217 at 320 -- and 141 against 119 at 128, where the decode kernels' 8-row groups stay; fewer experts
+// cross earlier (below).
 // Decided per product: gate / up (one type) and down each run on it when their type is one it takes; a layer with
 // a Q8_0 down stack (core/src/llm/moe/native.cpp:4611-4620; its activations are Q8_0 as well) keeps its two large
 // products on the matrix cores and sends the fp32 hidden rows through the Q8_0 launches.
@@ -1844,7 +1846,8 @@ static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
     if (ge->n_experts > 4096 || (ge->rows & 3) || (ge->cols & 3)) return false;
     // (256 + 1 experts, top-8, 2048 x 512, the expert-grouped decode launches against the GEMM with items of two tiles:
     // 106 / 135 us at 96 tokens, 119 / 141 at 128, 153 / 152 at 192, 186 / 158 at 256, 217 / 164 at 320)
-    // Below 192 tokens where the down product by itself takes it (moe_gemm_width), so that the layer and its stages agree.  Over 1,050
+    // Below 192 tokens where the down product by itself takes it (moe_gemm_width); the gate/up node asks for its own matrices, and comes to
+    // another choice for about one block in seven of 17 to 191 tokens.  Over 1,050
     // blocks of 8 to 128 experts, top-2 to 8, 9 to 190 tokens and five shapes: 0.82 of the decode launches' time, nowhere more than it
     // (16 experts, top-8, 2816 x 768 at 128 tokens 354 -> 78 us).
     return n >= 192 ? n * L->top_k >= 6 * ge->n_experts : moe_gemm_width(L->down_exps, n, L->top_k, 1);

@@ -113,7 +113,15 @@ int mq_quantize_q8k(const float* x_dev, int64_t n, int64_t ldx, int64_t k, void*
  * cb_gemv_custom (core/src/llm/matmul/gemv_exec.cpp:99, n == 1),
  * cb_gemv_batched_custom (core/src/llm/matmul/batched_exec.cpp:55, 2 <= n <= 16)
  * and CpuBackend::MatMulGgmlQuantizedTransB
- * (core/include/densecore/backend/cpu_backend.h:293-300, any n). */
+ * (core/include/densecore/backend/cpu_backend.h:293-300, any n).
+ *
+ * The width chooses the kernel.  Q4_K, Q5_K and Q6_K: decode kernels up to 16 rows, the int8 matrix-core GEMM from 65, and
+ * whichever is estimated to be clearly the faster one between (the GEMM from 48 rows, or 17 for matrices of 44 million weights -- 24 MB of
+ * Q4_K -- and more, unless the rows run as tiles of sixteen on the decode arithmetic; earlier or later where that is far off).  All decode kernels return the same
+ * bits: row i of y depends on row i of x alone, bit for bit, up to 16 rows -- and up to 47 rows where the rows of W have at most
+ * 1024 columns and W fewer weights than that.  The GEMM forms the same integers per super-block and adds them up in another order: results
+ * agree to rounding.  Q8_0: passes of eight rows (with the same property) up to eight rows, from nine to 33 rows on -- by estimated
+ * time -- a GEMM whose sums run over the super-blocks in another order, to rounding as well. */
 int mq_mul_mat_q4k(const mq_weight* w, const float* x_dev, int64_t n, int64_t ldx, float* y_dev, int64_t ldy,
                    void* stream);
 /* Several products of ONE activation row in one launch: y_dev[i][r] = w[i][r] . q8k(x), i < count <= 8, all
@@ -126,17 +134,15 @@ int mq_mul_mat_q4k(const mq_weight* w, const float* x_dev, int64_t n, int64_t ld
  * outputs of the list undefined. */
 int mq_mul_mat_q4k_multi(const mq_weight* const* w, int count, const float* x_dev, float* const* y_dev, void* stream);
 /* mq_mul_mat_q4k for callers that cannot allocate (code under HIP-graph capture, serving loops and harnesses that
- * forbid hipMalloc): the same product, bit for bit, for n <= 16 rows of cols <= 16384 (MQ_ERR_UNSUPPORTED beyond
+ * forbid hipMalloc): the same product, bit for bit (neither takes the GEMM there), for n <= 16 rows of cols <= 16384 (MQ_ERR_UNSUPPORTED beyond
  * that), Q4_K / Q5_K / Q6_K weights.  It calls no allocating routine: the quantized activations go to a fixed
  * 528,384-byte device array inside the library (one per GPU, held until the process ends) whose address mq_init
  * looks up.  It has no counterpart in the reference.  Every call on a GPU shares that GPU's array: calls that
  * overlap on one GPU (two streams, two threads' launches in flight together) race; order them on one stream. */
 int mq_mul_mat_q4k_noalloc(const mq_weight* w, const float* x_dev, int64_t n, int64_t ldx, float* y_dev, int64_t ldy,
                            void* stream);
-/* The same product computed by the matrix-core GEMM kernel whatever n is (mq_mul_mat_q4k switches to it
- * by itself from 48 rows up, from 17 for matrices of 24 MB and more; Q4_K products stay on the decode arithmetic up to
- * 32 rows, up to 64 where their rows pass through LDS in runs of super-blocks, Q5_K and Q6_K products likewise): weights are read once per 128 activation rows and the int8 MFMA
- * units do the arithmetic.  RunQ4KRawBatchedDenseGemm (core/src/backend/cpu_backend_q4k_dense.cpp:57-101),
+/* The same product computed by the matrix-core GEMM kernel whatever n is (mq_mul_mat_q4k switches to it by itself between 17 and 65
+ * rows, see there): weights are read once per 128 activation rows and the int8 MFMA units do the arithmetic.  RunQ4KRawBatchedDenseGemm (core/src/backend/cpu_backend_q4k_dense.cpp:57-101),
  * the A.shape[0] >= 4 branch of MatMulGgmlQuantizedTransBWithPath
  * (core/src/backend/cpu_backend_quantized_matmul.cpp:164-170).  Same integers per super-block as
  * mq_mul_mat_q4k; the fp32 update uses fused multiply-adds, so results agree to rounding, not bitwise. */
@@ -157,7 +163,8 @@ int mq_mul_mat_q4k_host(const mq_weight* w, const float* x_host, int64_t n, int6
  * (core/src/llm/matmul/gemv_exec.cpp:298-341, MatmulWorkState core/src/llm/runtime/work_state.h:86-89)
  * and with Qwen35SharedQ8RowsUserData (core/src/llm/moe/native.cpp:1027-1038).
  * create/free allocate and must stay outside a HIP-graph capture; quantize and the two products
- * only launch kernels.  n of the products is the n of the handle's last mq_acts_quantize. */
+ * only launch kernels.  n of the products is the n of the handle's last mq_acts_quantize (or mq_add_rmsnorm_q8k).  They stay
+ * on the decode kernels at every width: a row's bits are those of the row alone, whichever call filled the handle. */
 typedef struct mq_acts mq_acts;
 int mq_acts_create(int64_t max_rows, int64_t cols, mq_acts** out);
 int mq_acts_free(mq_acts* a);
@@ -170,9 +177,9 @@ int mq_swiglu_mul_mat_q4k_acts(const mq_weight* gate, const mq_weight* up, const
  * h[m][r] = silu(gate[r] . q8k(x[m])) * (up[r] . q8k(x[m])), one pass over both matrices.
  * FusedSwiGLUQ4KQ8KRows_Hwy (core/include/densecore/simd/hwy_ops.h:275-281,
  * core/src/kernels/hwy/hwy_moe_quant.cc:359-380) and RunMoEQ4KRawBatchedFusedSwiGLUImpl
- * (core/src/backend/cpu_backend_moe_raw_batched.inl:1629-1698).  Wherever mq_mul_mat_q4k would take the
- * matrix-core GEMM (Q4_K, 48 rows and more, 17 for matrices of 24 MB and more; 16-byte aligned h rows) the two
- * products run on it and a third launch forms h. */
+ * (core/src/backend/cpu_backend_moe_raw_batched.inl:1629-1698).  Kernels by width as in mq_mul_mat_q4k (the choice is
+ * made for the pair; below 48 rows and 44 million weights a matrix never the GEMM); on the GEMM (16-byte aligned h rows) one launch
+ * forms h, or two products and a third launch where that is faster. */
 int mq_swiglu_mul_mat_q4k(const mq_weight* gate, const mq_weight* up, const float* x_dev, int64_t n, int64_t ldx,
                           float* h_dev, int64_t ldh, int silu_mode, void* stream);
 
@@ -180,9 +187,9 @@ int mq_swiglu_mul_mat_q4k(const mq_weight* gate, const mq_weight* up, const floa
  * y = down( silu(gate x) * (up x) ), x_dev [n][hidden], y_dev [n][hidden].
  * gate/up: rows = inter, cols = hidden; down: rows = hidden, cols = inter.
  * The three smart_mul_mat calls plus cb_silu_mul_fused of a dense FFN block
- * (core/src/llm/graph/decoder.cpp:2662-2730, core/src/llm/graph/fused_ops.cpp:317-366).  Prefill widths (the
- * row counts from which mq_mul_mat_q4k takes the matrix-core GEMM for both shapes) run as three GEMMs, the SwiGLU
- * formed by the quantizer of the down product: 4096 -> 14336 -> 4096 at 512 / 2048 rows in 0.27 / 0.95 ms. */
+ * (core/src/llm/graph/decoder.cpp:2662-2730, core/src/llm/graph/fused_ops.cpp:317-366).  Each of the
+ * two steps (gate and up, down) takes the kernel that mq_swiglu_mul_mat_q4k and mq_mul_mat_q4k take for its shape and
+ * width; prefill widths run on the matrix-core GEMM throughout: 4096 -> 14336 -> 4096 at 512 / 2048 rows in 0.25 / 0.76 ms. */
 int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weight* down, const float* x_dev,
                       int64_t n, float* y_dev, int silu_mode, void* stream);
 
@@ -209,9 +216,11 @@ int mq_moe_weights_from_logits(const float* logits_dev, int64_t n_experts, int64
  * by expert on the device; nothing returns to the host.  y_dev fp32
  * [n][top_k][rows].  (ggml_mul_mat_id as emitted at
  * core/src/llm/moe/native_gemma.cpp:1509-1559.)  Prefill widths (192 tokens
- * and more with six rows per expert on average) run on the int8 matrix-core
- * GEMM in its expert-grouped form, as do mq_moe_gateup_swiglu_q4k and
- * mq_moe_down_weighted_q4k below. */
+ * and more with six rows per expert on average, and from 17 tokens with five rows
+ * per expert where an estimate says that it is clearly faster: few experts) run on
+ * the int8 matrix-core GEMM in its expert-grouped form, as do
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, each by its own
+ * matrices' estimate. */
 int mq_mul_mat_id_q4k(const mq_weight* w_exps, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
                       int top_k, float* y_dev, void* stream);
 
@@ -240,10 +249,12 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * Up to eight tokens (and 512 experts) two launches: gate/up + SwiGLU with the router and the Q8_K of x inside,
  * down with the Q8_K of the hidden rows and the weighted combine inside.  Above: router + expert grouping + Q8_K
  * of x, expert-grouped gate/up leaving its rows in Q8_K, expert-grouped down, combine.  Same bits either way.
- * Prefill widths (192 tokens and more with six routed rows per expert on average): the expert products run on the
+ * Prefill widths (192 tokens and more with six routed rows per expert on average; from 17 tokens with five where the down product's
+ * estimate says so, e.g. 16 experts, top-8, 2816 x 768 at 128 tokens): the expert products run on the
  * int8 matrix-core GEMM in an expert-grouped form (entries in 16-row tiles per expert), the shared expert as one more
  * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches; same routing, results within the fp32 tolerance of the other form (the
- * summation order differs), and mq_debug_moe_hidden does not apply. */
+ * summation order differs), and mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.  Between 17 and 191
+ * tokens mq_moe_gateup_swiglu_q4k decides by itself, so the layer and its nodes may take different forms there and agree to that tolerance. */
 typedef struct {
     const mq_weight* gate_exps; /* n_experts x [inter][hidden]  */
     const mq_weight* up_exps;

@@ -3,7 +3,7 @@
  *
  * Exported by the same library as the entry points of mi355_q4k.h, kept apart from them: a DenseCore host binds
  * mi355_q4k.h; tests and benchmarks also include this file.  None of these calls changes what a product entry point
- * computes; mq_debug_set_dense_lds selects between kernels that return the same bits.
+ * computes; mq_debug_set_dense_lds selects between kernels that return the same bits up to 16 rows and agree to rounding beyond.
  */
 #ifndef MI355_Q4K_DEBUG_H
 #define MI355_Q4K_DEBUG_H
@@ -65,9 +65,10 @@ int mq_census_read(int kind, double* avg_us, double* min_us, double* max_us, int
  * ones; bit 3 (on = 9) makes gate and up at prefill widths two GEMM launches and a SwiGLU pass instead of the
  * one launch that stores silu(gate) * up; bits 8..11 force the activation tiles per item of the expert-grouped GEMM (2,
  * 4 or 8; 0 = chosen by the rows per expert); bit 12 keeps dense products of nine to 64 rows on the kernels
- * that multiply them as token tiles of eight (or on the GEMM) instead of the one that takes them as tiles of sixteen.  All
- * return the same bits (tests/test_gpu_dense_lds.py, tests/test_gpu_grouped_lds.py, tests/test_gpu_prefill.py); returns the
- * previous setting of bit 0.  No counterpart in the reference. */
+ * that multiply them as token tiles of eight (or on the GEMM) instead of the one that takes them as tiles of sixteen.  They
+ * return the same bits (tests/test_gpu_dense_lds.py, tests/test_gpu_grouped_lds.py, tests/test_gpu_prefill.py), except that bits 0 and 12
+ * also turn off the choice by estimate between 17 and 64 rows, and bit 3 lets K be cut into runs: a product that so changes between
+ * the decode kernels and the GEMM, or its GEMM's shape, agrees to rounding.  Returns the previous setting of bit 0.  No counterpart in the reference. */
 int mq_debug_set_dense_lds(int on);
 
 /* Launch shape that the matrix-core GEMM takes for a product of n rows (pair 1: for gate and up in one launch, 2: ahead of a down product), for a 256-unit

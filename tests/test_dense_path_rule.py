@@ -19,6 +19,17 @@ def test_up_to_sixteen_rows_stay_on_the_decode_kernels():
         assert dense_path(wtype, rows, nb, 65, pair)[0] == GEMM
 
 
+def test_short_rows_and_pairs_of_ordinary_matrices_stay_on_the_decode_kernels_up_to_47_rows():
+    """Of fewer than 44 million weights (24 MB of Q4_K): rows of up to 1024 columns, and gate/up pairs of any."""
+    rng = random.Random(8)
+    for _ in range(20000):
+        wtype, pair, n = rng.choice((12, 13, 14)), rng.randint(0, 1), rng.randint(17, 47)
+        nb = rng.randint(1, 64 if pair else 4)
+        rows = int(2 ** rng.uniform(4, 15.4)) if not pair else rng.randint(1, (24 << 20) // (144 * nb))
+        if rows * nb * 144 < 24 << 20:
+            assert dense_path(wtype, rows, nb, n, pair)[0] != GEMM, (wtype, rows, nb, n, pair)
+
+
 def test_tiles_of_sixteen_split_a_row_like_the_passes():
     for wtype, rows, nb, pair in products(20000, 6):
         for n in (9, 16, 17, 33, 64):
