@@ -1034,7 +1034,8 @@ int mq_mul_mat_q4k_q8k(const mq_weight* w, const void* q8_dev, int64_t n, size_t
 // up to kStageInKernel bytes come over in a copy kernel; below that the runtime's own copy is as fast (it is a kernel too), above it
 // the copy engine is.  us per call, copies both ways | this, Q4_K: 4096 x 4096 at 1 / 2 / 8 / 48 rows 22.4 / 33.7 / 42.8 / 104 |
 // 20.7 / 23.8 / 31.7 / 100; 14336 x 4096 at 1 / 8 / 48 rows 33.2 / 63.0 / 206 | 25.6 / 49.3 / 197; a copy kernel at 786 KB or 1.5 MB
-// of rows costs 2 to 6 us more than the copy engine.  Larger outputs than 2.75 MB were not measured.
+// of rows costs 2 to 6 us more than the copy engine.  Larger results gain less and less: 3.3 / 4.0 / 5.2 / 8.0 MB 300 / 253 / 313 / 466 |
+// 293 / 247 / 310 / 459.
 constexpr size_t kStageInCopy = 16 << 10, kStageInKernel = 512 << 10, kStageOutDirect = 4 << 20;
 int mq_mul_mat_q4k_host(const mq_weight* w, const float* x_host, int64_t n, int64_t ldx, float* y_host, int64_t ldy) {
     if (int rc = check_ready()) return rc;

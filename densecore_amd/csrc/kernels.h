@@ -254,8 +254,8 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
 // Expert-grouped form of the GEMM (a MoE block at prefill widths): a plan lays the routed entries out in 16-row tiles
 // per expert (moe_gemm_plan_ints() int32 of workspace; sizes from the upper bounds entries = n * top_k and groups_max),
 // the GEMM multiplies every item by its expert's weights.  Its activations: gathered > 0: that many distinct rows in the row layout,
-// fetched by the plan's row list (a gather into tiles ahead of the GEMM cost 15 us of a block of 1500 tokens, top-8 and a shared
-// expert of 2048 columns: 264 -> 246 us without it); 0: tiles in the plan's order.
+// fetched by the plan's row list (without a launch that gathers them into tiles ahead of the GEMM: a block of 256 + 1 experts, top-8,
+// 2048 x 512 at 700 / 1500 tokens 179 / 258 -> 165 / 241 us); 0: tiles in the plan's order.
 // sh_tokens > 0 appends the shared expert as one more group of all tokens (weights w_shared, output slot slots - 1);
 // `entries` and `groups_max` then count its rows and its group as well.
 int64_t moe_gemm_tiles_max(int64_t entries, int64_t groups_max);

@@ -721,7 +721,8 @@ GemmShape choose_shape(const Pace* pace, bool pair, int64_t rows, int64_t nb, in
 // out_row[r] for row r of the tiles: the token whose activations it holds and the row of the per-(token, slot) output
 // it produces (token * slots + k), -1 for padding (src_per_slot: the activations are per (token, slot) rows too).
 // Workgroups past plan_wgs quantize the rows that the GEMM will gather: the plan is a chain of short dependent steps on a few compute
-// units, and the rows need nothing of it (256 + 1 experts, 2048 columns, 1500 tokens: 5.4 + 5.7 us as two launches, 6.9 as one).
+// units, and the rows need nothing of it (256 + 1 experts, 2048 columns, 1500 tokens: 5.4 + 5.7 us as two launches, 6.9 as one;
+// the block 235.9 -> 230.9).
 __global__ void __launch_bounds__(1024) moe_gemm_plan_kernel(const int32_t* __restrict__ n_groups, const int32_t* __restrict__ group_expert,
                                                              const int32_t* __restrict__ group_begin,
                                                              const int32_t* __restrict__ entry_token,
@@ -906,9 +907,9 @@ hipError_t raise_gemm_lds() {
 }
 // Where all super-blocks of an item's tiles fit the LDS of four workgroups to a unit (a down product of two super-blocks; of four with
 // items of two tiles), a workgroup keeps them and takes this many blocks of 64 rows: MoE block of 256 + 1 experts, top-8, 2048 x 512 at
-// 700 / 1500 tokens 171.9 / 257 us without, 169.5 / 253 with one block (a single barrier), 167.7 / 247 with two, 168.7 / 246 with four,
-// 172.3 / 253 with eight (whose last round of workgroups is long); at twice the LDS (two workgroups to a unit) 4096 x 1024 at 300
-// tokens 104 -> 114.
+// 700 / 1500 tokens 165.0 / 240.7 -> 163.4 / 235.0 us.  Shares of the time without, on another card: one block (a single barrier) 0.986 /
+// 0.984, two 0.976 / 0.961, four 0.981 / 0.957, eight 1.002 / 0.984 (their last round of workgroups is long); at twice the LDS (two
+// workgroups to a unit) 4096 x 1024 at 300 tokens 104 -> 114 us.
 constexpr int kResidentTiles = 8, kResidentRowBlocks = 2;
 constexpr int64_t kGatherMaxRows = ((int64_t)1 << 31) / kPRowBytes;  // a row's offset in its plane is a 32-bit one
 int pace_of(int wtype) { return wtype == kTypeQ6K ? 2 : wtype == kTypeQ5K ? 1 : 0; }
