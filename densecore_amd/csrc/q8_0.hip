@@ -267,8 +267,10 @@ __global__ void __launch_bounds__(256) quantize_q80_tiles_kernel(const float* __
 // super-block's sum, which is what bounds it (100 beside eight MFMAs per tile; twelve LDS reads).  A row's sum is two chains, over
 // the even and the odd super-blocks, of chains of eight blocks: against double, the same operands, its error is 0.35 to 0.95 of that of
 // the passes of eight, which split a row over one to eight wavefronts (40 products of 2048 to 14336 columns; 4096 columns on eight
-// wavefronts 0.82e-7 against 0.92e-7, 14336 1.16e-7 against 1.46e-7).  One chain over the row was 1.5 % faster and had up to 2.6 times
-// that error.  The launch of eight-row passes walks all rows
+// wavefronts 0.82e-7 against 0.92e-7, 14336 1.16e-7 against 1.46e-7).  One chain over the row had up to 2.6 times that error;
+// it took 0.97 of the time with one activation tile to a workgroup (154 products of 33 rows and more; at least 0.91, 4096 x 14336 at 64 rows),
+// the same with two, 0.995 with four.  Eight chains, one per block of a super-block, are slower yet with one and two tiles (1.010, 1.025).
+// The launch of eight-row passes walks all rows
 // in one workgroup per row tile: us, passes | this: 8075 x 13312 at 32 / 128 / 500 / 1100 rows 97 / 396 / 1561 / 3438 | 40 / 136 / 206 / 437
 // (541 TOP/s), 920 x 6912 26 / 92 / 369 / 811 | 22 / 23 / 27 / 43.
 template <int MT>
