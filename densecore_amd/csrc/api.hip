@@ -607,7 +607,13 @@ constexpr PathCost kPathCost[2][3] = {
      {{7.89f, 2.00f, 1.378f, 0.342f}, {10.17f, 0.498f, 0.562f, 0.000f, 0.146f}, {10.23f, 0.899f}}}};
 constexpr float kPathLess = 0.77f;
 constexpr int64_t kDecodeShortBlocks = 4;
-static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bool swiglu) {
+// The down product of an FFN whose gate and up run on the GEMM (behind_gemm): the kernel that is estimated to take the least, a row's
+// bits being the GEMM's already, with 2 us more for the decode kernels: they keep the SwiGLU out of the down product's quantizer (two
+// launches for gate and up instead of the pair then win more often).  90 FFNs of 17 to 64 rows whose down product has tiles of
+// sixteen: 0.959 of the time with those, 0.992 of it with the GEMM throughout, 1.006 of the faster one's (Q5_K 6144 -> 9472 at 23 rows 71.2 ->
+// 62.9 us; Q5_K 3072 -> 2816 at 48 rows stays at 37.9 against 42.5).
+constexpr float kBehindGemm = 2.0f;
+static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bool swiglu, bool behind_gemm = false) {
     if ((type != kTypeQ4K && type != kTypeQ5K && type != kTypeQ6K) || n <= 8) return kPasses;
     if (n > kSkinnyMaxRows) return kGemm;
     const int64_t rowtiles = (rows + 15) / 16;
@@ -626,8 +632,9 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         const float far = skinny16_one_run(nb, rowtiles, swiglu, n) ? 0.0f : c.sixteens[3];
         us[kSixteens] = c.sixteens[0] + stages(dense_waves(nb, rowtiles)) * (c.sixteens[1] + tiles * (c.sixteens[2] + far)) + c.sixteens[4] * mb;
     }
+    if (behind_gemm) us[kPasses] += kBehindGemm, us[kSixteens] += kBehindGemm;
     const float decode = us[kSixteens] < us[kPasses] ? us[kSixteens] : us[kPasses];
-    if (plain == kGemm || (n > kDecodeRows && !swiglu && nb > kDecodeShortBlocks && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
+    if (plain == kGemm || behind_gemm || (n > kDecodeRows && !swiglu && nb > kDecodeShortBlocks && decode > 12.0f)) {  // (no GEMM takes less: its search is not worth making)
         GemmShape shape;
         float gemm;
         if (swiglu && gemm_pair_shape(type, rows, nb, n, false, &shape)) {
@@ -639,7 +646,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         us[kGemm] = c.gemm[0] + c.gemm[1] * gemm;
     }
     const DensePath best = us[kGemm] < decode ? kGemm : us[kSixteens] < us[kPasses] ? kSixteens : kPasses;
-    return us[best] < kPathLess * us[plain] ? best : plain;
+    return behind_gemm || us[best] < kPathLess * us[plain] ? best : plain;
 }
 static DensePath dense_path(const mq_weight* w, int64_t n, bool swiglu) { return dense_path_of(w->type, w->rows, w->nb, n, swiglu); }
 constexpr int64_t kGemvFusedMaxRows = 4;  // widest product whose quantizer runs inside the GEMV kernel (measured: 8 loses)
@@ -1104,7 +1111,7 @@ int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weigh
     Entry entry(s);
     if (entry.rc) return entry.rc;
     g.hidden_rows = 0;
-    const DensePath gate_path = dense_path(gate, n, true), down_path = dense_path(down, n, false);
+    const DensePath gate_path = dense_path(gate, n, true), down_path = dense_path_of(down->type, down->rows, down->nb, n, false, gate_path == kGemm);
     if (gate_path == kGemm) {  // wide: the matrix-core GEMM for gate and up, and for down unless another kernel takes less
         MQ_HIP(g.mid.reserve((size_t)n * (size_t)inter * sizeof(float)));
         const int rc = ffn_wide_locked(gate, up, down_path == kGemm ? down : nullptr, x_dev, n, hidden, silu_mode, (float*)g.mid.ptr, inter, y_dev, hidden, s);
@@ -2242,9 +2249,9 @@ int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
         path_out[2] = q80_gemm_tiles(rows, n);
         return MQ_OK;
     }
-    path_out[0] = dense_path_of(wtype, rows, nb, n, pair != 0);
+    path_out[0] = dense_path_of(wtype, rows, nb, n, pair == 1, pair == 2);
     path_out[1] = dense_waves(nb, rowtiles);
-    path_out[2] = skinny16_applies(nb, rowtiles, pair != 0, n, wtype) ? dense_lds_wpr(nb, rowtiles) : 0;
+    path_out[2] = skinny16_applies(nb, rowtiles, pair == 1, n, wtype) ? dense_lds_wpr(nb, rowtiles) : 0;
     return MQ_OK;
 }
 

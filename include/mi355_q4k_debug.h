@@ -76,7 +76,8 @@ int mq_debug_set_dense_lds(int on);
  * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns. */
 int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);
 
-/* Kernels that a dense product of n rows (pair != 0: gate and up in one call) runs on, for a 256-unit device before mq_init.  path_out:
+/* Kernels that a dense product of n rows (pair 1: gate and up in one call; 2: the down product of an FFN whose gate and up run on the
+ * GEMM) runs on, for a 256-unit device before mq_init.  path_out:
  * 0 passes of eight or sixteen rows, 1 tiles of sixteen, 2 the matrix-core GEMM; wavefronts per row tile of the passes, and of the
  * tiles of sixteen (0: not built for this product).  Q8_0 (pair == 0): 0 or 2; wavefronts per row tile of the passes; activation tiles
  * per workgroup of the GEMM. */

@@ -37,6 +37,15 @@ def test_tiles_of_sixteen_split_a_row_like_the_passes():
             assert sixteens in (0, passes) and (path != SIXTEENS or sixteens), (wtype, rows, nb, n, pair)
 
 
+def test_down_product_behind_a_gemm_takes_the_faster_kernel():
+    """Alone it stays with the tiles of sixteen unless the GEMM is far ahead; behind gate and up on the GEMM it need not."""
+    for wtype, hidden, inter, n in ((14, 5120, 9216, 20), (12, 6144, 9472, 23), (13, 6144, 8704, 24), (12, 3840, 512, 54)):
+        assert dense_path(wtype, hidden, inter // 256, n)[0] == SIXTEENS
+        assert dense_path(wtype, hidden, inter // 256, n, 2)[0] == GEMM
+    for wtype, hidden, inter, n in ((13, 3072, 2816, 48), (14, 2816, 2048, 49), (12, 1536, 2048, 53)):
+        assert dense_path(wtype, hidden, inter // 256, n)[0] == dense_path(wtype, hidden, inter // 256, n, 2)[0] == SIXTEENS
+
+
 def test_q80_rule_has_no_single_widths():
     """The row count from which the GEMM takes a Q8_0 product, over row lengths that the passes split over one wavefront count (eight, and
     four of more than 128 row tiles): longer rows keep it waiting, none of them alone."""

@@ -25,7 +25,8 @@ def test_products_match_their_rows_eight_at_a_time(wtype, rows, nb):
     w.free()
 
 
-@pytest.mark.parametrize("wtype,down_type,hidden,inter", [(12, 12, 2560, 11008), (12, 14, 2816, 5888), (13, 12, 1280, 7424), (14, 13, 4864, 9984)])
+@pytest.mark.parametrize("wtype,down_type,hidden,inter", [(12, 12, 2560, 11008), (12, 14, 2816, 5888), (13, 12, 1280, 7424), (14, 13, 4864, 9984),
+                                                           (13, 14, 5120, 9216), (13, 13, 3072, 2816)])
 def test_ffn_with_each_product_on_its_own_kernel(wtype, down_type, hidden, inter):
     import torch
     from densecore_amd import ops
