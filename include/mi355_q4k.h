@@ -189,7 +189,7 @@ int mq_swiglu_mul_mat_q4k(const mq_weight* gate, const mq_weight* up, const floa
  * The three smart_mul_mat calls plus cb_silu_mul_fused of a dense FFN block
  * (core/src/llm/graph/decoder.cpp:2662-2730, core/src/llm/graph/fused_ops.cpp:317-366).  Each of the
  * two steps (gate and up, down) takes the kernel that mq_swiglu_mul_mat_q4k and mq_mul_mat_q4k take for its shape and
- * width; prefill widths run on the matrix-core GEMM throughout: 4096 -> 14336 -> 4096 at 512 / 2048 rows in 0.25 / 0.76 ms. */
+ * width, except that down, behind gate and up on the GEMM, takes the one estimated the fastest; prefill widths run on the matrix-core GEMM throughout: 4096 -> 14336 -> 4096 at 512 / 2048 rows in 0.25 / 0.76 ms. */
 int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weight* down, const float* x_dev,
                       int64_t n, float* y_dev, int silu_mode, void* stream);
 
