@@ -15,7 +15,8 @@ attention core left out.  Weights are random-init Q4_K generated on the device f
 whole step can be captured in one HIP graph (torch.cuda.CUDAGraph) and replayed.
 
 FusedDecodeStep runs the same layers through mq_decoder_step: one persistent kernel for the whole run of
-layers (n <= 8), whose results are bit-identical to DecodeStep's.
+layers (n <= 8), whose results are bit-identical to DecodeStep's where the separate launches split a row's super-blocks like it
+(rows of up to eight super-blocks), and equal to rounding elsewhere.
 """
 import ctypes as C
 from dataclasses import dataclass

@@ -282,7 +282,9 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* layer, const float* x_dev, const f
  * threads that meet at a barrier after each one; here one persistent kernel does, with device-wide barriers
  * between the phases, and returns bit for bit what the node-by-node entry points above return
  * (mq_add_rmsnorm_q8k, mq_mul_mat_q4k_acts, mq_mul_mat_q4k, mq_add_rmsnorm_f32, mq_router_logits_f32,
- * mq_moe_layer_q4k).  All weights Q4_K; every layer has layer 0's shapes; n_experts <= 512; top_k <= 8.
+ * mq_moe_layer_q4k) where those split a row's super-blocks over wavefronts as this kernel does, always over eight -- the 2048 x 512
+ * layer of 256 experts, rows of up to eight super-blocks in general -- and to rounding where they take another number
+ * (hidden 2560: five).  All weights Q4_K; every layer has layer 0's shapes; n_experts <= 512; top_k <= 8.
  * The kernel needs every compute unit of the device free for this process: a barrier that is not met within
  * 200 ms is abandoned, the launch drains, and mq_decoder_status reports it.  Steps of one handle, and steps of
  * different handles, must not overlap on the device (one stream, or streams ordered by events). */
