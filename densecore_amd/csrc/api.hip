@@ -1330,20 +1330,20 @@ int mq_mul_mat_id_q4k(const mq_weight* w, const float* x_dev, int64_t n, int x_s
     if (int rc = carve_route(n, top_k, w->n_experts, r)) return rc;
     // entries with ids outside [0, n_experts) are dropped by the grouping, so clear y first
     MQ_HIP(launch_fill_zero(y_dev, (size_t)n * top_k * (size_t)w->rows, s));
-    MQ_HIP(launch_build_groups(ids_dev, n, top_k, w->n_experts, r.group_expert, r.group_begin, r.n_groups,
-                               r.entry_token, r.entry_k, s));
     if (use_gemm) {
         const int64_t entries = n * top_k, E = w->n_experts;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
         const int mt = g_moe_item_tiles ? g_moe_item_tiles : moe_gemm_item_tiles(entries, E);  // tiles per item: the plan and every launch reading it
         // every row quantized once, gathered by the GEMM (a token's one row, broadcast over its slots, repeats top_k times)
         MQ_HIP(g.ap.reserve(prow_bytes(n * x_slots, w->nb)));
-        MQ_HIP(launch_moe_gemm_plan(r.n_groups, r.group_expert, r.group_begin, r.entry_token, r.entry_k, top_k, x_slots != 1, entries, E,
-                                    0, 0, (int32_t*)g.plan.ptr, s, mt, {x_dev, n * x_slots, w->cols, w->nb, (uint8_t*)g.ap.ptr}));
+        MQ_HIP(launch_moe_group_plan(ids_dev, n, top_k, E, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, top_k, x_slots != 1, 0, 0,
+                                     (int32_t*)g.plan.ptr, s, mt, {x_dev, n * x_slots, w->cols, w->nb, (uint8_t*)g.ap.ptr}));
         MQ_HIP(launch_prefill_gemm_grouped(w->data, w->type, w->expert_bytes, nullptr, w->rows, w->nb, (const uint8_t*)g.ap.ptr, n * x_slots, entries, E,
                                            (const int32_t*)g.plan.ptr, true, y_dev, w->rows, s, mt));
         return MQ_OK;
     }
+    MQ_HIP(launch_build_groups(ids_dev, n, top_k, w->n_experts, r.group_expert, r.group_begin, r.n_groups,
+                               r.entry_token, r.entry_k, s));
     MatmulArgs a;
     a.w0 = w->data;
     a.wtype = w->type;
@@ -1745,8 +1745,6 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
     RouteWs r;
     if (int rc = carve_route(n, top_k, gate_exps->n_experts, r)) return rc;
     MQ_HIP(launch_fill_zero(hidden_dev, (size_t)n * top_k * (size_t)gate_exps->rows, s));
-    MQ_HIP(launch_build_groups(ids_dev, n, top_k, gate_exps->n_experts, r.group_expert, r.group_begin, r.n_groups,
-                               r.entry_token, r.entry_k, s));
     if (moe_gemm_width(gate_exps, n, top_k, 2)) {  // gate and up share their type
         // prefill widths: both products on the expert-grouped GEMM, SwiGLU rows scattered to their (token, slot) places
         const int64_t entries = n * top_k, E = gate_exps->n_experts, inter = gate_exps->rows, hidden = gate_exps->cols;
@@ -1754,8 +1752,8 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
         const int mt = g_moe_item_tiles ? g_moe_item_tiles : moe_gemm_item_tiles(entries, E);  // tiles per item: the plan and every launch reading it
         const int32_t* plan = (const int32_t*)g.plan.ptr;
         MQ_HIP(g.ap.reserve(prow_bytes(n, hidden / kQK)));  // every token is a row of top_k experts: quantized once, gathered by the GEMM
-        MQ_HIP(launch_moe_gemm_plan(r.n_groups, r.group_expert, r.group_begin, r.entry_token, r.entry_k, top_k, false, entries, E,
-                                    0, 0, (int32_t*)g.plan.ptr, s, mt, {x_dev, n, hidden, hidden / kQK, (uint8_t*)g.ap.ptr}));
+        MQ_HIP(launch_moe_group_plan(ids_dev, n, top_k, E, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, top_k, false, 0, 0,
+                                     (int32_t*)g.plan.ptr, s, mt, {x_dev, n, hidden, hidden / kQK, (uint8_t*)g.ap.ptr}));
         const int64_t rows_max = moe_gemm_tiles_max(entries, E) * 16;
         if (g_gemm_pair && gate_exps->type == up_exps->type) {
             // one launch for gate and up, silu(gate) * up scattered to its (token, slot) place by the epilogue
@@ -1776,6 +1774,8 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
                                                   hidden_dev, inter, s));
         return MQ_OK;
     }
+    MQ_HIP(launch_build_groups(ids_dev, n, top_k, gate_exps->n_experts, r.group_expert, r.group_begin, r.n_groups,
+                               r.entry_token, r.entry_k, s));
     if (int rc = quantize_into(g.aq, g.ad, x_dev, n, gate_exps->cols, gate_exps->cols, s)) return rc;
     return run_moe_gateup(gate_exps, up_exps, SharedExpert{}, n, top_k, top_k, silu_mode, r, hidden_dev, false, s);
 }
@@ -1794,16 +1794,14 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
     if (entry.rc) return entry.rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, down_exps->n_experts, r)) return rc;
-    MQ_HIP(launch_build_groups(ids_dev, n, top_k, down_exps->n_experts, r.group_expert, r.group_begin, r.n_groups,
-                               r.entry_token, r.entry_k, s));
     if (moe_gemm_width(down_exps, n, top_k, 1)) {
         // prefill widths: the product on the expert-grouped GEMM into the per-(token, slot) rows, then the combine
         const int64_t entries = n * top_k, E = down_exps->n_experts, hidden = down_exps->rows, inter = down_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
         const int mt = g_moe_item_tiles ? g_moe_item_tiles : moe_gemm_item_tiles(entries, E);  // tiles per item: the plan and every launch reading it
         const int32_t* plan = (const int32_t*)g.plan.ptr;
-        MQ_HIP(launch_moe_gemm_plan(r.n_groups, r.group_expert, r.group_begin, r.entry_token, r.entry_k, top_k, true, entries, E,
-                                    0, 0, (int32_t*)g.plan.ptr, s, mt));
+        MQ_HIP(launch_moe_group_plan(ids_dev, n, top_k, E, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, top_k, true, 0, 0,
+                                     (int32_t*)g.plan.ptr, s, mt));
         MQ_HIP(g.ap2.reserve(pmajor_bytes(moe_gemm_tiles_max(entries, E) * 16, inter / kQK)));
         MQ_HIP(launch_quantize_q8k_pmajor_grouped(hidden_dev, nullptr, false, 0, inter, inter, entries, E, plan, (uint8_t*)g.ap2.ptr,
                                                   nullptr, 0, s));
@@ -1813,6 +1811,8 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
         MQ_HIP(launch_moe_combine((const float*)g.part.ptr, n, top_k, top_k, hidden, weights_dev, ids_dev, E, 0, nullptr, nullptr, y_dev, s));
         return MQ_OK;
     }
+    MQ_HIP(launch_build_groups(ids_dev, n, top_k, down_exps->n_experts, r.group_expert, r.group_begin, r.n_groups,
+                               r.entry_token, r.entry_k, s));
     return run_moe_down(down_exps, SharedExpert{}, hidden_dev, false, n, top_k, top_k, r, ids_dev, weights_dev, nullptr,
                         nullptr, y_dev, s);
 }
@@ -1931,15 +1931,13 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         const int64_t entries = n * K + (sh.gate ? n : 0), G = E + (sh.gate ? 1 : 0);
         MQ_HIP(g.part.reserve((size_t)n * slots * (size_t)hidden * sizeof(float)));
         float* part = (float*)g.part.ptr;
-        MQ_HIP(launch_route_and_group(logits_dev, E, n, K, L->route_mode, ids, wts, (uint32_t*)g.counters.ptr + 4095,
-                                      r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, true, nullptr, 0, 0,
-                                      nullptr, nullptr, s));
+        MQ_HIP(launch_route_topk(logits_dev, E, n, K, L->route_mode, ids, wts, s));
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, G) * sizeof(int32_t)));
         const int mt = g_moe_item_tiles ? g_moe_item_tiles : moe_gemm_item_tiles(entries, G);  // tiles per item: the plan and every launch reading it
         const int32_t* plan = (const int32_t*)g.plan.ptr;
         MQ_HIP(g.ap.reserve(prow_bytes(n, hidden / kQK)));  // every token is a row of top_k (+ the shared) experts: quantized once, gathered by the GEMM
-        MQ_HIP(launch_moe_gemm_plan(r.n_groups, r.group_expert, r.group_begin, r.entry_token, r.entry_k, slots, false, entries, G,
-                                    sh.gate ? n : 0, MQ_SILU_FAST_FMA, (int32_t*)g.plan.ptr, s, mt, {x_dev, n, hidden, hidden / kQK, (uint8_t*)g.ap.ptr}));
+        MQ_HIP(launch_moe_group_plan(ids, n, K, E, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, slots, false, sh.gate ? n : 0,
+                                     MQ_SILU_FAST_FMA, (int32_t*)g.plan.ptr, s, mt, {x_dev, n, hidden, hidden / kQK, (uint8_t*)g.ap.ptr}));
         const int64_t rows_max = moe_gemm_tiles_max(entries, G) * 16;
         MQ_HIP(g.mid2.reserve(2 * (size_t)rows_max * (size_t)inter * sizeof(float)));
         float* gbuf = (float*)g.mid2.ptr;

@@ -264,11 +264,11 @@ size_t moe_gemm_plan_ints(int64_t entries, int64_t groups_max);
 // activation tiles per item (2, 4 or 8) of an expert-grouped launch over `entries` rows in `groups` groups: the plan and
 // every launch that reads it take the same value
 int moe_gemm_item_tiles(int64_t entries, int64_t groups);
+// Groups the pairs of the given ids by expert (the lists of launch_build_groups) and lays the groups out as the plan.
 // rows (optional): quantized by the same launch.
-hipError_t launch_moe_gemm_plan(const int32_t* n_groups, const int32_t* group_expert, const int32_t* group_begin,
-                                const int32_t* entry_token, const int32_t* entry_k, int slots, bool src_per_slot, int64_t entries,
-                                int64_t groups_max, int64_t sh_tokens, int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt,
-                                const GroupedRows& rows = {});
+hipError_t launch_moe_group_plan(const int32_t* ids, int64_t n, int top_k, int64_t n_experts, int32_t* group_expert, int32_t* group_begin,
+                                 int32_t* n_groups, int32_t* entry_token, int32_t* entry_k, int slots, bool src_per_slot, int64_t sh_tokens,
+                                 int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt, const GroupedRows& rows = {});
 hipError_t launch_quantize_q8k_pmajor_grouped(const float* x, const float* x2, bool swiglu, int silu_mode, int64_t ldx, int64_t k,
                                               int64_t entries, int64_t groups_max, const int32_t* plan, uint8_t* ap, float* h_out,
                                               int64_t ldh, hipStream_t stream);

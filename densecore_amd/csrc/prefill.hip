@@ -570,6 +570,16 @@ __device__ __forceinline__ void quantize_prow(const GroupedRows& rows, int64_t r
     if (lane == 0) *reinterpret_cast<float*>(dst + kPRowScaleOff) = q.d;
 }
 
+// A workgroup of 1024 threads, number wg of wgs: sixteen rows of a super-block, one per wavefront, and again as many workgroups further
+__device__ __forceinline__ void quantize_prow_runs(const GroupedRows& rows, uint32_t wg, uint32_t wgs) {
+    const uint32_t per_block = (uint32_t)((rows.n + 15) / 16), runs = per_block * (uint32_t)rows.nb;  // < 2^31: host-checked
+    for (uint32_t q = wg; q < runs; q += wgs) {
+        const uint32_t b = q / per_block;
+        const int64_t row = (int64_t)(q - b * per_block) * 16 + (threadIdx.x >> 6);
+        if (row < rows.n) quantize_prow(rows, row, b, threadIdx.x & 63);
+    }
+}
+
 // y[tok][row] = plane 0 + plane 1 + ... in that order; four rows per thread (rows % 4 == 0)
 __global__ void __launch_bounds__(256) prefill_sum_planes_kernel(const float* __restrict__ part, int splits, int64_t n, int64_t rows,
                                                                  float* __restrict__ y, int64_t ldy) {
@@ -730,13 +740,8 @@ __global__ void __launch_bounds__(1024) moe_gemm_plan_kernel(const int32_t* __re
                                                              int groups_max, int sh_tokens, int sh_slot, int sh_silu_mode,
                                                              int32_t* __restrict__ plan, int32_t* __restrict__ row_src,
                                                              int32_t* __restrict__ out_row, int mt, int plan_wgs, GroupedRows rows) {
-    if ((int)blockIdx.x >= plan_wgs) {  // sixteen rows of a super-block, one per wavefront, and again as many workgroups further
-        const uint32_t per_block = (uint32_t)((rows.n + 15) / 16), runs = per_block * (uint32_t)rows.nb;  // < 2^31: host-checked
-        for (uint32_t q = blockIdx.x - (uint32_t)plan_wgs; q < runs; q += gridDim.x - (uint32_t)plan_wgs) {
-            const uint32_t b = q / per_block;
-            const int64_t row = (int64_t)(q - b * per_block) * 16 + (threadIdx.x >> 6);
-            if (row < rows.n) quantize_prow(rows, row, b, threadIdx.x & 63);
-        }
+    if ((int)blockIdx.x >= plan_wgs) {
+        quantize_prow_runs(rows, blockIdx.x - (uint32_t)plan_wgs, gridDim.x - (uint32_t)plan_wgs);
         return;
     }
     extern __shared__ int32_t plan_sh[];  // begin[g], tile0[g], item0[g]: groups_max + 2 each
@@ -817,6 +822,112 @@ __global__ void __launch_bounds__(1024) moe_gemm_plan_kernel(const int32_t* __re
     }
 }
 
+// Grouping of given ids and the plan above in one launch, a workgroup per expert (the last one stands for the shared expert): each
+// counts the pairs of every expert in LDS -- the ids are a few KB that the L2 hands out --, adds up what lies ahead of its own
+// expert, and places its own pairs in the order of the ids, so a repeated (token, expert) needs no case of its own.  The lists, the
+// plan and the quantizing workgroups are those of build_groups_kernel and moe_gemm_plan_kernel, which took two launches and
+// sixteen workgroups that placed every expert's pairs by bit masks over the tokens.
+// Latency: one read of the ids, LDS counters, two barriers, the scattered stores.  256 + 1 experts, top-8, 2048 x 512: the block at 256 / 1500
+// tokens 135.1 / 228.0 -> 132.6 / 223.6 us (12.2 + 7.5 us by trace in two launches); 64 experts, top-6, at 192 / 256 tokens 66.0 / 64.5 ->
+// 59.7 / 59.5, 16 experts, top-2, 1024 x 256 at 400 / 700 tokens 52.7 / 59.5 -> 43.8 / 44.9.
+__global__ void __launch_bounds__(1024) moe_group_plan_kernel(const int32_t* __restrict__ ids, int n_pairs, int top_k, uint32_t top_k_inverse, int n_experts,
+                                                              int32_t* __restrict__ group_expert, int32_t* __restrict__ group_begin,
+                                                              int32_t* __restrict__ n_groups, int32_t* __restrict__ entry_token,
+                                                              int32_t* __restrict__ entry_k, int slots, int src_per_slot, int sh_tokens,
+                                                              int sh_silu_mode, int32_t* __restrict__ plan, int32_t* __restrict__ row_src,
+                                                              int32_t* __restrict__ out_row, int mt, int plan_wgs, GroupedRows rows) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x >= plan_wgs) {
+        quantize_prow_runs(rows, blockIdx.x - (uint32_t)plan_wgs, gridDim.x - (uint32_t)plan_wgs);
+        return;
+    }
+    const int own = blockIdx.x;  // n_experts: the shared expert
+    extern __shared__ int32_t plan_sh[];  // pairs of every expert, of this one in every wavefront's run of ids, the sums of wavefront 0
+    int32_t* count = plan_sh;
+    int32_t* before = count + n_experts;
+    int32_t* sums = before + 16;
+    // wavefront w holds the pairs [w per, (w + 1) per); bit c of a lane's mine: pair 64 c + lane of them is this expert's
+    const int chunks = (n_pairs + 1023) / 1024, first = wave * chunks * 64 + lane;  // chunks <= 64: host-checked
+    constexpr int kRound = 16;  // requested together
+    int v[kRound];
+    auto request = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < kRound; ++u) {
+            const int i = first + (c0 + u) * 64;
+            v[u] = ids[i < n_pairs ? i : n_pairs - 1];
+        }
+    };
+    request(0);
+    for (int e = tid; e < n_experts; e += 1024) count[e] = 0;
+    __syncthreads();
+    uint64_t mine = 0;
+    int in_wave = 0;
+    for (int c0 = 0; c0 < chunks; c0 += kRound) {
+        if (c0 > 0) request(c0);
+#pragma unroll
+        for (int u = 0; u < kRound; ++u) {
+            const bool valid = c0 + u < chunks && first + (c0 + u) * 64 < n_pairs && (uint32_t)v[u] < (uint32_t)n_experts;
+            if (valid) atomicAdd(&count[v[u]], 1);
+            const bool is_mine = valid && v[u] == own;
+            if (is_mine) mine |= (uint64_t)1 << (c0 + u);
+            in_wave += __popcll(__ballot(is_mine));
+        }
+    }
+    if (lane == 0) before[wave] = in_wave;
+    __syncthreads();
+    // what lies ahead of this expert (and, for the totals, of every expert): pairs and tiles, groups and items side by side
+    // (at most 2^16 pairs, 2^13 tiles, 2^9 groups)
+    const int mt_shift = mt == 2 ? 1 : mt == 4 ? 2 : 3;
+    auto ahead_of = [&](int end, int32_t* out) {
+        uint32_t pt = 0, gi = 0;
+        for (int e = lane; e < end; e += 64) {
+            const uint32_t p = (uint32_t)count[e], t = (p + 15) >> 4;
+            pt += p | t << 17, gi += (p > 0 ? 1u : 0u) | ((t + mt - 1) >> mt_shift) << 10;
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) pt += __shfl_xor(pt, d, 64), gi += __shfl_xor(gi, d, 64);
+        if (lane == 0) out[0] = (int)(pt & 0x1ffffu), out[1] = (int)(pt >> 17), out[2] = (int)(gi & 0x3ffu), out[3] = (int)(gi >> 10);
+    };
+    if (wave == 0) ahead_of(own, sums);
+    if (wave == 1 && own == 0) ahead_of(n_experts, sums + 4);
+    __syncthreads();
+    const int begin = sums[0], tile0 = sums[1], group = sums[2], item0 = sums[3];
+    if (own == 0 && tid == 0) {
+        const int sh_tiles = (sh_tokens + 15) >> 4, tiles_all = sums[5];
+        *n_groups = sums[6], group_begin[sums[6]] = sums[4];
+        plan[0] = sums[7] + ((sh_tiles + mt - 1) >> mt_shift), plan[1] = tiles_all + sh_tiles, plan[2] = tiles_all, plan[3] = sh_silu_mode;
+    }
+    const bool shared = own == n_experts;
+    const int here = shared ? sh_tokens : count[own], tiles = (here + 15) >> 4;
+    if (here == 0) return;
+    if (!shared && tid == 0) group_expert[group] = own, group_begin[group] = begin;
+    for (int j = tid; j << mt_shift < tiles; j += 1024) {
+        int32_t* item = plan + 4 + 3 * (item0 + j);
+        const int t = j << mt_shift;
+        item[0] = shared ? -1 : own, item[1] = tile0 + t, item[2] = tiles - t < mt ? tiles - t : mt;
+    }
+    const int row0 = tile0 * 16;
+    for (int p = (shared ? 0 : here) + tid; p < tiles * 16; p += 1024) {  // padding rows, or all of the shared expert's
+        row_src[row0 + p] = p < here ? p : -1;
+        out_row[row0 + p] = p < here ? p * slots + slots - 1 : -1;
+    }
+    if (shared) return;
+    int at = 0;
+    for (int w = 0; w < wave; ++w) at += before[w];
+    for (int c = 0; c < chunks; ++c) {
+        const bool is_mine = (mine >> c) & 1;
+        const uint64_t lanes = __ballot(is_mine);
+        if (is_mine) {
+            const int pos = at + __popcll(lanes & (((uint64_t)1 << lane) - 1)), i = first + c * 64;
+            const int tok = top_k == 1 ? i : (int)__umulhi((uint32_t)i, top_k_inverse), k = i - tok * top_k;
+            entry_token[begin + pos] = tok, entry_k[begin + pos] = k;
+            const int dst = tok * slots + k;
+            row_src[row0 + pos] = src_per_slot ? dst : tok, out_row[row0 + pos] = dst;
+        }
+        at += __popcll(lanes);
+    }
+}
+
 }  // namespace
 
 // upper bounds: `entries` counts every row of the plan (the routed pairs and, with a shared expert, every token once
@@ -833,16 +944,28 @@ size_t moe_gemm_plan_ints(int64_t entries, int64_t groups_max) {
     return 4 + 3 * (size_t)moe_gemm_items_max(entries, groups_max) + 2 * 16 * (size_t)moe_gemm_tiles_max(entries, groups_max);
 }
 
-hipError_t launch_moe_gemm_plan(const int32_t* n_groups, const int32_t* group_expert, const int32_t* group_begin,
-                                const int32_t* entry_token, const int32_t* entry_k, int slots, bool src_per_slot, int64_t entries,
-                                int64_t groups_max, int64_t sh_tokens, int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt, const GroupedRows& rows) {
+// The grouping of the given ids and the plan over it.  One launch up to kGroupPlanExperts experts (a workgroup each, two to a compute
+// unit: all at once) and 64 x 1024 pairs (a lane's bits); beyond, two launches as before.
+constexpr int64_t kGroupPlanExperts = 512, kGroupPlanPairs = 64 * 1024;
+hipError_t launch_moe_group_plan(const int32_t* ids, int64_t n, int top_k, int64_t n_experts, int32_t* group_expert, int32_t* group_begin,
+                                 int32_t* n_groups, int32_t* entry_token, int32_t* entry_k, int slots, bool src_per_slot, int64_t sh_tokens,
+                                 int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt, const GroupedRows& rows) {
+    const int64_t entries = n * top_k + sh_tokens, groups_max = n_experts + (sh_tokens > 0 ? 1 : 0);
     // (a grid holds fewer than 2^32 threads, four million workgroups of 1024: beyond kQuantWgs a workgroup takes several runs of rows)
     constexpr int64_t kQuantWgs = 1 << 16;
     const int64_t quant_runs = rows.x ? (rows.n + 15) / 16 * rows.nb : 0, quant_wgs = quant_runs < kQuantWgs ? quant_runs : kQuantWgs;
     if (quant_runs >= (int64_t)1 << 31 || (rows.x && (rows.nb > 65535 || rows.n >= (int64_t)1 << 31))) return hipErrorInvalidValue;
     if (groups_max > 4097 || (mt != kMTilesSmall && mt != kMTilesMid && mt != kMTilesPerGroup)) return hipErrorInvalidValue;
+    if (entries == 0) return hipSuccess;
     int32_t* row_src = plan + 4 + 3 * moe_gemm_items_max(entries, groups_max);
     int32_t* out_row = row_src + 16 * moe_gemm_tiles_max(entries, groups_max);
+    if (n_experts <= kGroupPlanExperts && n * top_k <= kGroupPlanPairs) {
+        MQ_LAUNCH(moe_group_plan_kernel, dim3((unsigned)(groups_max + quant_wgs)), dim3(1024), (size_t)(n_experts + 24) * sizeof(int32_t), stream, ids,
+                  (int)(n * top_k), top_k, (uint32_t)((((uint64_t)1 << 32) + top_k - 1) / top_k), (int)n_experts, group_expert, group_begin, n_groups, entry_token, entry_k, slots, src_per_slot ? 1 : 0,
+                  (int)sh_tokens, sh_silu_mode, plan, row_src, out_row, mt, (int)groups_max, rows);
+        return hipGetLastError();
+    }
+    if (hipError_t e = launch_build_groups(ids, n, top_k, n_experts, group_expert, group_begin, n_groups, entry_token, entry_k, stream); e != hipSuccess) return e;
     const int64_t rows_max = 16 * moe_gemm_tiles_max(entries, groups_max);
     const unsigned wgs = (unsigned)(rows_max / 1024 < 1 ? 1 : (rows_max / 1024 > 64 ? 64 : rows_max / 1024));
     MQ_LAUNCH(moe_gemm_plan_kernel, dim3(wgs + (unsigned)quant_wgs), dim3(1024), 3 * (size_t)(groups_max + 2) * sizeof(int32_t), stream, n_groups,
