@@ -1286,28 +1286,48 @@ int mq_moe_weights_from_logits(const float* logits_dev, int64_t n_experts, int64
     return MQ_OK;
 }
 
-// Whether an expert product by itself (nmat: one matrix, or gate and up) runs on the matrix-core GEMM in its expert-grouped form: from
-// 192 tokens with six routed rows per expert on, and from 17 tokens where an estimate says it takes less than 0.90 of the decode launches
-// (0.85 for gate and up, whose estimate is the looser one), whose groups take their rows eight at a time (64 rows per expert: eight
-// passes).  us, with rpe rows per expert:
-//   decode  17.5 + 1.20 nmat (rpe / 8 + 1/2) (stages of a wavefront, times the rounds of workgroups)
-//   GEMM    20.9 + 0.013 MB of weights + 0.26 nmat per thousand (activation tile, row tile, super-block) + 0.51 super-blocks x rounds
-// Least squares over 1,080 nodes (8 to 128 experts, top-2 to 8, 9 to 190 tokens, five shapes and three types): the choice takes 0.78 of
-// the decode launches' time (gate and up of 512 x 2048, 64 experts, top-8, 128 tokens: 56.6 -> 36.2 us), over 1.03 of it on 10, at most 1.18.
+static bool moe_gemm_takes(const mq_weight* w) { return w->type == kTypeQ4K || w->type == kTypeQ5K || w->type == kTypeQ6K; }
 constexpr int64_t kMoeGemmMinTokens = 17;
-static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k, int nmat) {
-    if ((w->type != kTypeQ4K && w->type != kTypeQ5K && w->type != kTypeQ6K) || w->n_experts > 4096 || (w->rows & 3) || (w->cols & 3)) return false;
-    if (n >= 192) return n * top_k >= 6 * w->n_experts;
-    if (n < kMoeGemmMinTokens || n * top_k < 5 * w->n_experts) return false;
-    const float experts = (float)w->n_experts, rpe = (float)(n * top_k) / experts, rt = (float)w->rowtiles, nb = (float)w->nb, mats = (float)nmat;
-    const int waves = pick_waves(w->nb, w->rowtiles * w->n_experts), mt = moe_gemm_item_tiles(n * top_k, w->n_experts);
+// Whether the estimates say that one expert product of rows x 256 nb weights takes less than 0.90 of the time on the matrix-core GEMM in its
+// expert-grouped form that it takes on the decode launches, whose groups take their rows eight at a time (64 rows per expert: eight
+// passes).  us, with rpe rows per expert:
+//   decode  17.5 + 1.20 (rpe / 8 + 1/2) (stages of a wavefront, times the rounds of workgroups)
+//   GEMM    20.9 + 0.013 MB of weights + 0.26 per thousand (activation tile, row tile, super-block) + 0.51 super-blocks x rounds
+// Least squares over 1,080 nodes (8 to 128 experts, top-2 to 8, 9 to 190 tokens, five shapes and three types): the choice takes 0.78 of
+// the decode launches' time, over 1.03 of it on 10, at most 1.18.
+static bool moe_gemm_estimate(int64_t n_experts, int64_t rowtiles, int64_t rows, int64_t n_blocks, int64_t n, int top_k) {
+    const float experts = (float)n_experts, rpe = (float)(n * top_k) / experts, rt = (float)rowtiles, nb = (float)n_blocks;
+    const int waves = pick_waves(n_blocks, rowtiles * n_experts), mt = moe_gemm_item_tiles(n * top_k, n_experts);
     const float slots = 8.0f * (float)compute_units(), load = rt * experts * (float)waves / slots;
-    const float decode = 17.5f + 1.20f * mats * (rpe * 0.125f + 0.5f) * (nb / (float)waves) * (load > 1.0f ? load : 1.0f);
+    const float decode = 17.5f + 1.20f * (rpe * 0.125f + 0.5f) * (nb / (float)waves) * (load > 1.0f ? load : 1.0f);
     const float items = experts * (rpe > 16.0f * (float)mt ? rpe / (16.0f * (float)mt) : 1.0f);
-    const float wgs = items * (float)((w->rowtiles + 3) / 4) / (2.0f * (float)compute_units());
-    const float gemm = 20.9f + 0.0132f * mats * experts * (float)w->rows * nb * 144e-6f + 2.59e-4f * mats * experts * (rpe * 0.0625f + 0.5f) * rt * nb +
+    const float wgs = items * (float)((rowtiles + 3) / 4) / (2.0f * (float)compute_units());
+    const float gemm = 20.9f + 0.0132f * experts * (float)rows * nb * 144e-6f + 2.59e-4f * experts * (rpe * 0.0625f + 0.5f) * rt * nb +
                        0.507f * nb * (wgs > 1.0f ? wgs : 1.0f);
-    return gemm < (nmat == 1 ? 0.90f : 0.85f) * decode;
+    return gemm < 0.90f * decode;
+}
+// A product by itself (mul_mat_id): from 192 tokens with six routed rows per expert, and from 17 with five where the estimate says so.
+static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
+    if (!moe_gemm_takes(w) || w->n_experts > 4096 || (w->rows & 3) || (w->cols & 3)) return false;
+    if (n >= 192) return n * top_k >= 6 * w->n_experts;
+    return n >= kMoeGemmMinTokens && n * top_k >= 5 * w->n_experts && moe_gemm_estimate(w->n_experts, w->rowtiles, w->rows, w->nb, n, top_k);
+}
+// Whether a MoE block runs its expert products on the expert-grouped GEMM, by its shape alone, so that the layer and the two nodes it
+// is made of come to one choice (a product whose type the GEMM does not take stays where it is).  By the routed rows per expert rpe:
+// from inter <= 12 rpe^3 on (2.8 rows at 256, 3.5 at 512, 4.4 at 1024), from six, and where the down product's estimate says so.  The line
+// goes through 15,305 blocks (8 to 256 experts, top-2 to 8, 1024 to 4096 x 256 to 1024, every mix of Q4_K, Q5_K and Q6_K, with and without
+// a shared expert, 9 to 400 tokens) timed both ways: the choice takes 1.008 of the faster one's time (1.088 with six rows, or five and the
+// estimate below 192 tokens), on 0.3 % of them it costs over 3 %, on 0.1 % over 8 % more than that did (with 20 in place of 12: 1.005,
+// 0.5 and 0.2 %, but one pair of nodes in ten 3 to 8 % slower, whose GEMM pays for a launch that clears the rows).  Fewer than 64 pairs stay on the
+// decode launches: the GEMM's fixed part is the longer one (8 experts, top-2, 20 tokens 32 against 43 us).
+// 64 experts, top-6, 2048 x 512 at 64 tokens 65.8 -> 53.7 us, 16 experts, top-8, 2816 x 768 at 24 tokens 98.7 -> 42.4.
+static bool moe_block_takes_gemm(int64_t n_experts, int64_t hidden, int64_t inter, int64_t n, int top_k) {
+    const int64_t pairs = n * top_k;
+    if (n < kMoeGemmMinTokens || pairs < 64 || n_experts > 4096 || (hidden & 3) || (inter & 3)) return false;
+    const float rpe = (float)pairs / (float)n_experts;
+    if (12.0f * rpe * rpe * rpe >= (float)inter) return true;
+    if (n >= 192) return pairs >= 6 * n_experts;
+    return pairs >= 5 * n_experts && moe_gemm_estimate(n_experts, (hidden + 15) / 16, hidden, inter / kQK, n, top_k);
 }
 
 int mq_mul_mat_id_q4k(const mq_weight* w, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
@@ -1323,7 +1343,7 @@ int mq_mul_mat_id_q4k(const mq_weight* w, const float* x_dev, int64_t n, int x_s
     Entry entry(s);
     if (entry.rc) return entry.rc;
     // prefill widths: the matrix-core GEMM in its expert-grouped form (see mq_moe_layer_q4k)
-    const bool use_gemm = moe_gemm_width(w, n, top_k, 1);
+    const bool use_gemm = moe_gemm_width(w, n, top_k);
     if (!use_gemm)
         if (int rc = quantize_into(g.aq, g.ad, x_dev, n * x_slots, w->cols, w->cols, s)) return rc;
     RouteWs r;
@@ -1745,7 +1765,7 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
     RouteWs r;
     if (int rc = carve_route(n, top_k, gate_exps->n_experts, r)) return rc;
     MQ_HIP(launch_fill_zero(hidden_dev, (size_t)n * top_k * (size_t)gate_exps->rows, s));
-    if (moe_gemm_width(gate_exps, n, top_k, 2)) {  // gate and up share their type
+    if (moe_gemm_takes(gate_exps) && moe_block_takes_gemm(gate_exps->n_experts, gate_exps->cols, gate_exps->rows, n, top_k)) {  // gate and up share their type
         // prefill widths: both products on the expert-grouped GEMM, SwiGLU rows scattered to their (token, slot) places
         const int64_t entries = n * top_k, E = gate_exps->n_experts, inter = gate_exps->rows, hidden = gate_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
@@ -1794,7 +1814,7 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
     if (entry.rc) return entry.rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, down_exps->n_experts, r)) return rc;
-    if (moe_gemm_width(down_exps, n, top_k, 1)) {
+    if (moe_gemm_takes(down_exps) && moe_block_takes_gemm(down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k)) {
         // prefill widths: the product on the expert-grouped GEMM into the per-(token, slot) rows, then the combine
         const int64_t entries = n * top_k, E = down_exps->n_experts, hidden = down_exps->rows, inter = down_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
@@ -1840,25 +1860,18 @@ int decoder_grid(size_t lds_bytes, int* n_workgroups, long long* spin_ticks) {
 
 }  // namespace
 
-// The expert-grouped GEMM pays from six routed rows per expert on average (its workgroups multiply 16-row tiles, two,
-// four or eight of an expert at a time): 256 experts, top-8, 2048 x 512: 152 against 153 us per block at 192 tokens, 158
-// against 186 at 256, 164 against 217 at 320 -- and 141 against 119 at 128, where the decode kernels' 8-row groups stay; fewer experts
-// cross earlier (below).
-// Decided per product: gate / up (one type) and down each run on it when their type is one it takes; a layer with
+// Decided per product: gate / up (one type) and down each run on the expert-grouped GEMM when their type is one it takes; a layer with
 // a Q8_0 down stack (core/src/llm/moe/native.cpp:4611-4620; its activations are Q8_0 as well) keeps its two large
-// products on the matrix cores and sends the fp32 hidden rows through the Q8_0 launches.
-static bool moe_gemm_takes(const mq_weight* w) { return w->type == kTypeQ4K || w->type == kTypeQ5K || w->type == kTypeQ6K; }
+// products on the matrix cores from 192 tokens on and sends the fp32 hidden rows through the Q8_0 launches.
+// Up to this many tokens the GEMM's hidden rows lie at their (token, slot) places, as the decode launches leave them and where
+// mq_debug_moe_hidden finds them; more stay in its tiles, which its quantizer reads in order.
+constexpr int64_t kMoeRowsInPlaceTokens = 64;
 static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
     const mq_weight* ge = L->gate_exps;
-    if (!moe_gemm_takes(ge) || !moe_gemm_takes(L->up_exps)) return false;  // the shared expert has the stacks' types
-    if (ge->n_experts > 4096 || (ge->rows & 3) || (ge->cols & 3)) return false;
-    // (256 + 1 experts, top-8, 2048 x 512, the expert-grouped decode launches against the GEMM with items of two tiles:
-    // 106 / 135 us at 96 tokens, 119 / 141 at 128, 153 / 152 at 192, 186 / 158 at 256, 217 / 164 at 320)
-    // Below 192 tokens where the down product by itself takes it (moe_gemm_width); the gate/up node asks for its own matrices, and comes to
-    // another choice for about one block in seven of 17 to 191 tokens.  Over 1,050
-    // blocks of 8 to 128 experts, top-2 to 8, 9 to 190 tokens and five shapes: 0.82 of the decode launches' time, nowhere more than it
-    // (16 experts, top-8, 2816 x 768 at 128 tokens 354 -> 78 us).
-    return n >= 192 ? n * L->top_k >= 6 * ge->n_experts : moe_gemm_width(L->down_exps, n, L->top_k, 1);
+    // (a Q8_0 down stack's launches follow either way: 42 us a block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them)
+    if (n < 192 && !moe_gemm_takes(L->down_exps)) return false;
+    return moe_gemm_takes(ge) && moe_gemm_takes(L->up_exps) &&  // the shared expert has the stacks' types
+           moe_block_takes_gemm(ge->n_experts, ge->cols, ge->rows, n, L->top_k);
 }
 
 int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float* logits_dev, int64_t n, float* y_dev,
@@ -1955,10 +1968,19 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
                 g.hidden_rows = hidden_rows;
                 return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, false, n, K, slots, r, ids, wts, L->sh_gate_inp_dev, x_dev, y_dev, s);
             }
-            MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
-                                                    L->gate_exps->nb, (const uint8_t*)g.ap.ptr, n, entries, G, plan, false, L->silu_mode, gbuf, inter, s, mt));
             MQ_HIP(g.ap2.reserve(pmajor_bytes(rows_max, inter / kQK)));
-            MQ_HIP(launch_quantize_q8k_pmajor(gbuf, rows_max, inter, inter, (uint8_t*)g.ap2.ptr, s, plan));  // rows in the plan's order already
+            if (n <= kMoeRowsInPlaceTokens) {
+                MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
+                MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
+                                                        L->gate_exps->nb, (const uint8_t*)g.ap.ptr, n, entries, G, plan, true, L->silu_mode,
+                                                        (float*)g.mid.ptr, inter, s, mt));
+                g.hidden_rows = hidden_rows;
+                MQ_HIP(launch_quantize_q8k_pmajor_grouped((const float*)g.mid.ptr, nullptr, false, 0, inter, inter, entries, G, plan, (uint8_t*)g.ap2.ptr, nullptr, 0, s, true));
+            } else {
+                MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
+                                                        L->gate_exps->nb, (const uint8_t*)g.ap.ptr, n, entries, G, plan, false, L->silu_mode, gbuf, inter, s, mt));
+                MQ_HIP(launch_quantize_q8k_pmajor(gbuf, rows_max, inter, inter, (uint8_t*)g.ap2.ptr, s, plan));  // rows in the plan's order already
+            }
             MQ_HIP(launch_prefill_gemm_grouped(L->down_exps->data, L->down_exps->type, L->down_exps->expert_bytes, shd, hidden, L->down_exps->nb,
                                                (const uint8_t*)g.ap2.ptr, 0, entries, G, plan, true, part, hidden, s, mt));
             MQ_HIP(launch_moe_combine(part, n, K, slots, hidden, wts, ids, E, sh.gate ? 1 : 0, L->sh_gate_inp_dev, x_dev, y_dev, s));

@@ -271,7 +271,7 @@ hipError_t launch_moe_group_plan(const int32_t* ids, int64_t n, int top_k, int64
                                  int sh_silu_mode, int32_t* plan, hipStream_t stream, int mt, const GroupedRows& rows = {});
 hipError_t launch_quantize_q8k_pmajor_grouped(const float* x, const float* x2, bool swiglu, int silu_mode, int64_t ldx, int64_t k,
                                               int64_t entries, int64_t groups_max, const int32_t* plan, uint8_t* ap, float* h_out,
-                                              int64_t ldh, hipStream_t stream);
+                                              int64_t ldh, hipStream_t stream, bool x_in_place = false);
 hipError_t launch_prefill_gemm_grouped(const uint8_t* w, int wtype, int64_t expert_bytes, const uint8_t* w_shared, int64_t rows,
                                        int64_t nb, const uint8_t* ap, int64_t gathered, int64_t entries, int64_t groups_max, const int32_t* plan,
                                        bool scatter, float* y, int64_t ldy, hipStream_t stream, int mt = 8);

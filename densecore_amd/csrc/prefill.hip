@@ -974,12 +974,13 @@ hipError_t launch_moe_group_plan(const int32_t* ids, int64_t n, int top_k, int64
     return hipGetLastError();
 }
 
-// Rows of the plan's tiles in the P-major layout: gathered from x by the plan's row list (swiglu == false), or
+// Rows of the plan's tiles in the P-major layout: gathered from x by the plan's row list (swiglu == false; x_in_place: by its list of
+// output rows, x being what an expert-grouped launch scattered), or
 // silu(gate) * up of two planes that already are in the plan's row order (swiglu == true; h_out, if given, receives
 // those rows as fp32 at their per-(token, slot) places).
 hipError_t launch_quantize_q8k_pmajor_grouped(const float* x, const float* x2, bool swiglu, int silu_mode, int64_t ldx, int64_t k,
                                               int64_t entries, int64_t groups_max, const int32_t* plan, uint8_t* ap, float* h_out,
-                                              int64_t ldh, hipStream_t stream) {
+                                              int64_t ldh, hipStream_t stream, bool x_in_place) {
     const int64_t nb = k / kQK, m_tiles = moe_gemm_tiles_max(entries, groups_max);
     if (m_tiles == 0 || nb == 0) return hipSuccess;
     if (nb > 65535 || m_tiles >= (int64_t)1 << 31) return hipErrorInvalidValue;
@@ -990,7 +991,8 @@ hipError_t launch_quantize_q8k_pmajor_grouped(const float* x, const float* x2, b
                            row_src + 16 * m_tiles);
     } else {
         MQ_LAUNCH(quantize_q8k_pmajor_kernel<false>, dim3((unsigned)m_tiles, (unsigned)nb), dim3(256), 0, stream, x,
-                           (const float*)nullptr, 0, (float*)nullptr, (int64_t)0, m_tiles * 16, ldx, nb, m_tiles, ap, plan, row_src,
+                           (const float*)nullptr, 0, (float*)nullptr, (int64_t)0, m_tiles * 16, ldx, nb, m_tiles, ap, plan,
+                           x_in_place ? row_src + 16 * m_tiles : row_src,
                            (const int32_t*)nullptr);
     }
     return hipGetLastError();

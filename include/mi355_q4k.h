@@ -219,8 +219,8 @@ int mq_moe_weights_from_logits(const float* logits_dev, int64_t n_experts, int64
  * and more with six rows per expert on average, and from 17 tokens with five rows
  * per expert where an estimate says that it is clearly faster: few experts) run on
  * the int8 matrix-core GEMM in its expert-grouped form, as do
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, each by its own
- * matrices' estimate. */
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, which follow the
+ * rule of mq_moe_layer_q4k. */
 int mq_mul_mat_id_q4k(const mq_weight* w_exps, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
                       int top_k, float* y_dev, void* stream);
 
@@ -249,12 +249,14 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * Up to eight tokens (and 512 experts) two launches: gate/up + SwiGLU with the router and the Q8_K of x inside,
  * down with the Q8_K of the hidden rows and the weighted combine inside.  Above: router + expert grouping + Q8_K
  * of x, expert-grouped gate/up leaving its rows in Q8_K, expert-grouped down, combine.  Same bits either way.
- * Prefill widths (192 tokens and more with six routed rows per expert on average; from 17 tokens with five where the down product's
- * estimate says so, e.g. 16 experts, top-8, 2816 x 768 at 128 tokens): the expert products run on the
+ * From 17 tokens with 64 routed pairs on, where the routed rows per expert r satisfy inter <= 12 r^3 (2.8 rows at 256 hidden
+ * values per expert, 3.5 at 512, 4.4 at 1024) or r >= 6 (below 192 tokens r >= 5 and an estimate), the expert products run on the
  * int8 matrix-core GEMM in an expert-grouped form (entries in 16-row tiles per expert), the shared expert as one more
- * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches; same routing, results within the fp32 tolerance of the other form (the
- * summation order differs), and mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.  Between 17 and 191
- * tokens mq_moe_gateup_swiglu_q4k decides by itself, so the layer and its nodes may take different forms there and agree to that tolerance. */
+ * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches (from 192 tokens); same
+ * routing, results within the fp32 tolerance of the other form (the
+ * summation order differs), and above 64 tokens mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same rule, so the layer is the composition of its two nodes bit for
+ * bit there (with a Q8_0 down stack from 192 tokens on). */
 typedef struct {
     const mq_weight* gate_exps; /* n_experts x [inter][hidden]  */
     const mq_weight* up_exps;
