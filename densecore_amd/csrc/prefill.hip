@@ -111,7 +111,7 @@ __device__ __forceinline__ void request_a_rows(const GatherOffsets<MT>& off, con
 // comes with two (items of 32 rows): with a dozen or two routed rows per expert a workgroup has one or two tiles, its
 // accumulators for eight only cost registers and LDS -- and how many workgroups a compute unit holds is what hides the
 // latency of a workgroup that walks eight super-blocks with a barrier each.
-template <int kWTilesPerWave, int WT = kWtQ4, bool PAIR = false, int MT = kMTilesPerGroup, bool GATHER = false>
+template <int kWTilesPerWave, int WT = kWtQ4, bool PAIR = false, int MT = kMTilesPerGroup, bool GATHER = false, bool kDense = false>
 __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __restrict__ w, int64_t rowtiles, int64_t rows,
                                                            int64_t nb, const uint8_t* __restrict__ ap, int64_t m_tiles,
                                                            int64_t n_tokens, float* __restrict__ y, int64_t ldy, int sb_split,
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
         // the zero bytes behind every tile of both buffers: no request writes them
         if (tid < 2 * MT * 4) *reinterpret_cast<uint32_t*>(a_lds + (tid >> 2) * kPTileBytes + kPZeroOff + (tid & 3) * 4) = 0u;
     }
-    constexpr bool kByLane = MT == kMTilesPerGroup && !PAIR && (kWTilesPerWave == 1) == (WT != kWtQ5);
+    constexpr bool kByLane = MT > kMTilesMid && !PAIR && kWTilesPerWave == 1 && WT != kWtQ5;
     auto request_a = [&](int64_t b) {
         uint8_t* buf = a_lds + (b & 1) * kBufBytes;
         if constexpr (GATHER) request_a_rows<MT>(gather, a_src + (size_t)b * a_stride, buf, mt_count, wave, lane);
@@ -212,122 +212,155 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
     request_a(b_begin);
     request_w(b_begin);
 
-    for (int64_t b = b_begin; b < b_end; ++b) {
-        // everything this thread requested for super-block b has landed ...
-        __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xF << 8));  // vmcnt(0)
-        // ... and after the barrier so has everybody else's share of the activation tiles; every wave
-        // is also done reading the other buffer (super-block b-1), which the next requests overwrite
-        __syncthreads();
-        if constexpr (PAIR && MT <= 4) {
-            // Few activation tiles: the two weight tiles are expanded and multiplied one after the other, so that one
-            // expanded tile is live at a time (38 registers less: three wavefronts per SIMD instead of two, which is
-            // what a launch of many short workgroups needs); the activation operands are read from LDS once per tile.
-            if (b + 1 < b_end) request_a(b + 1);
-            const uint8_t* a_buf = a_lds + (b & 1) * kBufBytes;
+    struct ATile {
+        v4i a[4];
+        v4f yd;
+        v8h dg;
+    };
+    auto read_a = [&](ATile& t, const uint8_t* at) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                WTile w1;
-                if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, w1);
-                else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, w1);
-                if (b + 1 < b_end) request_w(b + 1, t);  // the raw tile's registers are free again
+        for (int j = 0; j < 4; ++j) t.a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+        t.yd = *reinterpret_cast<const v4f*>(at + kPScaleOff + kq * 16);
+        if constexpr (!Q6) t.dg = *reinterpret_cast<const v8h*>(at + digit_off);
+    };
+    // The LDS operands of the next activation tile are requested while this one is multiplied.  One weight tile to a wavefront: by hand, the
+    // 24 registers are there (kAhead).  Two: they are not (eight to twelve spill), but without a branch round every tile the compiler
+    // finds room for them in turn (kAll: a workgroup whose tiles are all there; a form of its own for five, six, seven and eight).  Two
+    // wavefronts to a SIMD waited 30 % of their time, much of it for these reads.  Against a read ahead of every tile's products, same
+    // bits: 198 products of 64-row workgroups at 70 to 512 rows 0.951 of the time (Q4_K 2048 x 2048 at 128 rows 13.0 -> 12.1 us, Q5_K 4096 x 4096
+    // at 100 rows 21.0 -> 19.0), 366 products and FFNs at 70 to 2048 rows 0.968 (Q4_K 14336 x 4096 at 700 rows 111 -> 99 us, Q6_K at
+    // 2048 rows 0.96); least where the card's power is the limit (Q4_K from 1500 rows on: 0.98 to 1.0).  Without branches and without kAhead
+    // one weight tile gains less and loses up to 9 % where the last column is short.
+    constexpr bool kAhead = kDense && kWTilesPerWave == 1;
+    auto multiply = [&](auto all_c) {
+        constexpr bool kAll = decltype(all_c)::value;
+        for (int64_t b = b_begin; b < b_end; ++b) {
+            // everything this thread requested for super-block b has landed ...
+            __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xF << 8));  // vmcnt(0)
+            // ... and after the barrier so has everybody else's share of the activation tiles; every wave
+            // is also done reading the other buffer (super-block b-1), which the next requests overwrite
+            __syncthreads();
+            if constexpr (PAIR && MT <= 4) {
+                // Few activation tiles: the two weight tiles are expanded and multiplied one after the other, so that one
+                // expanded tile is live at a time (38 registers less: three wavefronts per SIMD instead of two, which is
+                // what a launch of many short workgroups needs); the activation operands are read from LDS once per tile.
+                if (b + 1 < b_end) request_a(b + 1);
+                const uint8_t* a_buf = a_lds + (b & 1) * kBufBytes;
 #pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    if (m < mt_count) {  // uniform over the workgroup
-                        const uint8_t* at = a_buf + m * kPTileBytes;
-                        v4i a[4];
+                for (int t = 0; t < 2; ++t) {
+                    WTile w1;
+                    if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, w1);
+                    else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, w1);
+                    if (b + 1 < b_end) request_w(b + 1, t);  // the raw tile's registers are free again
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
-                        const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
-                        const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
-                        const v4i zero = {0, 0, 0, 0};
-                        const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
-                        v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.hi[0], zero, 0, 0, 0);
-                        v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.lo[0], zero, 0, 0, 0);
-                        v4i b5 = zero;
-                        if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.b5[0], zero, 0, 0, 0);
-                        v4f mn = zero_f;
-                        if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(at + digit_off), w1.mins, zero_f, 0, 0, 0);
+                    for (int m = 0; m < MT; ++m) {
+                        if (kAll || m < mt_count) {  // uniform over the workgroup
+                            const uint8_t* at = a_buf + m * kPTileBytes;
+                            v4i a[4];
 #pragma unroll
-                        for (int j = 1; j < 4; ++j) {
-                            hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.hi[j], hi, 0, 0, 0);
-                            lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.lo[j], lo, 0, 0, 0);
-                            if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.b5[j], b5, 0, 0, 0);
-                        }
+                            for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+                            const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
+                            const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
+                            const v4i zero = {0, 0, 0, 0};
+                            const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
+                            v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.hi[0], zero, 0, 0, 0);
+                            v4i lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.lo[0], zero, 0, 0, 0);
+                            v4i b5 = zero;
+                            if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.b5[0], zero, 0, 0, 0);
+                            v4f mn = zero_f;
+                            if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(at + digit_off), w1.mins, zero_f, 0, 0, 0);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {  // the arithmetic of the two-tiles-at-once form below
-                            const int dot = join_digits<WT, MT>(hi[i], lo[i], b5[i]);
-                            if constexpr (Q6) {
-                                acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], w1.d), (float)dot, acc[t][m][i]);
-                            } else {
-                                const float v = __fmaf_rn(-w1.dmin, mn[i], __fmul_rn(w1.d, (float)dot));
-                                acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                            for (int j = 1; j < 4; ++j) {
+                                hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.hi[j], hi, 0, 0, 0);
+                                lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.lo[j], lo, 0, 0, 0);
+                                if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.b5[j], b5, 0, 0, 0);
+                            }
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {  // the arithmetic of the two-tiles-at-once form below
+                                const int dot = join_digits<WT, MT>(hi[i], lo[i], b5[i]);
+                                if constexpr (Q6) {
+                                    acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], w1.d), (float)dot, acc[t][m][i]);
+                                } else {
+                                    const float v = __fmaf_rn(-w1.dmin, mn[i], __fmul_rn(w1.d, (float)dot));
+                                    acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                                }
                             }
                         }
                     }
                 }
+                continue;
             }
-            continue;
-        }
-        WTile wt[kWTilesPerWave];
+            WTile wt[kWTilesPerWave];
 #pragma unroll
-        for (int t = 0; t < kWTilesPerWave; ++t) {
-            if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, wt[t]);
-            else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, wt[t]);
-        }
-        if (b + 1 < b_end) {
-            request_a(b + 1);
-            request_w(b + 1);
-        }
-        const uint8_t* a_buf = a_lds + (b & 1) * kBufBytes;
+            for (int t = 0; t < kWTilesPerWave; ++t) {
+                if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, wt[t]);
+                else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, wt[t]);
+            }
+            if (b + 1 < b_end) {
+                request_a(b + 1);
+                request_w(b + 1);
+            }
+            const uint8_t* a_buf = a_lds + (b & 1) * kBufBytes;
 
+            ATile at[kAhead ? 2 : 1];
+            if constexpr (kAhead) read_a(at[0], a_buf);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m < mt_count) {  // uniform over the workgroup
-                const uint8_t* at = a_buf + m * kPTileBytes;
-                v4i a[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
-                const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
-                const v4i zero = {0, 0, 0, 0};
-                const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
-                const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
-                v4i hi[kWTilesPerWave], lo[kWTilesPerWave], b5[kWTilesPerWave];
-                v4f mn[kWTilesPerWave];
-                v8h dg;
-                if constexpr (!Q6) dg = *reinterpret_cast<const v8h*>(at + digit_off);
-#pragma unroll
-                for (int t = 0; t < kWTilesPerWave; ++t) {
-                    hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].hi[0], zero, 0, 0, 0);
-                    lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].lo[0], zero, 0, 0, 0);
-                    b5[t] = zero;
-                    if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].b5[0], zero, 0, 0, 0);
-                    if constexpr (!Q6) mn[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, wt[t].mins, zero_f, 0, 0, 0);
-                }
-#pragma unroll
-                for (int j = 1; j < 4; ++j)
+            for (int m = 0; m < MT; ++m) {
+                if (kAll || m < mt_count) {  // uniform over the workgroup
+                    if constexpr (kAhead) {
+                        if (m + 1 < MT) read_a(at[(m + 1) & 1], a_buf + (m + 1) * kPTileBytes);  // (past mt_count: read and not used)
+                        __builtin_amdgcn_sched_barrier(0);  // ahead of this tile's products
+                    } else {
+                        read_a(at[0], a_buf + m * kPTileBytes);
+                    }
+                    const ATile& now = at[kAhead ? m & 1 : 0];
+                    const v4i (&a)[4] = now.a;
+                    const float ydv[4] = {now.yd.x, now.yd.y, now.yd.z, now.yd.w};
+                    const v8h dg = now.dg;
+                    const v4i zero = {0, 0, 0, 0};
+                    const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
+                    v4i hi[kWTilesPerWave], lo[kWTilesPerWave], b5[kWTilesPerWave];
+                    v4f mn[kWTilesPerWave];
 #pragma unroll
                     for (int t = 0; t < kWTilesPerWave; ++t) {
-                        hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].hi[j], hi[t], 0, 0, 0);
-                        lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].lo[j], lo[t], 0, 0, 0);
-                        if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].b5[j], b5[t], 0, 0, 0);
+                        hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].hi[0], zero, 0, 0, 0);
+                        lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].lo[0], zero, 0, 0, 0);
+                        b5[t] = zero;
+                        if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], wt[t].b5[0], zero, 0, 0, 0);
+                        if constexpr (!Q6) mn[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, wt[t].mins, zero_f, 0, 0, 0);
                     }
 #pragma unroll
-                for (int t = 0; t < kWTilesPerWave; ++t)
+                    for (int j = 1; j < 4; ++j)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int dot = join_digits<WT, MT>(hi[t][i], lo[t][i], b5[t][i]);
-                        if constexpr (Q6) {
-                            // the integer of the reference's kernel (times 4, taken out of d), then its one fused multiply-add
-                            // per block (core/src/llm/matmul/q6_small_batch.h:84-86)
-                            acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], wt[t].d), (float)dot, acc[t][m][i]);
-                        } else {
-                            // yd * (d * dot - dmin * min_dot): three fp32 operations per output and super-block
-                            const float v = __fmaf_rn(-wt[t].dmin, mn[t][i], __fmul_rn(wt[t].d, (float)dot));
-                            acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                        for (int t = 0; t < kWTilesPerWave; ++t) {
+                            hi[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].hi[j], hi[t], 0, 0, 0);
+                            lo[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].lo[j], lo[t], 0, 0, 0);
+                            if constexpr (kFifthChain<WT, MT>) b5[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt[t].b5[j], b5[t], 0, 0, 0);
                         }
-                    }
+#pragma unroll
+                    for (int t = 0; t < kWTilesPerWave; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int dot = join_digits<WT, MT>(hi[t][i], lo[t][i], b5[t][i]);
+                            if constexpr (Q6) {
+                                // the integer of the reference's kernel (times 4, taken out of d), then its one fused multiply-add
+                                // per block (core/src/llm/matmul/q6_small_batch.h:84-86)
+                                acc[t][m][i] = __fmaf_rn(__fmul_rn(ydv[i], wt[t].d), (float)dot, acc[t][m][i]);
+                            } else {
+                                // yd * (d * dot - dmin * min_dot): three fp32 operations per output and super-block
+                                const float v = __fmaf_rn(-wt[t].dmin, mn[t][i], __fmul_rn(wt[t].d, (float)dot));
+                                acc[t][m][i] = __fmaf_rn(ydv[i], v, acc[t][m][i]);
+                            }
+                        }
+                }
             }
         }
+    };
+    if constexpr (kDense && kWTilesPerWave == 2) {
+        if (mt_count == MT) multiply(std::true_type{});
+        else multiply(std::false_type{});
+    } else {
+        multiply(std::false_type{});
     }
 
     if constexpr (PAIR) {  // one output per (token, row): silu(gate) * up
@@ -1016,16 +1049,19 @@ namespace {
 hipError_t raise_gemm_lds() {
     static bool raised = false;
     if (raised) return hipSuccess;
-#define MQ_FORM(KW, WT_, PAIR_) reinterpret_cast<const void*>(&prefill_gemm_kernel<KW, WT_, PAIR_>)
+#define MQ_TILES(KW, WT_, PAIR_, MT_) reinterpret_cast<const void*>(&prefill_gemm_kernel<KW, WT_, PAIR_, MT_, false, true>)
+#define MQ_FORM(KW, WT_, PAIR_) MQ_TILES(KW, WT_, PAIR_, 5), MQ_TILES(KW, WT_, PAIR_, 6), MQ_TILES(KW, WT_, PAIR_, 7), MQ_TILES(KW, WT_, PAIR_, 8)
 #define MQ_GATHER_FORM(WT_, PAIR_) reinterpret_cast<const void*>(&prefill_gemm_kernel<2, WT_, PAIR_, kMTilesPerGroup, true>)
     for (const void* k : {MQ_FORM(1, kWtQ4, false), MQ_FORM(2, kWtQ4, false), MQ_FORM(2, kWtQ4, true), MQ_FORM(1, kWtQ5, false), MQ_FORM(2, kWtQ5, false),
                           MQ_FORM(2, kWtQ5, true), MQ_FORM(1, kWtQ6, false), MQ_FORM(2, kWtQ6, false), MQ_FORM(2, kWtQ6, true),
-                          MQ_GATHER_FORM(kWtQ4, false), MQ_GATHER_FORM(kWtQ5, false), MQ_GATHER_FORM(kWtQ6, false),
+                          reinterpret_cast<const void*>(&prefill_gemm_kernel<2, kWtQ4>), reinterpret_cast<const void*>(&prefill_gemm_kernel<2, kWtQ5>),
+                          reinterpret_cast<const void*>(&prefill_gemm_kernel<2, kWtQ6>), MQ_GATHER_FORM(kWtQ4, false), MQ_GATHER_FORM(kWtQ5, false), MQ_GATHER_FORM(kWtQ6, false),
                           MQ_GATHER_FORM(kWtQ4, true), MQ_GATHER_FORM(kWtQ5, true), MQ_GATHER_FORM(kWtQ6, true)}) {
         hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * kMTilesPerGroup * kPTileBytes);
         if (e != hipSuccess) return e;
     }
 #undef MQ_FORM
+#undef MQ_TILES
 #undef MQ_GATHER_FORM
     raised = true;
     return hipSuccess;
@@ -1045,6 +1081,17 @@ bool gemm_type(int wtype) { return wtype == kTypeQ4K || wtype == kTypeQ5K || wty
         if ((wtype) == kTypeQ6K) GO(kWtQ6); \
         else if ((wtype) == kTypeQ5K) GO(kWtQ5); \
         else GO(kWtQ4);                    \
+    } while (0)
+// LDS of a dense GEMM's workgroup, whatever its tiles: two to a compute unit, as the estimate of a shape has it.  With as many as fit, 448
+// workgroups of fewer tiles come to lie three to a unit beside units with one (Q6_K 14336 x 4096 at 200 rows 41.8 -> 46.1 us).
+constexpr size_t kGemmLds = 2 * kMTilesPerGroup * kPTileBytes;
+// GO(type, activation tiles of the form): five to eight tiles of a workgroup in a form of their own, fewer in that of five
+#define MQ_BY_COUNT(tiles, GO, WT_)        \
+    do {                                   \
+        if ((tiles) >= 8) GO(WT_, 8);      \
+        else if ((tiles) == 7) GO(WT_, 7); \
+        else if ((tiles) == 6) GO(WT_, 6); \
+        else GO(WT_, 5);                   \
     } while (0)
 }  // namespace
 
@@ -1118,12 +1165,14 @@ hipError_t launch_prefill_gemm_pair(const uint8_t* gate, const uint8_t* up, int 
     if (rowtiles == 0 || m_tiles == 0) return hipSuccess;
     if (!gemm_type(wtype) || ps.splits != 1 || ps.groups > 65535u) return hipErrorInvalidValue;
     if (hipError_t e = raise_gemm_lds(); e != hipSuccess) return e;
-#define MQ_GO(WT_)                                                                                                                        \
-    MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, \
+#define MQ_PAIR(WT_, MT_)                                                                                                                 \
+    MQ_LAUNCH((prefill_gemm_kernel<2, WT_, true, MT_, false, true>), dim3(ps.row_wgs, ps.groups, 1u), dim3(256), kGemmLds, stream, \
               gate, rowtiles, rows, nb, ap, m_tiles, n, h, ldh, (int)nb, (int64_t)0, (const int32_t*)nullptr, (int64_t)0,               \
               (const int32_t*)nullptr, (const uint8_t*)nullptr, up, (const uint8_t*)nullptr, silu_mode, ps.tiles_per_wg)
+#define MQ_GO(WT_) MQ_BY_COUNT(ps.tiles_per_wg, MQ_PAIR, WT_)
     MQ_BY_TYPE(wtype, MQ_GO);
 #undef MQ_GO
+#undef MQ_PAIR
     return hipGetLastError();
 }
 
@@ -1203,15 +1252,19 @@ hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_
     const int64_t ld = split ? rows : ldy;
     const int64_t stride = split ? n * rows : 0;
     const dim3 grid(ps.row_wgs, ps.groups, (unsigned)ps.splits);
-#define MQ_DENSE(KW, WT_)                                                                                                                 \
-    MQ_LAUNCH((prefill_gemm_kernel<KW, WT_>), grid, dim3(256), 2 * kMTilesPerGroup * kPTileBytes, stream, w, rowtiles, rows, nb, ap, m_tiles, \
+#define MQ_WIDE(WT_, MT_) MQ_DENSE(2, WT_, MT_)
+#define MQ_NARROW(WT_, MT_) MQ_DENSE(1, WT_, MT_)
+#define MQ_DENSE(KW, WT_, MT_)                                                                                                            \
+    MQ_LAUNCH((prefill_gemm_kernel<KW, WT_, false, MT_, false, true>), grid, dim3(256), kGemmLds, stream, w, rowtiles, rows, nb, ap, m_tiles, \
               n, out, ld, ps.sb_split, stride, (const int32_t*)nullptr, (int64_t)0, (const int32_t*)nullptr, (const uint8_t*)nullptr, \
               (const uint8_t*)nullptr, (const uint8_t*)nullptr, 0, ps.tiles_per_wg)
 #define MQ_GO(WT_)                       \
-    if (ps.narrow) MQ_DENSE(1, WT_);     \
-    else MQ_DENSE(2, WT_)
+    if (ps.narrow) MQ_BY_COUNT(ps.tiles_per_wg, MQ_NARROW, WT_); \
+    else MQ_BY_COUNT(ps.tiles_per_wg, MQ_WIDE, WT_)
     MQ_BY_TYPE(wtype, MQ_GO);
 #undef MQ_GO
+#undef MQ_NARROW
+#undef MQ_WIDE
 #undef MQ_DENSE
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (split) {
