@@ -112,7 +112,7 @@ __device__ __forceinline__ void request_a_rows(const GatherOffsets<MT>& off, con
 // accumulators for eight only cost registers and LDS -- and how many workgroups a compute unit holds is what hides the
 // latency of a workgroup that walks eight super-blocks with a barrier each.
 template <int kWTilesPerWave, int WT = kWtQ4, bool PAIR = false, int MT = kMTilesPerGroup, bool GATHER = false, bool kDense = false>
-__global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __restrict__ w, int64_t rowtiles, int64_t rows,
+__global__ void __launch_bounds__(256, PAIR && MT == kMTilesMid && WT != kWtQ5 ? 3 : 2) prefill_gemm_kernel(const uint8_t* __restrict__ w, int64_t rowtiles, int64_t rows,
                                                            int64_t nb, const uint8_t* __restrict__ ap, int64_t m_tiles,
                                                            int64_t n_tokens, float* __restrict__ y, int64_t ldy, int sb_split,
                                                            int64_t split_stride, const int32_t* __restrict__ plan,
@@ -232,6 +232,7 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
     // 2048 rows 0.96); least where the card's power is the limit (Q4_K from 1500 rows on: 0.98 to 1.0).  Without branches and without kAhead
     // one weight tile gains less and loses up to 9 % where the last column is short.
     constexpr bool kAhead = kDense && kWTilesPerWave == 1;
+    constexpr int kFirst = MT != kMTilesMid || Q5 ? 0 : Q6 ? 2 : 1;
     auto multiply = [&](auto all_c) {
         constexpr bool kAll = decltype(all_c)::value;
         for (int64_t b = b_begin; b < b_end; ++b) {
@@ -252,15 +253,30 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                     if constexpr (Q6) expand_tile6(seg0[t], seg1[t], qh6[t], hdr[t], d6[t], kq, w1);
                     else expand_tile<Q5, kFifthChain<WT, MT>>(seg0[t], seg1[t], hdr[t], qh[t], kq, w1);
                     if (b + 1 < b_end) request_w(b + 1, t);  // the raw tile's registers are free again
+                    // The first kFirst of a tile's four operands are read a tile ahead: as many as leave three wavefronts to a SIMD (none of Q5_K's).
+                    // With the same in prefill_gemm_resident_kernel, 84 blocks of 31 to 158 rows per expert take 0.982 of the time (16 experts,
+                    // top-4, 2816 x 768, Q6_K down at 180 tokens 60.5 -> 56.2 us; 256 + 1, top-8, 2048 x 512 at 1500 tokens 224 -> 221).
+                    v4i first[2][kFirst + 1];
+                    auto read_first = [&](v4i (&f)[kFirst + 1], const uint8_t* at) {
+#pragma unroll
+                        for (int j = 0; j < kFirst; ++j) f[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+                    };
+                    read_first(first[0], a_buf);
 #pragma unroll
                     for (int m = 0; m < MT; ++m) {
                         if (kAll || m < mt_count) {  // uniform over the workgroup
                             const uint8_t* at = a_buf + m * kPTileBytes;
-                            v4i a[4];
+                            ATile now;
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
-                            const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
-                            const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
+                            for (int j = 0; j < 4; ++j) now.a[j] = j < kFirst ? first[m & 1][j < kFirst ? j : 0] : *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+                            if constexpr (!Q6) now.dg = *reinterpret_cast<const v8h*>(at + digit_off);
+                            now.yd = *reinterpret_cast<const v4f*>(at + kPScaleOff + kq * 16);
+                            if constexpr (kFirst > 0) {
+                                if (m + 1 < MT) read_first(first[(m + 1) & 1], at + kPTileBytes);  // (past mt_count: read and not used)
+                                __builtin_amdgcn_sched_barrier(0);  // ahead of this tile's products
+                            }
+                            const v4i (&a)[4] = now.a;
+                            const float ydv[4] = {now.yd.x, now.yd.y, now.yd.z, now.yd.w};
                             const v4i zero = {0, 0, 0, 0};
                             const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
                             v4i hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.hi[0], zero, 0, 0, 0);
@@ -268,7 +284,7 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(const uint8_t* __r
                             v4i b5 = zero;
                             if constexpr (kFifthChain<WT, MT>) b5 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0], w1.b5[0], zero, 0, 0, 0);
                             v4f mn = zero_f;
-                            if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(at + digit_off), w1.mins, zero_f, 0, 0, 0);
+                            if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(now.dg, w1.mins, zero_f, 0, 0, 0);
 #pragma unroll
                             for (int j = 1; j < 4; ++j) {
                                 hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], w1.hi[j], hi, 0, 0, 0);
@@ -418,6 +434,7 @@ __global__ void __launch_bounds__(256, 3) prefill_gemm_resident_kernel(const uin
     extern __shared__ __align__(16) uint8_t a_lds[];  // nb buffers of MT * kPTileBytes bytes, then the output row of each of the tiles' rows
     constexpr int kBufBytes = MT * kPTileBytes;
     constexpr bool Q5 = WT == kWtQ5, Q6 = WT == kWtQ6;
+    constexpr int kFirst = MT == kMTilesMid && !Q5 ? 2 : 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
     const int item = blockIdx.y;
@@ -466,20 +483,32 @@ __global__ void __launch_bounds__(256, 3) prefill_gemm_resident_kernel(const uin
             if (b + 1 < nb) request_w(rt, b + 1);
             else if (rt + 4 < rt_end) request_w(rt + 4, 0);
             const uint8_t* a_buf = a_lds + b * kBufBytes;
+            v4i first[2][kFirst + 1];  // the first kFirst of a tile's four operands, one tile ahead
+            auto read_first = [&](v4i (&f)[kFirst + 1], const uint8_t* at) {
+#pragma unroll
+                for (int j = 0; j < kFirst; ++j) f[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+            };
+            read_first(first[0], a_buf);
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
                 if (m < mt_count) {  // uniform over the workgroup
                     const uint8_t* at = a_buf + m * kPTileBytes;
                     v4i a[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
+                    for (int j = 0; j < 4; ++j) a[j] = j < kFirst ? first[m & 1][j < kFirst ? j : 0] : *reinterpret_cast<const v4i*>(at + j * 1024 + lane * 16);
                     const float4 yd = *reinterpret_cast<const float4*>(at + kPScaleOff + kq * 16);
+                    v8h dg;
+                    if constexpr (!Q6) dg = *reinterpret_cast<const v8h*>(at + digit_off);
+                    if constexpr (kFirst > 0) {
+                        if (m + 1 < MT) read_first(first[(m + 1) & 1], at + kPTileBytes);  // (past mt_count: read and not used)
+                        __builtin_amdgcn_sched_barrier(0);  // ahead of this tile's products
+                    }
                     const float ydv[4] = {yd.x, yd.y, yd.z, yd.w};
                     const v4i zero = {0, 0, 0, 0};
                     const v4f zero_f = {0.0f, 0.0f, 0.0f, 0.0f};
                     v4i hi = zero, lo = zero, b5 = zero;
                     v4f mn = zero_f;
-                    if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const v8h*>(at + digit_off), wt.mins, zero_f, 0, 0, 0);
+                    if constexpr (!Q6) mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(dg, wt.mins, zero_f, 0, 0, 0);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], wt.hi[j], hi, 0, 0, 0);
