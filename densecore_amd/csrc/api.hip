@@ -640,7 +640,7 @@ static DensePath dense_path_of(int type, int64_t rows, int64_t nb, int64_t n, bo
         if (swiglu && gemm_pair_shape(type, rows, nb, n, false, &shape)) {
             gemm = shape.us + 0.25e-6f * (float)(n * rows);
         } else {
-            gemm = gemm_shape(type, rows, nb, n).us;
+            gemm = gemm_launch_shape(type, rows, nb, n).us;
             if (swiglu) gemm = 2.0f * gemm + 8.5f + 3.15e-6f * (float)(n * rows);
         }
         us[kGemm] = c.gemm[0] + c.gemm[1] * gemm;
@@ -663,7 +663,7 @@ constexpr int64_t kNormFusedMaxRows = 2;
 
 // A product of rows that are in the P-major layout already
 static int gemm_quantized_locked(const mq_weight* w, const uint8_t* ap, int64_t n, float* y_dev, int64_t ldy, hipStream_t s) {
-    const GemmShape shape = gemm_shape(w->type, w->rows, w->nb, n);
+    const GemmShape shape = gemm_launch_shape(w->type, w->rows, w->nb, n);
     const size_t part_bytes = gemm_part_bytes(shape, w->rows, n);
     if (part_bytes) MQ_HIP(g.kpart.reserve(part_bytes));
     MQ_HIP(launch_prefill_gemm(w->data, w->type, w->rows, w->nb, ap, n, y_dev, ldy, part_bytes ? (float*)g.kpart.ptr : nullptr, shape, s));

@@ -237,6 +237,7 @@ struct GemmShape {
     float us = 0.0f;  // its estimate
 };
 GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n);
+GemmShape gemm_launch_shape(int wtype, int64_t rows, int64_t nb, int64_t n);  // ... or that of the rows padded to four, if they do not divide and it is the shorter one
 size_t gemm_part_bytes(const GemmShape& shape, int64_t rows, int64_t n);
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
                                int64_t ldy, float* part, const GemmShape& shape, hipStream_t stream);

@@ -73,7 +73,9 @@ int mq_debug_set_dense_lds(int on);
 
 /* Launch shape that the matrix-core GEMM takes for a product of n rows (pair 1: for gate and up in one launch, 2: ahead of a down product), for a 256-unit
  * device before mq_init.  shape_out: 64-row workgroups (1) or 128-row ones (0), runs of K, super-blocks per run, activation tiles per
- * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns. */
+ * workgroup, workgroup rows, workgroup columns, whether the one launch is taken (1 where pair == 0), the estimate in ns.  Planes of
+ * partial sums have rows of four floats, so for a row count that does not divide by four this is the best shape without runs; a product of
+ * such a matrix is launched in the shape of the row count padded to four where that one's estimate is less. */
 int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);
 
 /* Kernels that a dense product of n rows (pair 1: gate and up in one call; 2: the down product of an FFN whose gate and up run on the
