@@ -353,7 +353,8 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
 // Activation tiles to a workgroup: as many as leave two workgroups for every unit
 int q80_gemm_tiles(int64_t rows, int64_t n) {
     const int64_t row_wgs = ((rows + 15) / 16 + 3) / 4, m_tiles = (n + 15) / 16, enough = 2 * (int64_t)compute_units();
-    return row_wgs * ((m_tiles + 3) / 4) >= enough ? 4 : row_wgs * ((m_tiles + 1) / 2) >= enough ? 2 : 1;
+    // (no more than there are: the form of four holds two workgroups fewer to a unit)
+    return m_tiles > 2 && row_wgs * ((m_tiles + 3) / 4) >= enough ? 4 : m_tiles > 1 && row_wgs * ((m_tiles + 1) / 2) >= enough ? 2 : 1;
 }
 
 size_t q80_tiles_bytes(int64_t n, int64_t nb) { return (size_t)((n + 15) / 16) * (size_t)nb * kQ80ATileBytes; }
