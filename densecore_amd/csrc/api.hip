@@ -661,11 +661,20 @@ static bool gemvn_fused_pays(const mq_weight* w, int64_t n) {
 // its own that emits Q8_K for the LDS-staged product: 36.0 / 36.2 us at two rows, 43.9 / 42.4 at three, 48.6 / 45.7 at four.
 constexpr int64_t kNormFusedMaxRows = 2;
 
+// Room for the planes of a K in runs.  Where there is none -- under graph capture nothing can be allocated, and a call of a larger shape
+// before it may have had K whole -- the product is launched with K whole, which needs none.
+static bool planes_fit(size_t bytes, hipStream_t s) {
+    if (bytes <= g.kpart.cap) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone && g.kpart.reserve(bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
 // A product of rows that are in the P-major layout already
 static int gemm_quantized_locked(const mq_weight* w, const uint8_t* ap, int64_t n, float* y_dev, int64_t ldy, hipStream_t s) {
-    const GemmShape shape = gemm_launch_shape(w->type, w->rows, w->nb, n);
-    const size_t part_bytes = gemm_part_bytes(shape, w->rows, n);
-    if (part_bytes) MQ_HIP(g.kpart.reserve(part_bytes));
+    GemmShape shape = gemm_launch_shape(w->type, w->rows, w->nb, n);
+    size_t part_bytes = gemm_part_bytes(shape, w->rows, n);
+    if (part_bytes && !planes_fit(part_bytes, s)) shape = gemm_whole_k(shape, w->nb), part_bytes = 0;
     MQ_HIP(launch_prefill_gemm(w->data, w->type, w->rows, w->nb, ap, n, y_dev, ldy, part_bytes ? (float*)g.kpart.ptr : nullptr, shape, s));
     return MQ_OK;
 }
@@ -760,7 +769,9 @@ static int ffn_down_locked(const mq_weight* down, int64_t n, bool one_row, float
 // were not fitted: 0.575 of the passes' time, 0.7 % over 3 % behind, at most 9 % (263 x 9984 at 17 rows 26.9 -> 29.2).  us, passes | GEMM:
 // 13611 x 4096 at 9 / 17 / 64 rows 28 / 41 / 116 | 17 / 21 / 42, 1041 x 12288 at 17 / 25 / 33 rows 31.6 / 40.0 / 49.6 | 36.0 / 36.0 / 36.6,
 // 155 x 5632 at 9 / 17 rows 16.3 / 22.6 | 17.7 / 18.2.  Two million products and less are the cost of two launches either way and stay
-// with the passes, as do up to eight rows, whose bits are those of the row alone.
+// with the passes, as do up to eight rows, whose bits are those of the row alone.  The tiles to a workgroup are those there are (with four
+// counted for one or two, matrices of 100,000 rows stayed with the passes: 125313 x 1280 at 10 / 24 rows 89 / 144 us, the GEMM 30 / 33), and
+// the line stays that of K in one run: a product that takes the GEMM by it only gains by runs.
 constexpr int64_t kQ80GemmMaxRows = 16 * 65535, kQ80GemmMinProducts = 1 << 21;
 static bool q80_gemm_applies(int64_t rows, int64_t nb, int64_t n) {
     if (n <= 8 || n > kQ80GemmMaxRows || nb > 65535 || rows * nb * kQK * n < kQ80GemmMinProducts) return false;
@@ -777,7 +788,9 @@ static int mul_mat_q80_locked(const mq_weight* w, const float* x_dev, int64_t n,
         return fail(MQ_ERR_INVALID, "Q8_0 product: activation rows must be 16-byte aligned (ldx %% 4 == 0)");
     if (!dbg_sum && q80_gemm_applies(w->rows, w->nb, n)) {
         MQ_HIP(g.ap.reserve(q80_tiles_bytes(n, w->nb)));
-        MQ_HIP(launch_q80_gemm(w->data, w->rows, w->nb, x_dev, n, ldx, (uint8_t*)g.ap.ptr, y_dev, ldy, s));
+        int runs = q80_gemm_runs(w->rows, w->nb, n);
+        if (runs > 1 && !planes_fit(planes_bytes(runs, w->rows, n), s)) runs = 1;
+        MQ_HIP(launch_q80_gemm(w->data, w->rows, w->nb, x_dev, n, ldx, (uint8_t*)g.ap.ptr, y_dev, ldy, runs > 1 ? (float*)g.kpart.ptr : nullptr, runs, s));
         return MQ_OK;
     }
     MQ_HIP(g.aq.reserve(aq_bytes(n, w->nb)));

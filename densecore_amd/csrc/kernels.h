@@ -176,10 +176,12 @@ struct Q80MatmulArgs {
 size_t q80_scale_bytes(int64_t n, int64_t nb);
 // x rows 16-byte aligned (ldx % 4 == 0), cols % 256 == 0
 hipError_t launch_quantize_q80(const float* x, int64_t n, int64_t ldx, int64_t cols, uint8_t* aq, uint16_t* ah, hipStream_t stream);
-// Dense Q8_0 product of many rows: quantizer into tiles of sixteen rows (q80_tiles_bytes(n, nb) bytes at ap), then the GEMM.
+// Dense Q8_0 product of many rows: quantizer into tiles of sixteen rows (q80_tiles_bytes(n, nb) bytes at ap), then the GEMM, K whole or in
+// up to q80_gemm_runs() runs whose sums go to planes of `part` (planes_bytes(runs, rows, n) bytes).
+int q80_gemm_runs(int64_t rows, int64_t nb, int64_t n);
 size_t q80_tiles_bytes(int64_t n, int64_t nb);
 int q80_gemm_tiles(int64_t rows, int64_t n);  // activation tiles that a workgroup takes: 1, 2 or 4
-hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy,
+hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy, float* part, int runs,
                            hipStream_t stream);
 hipError_t launch_q80_matmul(const Q80MatmulArgs& a, hipStream_t stream);
 
@@ -239,6 +241,15 @@ struct GemmShape {
 GemmShape gemm_shape(int wtype, int64_t rows, int64_t nb, int64_t n);
 GemmShape gemm_launch_shape(int wtype, int64_t rows, int64_t nb, int64_t n);  // ... or that of the rows padded to four, if they do not divide and it is the shorter one
 size_t gemm_part_bytes(const GemmShape& shape, int64_t rows, int64_t n);
+// The same workgroups with K whole
+inline GemmShape gemm_whole_k(GemmShape shape, int64_t nb) {
+    shape.splits = 1, shape.sb_split = (int)nb;
+    return shape;
+}
+// Planes of partial sums: `splits` of n rows, each plane_pitch(rows) floats long, added in order into y
+inline int64_t plane_pitch(int64_t rows) { return (rows + 3) & ~(int64_t)3; }
+size_t planes_bytes(int splits, int64_t rows, int64_t n);
+hipError_t launch_sum_planes(const float* part, int splits, int64_t n, int64_t rows, float* y, int64_t ldy, hipStream_t stream);
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
                                int64_t ldy, float* part, const GemmShape& shape, hipStream_t stream);
 // silu(gate . x) * (up . x) from ONE launch (prefill.hip: the pair form of the GEMM kernel), dense and expert-grouped.

@@ -1107,7 +1107,6 @@ hipError_t raise_gemm_lds() {
 // workgroups to a unit) 4096 x 1024 at 300 tokens 104 -> 114 us.
 constexpr int kResidentTiles = 8, kResidentRowBlocks = 2;
 constexpr int64_t kGatherMaxRows = ((int64_t)1 << 31) / kPRowBytes;  // a row's offset in its plane is a 32-bit one
-int64_t plane_pitch(int64_t rows) { return (rows + 3) & ~(int64_t)3; }
 int pace_of(int wtype) { return wtype == kTypeQ6K ? 2 : wtype == kTypeQ5K ? 1 : 0; }
 bool gemm_type(int wtype) { return wtype == kTypeQ4K || wtype == kTypeQ5K || wtype == kTypeQ6K; }
 // GO(form constant) for the weight type of a launch
@@ -1250,7 +1249,7 @@ hipError_t launch_prefill_gemm_grouped_pair(const uint8_t* gate, const uint8_t* 
 }
 
 size_t gemm_part_bytes(const GemmShape& ps, int64_t rows, int64_t n) {
-    return ps.splits > 1 ? (size_t)ps.splits * (size_t)n * (size_t)plane_pitch(rows) * sizeof(float) : 0;
+    return ps.splits > 1 ? planes_bytes(ps.splits, rows, n) : 0;
 }
 
 size_t prow_bytes(int64_t n, int64_t nb) { return (size_t)n * (size_t)nb * kPRowBytes; }
@@ -1285,6 +1284,14 @@ hipError_t launch_swiglu_quantize_q8k_pmajor(const float* gate, const float* up,
     return hipGetLastError();
 }
 
+size_t planes_bytes(int splits, int64_t rows, int64_t n) { return (size_t)splits * (size_t)n * (size_t)plane_pitch(rows) * sizeof(float); }
+
+hipError_t launch_sum_planes(const float* part, int splits, int64_t n, int64_t rows, float* y, int64_t ldy, hipStream_t stream) {
+    const int64_t pitch = plane_pitch(rows), units = n * (pitch >> 2);
+    MQ_LAUNCH(prefill_sum_planes_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, part, splits, n, rows, pitch, y, ldy);
+    return hipGetLastError();
+}
+
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
                                int64_t ldy, float* part, const GemmShape& ps, hipStream_t stream) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16;
@@ -1314,9 +1321,7 @@ hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_
 #undef MQ_DENSE
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (split) {
-        const int64_t units = n * (ld >> 2);
-        MQ_LAUNCH(prefill_sum_planes_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, part, ps.splits, n,
-                           rows, ld, y, ldy);
+        return launch_sum_planes(part, ps.splits, n, rows, y, ldy, stream);
     }
     return hipGetLastError();
 }

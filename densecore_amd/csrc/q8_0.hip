@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(256) quantize_q80_tiles_kernel(const float* __
 // (541 TOP/s), 920 x 6912 26 / 92 / 369 / 811 | 22 / 23 / 27 / 43.
 template <int MT>
 __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restrict__ w, int64_t rowtiles, int64_t rows, int nb, const uint8_t* __restrict__ ap,
-                                                          int64_t m_tiles, int64_t n, float* __restrict__ y, int64_t ldy) {
+                                                          int64_t m_tiles, int64_t n, float* __restrict__ y, int64_t ldy, int sb_run, int64_t plane) {
     __shared__ __align__(16) uint8_t a_lds[2][MT * kQ80ATileBytes];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, kq = lane >> 4;
@@ -283,30 +283,33 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
     const int mt_count = (int)(m_tiles - mt0 < MT ? m_tiles - mt0 : MT);
     const int64_t rt = (int64_t)blockIdx.x * 4 + wave;  // row tiles past the end: the last one again, not stored
     const uint8_t* tile = w + tile_offset(rt < rowtiles ? rt : rowtiles - 1, 0, nb, kTile80Bytes);
-    float even[MT][4], odd[MT][4];  // sums over the even and the odd super-blocks
+    // K in runs over grid.z: super-blocks [begin, end) into plane blockIdx.z
+    const int begin = (int)blockIdx.z * sb_run, end = begin + sb_run < nb ? begin + sb_run : nb;
+    y += (size_t)blockIdx.z * (size_t)plane;
+    float even[MT][4], odd[MT][4];  // sums over the run's even and odd super-blocks
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int i = 0; i < 4; ++i) even[m][i] = odd[m][i] = 0.0f;
     Tile80 next;
     auto request = [&](int b) {
-        request_a_tiles(ap + ((size_t)b * (size_t)m_tiles + (size_t)mt0) * kQ80ATileBytes, a_lds[b & 1], mt_count * kQ80ATileWords, wave, lane);
+        request_a_tiles(ap + ((size_t)b * (size_t)m_tiles + (size_t)mt0) * kQ80ATileBytes, a_lds[(b - begin) & 1], mt_count * kQ80ATileWords, wave, lane);
 #pragma unroll
         for (int c = 0; c < 4; ++c) next.q[c] = load16(tile + (size_t)b * kTile80Bytes + c * 1024 + lane * 16);
         next.sc = load16(tile + (size_t)b * kTile80Bytes + kTile80SOff + r * 16);
     };
-    request(0);
+    request(begin);
     auto step = [&](int b, float (&sum)[MT][4]) {
         __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xF << 8));  // vmcnt(0): what this thread asked for has landed ...
         __syncthreads();                                          // ... and everybody else's; the other buffer is free
         const Tile80 cur = next;
-        if (b + 1 < nb) request(b + 1);
+        if (b + 1 < end) request(b + 1);
         float dx[8];
         unpack_halves(cur.sc, dx);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             if (m < mt_count) {  // uniform over the workgroup
-                const uint8_t* at = a_lds[b & 1] + m * kQ80ATileBytes;
+                const uint8_t* at = a_lds[(b - begin) & 1] + m * kQ80ATileBytes;
                 float part[4];  // the super-block's sum
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
@@ -331,12 +334,12 @@ __global__ void __launch_bounds__(256, 4) q80_gemm_kernel(const uint8_t* __restr
             }
         }
     };
-    int b = 0;
-    for (; b + 1 < nb; b += 2) {
+    int b = begin;
+    for (; b + 1 < end; b += 2) {
         step(b, even);
         step(b + 1, odd);
     }
-    if (b < nb) step(b, even);
+    if (b < end) step(b, even);
     const int64_t row = rt * 16 + r;
     if (rt >= rowtiles || row >= rows) return;
 #pragma unroll
@@ -357,23 +360,48 @@ int q80_gemm_tiles(int64_t rows, int64_t n) {
     return m_tiles > 2 && row_wgs * ((m_tiles + 3) / 4) >= enough ? 4 : m_tiles > 1 && row_wgs * ((m_tiles + 1) / 2) >= enough ? 2 : 1;
 }
 
+// K in runs of at least four super-blocks where the estimate of the GEMM (api.hip) for a run, with a launch and the planes written and read,
+// is under 0.9 of that of K whole: a workgroup walks its super-blocks one after the other, half a microsecond each, whatever units that
+// leaves idle.  us before | after: 527 x 12544 at 148 rows 39.0 | 20.2, 1866 x 10240 at 27 31.3 | 16.0, 1140 x 13056 at 61 39.4 | 19.4,
+// 6315 x 6912 at 15 23.0 | 15.6, 5903 x 12544 at 28 38.4 | 31.1; 137 products 0.949 of the time, those left whole 1.000.
+int q80_gemm_runs(int64_t rows, int64_t nb, int64_t n) {
+    const int64_t m_tiles = (n + 15) / 16, mt = q80_gemm_tiles(rows, n), wgs = ((rows + 15) / 16 + 3) / 4 * ((m_tiles + mt - 1) / mt);
+    float best = 0.0f;
+    int runs = 1;
+    for (int s = 1; s <= 16 && (s == 1 || nb >= 4 * s); ++s) {
+        const int64_t sb = (nb + s - 1) / s;
+        if ((nb + sb - 1) / sb != s) continue;  // a count that leaves no empty run
+        const float load = (float)(wgs * s) / (float)(2 * compute_units()), k = (float)sb;
+        float us = 6.8f + 0.51f * k + (load > 1.0f ? 1.18f * k * (float)mt * (load - 1.0f) : 0.0f) + 19e-6f * (float)rows * (float)nb;
+        if (s > 1) us += 2.8f + 0.55e-6f * (float)s * (float)(n * rows);
+        if (s == 1 || us < best) best = s == 1 ? 0.9f * us : us, runs = s;
+        if (load > 2.0f) break;  // two rounds: further runs only add planes
+    }
+    return runs;
+}
+
 size_t q80_tiles_bytes(int64_t n, int64_t nb) { return (size_t)((n + 15) / 16) * (size_t)nb * kQ80ATileBytes; }
 
-hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy, hipStream_t stream) {
+hipError_t launch_q80_gemm(const uint8_t* w, int64_t rows, int64_t nb, const float* x, int64_t n, int64_t ldx, uint8_t* ap, float* y, int64_t ldy, float* part,
+                           int runs, hipStream_t stream) {
     const int64_t rowtiles = (rows + 15) / 16, m_tiles = (n + 15) / 16, row_wgs = (rowtiles + 3) / 4;
     if (rows <= 0 || nb <= 0 || n <= 0 || !w || !x || !ap || !y || ldy < rows || ldx < nb * kQK) return hipErrorInvalidValue;
     if (nb > 65535 || m_tiles > 65535 || (ldx & 3) || (reinterpret_cast<uintptr_t>(x) & 15u)) return hipErrorInvalidValue;
     MQ_LAUNCH(quantize_q80_tiles_kernel, dim3((unsigned)m_tiles, (unsigned)nb), dim3(256), 0, stream, x, n, ldx, m_tiles, ap);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    const int tiles = q80_gemm_tiles(rows, n);
+    const int tiles = q80_gemm_tiles(rows, n), sb_run = (int)((nb + runs - 1) / runs);
+    if (runs < 1 || (runs > 1 && !part)) return hipErrorInvalidValue;
+    float* out = runs > 1 ? part : y;
+    const int64_t ld = runs > 1 ? plane_pitch(rows) : ldy, plane = runs > 1 ? n * ld : 0;
 #define MQ_Q80(MT)                                                                                                                     \
-    MQ_LAUNCH(q80_gemm_kernel<MT>, dim3((unsigned)row_wgs, (unsigned)((m_tiles + MT - 1) / MT)), dim3(256), 0, stream, w, rowtiles, rows, (int)nb, \
-              (const uint8_t*)ap, m_tiles, n, y, ldy)
+    MQ_LAUNCH(q80_gemm_kernel<MT>, dim3((unsigned)row_wgs, (unsigned)((m_tiles + MT - 1) / MT), (unsigned)runs), dim3(256), 0, stream, w, rowtiles, rows, (int)nb, \
+              (const uint8_t*)ap, m_tiles, n, out, ld, sb_run, plane)
     if (tiles == 4) MQ_Q80(4);
     else if (tiles == 2) MQ_Q80(2);
     else MQ_Q80(1);
 #undef MQ_Q80
-    return hipGetLastError();
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || runs == 1) return e;
+    return launch_sum_planes(part, runs, n, rows, y, ldy, stream);
 }
 
 size_t q80_scale_bytes(int64_t n, int64_t nb) { return ad_count(n, nb) * 8 * sizeof(uint16_t); }
