@@ -1333,14 +1333,16 @@ static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
 // estimate below 192 tokens), on 0.3 % of them it costs over 3 %, on 0.1 % over 8 % more than that did (with 20 in place of 12: 1.005,
 // 0.5 and 0.2 %, but one pair of nodes in ten 3 to 8 % slower, whose GEMM pays for a launch that clears the rows).  Fewer than 64 pairs stay on the
 // decode launches: the GEMM's fixed part is the longer one (8 experts, top-2, 20 tokens 32 against 43 us).
-// Nine to sixteen tokens, which are two groups of eight rows an expert at most: where there are over five rows an expert and a wavefront of
-// the decode launch has two super-blocks of a row or more one after the other.  110 random blocks of 8 to 64 experts on the GEMM and on the
-// decode launches: 0.50 to 0.96 of the time where the rule takes it, 0.62 to 1.27 elsewhere; 8 experts, top-8, 3840 x 1536 at 11 tokens
-// 83.2 -> 41.3 us, top-4, 2048 x 512 at 16 (one super-block to a wavefront) 28.8 against 36.5.
+// Nine to sixteen tokens, which are two groups of eight rows an expert at most: where there are six rows an expert and a wavefront of the
+// decode launch has five super-blocks of a row or more one after the other.  110 random blocks of 8 to 64 experts on the GEMM and on the
+// decode launches: 0.50 to 0.88 of the time where the rule takes it, 0.57 to 1.27 elsewhere; 8 experts, top-8, 3840 x 1536 at 11 tokens
+// 83.2 -> 41.3 us, top-4, 2048 x 512 at 16 (one super-block to a wavefront) 28.8 against 36.5.  With five rows and two super-blocks the
+// blocks gained too (0.50 to 0.96), but a gate/up node by itself took up to 1.4 of the time (8 experts, top-6, 3840 x 512 at 13 tokens, three
+// super-blocks to a wavefront, 23 -> 33 us).
 // 64 experts, top-6, 2048 x 512 at 64 tokens 65.8 -> 53.7 us, 16 experts, top-8, 2816 x 768 at 24 tokens 98.7 -> 42.4.
 static bool moe_block_takes_gemm(int64_t n_experts, int64_t hidden, int64_t inter, int64_t n, int top_k) {
     const int64_t pairs = n * top_k;
-    if (n < kMoeGemmMinTokens && (n <= 8 || pairs <= 5 * n_experts || hidden / kQK < 2 * pick_waves(hidden / kQK, (inter + 15) / 16 * n_experts))) return false;
+    if (n < kMoeGemmMinTokens && (n <= 8 || pairs < 6 * n_experts || hidden / kQK < 5 * pick_waves(hidden / kQK, (inter + 15) / 16 * n_experts))) return false;
     if (pairs < 64 || n_experts > 4096 || (hidden & 3) || (inter & 3)) return false;
     const float rpe = (float)pairs / (float)n_experts;
     if (12.0f * rpe * rpe * rpe >= (float)inter) return true;

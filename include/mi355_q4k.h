@@ -250,8 +250,8 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * down with the Q8_K of the hidden rows and the weighted combine inside.  Above: router + expert grouping + Q8_K
  * of x, expert-grouped gate/up leaving its rows in Q8_K, expert-grouped down, combine.  Same bits either way.
  * From 17 tokens with 64 routed pairs on, where the routed rows per expert r satisfy inter <= 12 r^3 (2.8 rows at 256 hidden
- * values per expert, 3.5 at 512, 4.4 at 1024) or r >= 6 (below 192 tokens r >= 5 and an estimate) -- from nine tokens where also r > 5 and the decode launch would
- * give a wavefront two super-blocks of a row or more --, the expert products run on the
+ * values per expert, 3.5 at 512, 4.4 at 1024) or r >= 6 (below 192 tokens r >= 5 and an estimate) -- from nine tokens where r >= 6 and the decode launch would
+ * give a wavefront five super-blocks of a row or more --, the expert products run on the
  * int8 matrix-core GEMM in an expert-grouped form (entries in 16-row tiles per expert), the shared expert as one more
  * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches (from 192 tokens); same
  * routing, results within the fp32 tolerance of the other form (the
