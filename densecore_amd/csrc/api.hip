@@ -1880,12 +1880,13 @@ int decoder_grid(size_t lds_bytes, int* n_workgroups, long long* spin_ticks) {
 
 }  // namespace
 
-// Decided per product: gate / up (one type) and down each run on the expert-grouped GEMM when their type is one it takes; a layer with
-// a Q8_0 down stack (core/src/llm/moe/native.cpp:4611-4620; its activations are Q8_0 as well) keeps its two large
-// products on the matrix cores from 192 tokens on and sends the fp32 hidden rows through the Q8_0 launches.
 // Up to this many tokens the GEMM's hidden rows lie at their (token, slot) places, as the decode launches leave them and where
 // mq_debug_moe_hidden finds them; more stay in its tiles, which its quantizer reads in order.
 constexpr int64_t kMoeRowsInPlaceTokens = 64;
+
+// Decided per product: gate / up (one type) and down each run on the expert-grouped GEMM when their type is one it takes; a layer with
+// a Q8_0 down stack (core/src/llm/moe/native.cpp:4611-4620; its activations are Q8_0 as well) keeps its two large
+// products on the matrix cores from 192 tokens on and sends the fp32 hidden rows through the Q8_0 launches.
 static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
     const mq_weight* ge = L->gate_exps;
     // (a Q8_0 down stack's launches follow either way: 42 us a block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them)
