@@ -257,13 +257,14 @@ hipError_t census_launch(const MatmulArgs& a, hipStream_t s) {
 // counters) are one set per process, so a call on stream B must not start on the device before the previous call on
 // stream A has finished with them.  A stream under graph capture is left alone (an event recorded outside the capture
 // cannot be waited on inside it): a graph's replays are ordered by whoever launches them.
-int order_stream(hipStream_t s) {
+int order_stream(hipStream_t s, bool* capturing) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess) {
         (void)hipGetLastError();
         st = hipStreamCaptureStatusNone;
     }
-    if (st != hipStreamCaptureStatusNone) {
+    *capturing = st != hipStreamCaptureStatusNone;
+    if (*capturing) {
         g_graph_seen = true;
         return MQ_OK;
     }
@@ -285,9 +286,17 @@ int order_stream(hipStream_t s) {
 }
 struct Entry {
     std::lock_guard<std::recursive_mutex> lock;
+    bool capturing = false;
     int rc;
-    explicit Entry(hipStream_t s) : lock(g.mu), rc(order_stream(s)) {}
+    explicit Entry(hipStream_t s) : lock(g.mu), rc(order_stream(s, &capturing)) {}
 };
+
+// Room that a smaller call under graph capture, where nothing can be allocated, may need and this one does not: one eager call of the
+// largest shape serves every smaller width, whichever kernels that takes (outside a capture only; at an entry point's start, before anything
+// lies in the workspaces: one that grows loses what it holds).  No room for it is no error of this call.
+void reserve_ahead(const Entry& entry, Buffer& b, size_t bytes) {
+    if (!entry.capturing && b.reserve(bytes) != hipSuccess) (void)hipGetLastError();
+}
 
 int check_ready() {
     if (!g.ready) return fail(MQ_ERR_STATE, "mq_init has not been called (or no GPU is present)");
@@ -1963,6 +1972,8 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         // expert as a dense FFN on it; per-(token, slot) rows and the combine as at the other widths.
         // The shared expert rides along as one more group of all tokens (its own weights, its own SiLU form, output slot K).
         const int64_t entries = n * K + (sh.gate ? n : 0), G = E + (sh.gate ? 1 : 0);
+        // (rows in place are in mid, those of this many tokens in mid2)
+        if (n > kMoeRowsInPlaceTokens) reserve_ahead(entry, g.mid, (size_t)kMoeRowsInPlaceTokens * (size_t)slots * (size_t)inter * sizeof(float));
         MQ_HIP(g.part.reserve((size_t)n * slots * (size_t)hidden * sizeof(float)));
         float* part = (float*)g.part.ptr;
         MQ_HIP(launch_route_topk(logits_dev, E, n, K, L->route_mode, ids, wts, s));
