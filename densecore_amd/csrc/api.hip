@@ -1359,6 +1359,47 @@ static bool moe_block_takes_gemm(int64_t n_experts, int64_t hidden, int64_t inte
     return pairs >= 5 * n_experts && moe_gemm_estimate(n_experts, (hidden + 15) / 16, hidden, inter / kQK, n, top_k);
 }
 
+// Room for expert-grouped calls of up to n tokens (reserve_ahead): for the decode launches, which take fewer than 192 tokens or six rows per
+// expert, and for the GEMM, which takes no block on the lower side of both its lines (five rows per expert, inter <= 12 r^3).
+struct MoeAhead {
+    int64_t n_experts, n;
+    int top_k, slots;
+    int64_t in_cols, in_rows;     // quantized input rows: columns (0: none), rows per token
+    int64_t inter, hidden;        // hidden rows (0: none) and the outputs of the down product on them (0: none)
+    bool layer, gemm;             // the hidden rows stay inside the call; the expert-grouped GEMM takes its types
+};
+static int moe_reserve_ahead(const Entry& entry, const MoeAhead& m) {
+    if (entry.capturing) return MQ_OK;
+    const int64_t decode_most = 6 * m.n_experts / m.top_k > 191 ? 6 * m.n_experts / m.top_k : 191, few = m.n < decode_most ? m.n : decode_most;
+    const int64_t in_nb = m.in_cols / kQK, mid_nb = m.inter / kQK;
+    if (in_nb) {
+        reserve_ahead(entry, g.aq, aq_bytes(few * m.in_rows, in_nb));
+        reserve_ahead(entry, g.ad, ad_count(few * m.in_rows, in_nb) * sizeof(float));
+    }
+    if (mid_nb && m.hidden) {
+        reserve_ahead(entry, g.aq2, aq_bytes(few * m.slots, mid_nb));
+        reserve_ahead(entry, g.ad2, ad_count(few * m.slots, mid_nb) * sizeof(float));
+        reserve_ahead(entry, g.part, (size_t)(few * m.slots) * (size_t)m.hidden * sizeof(float));
+    }
+    if (m.layer) {
+        reserve_ahead(entry, g.mid, (size_t)(few * m.slots) * (size_t)m.inter * sizeof(float));
+        const int64_t pairs = few * m.top_k, groups = (pairs < m.n_experts ? pairs : m.n_experts) + (few + 7) / 8;
+        if (int rc = reserve_counters((size_t)(groups * mid_nb > 4096 ? groups * mid_nb : 4096))) return rc;
+    }
+    const float rpe = (float)(m.n * m.top_k) / (float)m.n_experts;
+    if (!m.gemm || m.n_experts > 4096 || (rpe < 5.0f && (!m.inter || 12.0f * rpe * rpe * rpe < (float)m.inter))) return MQ_OK;
+    const bool shared = m.slots > m.top_k;
+    const int64_t entries = m.n * m.slots, groups = m.n_experts + (shared ? 1 : 0), rows_max = 16 * moe_gemm_tiles_max(entries, groups);
+    reserve_ahead(entry, g.plan, moe_gemm_plan_ints(entries, groups) * sizeof(int32_t));
+    if (in_nb) reserve_ahead(entry, g.ap, prow_bytes(m.n * m.in_rows, in_nb));
+    if (mid_nb && m.hidden) {
+        reserve_ahead(entry, g.ap2, pmajor_bytes(rows_max, mid_nb));
+        reserve_ahead(entry, g.part, (size_t)(m.n * m.slots) * (size_t)m.hidden * sizeof(float));
+    }
+    if (m.layer) reserve_ahead(entry, g.mid2, 2 * (size_t)rows_max * (size_t)m.inter * sizeof(float));
+    return MQ_OK;
+}
+
 int mq_mul_mat_id_q4k(const mq_weight* w, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
                       int top_k, float* y_dev, void* stream) {
     if (int rc = check_ready()) return rc;
@@ -1371,6 +1412,7 @@ int mq_mul_mat_id_q4k(const mq_weight* w, const float* x_dev, int64_t n, int x_s
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    if (int rc = moe_reserve_ahead(entry, {w->n_experts, n, top_k, top_k, w->cols, x_slots, 0, 0, false, moe_gemm_takes(w)})) return rc;
     // prefill widths: the matrix-core GEMM in its expert-grouped form (see mq_moe_layer_q4k)
     const bool use_gemm = moe_gemm_width(w, n, top_k);
     if (!use_gemm)
@@ -1791,6 +1833,8 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    if (int rc = moe_reserve_ahead(entry, {gate_exps->n_experts, n, top_k, top_k, gate_exps->cols, 1, gate_exps->rows, 0, false, moe_gemm_takes(gate_exps)}))
+        return rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, gate_exps->n_experts, r)) return rc;
     MQ_HIP(launch_fill_zero(hidden_dev, (size_t)n * top_k * (size_t)gate_exps->rows, s));
@@ -1841,6 +1885,8 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    if (int rc = moe_reserve_ahead(entry, {down_exps->n_experts, n, top_k, top_k, 0, 0, down_exps->cols, down_exps->rows, false, moe_gemm_takes(down_exps)}))
+        return rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, down_exps->n_experts, r)) return rc;
     if (moe_gemm_takes(down_exps) && moe_block_takes_gemm(down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k)) {
@@ -1942,6 +1988,7 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
     const int slots = K + (sh.gate ? 1 : 0);  // hidden / partial rows per token
     const size_t hidden_rows = (size_t)n * (size_t)slots * (size_t)inter;
     g.hidden_rows = 0;
+    if (int rc = moe_reserve_ahead(entry, {E, n, K, slots, hidden, 1, inter, hidden, true, moe_gemm_takes(L->gate_exps)})) return rc;
     RouteWs r;
     if (int rc = carve_route(n, K, E, r)) return rc;
     // ids and weights go straight to the caller's buffers when it wants them
@@ -1972,8 +2019,6 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         // expert as a dense FFN on it; per-(token, slot) rows and the combine as at the other widths.
         // The shared expert rides along as one more group of all tokens (its own weights, its own SiLU form, output slot K).
         const int64_t entries = n * K + (sh.gate ? n : 0), G = E + (sh.gate ? 1 : 0);
-        // (rows in place are in mid, those of this many tokens in mid2)
-        if (n > kMoeRowsInPlaceTokens) reserve_ahead(entry, g.mid, (size_t)kMoeRowsInPlaceTokens * (size_t)slots * (size_t)inter * sizeof(float));
         MQ_HIP(g.part.reserve((size_t)n * slots * (size_t)hidden * sizeof(float)));
         float* part = (float*)g.part.ptr;
         MQ_HIP(launch_route_topk(logits_dev, E, n, K, L->route_mode, ids, wts, s));
