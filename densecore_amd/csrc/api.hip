@@ -670,20 +670,42 @@ static bool gemvn_fused_pays(const mq_weight* w, int64_t n) {
 // its own that emits Q8_K for the LDS-staged product: 36.0 / 36.2 us at two rows, 43.9 / 42.4 at three, 48.6 / 45.7 at four.
 constexpr int64_t kNormFusedMaxRows = 2;
 
-// Room for the planes of a K in runs.  Where there is none -- under graph capture nothing can be allocated, and a call of a larger shape
-// before it may have had K whole -- the product is launched with K whole, which needs none.
-static bool planes_fit(size_t bytes, hipStream_t s) {
-    if (bytes <= g.kpart.cap) return true;
+// Workspaces of a dense product of up to n rows (reserve_ahead): rows for the decode kernels, which take up to kSkinnyMaxRows of them
+// (Q8_0's passes more of a matrix that is too small for its GEMM), rows and planes for the GEMM.
+constexpr int64_t kQ80GemmMaxRows = 16 * 65535, kQ80GemmMinProducts = 1 << 21;
+static void dense_reserve_ahead(const Entry& entry, const mq_weight* w, int64_t n) {
+    const bool q80 = w->type == kTypeQ80;
+    const int64_t tiny = q80 ? kQ80GemmMinProducts / (w->rows * w->cols) + 1 : 0, most = tiny > kSkinnyMaxRows ? tiny : kSkinnyMaxRows, few = n < most ? n : most;
+    reserve_ahead(entry, g.aq, aq_bytes(few, w->nb));
+    reserve_ahead(entry, g.ad, q80 ? q80_scale_bytes(few, w->nb) : ad_count(few, w->nb) * sizeof(float));
+    if (n <= 8) return;
+    reserve_ahead(entry, g.ap, q80 ? q80_tiles_bytes(n, w->nb) : pmajor_bytes(n, w->nb));
+    reserve_ahead(entry, g.kpart, planes_most(w->rows, w->nb, n));
+}
+// Room for what only one of two forms of a product needs (planes of a K in runs, gate and up as two products): reserved ahead by the eager
+// calls.  Where there is none all the same -- a captured call of a matrix that no eager call had at this width or above, or no memory --
+// the other form is launched, which needs none: K whole, gate and up in one launch.  The sums are in another order then, and it takes longer.
+static bool room_for(Buffer& b, size_t bytes, hipStream_t s) {
+    if (bytes <= b.cap) return true;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone && g.kpart.reserve(bytes) == hipSuccess) return true;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone && b.reserve(bytes) == hipSuccess) return true;
     (void)hipGetLastError();
     return false;
+}
+// ... of gate and up: two products of up to kTwoProductsMost outputs each (the pair launch takes all but a few pairs of more)
+constexpr int64_t kTwoProductsMost = 4 << 20;
+static void pair_reserve_ahead(const Entry& entry, const mq_weight* gate, int64_t n) {
+    dense_reserve_ahead(entry, gate, n);
+    if (n <= kDecodeRows) return;
+    const int64_t outputs = n * gate->rows < kTwoProductsMost ? n * gate->rows : kTwoProductsMost;
+    reserve_ahead(entry, g.mid2, 2 * (size_t)outputs * sizeof(float));
+    if (gate->rows % kQK == 0) reserve_ahead(entry, g.ap2, pmajor_bytes(n, gate->rows / kQK));
 }
 // A product of rows that are in the P-major layout already
 static int gemm_quantized_locked(const mq_weight* w, const uint8_t* ap, int64_t n, float* y_dev, int64_t ldy, hipStream_t s) {
     GemmShape shape = gemm_launch_shape(w->type, w->rows, w->nb, n);
     size_t part_bytes = gemm_part_bytes(shape, w->rows, n);
-    if (part_bytes && !planes_fit(part_bytes, s)) shape = gemm_whole_k(shape, w->nb), part_bytes = 0;
+    if (part_bytes && !room_for(g.kpart, part_bytes, s)) shape = gemm_whole_k(shape, w->nb), part_bytes = 0;
     MQ_HIP(launch_prefill_gemm(w->data, w->type, w->rows, w->nb, ap, n, y_dev, ldy, part_bytes ? (float*)g.kpart.ptr : nullptr, shape, s));
     return MQ_OK;
 }
@@ -704,7 +726,9 @@ static int ffn_wide_locked(const mq_weight* gate, const mq_weight* up, const mq_
     MQ_HIP(g.ap.reserve(pmajor_bytes(n, gate->nb)));
     MQ_HIP(launch_quantize_q8k_pmajor(x_dev, n, ldx, gate->cols, (uint8_t*)g.ap.ptr, s));
     GemmShape pair;
-    if (g_gemm_pair && gate->type == up->type && gemm_pair_shape(gate->type, inter, gate->nb, n, down != nullptr, &pair)) {
+    const size_t two_bytes = 2 * (size_t)n * (size_t)inter * sizeof(float);
+    if (g_gemm_pair && gate->type == up->type &&
+        (gemm_pair_shape(gate->type, inter, gate->nb, n, down != nullptr, &pair) || !room_for(g.mid2, two_bytes, s))) {
         // gate and up in one launch that stores silu(gate) * up: no fp32 planes, no pass that reads them back
         MQ_HIP(launch_prefill_gemm_pair(gate->data, up->data, gate->type, inter, gate->nb, (const uint8_t*)g.ap.ptr, n, silu_mode, h_dev, ldh, pair, s));
         if (!down) return MQ_OK;
@@ -712,7 +736,7 @@ static int ffn_wide_locked(const mq_weight* gate, const mq_weight* up, const mq_
         MQ_HIP(launch_quantize_q8k_pmajor(h_dev, n, ldh, inter, (uint8_t*)g.ap2.ptr, s));
         return gemm_quantized_locked(down, (const uint8_t*)g.ap2.ptr, n, y_dev, ldy, s);
     }
-    MQ_HIP(g.mid2.reserve(2 * (size_t)n * (size_t)inter * sizeof(float)));
+    MQ_HIP(g.mid2.reserve(two_bytes));
     float* gbuf = (float*)g.mid2.ptr;
     float* ubuf = gbuf + (size_t)n * (size_t)inter;
     if (const int rc = gemm_quantized_locked(gate, (const uint8_t*)g.ap.ptr, n, gbuf, inter, s); rc != MQ_OK) return rc;
@@ -781,7 +805,6 @@ static int ffn_down_locked(const mq_weight* down, int64_t n, bool one_row, float
 // with the passes, as do up to eight rows, whose bits are those of the row alone.  The tiles to a workgroup are those there are (with four
 // counted for one or two, matrices of 100,000 rows stayed with the passes: 125313 x 1280 at 10 / 24 rows 89 / 144 us, the GEMM 30 / 33), and
 // the line stays that of K in one run: a product that takes the GEMM by it only gains by runs.
-constexpr int64_t kQ80GemmMaxRows = 16 * 65535, kQ80GemmMinProducts = 1 << 21;
 static bool q80_gemm_applies(int64_t rows, int64_t nb, int64_t n) {
     if (n <= 8 || n > kQ80GemmMaxRows || nb > 65535 || rows * nb * kQK * n < kQ80GemmMinProducts) return false;
     const int64_t rowtiles = (rows + 15) / 16, units = compute_units(), w = pick_waves(nb, rowtiles), mt = q80_gemm_tiles(rows, n);
@@ -798,7 +821,7 @@ static int mul_mat_q80_locked(const mq_weight* w, const float* x_dev, int64_t n,
     if (!dbg_sum && q80_gemm_applies(w->rows, w->nb, n)) {
         MQ_HIP(g.ap.reserve(q80_tiles_bytes(n, w->nb)));
         int runs = q80_gemm_runs(w->rows, w->nb, n);
-        if (runs > 1 && !planes_fit(planes_bytes(runs, w->rows, n), s)) runs = 1;
+        if (runs > 1 && !room_for(g.kpart, planes_bytes(runs, w->rows, n), s)) runs = 1;
         MQ_HIP(launch_q80_gemm(w->data, w->rows, w->nb, x_dev, n, ldx, (uint8_t*)g.ap.ptr, y_dev, ldy, runs > 1 ? (float*)g.kpart.ptr : nullptr, runs, s));
         return MQ_OK;
     }
@@ -831,6 +854,7 @@ int mq_gemm_q4k(const mq_weight* w, const float* x_dev, int64_t n, int64_t ldx, 
     if (!y_dev || ldy < w->rows) return fail(MQ_ERR_INVALID, "mq_gemm_q4k: null output or ldy < rows");
     Entry entry((hipStream_t)stream);
     if (entry.rc) return entry.rc;
+    dense_reserve_ahead(entry, w, n);
     return gemm_locked(w, x_dev, n, ldx, y_dev, ldy, (hipStream_t)stream);
 }
 
@@ -845,6 +869,7 @@ int mq_mul_mat_q4k(const mq_weight* w, const float* x_dev, int64_t n, int64_t ld
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    dense_reserve_ahead(entry, w, n);
     if (w->type == kTypeQ80) return mul_mat_q80_locked(w, x_dev, n, ldx, y_dev, ldy, nullptr, s);
     const DensePath path = dense_path(w, n, false);
     if (path == kGemm) return gemm_locked(w, x_dev, n, ldx, y_dev, ldy, s);
@@ -994,6 +1019,12 @@ int mq_rmsnorm_mul_mat_q4k(const mq_weight* w, const float* x_dev, const float* 
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    dense_reserve_ahead(entry, w, n);
+    if (n > kDecodeRows) {
+        const size_t normed = (size_t)n * (size_t)w->cols * sizeof(float);
+        if (normed > g.mid.cap) g.hidden_rows = 0;  // (rows that lie there are lost)
+        reserve_ahead(entry, g.mid, normed);
+    }
     if (n == 1 && w->type == kTypeQ4K) {  // one row, short K per wave: norm and quantizer run inside the GEMV kernel
         const int waves = dense_waves(w->nb, w->rowtiles);
         if (gemv1_fused_applies(w->nb, waves)) {
@@ -1133,6 +1164,12 @@ int mq_ffn_swiglu_q4k(const mq_weight* gate, const mq_weight* up, const mq_weigh
     Entry entry(s);
     if (entry.rc) return entry.rc;
     g.hidden_rows = 0;
+    pair_reserve_ahead(entry, gate, n);
+    const int64_t few = n < kSkinnyMaxRows ? n : kSkinnyMaxRows;
+    dense_reserve_ahead(entry, down, few);
+    reserve_ahead(entry, g.kpart, planes_most(down->rows, down->nb, n));
+    reserve_ahead(entry, g.aq2, aq_bytes(few, down->nb));
+    reserve_ahead(entry, g.ad2, ad_count(few, down->nb) * sizeof(float));
     const DensePath gate_path = dense_path(gate, n, true), down_path = dense_path_of(down->type, down->rows, down->nb, n, false, gate_path == kGemm);
     if (gate_path == kGemm) {  // wide: the matrix-core GEMM for gate and up, and for down unless another kernel takes less
         MQ_HIP(g.mid.reserve((size_t)n * (size_t)inter * sizeof(float)));
@@ -1694,6 +1731,7 @@ int mq_swiglu_mul_mat_q4k(const mq_weight* gate, const mq_weight* up, const floa
     hipStream_t s = (hipStream_t)stream;
     Entry entry(s);
     if (entry.rc) return entry.rc;
+    pair_reserve_ahead(entry, gate, n);
     const DensePath path = dense_path(gate, n, true);
     if (path == kGemm && !(ldh & 3) && !(reinterpret_cast<uintptr_t>(h_dev) & 15u))
         return ffn_wide_locked(gate, up, nullptr, x_dev, n, ldx, silu_mode, h_dev, ldh, nullptr, 0, s);

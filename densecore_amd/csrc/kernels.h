@@ -249,6 +249,7 @@ inline GemmShape gemm_whole_k(GemmShape shape, int64_t nb) {
 // Planes of partial sums: `splits` of n rows, each plane_pitch(rows) floats long, added in order into y
 inline int64_t plane_pitch(int64_t rows) { return (rows + 3) & ~(int64_t)3; }
 size_t planes_bytes(int splits, int64_t rows, int64_t n);
+size_t planes_most(int64_t rows, int64_t nb, int64_t n);  // ... of any product of up to n rows
 hipError_t launch_sum_planes(const float* part, int splits, int64_t n, int64_t rows, float* y, int64_t ldy, hipStream_t stream);
 hipError_t launch_prefill_gemm(const uint8_t* w, int wtype, int64_t rows, int64_t nb, const uint8_t* ap, int64_t n, float* y,
                                int64_t ldy, float* part, const GemmShape& shape, hipStream_t stream);

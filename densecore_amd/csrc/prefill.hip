@@ -1286,6 +1286,15 @@ hipError_t launch_swiglu_quantize_q8k_pmajor(const float* gate, const float* up,
 
 size_t planes_bytes(int splits, int64_t rows, int64_t n) { return (size_t)splits * (size_t)n * (size_t)plane_pitch(rows) * sizeof(float); }
 
+// A run has at least four super-blocks, and one run fewer would leave at most four workgroups to a unit (choose_shape, q80_gemm_runs), each
+// of at most 128 rows of outputs by 128: (runs - 1) times the outputs is at most `most`, and so are the outputs of a product in runs.
+size_t planes_most(int64_t rows, int64_t nb, int64_t n) {
+    const int64_t most = 4 * (int64_t)compute_units() * 128 * 128, outputs = n * plane_pitch(rows);
+    if (nb < 8) return 0;
+    const int64_t by_units = (outputs < most ? outputs : most) + most;
+    return (size_t)(nb / 4 > by_units / outputs ? by_units : nb / 4 * outputs) * sizeof(float);
+}
+
 hipError_t launch_sum_planes(const float* part, int splits, int64_t n, int64_t rows, float* y, int64_t ldy, hipStream_t stream) {
     const int64_t pitch = plane_pitch(rows), units = n * (pitch >> 2);
     MQ_LAUNCH(prefill_sum_planes_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, part, splits, n, rows, pitch, y, ldy);

@@ -8,6 +8,15 @@
  * as void* (NULL = the default stream).  All launches are stream-ordered and
  * return without synchronising unless the name ends in _host.
  *
+ * Scratch grows on eager calls and never under HIP-graph capture, where nothing
+ * can be allocated.  One eager call of an entry point with its weights at the
+ * largest width makes room for every smaller width: a captured call then runs
+ * the kernels of the eager one and returns its bits.  Without such a call the
+ * capture fails, or -- where another call's scratch holds all but the planes of
+ * partial sums, or gate and up as two products -- a dense product is recorded
+ * in the form that needs neither: the same integers, fp32 sums in another
+ * order, and up to 2.7 times the time.
+ *
  * Each declaration cites the DenseCore interface it stands in for
  * (paths relative to the DenseCore tree).
  */

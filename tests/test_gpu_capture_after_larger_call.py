@@ -96,3 +96,62 @@ def test_expert_nodes_at_every_width(ops, node, experts, k, hidden, inter, down,
         captured_equals_eager(lambda: (call(n),))
     for m in (G, U, D):
         m.free()
+
+
+# K in runs at the captured width and whole at the eager one; every kernel of a dense product below
+@pytest.mark.parametrize("wtype,rows,cols,eager,widths", [(12, 2000, 16384, 4096, (1, 3, 9, 17, 40, 65, 100, 700)), (12, 2001, 16384, 4096, (2, 33, 100)),
+                                                          (13, 4096, 4096, 600, (1, 8, 16, 24, 50, 64, 100)), (14, 6144, 1024, 300, (4, 12, 33, 48, 70)),
+                                                          (8, 2000, 16384, 4096, (1, 8, 9, 17, 40, 100)), (8, 16, 256, 3000, (1, 30, 100, 400))])
+def test_product_at_every_width(ops, wtype, rows, cols, eager, widths):
+    import torch
+    w = ops.Q4KWeight.synthetic(rows, rows, cols, 1, wtype)
+    x = torch.randn((eager, cols), device="cuda")
+    ops.mul_mat(w, x)
+    for n in widths:
+        captured_equals_eager(lambda: (ops.mul_mat(w, x[:n]),))
+    w.free()
+
+
+@pytest.mark.parametrize("types,hidden,inter,eager,widths", [((12, 14), 1024, 4096, 1000, (1, 2, 5, 9, 13, 17, 33, 50, 64, 65, 130, 391)),
+                                                             ((13, 12), 5120, 1024, 300, (1, 8, 16, 30, 64, 100)), ((14, 13), 768, 2816, 64, (1, 4, 12, 17, 40))])
+def test_ffn_and_pair_at_every_width(ops, types, hidden, inter, eager, widths):
+    import torch
+    G, U = (ops.Q4KWeight.synthetic(s, inter, hidden, 1, types[0]) for s in (1, 2))
+    D = ops.Q4KWeight.synthetic(3, hidden, inter, 1, types[1])
+    x = torch.randn((eager, hidden), device="cuda")
+    ops.ffn_swiglu(G, U, D, x)
+    for n in widths:
+        captured_equals_eager(lambda: (ops.ffn_swiglu(G, U, D, x[:n]),))
+    for m in (G, U, D):
+        m.free()
+
+
+@pytest.mark.parametrize("wtype,rows,cols,eager,widths", [(12, 4096, 14336, 400, (1, 9, 20, 42, 64, 100, 140)), (13, 513, 6144, 300, (3, 17, 50, 100))])
+def test_pair_by_itself_at_every_width(ops, wtype, rows, cols, eager, widths):
+    import torch
+    G, U = (ops.Q4KWeight.synthetic(s, rows, cols, 1, wtype) for s in (1, 2))
+    x = torch.randn((eager, cols), device="cuda")
+    ops.swiglu_mul_mat(G, U, x, ops.SILU_FAST)
+    for n in widths:
+        captured_equals_eager(lambda: (ops.swiglu_mul_mat(G, U, x[:n], ops.SILU_FAST),))
+    for m in (G, U):
+        m.free()
+
+
+@pytest.mark.parametrize("eager,widths", [(300, (1, 2, 5, 16, 20, 48, 64, 100))])
+def test_norm_and_product_at_every_width(ops, eager, widths):
+    import torch
+    from densecore_amd import _lib
+    rows, cols = 4096, 2560
+    w = ops.Q4KWeight.synthetic(5, rows, cols)
+    x, g = torch.randn((eager, cols), device="cuda"), torch.randn(cols, device="cuda")
+
+    def call(n):
+        y = torch.empty((n, rows), device="cuda")
+        _lib.check(_lib.lib().mq_rmsnorm_mul_mat_q4k(w._h, x.data_ptr(), None, g.data_ptr(), n, 1e-6, None, y.data_ptr(), rows,
+                                                     torch.cuda.current_stream().cuda_stream), "mq_rmsnorm_mul_mat_q4k")
+        return (y,)
+    call(eager)
+    for n in widths:
+        captured_equals_eager(lambda: call(n))
+    w.free()

@@ -39,7 +39,8 @@ def test_matches_eight_rows_at_a_time(rows, cols, n, tiles):
 
 @pytest.mark.parametrize("wtype,rows", [(Q80, 2000), (12, 2001), (12, 2000)])
 def test_planes_that_cannot_grow_under_capture_leave_k_whole(wtype, rows):
-    """Eager calls of more rows had K whole: the captured one, whose runs would need planes, is taken all the same."""
+    """No eager call had this matrix (one of four rows made room for the activations alone): the captured product, whose runs would need
+    planes, is taken all the same, with K whole, and its sums are in another order than the eager one's."""
     import torch
     from densecore_amd import _lib, ops
     torch.cuda.synchronize()
@@ -47,9 +48,9 @@ def test_planes_that_cannot_grow_under_capture_leave_k_whole(wtype, rows):
     _lib.check(_lib.lib().mq_init(torch.cuda.current_device()), "mq_init")
     cols, n, padded = 16384, 100, (rows + 3) // 4 * 4
     assert wtype == Q80 or (gemm_shape(wtype, padded, cols, 4096)["runs"] == 1 and gemm_shape(wtype, padded, cols, n)["runs"] > 1)
-    w = ops.Q4KWeight.synthetic(rows, rows, cols, 1, wtype)
+    w, other = (ops.Q4KWeight.synthetic(rows, r, cols, 1, wtype) for r in (rows, 4))
     x = torch.randn(4096, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
-    ops.mul_mat(w, x)
+    ops.mul_mat(other, x)
     side, out, graph = torch.cuda.Stream(), torch.empty(n, rows, device="cuda"), torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
         ops.mul_mat(w, x[:n], out)
@@ -57,4 +58,6 @@ def test_planes_that_cannot_grow_under_capture_leave_k_whole(wtype, rows):
     want = ops.mul_mat(w, x[:n])
     torch.cuda.synchronize()
     assert (out - want).abs().max().item() <= 2 * cols / 32 * 2.0 ** -24 * want.abs().max().item()
-    w.free()
+    assert not torch.equal(out, want)
+    for m in (w, other):
+        m.free()
