@@ -230,7 +230,10 @@ __global__ void __launch_bounds__(256, PAIR && MT == kMTilesMid && WT != kWtQ5 ?
     // bits: 198 products of 64-row workgroups at 70 to 512 rows 0.951 of the time (Q4_K 2048 x 2048 at 128 rows 13.0 -> 12.1 us, Q5_K 4096 x 4096
     // at 100 rows 21.0 -> 19.0), 366 products and FFNs at 70 to 2048 rows 0.968 (Q4_K 14336 x 4096 at 700 rows 111 -> 99 us, Q6_K at
     // 2048 rows 0.96); least where the card's power is the limit (Q4_K from 1500 rows on: 0.98 to 1.0).  Without branches and without kAhead
-    // one weight tile gains less and loses up to 9 % where the last column is short.
+    // one weight tile gains less and loses up to 9 % where the last column is short.  Q5_K's form of six tiles keeps the branches: without them
+    // eight registers spill, and products with K in runs took up to 1.05 of the time with the branches of the form of eight (11088 x 6400 at 187
+    // rows 61.0 -> 64.2 us); with its own it takes 0.987 of that time over 40 products and 0.961 over 24 pairs (61.4; pair 6832 x 1024 at 166 rows
+    // 21.7 -> 20.3).
     constexpr bool kAhead = kDense && kWTilesPerWave == 1;
     constexpr int kFirst = MT != kMTilesMid || Q5 ? 0 : Q6 ? 2 : 1;
     auto multiply = [&](auto all_c) {
@@ -372,7 +375,7 @@ __global__ void __launch_bounds__(256, PAIR && MT == kMTilesMid && WT != kWtQ5 ?
             }
         }
     };
-    if constexpr (kDense && kWTilesPerWave == 2) {
+    if constexpr (kDense && kWTilesPerWave == 2 && !(Q5 && MT == 6)) {
         if (mt_count == MT) multiply(std::true_type{});
         else multiply(std::false_type{});
     } else {
