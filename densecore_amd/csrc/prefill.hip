@@ -1203,7 +1203,7 @@ bool gemm_pair_shape(int wtype, int64_t rows, int64_t nb, int64_t n, bool then_q
     if (!gemm_type(wtype) || rows <= 0 || n <= 0) return false;
     *shape = choose_shape(kPace[pace_of(wtype)], true, rows, nb, n);
     const float out = 1e-6f * (float)(n * rows), one_launch = shape->us + 0.25f * out + 8.0f;
-    const float two_launches = 2.0f * gemm_shape(wtype, rows, nb, n).us + 8.5f + 3.15f * out + 8.0f;
+    const float two_launches = 2.0f * gemm_launch_shape(wtype, rows, nb, n).us + 8.5f + 3.15f * out + 8.0f;
     return two_launches >= (then_quantized ? one_launch + 4.0f + 0.82f * out : 0.94f * one_launch);
 }
 

@@ -73,3 +73,17 @@ def test_few_rows_of_a_long_k_take_two_launches(wtype, n):
     """Gate and up of 4096 x 14336: two launches with K in runs against the one that cannot split it, 44.0 | 62.3, 48.6 | 89.4,
     86.5 | 115.7, 67.8 | 104.7, 83.4 | 114.6 us."""
     assert shape(wtype, 4096, 14336, n, 1)["taken"] == 0
+
+
+@pytest.mark.parametrize("wtype,rows,cols,n", [(Q4, 513, 14336, 100), (Q5, 513, 14336, 100), (Q6, 513, 14336, 100), (Q5, 389, 10240, 79), (Q4, 283, 7936, 472),
+                                               (Q5, 287, 12032, 476), (Q4, 915, 12032, 306)])
+def test_few_ragged_rows_of_a_long_k_take_two_launches(wtype, rows, cols, n):
+    """Gate and up of rows that do not divide by four: their two launches have K in runs over the padded rows.  Two launches | one, us:
+    35.8 | 70.4, 38.1 | 99.1, 37.3 | 98.2, 29.9 | 63.0, 37.0 | 61.3, 44.7 | 111.2, 50.3 | 74.9."""
+    assert shape(wtype, rows, cols, n, 1)["taken"] == 0
+
+
+@pytest.mark.parametrize("wtype,rows,cols,n", [(Q4, 5633, 2048, 300), (Q4, 2047, 4096, 100), (Q5, 5605, 1536, 648), (Q6, 7587, 4096, 150), (Q4, 577, 3072, 67)])
+def test_ragged_pairs_of_a_short_k_stay_in_one_launch(wtype, rows, cols, n):
+    """One launch | two, us: 33.0 | 42.0, 27.5 | 29.9, 49.6 | 60.4, 47.5 | 59.5, 19.4 | 23.1."""
+    assert shape(wtype, rows, cols, n, 1)["taken"] == 1
