@@ -1371,8 +1371,8 @@ static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
     if (n >= 192) return n * top_k >= 6 * w->n_experts;
     return n >= kMoeGemmMinTokens && n * top_k >= 5 * w->n_experts && moe_gemm_estimate(w->n_experts, w->rowtiles, w->rows, w->nb, n, top_k);
 }
-// Whether a MoE block runs its expert products on the expert-grouped GEMM, by its shape alone, so that the layer and the two nodes it
-// is made of come to one choice (a product whose type the GEMM does not take stays where it is).  By the routed rows per expert rpe:
+// Whether a MoE block runs its expert products on the expert-grouped GEMM, by its shape alone (a product whose type the GEMM does not take
+// stays where it is).  By the routed rows per expert rpe:
 // from inter <= 12 rpe^3 on (2.8 rows at 256, 3.5 at 512, 4.4 at 1024), from six, and where the down product's estimate says so.  The line
 // goes through 15,305 blocks (8 to 256 experts, top-2 to 8, 1024 to 4096 x 256 to 1024, every mix of Q4_K, Q5_K and Q6_K, with and without
 // a shared expert, 9 to 400 tokens) timed both ways: the choice takes 1.008 of the faster one's time (1.088 with six rows, or five and the
@@ -1386,14 +1386,55 @@ static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
 // blocks gained too (0.50 to 0.96), but a gate/up node by itself took up to 1.4 of the time (8 experts, top-6, 3840 x 512 at 13 tokens, three
 // super-blocks to a wavefront, 23 -> 33 us).
 // 64 experts, top-6, 2048 x 512 at 64 tokens 65.8 -> 53.7 us, 16 experts, top-8, 2816 x 768 at 24 tokens 98.7 -> 42.4.
-static bool moe_block_takes_gemm(int64_t n_experts, int64_t hidden, int64_t inter, int64_t n, int top_k) {
-    const int64_t pairs = n * top_k;
-    if (n < kMoeGemmMinTokens && (n <= 8 || pairs < 6 * n_experts || hidden / kQK < 5 * pick_waves(hidden / kQK, (inter + 15) / 16 * n_experts))) return false;
-    if (pairs < 64 || n_experts > 4096 || (hidden & 3) || (inter & 3)) return false;
-    const float rpe = (float)pairs / (float)n_experts;
-    if (12.0f * rpe * rpe * rpe >= (float)inter) return true;
-    if (n >= 192) return pairs >= 6 * n_experts;
-    return pairs >= 5 * n_experts && moe_gemm_estimate(n_experts, (hidden + 15) / 16, hidden, inter / kQK, n, top_k);
+struct MoeShape {
+    int64_t n_experts, hidden, inter, n;
+    int top_k;
+    int64_t pairs() const { return n * top_k; }
+    float rows() const { return (float)pairs() / (float)n_experts; }  // per expert
+    bool over_line() const { return 12.0f * rows() * rows() * rows() >= (float)inter; }
+    int64_t gateup_stages() const { return hidden / kQK / pick_waves(hidden / kQK, (inter + 15) / 16 * n_experts); }  // of a wavefront of the decode launch
+    bool sizes() const { return n_experts <= 4096 && !(hidden & 3) && !(inter & 3); }
+    bool enough() const {
+        if (n < kMoeGemmMinTokens && (n <= 8 || pairs() < 6 * n_experts || gateup_stages() < 5)) return false;
+        return pairs() >= 64 && sizes();
+    }
+    bool down_estimate() const { return pairs() >= 5 * n_experts && moe_gemm_estimate(n_experts, (hidden + 15) / 16, hidden, inter / kQK, n, top_k); }
+};
+static bool moe_block_takes_gemm(const MoeShape& m) {
+    if (!m.enough()) return false;
+    if (m.over_line()) return true;
+    return m.n >= 192 ? m.pairs() >= 6 * m.n_experts : m.down_estimate();
+}
+// Time of gate and up of a block of fewer than 192 tokens on the GEMM, its plan included, over that on the decode launches, estimated:
+//   decode  14.6 + a (rpe / 8 + 0.36) stages of a wavefront x max(0.69, workgroups over those that run at once)
+//   GEMM    12.7 + b super-blocks x rounds + c per thousand (activation tile, row tile, super-block) + 0.028 MB as Q4_K
+// Least squares over 1,371 random nodes (8 to 256 experts, top-2 to 8, 1024 to 4096 x 256 to 1024, 9 to 191 tokens, 1.5 to 40 rows per
+// expert) timed both ways, 449 others beside them: residuals 9.6 and 6.4 % on both.  The GEMM walks a row's super-blocks one after the
+// other; few experts of a small inner size leave most units idle, where the decode launches give a row to several wavefronts.
+static float moe_gateup_ratio(int type, const MoeShape& m) {
+    constexpr float kDecode[3] = {2.13f, 2.60f, 3.26f}, kWalk[3] = {0.766f, 1.06f, 1.02f}, kTile[3] = {0.144e-3f, 0.24e-3f, 0.36e-3f};
+    const int t = type == kTypeQ6K ? 2 : type == kTypeQ5K ? 1 : 0;
+    const int64_t rowtiles = (m.inter + 15) / 16;
+    const float experts = (float)m.n_experts, rt = (float)rowtiles, nb = (float)(m.hidden / kQK), rpe = m.rows(), units = (float)compute_units();
+    const float waves = (float)pick_waves(m.hidden / kQK, rowtiles * m.n_experts), load = rt * experts * waves / (8.0f * units);
+    const float decode = 14.6f + kDecode[t] * (rpe * 0.125f + 0.36f) * (nb / waves) * (load > 0.69f ? load : 0.69f);
+    const float tiles = 16.0f * (float)moe_gemm_item_tiles(m.pairs(), m.n_experts), items = experts * (rpe > tiles ? rpe / tiles : 1.0f);
+    const float rounds = items * (float)((rowtiles + 3) / 4) / (2.0f * units);
+    const float gemm = 12.7f + kWalk[t] * nb * (rounds > 1.0f ? rounds : 1.0f) + kTile[t] * 2.0f * experts * (rpe * 0.0625f + 0.5f) * rt * nb +
+                       0.028f * 2.0f * experts * (float)m.inter * nb * 144e-6f;
+    return gemm / decode;
+}
+// The gate/up node by itself: the block's lines, and below 192 tokens the estimate for its own product, whatever follows it -- ahead of a down
+// stack that the GEMM does not take, Q8_0, nothing makes up for what it loses.  Over those 1,820 nodes the choice takes 0.910 of the decode
+// launches' time (0.920 by the block's rule), over 1.03 of it on 27 (194), at most 1.18 (1.55: Q5_K, 16 experts, top-4, 3072 x 256 at 18
+// tokens 17.9 -> 27.1 us).  From five rows on fewer than 64 pairs take it as well where the decode launch walks long rows (Q4_K, 8 experts,
+// top-2, 1280 x 768 at 27 tokens 0.65 of the time).
+static bool moe_gateup_takes_gemm(int type, const MoeShape& m) {
+    const bool enough = m.enough();
+    if (m.n >= 192) return enough && (m.over_line() || m.pairs() >= 6 * m.n_experts);
+    const bool asked = enough ? m.n < kMoeGemmMinTokens || m.over_line() || m.rows() >= 5.0f
+                              : m.n >= kMoeGemmMinTokens && m.sizes() && m.rows() >= 5.0f && m.gateup_stages() >= 5;
+    return asked && moe_gateup_ratio(type, m) < 0.97f;
 }
 
 // Room for expert-grouped calls of up to n tokens (reserve_ahead): for the decode launches, which take fewer than 192 tokens or six rows per
@@ -1876,7 +1917,7 @@ int mq_moe_gateup_swiglu_q4k(const mq_weight* gate_exps, const mq_weight* up_exp
     RouteWs r;
     if (int rc = carve_route(n, top_k, gate_exps->n_experts, r)) return rc;
     MQ_HIP(launch_fill_zero(hidden_dev, (size_t)n * top_k * (size_t)gate_exps->rows, s));
-    if (moe_gemm_takes(gate_exps) && moe_block_takes_gemm(gate_exps->n_experts, gate_exps->cols, gate_exps->rows, n, top_k)) {  // gate and up share their type
+    if (moe_gemm_takes(gate_exps) && moe_gateup_takes_gemm(gate_exps->type, {gate_exps->n_experts, gate_exps->cols, gate_exps->rows, n, top_k})) {  // gate and up share their type
         // prefill widths: both products on the expert-grouped GEMM, SwiGLU rows scattered to their (token, slot) places
         const int64_t entries = n * top_k, E = gate_exps->n_experts, inter = gate_exps->rows, hidden = gate_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
@@ -1927,7 +1968,7 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
         return rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, down_exps->n_experts, r)) return rc;
-    if (moe_gemm_takes(down_exps) && moe_block_takes_gemm(down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k)) {
+    if (moe_gemm_takes(down_exps) && moe_block_takes_gemm({down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k})) {
         // prefill widths: the product on the expert-grouped GEMM into the per-(token, slot) rows, then the combine
         const int64_t entries = n * top_k, E = down_exps->n_experts, hidden = down_exps->rows, inter = down_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
@@ -1985,7 +2026,7 @@ static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
     // (a Q8_0 down stack's launches follow either way: 42 us a block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them)
     if (n < 192 && !moe_gemm_takes(L->down_exps)) return false;
     return moe_gemm_takes(ge) && moe_gemm_takes(L->up_exps) &&  // the shared expert has the stacks' types
-           moe_block_takes_gemm(ge->n_experts, ge->cols, ge->rows, n, L->top_k);
+           moe_block_takes_gemm({ge->n_experts, ge->cols, ge->rows, n, L->top_k});
 }
 
 int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float* logits_dev, int64_t n, float* y_dev,
@@ -2387,6 +2428,23 @@ int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
     path_out[0] = dense_path_of(wtype, rows, nb, n, pair == 1, pair == 2);
     path_out[1] = dense_waves(nb, rowtiles);
     path_out[2] = skinny16_applies(nb, rowtiles, pair == 1, n, wtype) ? dense_lds_wpr(nb, rowtiles) : 0;
+    return MQ_OK;
+}
+
+int mq_debug_moe_path(int gate_type, int down_type, int64_t n_experts, int64_t hidden, int64_t inter, int64_t n, int top_k, int* path_out) {
+    auto known = [](int t) { return t == kTypeQ4K || t == kTypeQ5K || t == kTypeQ6K; };
+    if (!known(gate_type) || (!known(down_type) && down_type != kTypeQ80) || n_experts <= 0 || hidden <= 0 || hidden % kQK || inter <= 0 || inter % kQK ||
+        n <= 0 || top_k <= 0 || !path_out)
+        return fail(MQ_ERR_INVALID, "mq_debug_moe_path: bad type, size or pointer");
+    mq_weight gate, down;
+    gate.type = gate_type, gate.n_experts = n_experts, gate.rows = inter, gate.cols = hidden;
+    down.type = down_type, down.n_experts = n_experts, down.rows = hidden, down.cols = inter;
+    mq_moe_layer_desc layer = {};
+    layer.gate_exps = layer.up_exps = &gate, layer.down_exps = &down, layer.top_k = top_k;
+    const MoeShape m = {n_experts, hidden, inter, n, top_k};
+    path_out[0] = moe_gemm_applies(&layer, n);
+    path_out[1] = moe_gateup_takes_gemm(gate_type, m);
+    path_out[2] = known(down_type) && moe_block_takes_gemm(m);
     return MQ_OK;
 }
 

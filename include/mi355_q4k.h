@@ -228,8 +228,8 @@ int mq_moe_weights_from_logits(const float* logits_dev, int64_t n_experts, int64
  * and more with six rows per expert on average, and from 17 tokens with five rows
  * per expert where an estimate says that it is clearly faster: few experts) run on
  * the int8 matrix-core GEMM in its expert-grouped form, as do
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, which follow the
- * rule of mq_moe_layer_q4k. */
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, by the lines of
+ * mq_moe_layer_q4k. */
 int mq_mul_mat_id_q4k(const mq_weight* w_exps, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
                       int top_k, float* y_dev, void* stream);
 
@@ -265,8 +265,9 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches (from 192 tokens); same
  * routing, results within the fp32 tolerance of the other form (the
  * summation order differs), and above 64 tokens mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same rule, so the layer is the composition of its two nodes bit for
- * bit there (with a Q8_0 down stack from 192 tokens on). */
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same lines; the former only where its own product is estimated to gain
+ * below 192 tokens.  Where they run on the GEMM if the layer does -- always from 192 tokens on --, the layer is their composition bit for
+ * bit, elsewhere within that tolerance. */
 typedef struct {
     const mq_weight* gate_exps; /* n_experts x [inter][hidden]  */
     const mq_weight* up_exps;
