@@ -1371,8 +1371,7 @@ static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
     if (n >= 192) return n * top_k >= 6 * w->n_experts;
     return n >= kMoeGemmMinTokens && n * top_k >= 5 * w->n_experts && moe_gemm_estimate(w->n_experts, w->rowtiles, w->rows, w->nb, n, top_k);
 }
-// Whether a MoE block runs its expert products on the expert-grouped GEMM, by its shape alone (a product whose type the GEMM does not take
-// stays where it is).  By the routed rows per expert rpe:
+// Whether a MoE block runs its expert products on the expert-grouped GEMM (a product whose type the GEMM does not take stays where it is).  By the routed rows per expert rpe:
 // from inter <= 12 rpe^3 on (2.8 rows at 256, 3.5 at 512, 4.4 at 1024), from six, and where the down product's estimate says so.  The line
 // goes through 15,305 blocks (8 to 256 experts, top-2 to 8, 1024 to 4096 x 256 to 1024, every mix of Q4_K, Q5_K and Q6_K, with and without
 // a shared expert, 9 to 400 tokens) timed both ways: the choice takes 1.008 of the faster one's time (1.088 with six rows, or five and the
@@ -1400,11 +1399,6 @@ struct MoeShape {
     }
     bool down_estimate() const { return pairs() >= 5 * n_experts && moe_gemm_estimate(n_experts, (hidden + 15) / 16, hidden, inter / kQK, n, top_k); }
 };
-static bool moe_block_takes_gemm(const MoeShape& m) {
-    if (!m.enough()) return false;
-    if (m.over_line()) return true;
-    return m.n >= 192 ? m.pairs() >= 6 * m.n_experts : m.down_estimate();
-}
 // Time of gate and up of a block of fewer than 192 tokens on the GEMM, its plan included, over that on the decode launches, estimated:
 //   decode  14.6 + a (rpe / 8 + 0.36) stages of a wavefront x max(0.69, workgroups over those that run at once)
 //   GEMM    12.7 + b super-blocks x rounds + c per thousand (activation tile, row tile, super-block) + 0.028 MB as Q4_K
@@ -1423,6 +1417,26 @@ static float moe_gateup_ratio(int type, const MoeShape& m) {
     const float gemm = 12.7f + kWalk[t] * nb * (rounds > 1.0f ? rounds : 1.0f) + kTile[t] * 2.0f * experts * (rpe * 0.0625f + 0.5f) * rt * nb +
                        0.028f * 2.0f * experts * (float)m.inter * nb * 144e-6f;
     return gemm / decode;
+}
+// Below 192 tokens not every block over the line gains.  Few rows for a gate/up product that loses by itself, and down products that the decode
+// launch gives to several wavefronts a row (which hold off the GEMM by 5 to 18 % up to ten rows per expert and more), stay off it: over 1,820 blocks of that
+// width timed both ways, 916 of which the lines alone take, the GEMM costs over 3 % on 29 instead of 49, at most 1.14 times the time
+// instead of 1.19 (Q6_K, 32 experts, top-2, 3072 x 256 at 47 tokens 39.0 -> 46.3 us), at one block that loses 18 % by it.
+static bool moe_block_loses(int type, const MoeShape& m) {
+    const float ratio = moe_gateup_ratio(type, m);
+    return ratio > 1.0f && (pick_waves(m.inter / kQK, (m.hidden + 15) / 16 * m.n_experts) > 1 || ratio > 0.6f + 0.1f * m.rows() + (float)m.pairs() * (1.0f / 350.0f));
+}
+static bool moe_layer_takes_gemm(int type, const MoeShape& m) {
+    if (!m.enough()) return false;
+    if (m.n >= 192) return m.over_line() || m.pairs() >= 6 * m.n_experts;
+    return (m.over_line() && !moe_block_loses(type, m)) || m.down_estimate();
+}
+// The down node by itself: the line ends at inter <= 60 rpe^2 (4.1 rows at 1024) and leaves out products of several wavefronts a row: over 1.03 of
+// the time of six rows, or five and the estimate, on 31 of those 1,820 nodes instead of 100.
+static bool moe_down_takes_gemm(const MoeShape& m) {
+    if (!m.enough()) return false;
+    if (m.n >= 192) return m.over_line() || m.pairs() >= 6 * m.n_experts;
+    return (m.over_line() && 60.0f * m.rows() * m.rows() >= (float)m.inter && pick_waves(m.inter / kQK, (m.hidden + 15) / 16 * m.n_experts) == 1) || m.down_estimate();
 }
 // The gate/up node by itself: the block's lines, and below 192 tokens the estimate for its own product, whatever follows it -- ahead of a down
 // stack that the GEMM does not take, Q8_0, nothing makes up for what it loses.  Over those 1,820 nodes the choice takes 0.910 of the decode
@@ -1968,7 +1982,7 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
         return rc;
     RouteWs r;
     if (int rc = carve_route(n, top_k, down_exps->n_experts, r)) return rc;
-    if (moe_gemm_takes(down_exps) && moe_block_takes_gemm({down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k})) {
+    if (moe_gemm_takes(down_exps) && moe_down_takes_gemm({down_exps->n_experts, down_exps->rows, down_exps->cols, n, top_k})) {
         // prefill widths: the product on the expert-grouped GEMM into the per-(token, slot) rows, then the combine
         const int64_t entries = n * top_k, E = down_exps->n_experts, hidden = down_exps->rows, inter = down_exps->cols;
         MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, E) * sizeof(int32_t)));
@@ -2026,7 +2040,7 @@ static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
     // (a Q8_0 down stack's launches follow either way: 42 us a block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them)
     if (n < 192 && !moe_gemm_takes(L->down_exps)) return false;
     return moe_gemm_takes(ge) && moe_gemm_takes(L->up_exps) &&  // the shared expert has the stacks' types
-           moe_block_takes_gemm({ge->n_experts, ge->cols, ge->rows, n, L->top_k});
+           moe_layer_takes_gemm(ge->type, {ge->n_experts, ge->cols, ge->rows, n, L->top_k});
 }
 
 int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float* logits_dev, int64_t n, float* y_dev,
@@ -2444,7 +2458,7 @@ int mq_debug_moe_path(int gate_type, int down_type, int64_t n_experts, int64_t h
     const MoeShape m = {n_experts, hidden, inter, n, top_k};
     path_out[0] = moe_gemm_applies(&layer, n);
     path_out[1] = moe_gateup_takes_gemm(gate_type, m);
-    path_out[2] = known(down_type) && moe_block_takes_gemm(m);
+    path_out[2] = known(down_type) && moe_down_takes_gemm(m);
     return MQ_OK;
 }
 

@@ -265,9 +265,10 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches (from 192 tokens); same
  * routing, results within the fp32 tolerance of the other form (the
  * summation order differs), and above 64 tokens mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same lines; the former only where its own product is estimated to gain
- * below 192 tokens.  Where they run on the GEMM if the layer does -- always from 192 tokens on --, the layer is their composition bit for
- * bit, elsewhere within that tolerance. */
+ * Below 192 tokens blocks within these lines stay on the decode launches where an estimate says that they lose: few rows of few experts.
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same lines, below 192 tokens each by what its own product gains.  Where they
+ * run on the GEMM if the layer does -- always from 192 tokens on --, the layer is their composition bit for bit, elsewhere within that
+ * tolerance. */
 typedef struct {
     const mq_weight* gate_exps; /* n_experts x [inter][hidden]  */
     const mq_weight* up_exps;

@@ -46,3 +46,32 @@ def test_a_q80_down_stack_keeps_the_layer_on_the_decode_launches_below_192_token
         experts, n = rng.choice((8, 32, 256)), rng.randint(1, 400)
         p = moe_path(Q4, Q80, experts, 2048, 512, n, 8)
         assert p["down"] == 0 and p["layer"] == (moe_path(Q4, Q4, experts, 2048, 512, n, 8)["layer"] if n >= 192 else 0)
+
+
+# us of the layer on the decode launches | on the GEMM
+@pytest.mark.parametrize("block", [(Q6, 32, 2, 3072, 256, 47),   # 39.0 | 46.3
+                                   (Q6, 32, 2, 4096, 256, 52),   # 1.17 of the time
+                                   (Q6, 8, 2, 2048, 512, 47),    # 1.11
+                                   (Q5, 8, 2, 1280, 512, 35)])   # 29.8 | 33.5
+def test_a_layer_that_loses_on_the_gemm_stays_off_it(block):
+    t, experts, k, hidden, inter, n = block
+    assert moe_path(t, t, experts, hidden, inter, n, k)["layer"] == 0
+
+
+@pytest.mark.parametrize("block", [(Q6, 32, 2, 2048, 256, 77),   # 49.1 | 39.5
+                                   (Q4, 8, 4, 2048, 256, 26),    # 41.9 | 33.0
+                                   (Q4, 16, 8, 2816, 768, 24),   # 98.7 | 42.4
+                                   (Q4, 64, 6, 2048, 512, 64)])  # 65.8 | 53.7
+def test_a_layer_that_gains_takes_it(block):
+    t, experts, k, hidden, inter, n = block
+    assert moe_path(t, t, experts, hidden, inter, n, k)["layer"] == 1
+
+
+@pytest.mark.parametrize("block,gemm", [((8, 2, 2048, 1024, 33), 0),   # 1.09 of the decode launches' time
+                                        ((16, 2, 1024, 512, 32), 0),   # 1.05
+                                        ((8, 2, 1280, 512, 35), 0),    # 1.07
+                                        ((32, 2, 3072, 256, 47), 1),   # 0.93
+                                        ((8, 4, 2048, 256, 26), 1)])   # 0.66
+def test_the_down_node_goes_by_its_own_product(block, gemm):
+    experts, k, hidden, inter, n = block
+    assert moe_path(Q4, Q4, experts, hidden, inter, n, k)["down"] == gemm
