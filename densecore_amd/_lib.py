@@ -24,7 +24,7 @@ EXPORTS = [
 ]
 # every symbol include/mi355_q4k_debug.h declares (verification hooks and measurement instruments)
 DEBUG_EXPORTS = [
-    "mq_debug_block_sums", "mq_debug_moe_groups", "mq_debug_moe_hidden", "mq_debug_decoder_buffers",
+    "mq_debug_block_sums", "mq_debug_moe_groups", "mq_debug_moe_plan", "mq_debug_moe_hidden", "mq_debug_decoder_buffers",
     "mq_census_enable", "mq_census_reset", "mq_census_read", "mq_debug_set_dense_lds", "mq_debug_gemm_shape", "mq_debug_dense_path", "mq_debug_moe_path", "mq_debug_set_skeleton",
 ]
 
@@ -91,6 +91,7 @@ def load() -> C.CDLL:
     L.mq_moe_layer_q4k.argtypes = [C.POINTER(MoELayerDesc), vp, vp, i64, vp, vp, vp, vp]
     L.mq_debug_block_sums.argtypes = [vp, vp, i64, i64, vp, vp, vp, i64, vp]
     L.mq_debug_moe_groups.argtypes = [vp, vp, i64, i64, ci, vp, vp, vp]
+    L.mq_debug_moe_plan.argtypes = [vp, i64, i64, ci, ci, ci, vp, vp, vp, C.POINTER(i64), vp]
     L.mq_debug_moe_hidden.argtypes = [vp, sz, vp]
     L.mq_debug_decoder_buffers.argtypes = [vp] + [C.POINTER(vp)] * 5
     L.mq_silu_mul_f32.argtypes = [vp, vp, i64, i64, i64, i64, vp, i64, ci, vp]

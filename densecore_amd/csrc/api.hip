@@ -1579,6 +1579,27 @@ int mq_debug_moe_groups(const float* logits_dev, const int32_t* ids_dev, int64_t
     return MQ_OK;
 }
 
+int mq_debug_moe_plan(const int32_t* ids_dev, int64_t n_experts, int64_t n, int top_k, int shared, int item_tiles, int32_t* triples_dev,
+                      int32_t* count_dev, int32_t* plan_dev, int64_t* layout_out, void* stream) {
+    if (int rc = check_ready()) return rc;
+    if (n <= 0 || top_k <= 0 || top_k > 8 || n_experts <= 0 || n_experts > 4096 || (item_tiles != 2 && item_tiles != 4 && item_tiles != 8) || !layout_out)
+        return fail(MQ_ERR_INVALID, "mq_debug_moe_plan: need n > 0, 0 < top_k <= 8, 0 < n_experts <= 4096, items of 2, 4 or 8 tiles");
+    const int64_t entries = n * top_k + (shared ? n : 0), groups = n_experts + (shared ? 1 : 0);
+    layout_out[2] = (int64_t)moe_gemm_plan_ints(entries, groups);
+    layout_out[0] = 4 + 3 * moe_gemm_items_max(entries, groups), layout_out[1] = layout_out[0] + 16 * moe_gemm_tiles_max(entries, groups);
+    if (!plan_dev) return MQ_OK;
+    if (!ids_dev || !triples_dev || !count_dev) return fail(MQ_ERR_INVALID, "mq_debug_moe_plan: null pointer");
+    hipStream_t s = (hipStream_t)stream;
+    Entry entry(s);
+    if (entry.rc) return entry.rc;
+    RouteWs r;
+    if (int rc = carve_route(n, top_k, n_experts, r)) return rc;
+    MQ_HIP(launch_moe_group_plan(ids_dev, n, top_k, n_experts, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, top_k + (shared ? 1 : 0), false,
+                                 shared ? n : 0, MQ_SILU_FAST_FMA, plan_dev, s, item_tiles));
+    MQ_HIP(launch_flatten_groups(r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, (int)(n * top_k), triples_dev, count_dev, s));
+    return MQ_OK;
+}
+
 namespace {
 
 struct SharedExpert {

@@ -626,9 +626,8 @@ hipError_t launch_route_and_group(const float* logits, int64_t n_experts, int64_
     // one bit per (expert, token) for the grouping (see launch_build_groups)
     const int mask_words = n <= 4096 ? (int)((n + 31) / 32) : 0;
     const size_t lds_group = (size_t)n_experts * 4 + (size_t)n * top_k * 4 + (mask_words ? ((size_t)n_experts * (mask_words | 1) + 1) * 4 : 0);
-    // Prefill widths: route, then group over several workgroups, quantize on its own.  With nothing to quantize from 1536 pairs on: the
-    // one launch groups in its last workgroup, 14.1 us at 1600 pairs against 4.6 + 5.2 for the two (11.0 against 4.5 + 5.1 at 1040).
-    if (lds_group > 60 * 1024 || n * top_k >= (qx ? 3072 : 1536)) {
+    // Prefill widths: route, then group over several workgroups, quantize on its own.
+    if (lds_group > 60 * 1024 || n * top_k >= 3072) {
         hipError_t e = launch_route_topk(logits, n_experts, n, top_k, mode, ids, weights, stream);
         if (e != hipSuccess) return e;
         e = launch_build_groups(ids, n, top_k, n_experts, group_expert, group_begin, n_groups, entry_token, entry_k,

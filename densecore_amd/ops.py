@@ -216,6 +216,23 @@ def debug_moe_groups(n_experts: int, top_k: int, ids: torch.Tensor = None, logit
     return triples.cpu().numpy()[:int(count.item())]
 
 
+def debug_moe_plan(n_experts: int, top_k: int, ids: torch.Tensor, shared: bool, item_tiles: int):
+    """The expert-grouped GEMM's plan for ids int32 [n, top_k]: (work list as debug_moe_groups gives it, header of four, items [i, 3], source
+    token and output row of each of the tiles' rows)."""
+    n = ids.shape[0]
+    layout = (C.c_int64 * 3)()
+    _lib.check(_lib.lib().mq_debug_moe_plan(None, n_experts, n, top_k, int(shared), item_tiles, None, None, None, layout, _stream()), "mq_debug_moe_plan")
+    triples = torch.full((n * top_k, 3), -7, dtype=torch.int32, device=ids.device)
+    count = torch.zeros(1, dtype=torch.int32, device=ids.device)
+    plan = torch.full((layout[2],), -7, dtype=torch.int32, device=ids.device)
+    _lib.check(_lib.lib().mq_debug_moe_plan(_ptr(ids.contiguous()), n_experts, n, top_k, int(shared), item_tiles, _ptr(triples), _ptr(count), _ptr(plan),
+                                            layout, _stream()), "mq_debug_moe_plan")
+    plan = plan.cpu().numpy()
+    items, rows = int(plan[0]), 16 * int(plan[1])
+    return (triples.cpu().numpy()[:int(count.item())], plan[:4], plan[4:4 + 3 * items].reshape(items, 3), plan[layout[0]:layout[0] + rows],
+            plan[layout[1]:layout[1] + rows])
+
+
 def debug_moe_hidden(shape) -> torch.Tensor:
     """The fp32 intermediate of the last moe_layer / ffn_swiglu call (hidden rows [n, slots, inter] / [n, inter])."""
     out = torch.empty(shape, dtype=torch.float32, device="cuda")

@@ -27,10 +27,18 @@ int mq_debug_block_sums(const mq_weight* w, const float* x_dev, int64_t n, int64
  * entry: triples_dev int32 [n * top_k][3] = (expert, token, k) in list order, count_dev int32 [1] = entries (pairs
  * whose id is outside [0, n_experts) are dropped).  The reference's list is sorted by (expert, token, k)
  * (Qwen35BuildMoEAssignments, core/src/llm/moe/native.cpp:1664-1733).  Pass ids_dev int32 [n][top_k] to group given
- * ids (the grouping launch of mq_mul_mat_id_q4k and of the two expert nodes) or logits_dev fp32 [n][n_experts] to
+ * ids (the grouping launch of mq_mul_mat_id_q4k and of the two expert nodes on the decode launches) or logits_dev fp32 [n][n_experts] to
  * route and group in the one launch mq_moe_layer_q4k uses above eight tokens; the other pointer NULL. */
 int mq_debug_moe_groups(const float* logits_dev, const int32_t* ids_dev, int64_t n_experts, int64_t n, int top_k,
                         int32_t* triples_dev, int32_t* count_dev, void* stream);
+
+/* The plan of the expert-grouped GEMM as its launch (or, beyond 512 experts or 65,536 pairs, its two launches) lays it out for the given
+ * ids, with every token of a shared expert as one more group if asked for: plan_dev int32 [layout_out[2]], and the work list it leaves for
+ * a down stack that the GEMM does not take, as mq_debug_moe_groups writes it.  plan[0] items, [1] tiles of sixteen rows, [2] those of routed
+ * pairs, [4 + 3 i ..] expert (-1: the shared one), first tile and tiles of item i; from layout_out[0] on the token of each of the tiles' rows,
+ * from layout_out[1] on its output row token * slots + slot, -1 for padding.  plan_dev NULL: the layout alone. */
+int mq_debug_moe_plan(const int32_t* ids_dev, int64_t n_experts, int64_t n, int top_k, int shared, int item_tiles, int32_t* triples_dev,
+                      int32_t* count_dev, int32_t* plan_dev, int64_t* layout_out, void* stream);
 
 /* The fp32 intermediate the last mq_moe_layer_q4k / mq_ffn_swiglu_q4k call on this stream left in the library's
  * workspace, copied out: for the MoE layer the hidden rows silu(gate . x) * (up . x) as [n][top_k (+1 with a shared

@@ -65,3 +65,39 @@ def test_route_and_group_in_one_launch(ops, n, e, k):
     ids, _ = orc.route_topk(logits, k, 0)
     got = ops.debug_moe_groups(e, k, logits=cu(logits))
     assert np.array_equal(got, orc.build_assignments(ids, e))
+
+
+# one launch up to 512 experts and 65,536 pairs, two beyond; experts without rows, with one row, with tiles of 16 rows in full and one row more
+@pytest.mark.parametrize("n,e,k,shared", [(17, 8, 8, False), (9, 8, 8, True), (64, 64, 6, True), (193, 1, 1, False), (257, 256, 8, True), (512, 256, 8, False), (1500, 256, 8, True),
+                                          (1100, 512, 8, True), (1100, 513, 8, True), (300, 2000, 4, False), (8192, 16, 8, False), (8193, 16, 8, True)])
+@pytest.mark.parametrize("tiles", [2, 4, 8])
+@pytest.mark.parametrize("invalid", [False, True])
+def test_plan_of_the_expert_grouped_gemm(ops, n, e, k, shared, tiles, invalid):
+    """Items, rows and work list of launch_moe_group_plan against the sorted assignments: every expert's rows in (token, k) order from a tile
+    of its own on, in items of up to `tiles` tiles, padding marked, the shared expert's tokens behind them."""
+    rng = np.random.default_rng(n + e + tiles)
+    if invalid:
+        ids = rng.integers(0, e, size=(n, k)).astype(np.int32)  # repeats inside a token are likely
+        ids[0, 0], ids[n - 1, k - 1], ids[n // 2, k // 2] = -1, e, e + 1000
+        ids[1, :] = e // 3
+    else:
+        ids = np.argsort(rng.random((n, e)), axis=1)[:, :k].astype(np.int32)
+    want = orc.build_assignments(ids, e)
+    got, head, items, src, out = ops.debug_moe_plan(e, k, cu(ids), shared, tiles)
+    assert np.array_equal(got, want)
+    slots, want_items, want_src, want_out, tile = k + shared, [], [], [], 0
+    groups = [(x, want[want[:, 0] == x]) for x in np.unique(want[:, 0])]
+    if shared:
+        groups.append((-1, np.stack([np.full(n, -1), np.arange(n), np.full(n, k)], 1)))
+    for expert, rows in groups:
+        if expert >= 0:
+            routed = tile + (len(rows) + 15) // 16
+        count = (len(rows) + 15) // 16
+        want_items += [(expert, tile + t, min(tiles, count - t)) for t in range(0, count, tiles)]
+        pad = [-1] * (16 * count - len(rows))
+        want_src += list(rows[:, 1]) + pad
+        want_out += list(rows[:, 1] * slots + rows[:, 2]) + pad
+        tile += count
+    assert (head[0], head[1], head[2]) == (len(want_items), tile, routed)
+    assert np.array_equal(items[np.argsort(items[:, 1])], np.array(want_items))
+    assert np.array_equal(src, want_src) and np.array_equal(out, want_out)
