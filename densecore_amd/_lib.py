@@ -25,7 +25,7 @@ EXPORTS = [
 # every symbol include/mi355_q4k_debug.h declares (verification hooks and measurement instruments)
 DEBUG_EXPORTS = [
     "mq_debug_block_sums", "mq_debug_moe_groups", "mq_debug_moe_plan", "mq_debug_moe_hidden", "mq_debug_decoder_buffers",
-    "mq_census_enable", "mq_census_reset", "mq_census_read", "mq_debug_set_dense_lds", "mq_debug_gemm_shape", "mq_debug_dense_path", "mq_debug_moe_path", "mq_debug_set_skeleton",
+    "mq_census_enable", "mq_census_reset", "mq_census_read", "mq_debug_set_dense_lds", "mq_debug_gemm_shape", "mq_debug_gemm_launch", "mq_debug_dense_path", "mq_debug_moe_path", "mq_debug_set_skeleton",
 ]
 
 
@@ -114,6 +114,7 @@ def load() -> C.CDLL:
     L.mq_swiglu_mul_mat_q4k_acts.argtypes = [vp, vp, vp, vp, i64, ci, vp]
     L.mq_census_enable.argtypes = [ci]
     L.mq_debug_gemm_shape.argtypes = [ci, i64, i64, i64, ci, C.POINTER(ci)]
+    L.mq_debug_gemm_launch.argtypes = [ci, i64, i64, i64, C.POINTER(ci)]
     L.mq_debug_dense_path.argtypes = [ci, i64, i64, i64, ci, C.POINTER(ci)]
     L.mq_debug_moe_path.argtypes = [ci, ci, i64, i64, i64, i64, ci, C.POINTER(ci)]
     L.mq_debug_set_skeleton.argtypes = [ci]

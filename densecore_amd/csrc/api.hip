@@ -2449,6 +2449,23 @@ int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pa
     return MQ_OK;
 }
 
+int mq_debug_gemm_launch(int wtype, int64_t rows, int64_t cols, int64_t n, int* shape_out) {
+    const bool q80 = wtype == kTypeQ80;
+    if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K && !q80) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !shape_out)
+        return fail(MQ_ERR_INVALID, "mq_debug_gemm_launch: bad type, size or pointer");
+    const int64_t nb = cols / kQK;
+    if (q80) {
+        const int runs = q80_gemm_runs(rows, nb, n), tiles = q80_gemm_tiles(rows, n);
+        shape_out[0] = 1, shape_out[1] = runs, shape_out[2] = (int)((nb + runs - 1) / runs), shape_out[3] = tiles;
+        shape_out[4] = (int)((rows + 63) / 64), shape_out[5] = (int)(((n + 15) / 16 + tiles - 1) / tiles);
+        return MQ_OK;
+    }
+    const GemmShape s = gemm_launch_shape(wtype, rows, nb, n);
+    shape_out[0] = s.narrow, shape_out[1] = s.splits, shape_out[2] = s.sb_split, shape_out[3] = s.tiles_per_wg;
+    shape_out[4] = (int)s.row_wgs, shape_out[5] = (int)s.groups;
+    return MQ_OK;
+}
+
 int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out) {
     const bool q80 = wtype == kTypeQ80 && !pair;
     if ((wtype != kTypeQ4K && wtype != kTypeQ5K && wtype != kTypeQ6K && !q80) || rows <= 0 || cols <= 0 || cols % kQK || n <= 0 || !path_out)

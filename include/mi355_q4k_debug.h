@@ -86,6 +86,9 @@ int mq_debug_set_dense_lds(int on);
  * such a matrix is launched in the shape of the row count padded to four where that one's estimate is less. */
 int mq_debug_gemm_shape(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* shape_out);
 
+/* The first six of these for the launch that a GEMM product by itself makes, padded rows and Q8_0 weights included. */
+int mq_debug_gemm_launch(int wtype, int64_t rows, int64_t cols, int64_t n, int* shape_out);
+
 /* Kernels that a dense product of n rows (pair 1: gate and up in one call; 2: the down product of an FFN whose gate and up run on the
  * GEMM) runs on, for a 256-unit device before mq_init.  path_out:
  * 0 passes of eight or sixteen rows, 1 tiles of sixteen, 2 the matrix-core GEMM; wavefronts per row tile of the passes, and of the

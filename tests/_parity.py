@@ -35,6 +35,16 @@ def gemm_shape(wtype: int, rows: int, cols: int, n: int, pair: int = 0) -> dict:
     return dict(zip(("narrow", "runs", "sb_run", "tiles", "row_wgs", "columns", "taken", "ns"), out))
 
 
+def gemm_launch(wtype: int, rows: int, cols: int, n: int) -> dict:
+    """The shape in which a GEMM product is launched: rows padded to four where that is the shorter one, Q8_0 included."""
+    import ctypes as C
+
+    from densecore_amd import _lib
+    out = (C.c_int * 6)()
+    assert _lib.load().mq_debug_gemm_launch(wtype, rows, cols, n, out) == 0
+    return dict(zip(("narrow", "runs", "sb_run", "tiles", "row_wgs", "columns"), out))
+
+
 PASSES, SIXTEENS, GEMM = 0, 1, 2
 
 

@@ -1,7 +1,7 @@
 """Matrices whose rows do not divide by four: K in runs over the rows padded to four, whose sums leave the padding out."""
 import pytest
 
-from tests._parity import gemm_shape
+from tests._parity import gemm_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -18,13 +18,12 @@ def ops():
 @pytest.mark.parametrize("rows,cols,n", [(1, 4096, 65), (15, 4096, 70), (535, 12800, 108), (537, 8192, 66), (642, 8192, 130), (1023, 4096, 257),
                                          (2047, 5120, 391), (4097, 14336, 100), (4098, 14336, 67), (701, 2048, 100)])
 def test_ragged_rows(ops, wtype, rows, cols, n):
-    """Against the decode kernels (same integers, another order of the fp32 sums), and against the launch in one run over some of the rows of
-    the matrix that do divide; a padded output keeps its padding, the last row included."""
+    """Against the decode kernels: the same integers, another order of the fp32 sums; a padded output keeps its padding, the last row included."""
     import torch
     w = ops.Q4KWeight.synthetic(rows + n, rows, cols, 1, wtype)
     x = torch.randn((n, cols), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
-    ragged, padded = gemm_shape(wtype, rows, cols, n), gemm_shape(wtype, (rows + 3) // 4 * 4, cols, n)
-    assert ragged["runs"] == 1 and (padded["runs"] > 1 or cols <= 2048)
+    launch = gemm_launch(wtype, rows, cols, n)
+    assert launch["runs"] > 1 if cols > 2048 else launch["runs"] == (1 if wtype == 12 else 2)
     few = torch.cat([ops.mul_mat(w, x[i:i + 8].contiguous()) for i in range(0, n, 8)])
     wide = torch.full((n + 1, rows + 5), 7.0, device="cuda")
     for y, out in ((ops.gemm(w, x), None), (None, wide[:n, :rows])):

@@ -45,17 +45,20 @@ def test_a_row_does_not_depend_on_the_form(ops, wtype, rows, cols, n, form):
     w.free()
 
 
+# whole and short last columns of every form, and workgroups of fewer tiles than the form of five
 @pytest.mark.parametrize("wtype", [12, 13, 14])
-@pytest.mark.parametrize("n", [80, 96, 112, 128, 129, 177, 391])
-def test_pair_rows_do_not_depend_on_the_form(ops, wtype, n):
+@pytest.mark.parametrize("rows,cols,n,tiles", [(5648, 512, 80, 3), (5648, 512, 96, 3), (5648, 512, 112, 4), (5648, 512, 128, 4), (5648, 512, 129, 5), (5648, 512, 177, 6),
+                                               (5648, 512, 195, 7), (5648, 512, 255, 8), (5648, 512, 391, 5), (14336, 1024, 112, 7), (14336, 1024, 330, 8)])
+def test_pair_rows_do_not_depend_on_the_form(ops, wtype, rows, cols, n, tiles):
     """gate and up in one launch: the rows of a prefix of the tokens, bit for bit (a pair has no runs)."""
     import torch
-    rows, cols = 5648, 512
+    shape = gemm_shape(wtype, rows, cols, n, 1)
+    assert shape["taken"] and shape["tiles"] == tiles
     g, u = (ops.Q4KWeight.synthetic(s, rows, cols, 1, wtype) for s in (1, 2))
     x = torch.randn((n, cols), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
     h = ops.swiglu_mul_mat(g, u, x, ops.SILU_FAST)
     for count in (66, n - 1):
-        if gemm_shape(wtype, rows, cols, count, 1)["taken"] and gemm_shape(wtype, rows, cols, n, 1)["taken"]:
-            assert torch.equal(h[:count], ops.swiglu_mul_mat(g, u, x[:count].contiguous(), ops.SILU_FAST)), count
+        assert gemm_shape(wtype, rows, cols, count, 1)["taken"]
+        assert torch.equal(h[:count], ops.swiglu_mul_mat(g, u, x[:count].contiguous(), ops.SILU_FAST)), count
     for w in (g, u):
         w.free()

@@ -1,6 +1,8 @@
 """MoE blocks on either side of the line between the decode launches and the expert-grouped GEMM."""
 import pytest
 
+from tests._parity import moe_path
+
 pytestmark = pytest.mark.gpu
 
 
@@ -22,20 +24,21 @@ def near(got, want):
     assert bool(torch.isfinite(got).all())
 
 
-# (tokens, experts, top_k, hidden, inter): the fewest tokens with rows enough and one token less; the fewest pairs and fewer; rows per
+# (tokens, experts, top_k, hidden, inter, on the GEMM): the fewest tokens with rows enough and one token less; the fewest pairs and fewer; rows per
 # expert at the line (17 x 4 over 24 experts: 2.83 of 2.78 rows at inter 256) and below it; hidden rows in place and in tiles; few rows
-# per expert at prefill width; items of four tiles, whole and short; nine and sixteen tokens with five super-blocks of a row and more to a wavefront,
-# six rows per expert and fewer
-@pytest.mark.parametrize("n,experts,k,hidden,inter", [(17, 8, 8, 512, 256), (16, 8, 8, 512, 256), (32, 4, 2, 512, 256), (31, 4, 2, 512, 256),
-                                                      (17, 24, 4, 512, 256), (17, 25, 4, 512, 256), (64, 40, 4, 768, 512), (65, 40, 4, 768, 512),
-                                                      (200, 200, 4, 512, 512), (193, 256, 4, 512, 256),
-                                                      (200, 12, 4, 768, 512), (131, 9, 4, 512, 768), (333, 9, 2, 512, 256),
-                                                      (9, 8, 8, 2304, 512), (16, 10, 4, 1792, 512), (16, 11, 4, 1792, 512)])
+# per expert at prefill width; items of four tiles, whole and short; nine and sixteen tokens with three super-blocks of a row and with
+# seven to a wavefront, six rows per expert and fewer
+@pytest.mark.parametrize("n,experts,k,hidden,inter,gemm", [(17, 8, 8, 512, 256, 1), (16, 8, 8, 512, 256, 0), (32, 4, 2, 512, 256, 1), (31, 4, 2, 512, 256, 0),
+                                                           (17, 24, 4, 512, 256, 1), (17, 25, 4, 512, 256, 0), (64, 40, 4, 768, 512, 1), (65, 40, 4, 768, 512, 1),
+                                                           (200, 200, 4, 512, 512, 1), (193, 256, 4, 512, 256, 1),
+                                                           (200, 12, 4, 768, 512, 1), (131, 9, 4, 512, 768, 1), (333, 9, 2, 512, 256, 1),
+                                                           (9, 8, 8, 2304, 512, 0), (9, 8, 8, 1792, 768, 1), (16, 10, 4, 1792, 512, 1), (16, 11, 4, 1792, 512, 0)])
 @pytest.mark.parametrize("types", [("q4_k", "q4_k"), ("q6_k", "q5_k"), ("q5_k", "q6_k")])
-def test_layer_is_its_nodes_and_agrees_with_one_token_at_a_time(ops, n, experts, k, hidden, inter, types):
+def test_layer_is_its_nodes_and_agrees_with_one_token_at_a_time(ops, n, experts, k, hidden, inter, gemm, types):
     import torch
     T = {"q4_k": ops.GGML_TYPE_Q4_K, "q5_k": ops.GGML_TYPE_Q5_K, "q6_k": ops.GGML_TYPE_Q6_K}
     gu, dn = T[types[0]], T[types[1]]
+    assert set(moe_path(gu, dn, experts, hidden, inter, n, k).values()) == {gemm}
     G, U = (ops.Q4KWeight.synthetic(s, inter, hidden, experts, gu) for s in (1, 2))
     D = ops.Q4KWeight.synthetic(3, hidden, inter, experts, dn)
     sh = (ops.Q4KWeight.synthetic(4, inter, hidden, 1, gu), ops.Q4KWeight.synthetic(5, inter, hidden, 1, gu), ops.Q4KWeight.synthetic(6, hidden, inter, 1, dn))

@@ -2,22 +2,22 @@
 import pytest
 
 from densecore_amd import synth
-from tests._parity import GEMM, dense_path, gemm_shape
+from tests._parity import GEMM, dense_path, gemm_launch, gemm_shape
 
 pytestmark = pytest.mark.gpu
 Q80 = synth.GGML_TYPE_Q8_0
 
 
 # row counts that leave 0 .. 3 rows beside whole groups of four, an odd last run, up to sixteen runs; one and two tiles to a workgroup
-@pytest.mark.parametrize("rows,cols,n,tiles", [(64, 16384, 100, 1), (65, 16384, 40, 1), (527, 12544, 148, 1), (529, 8192, 33, 1), (1866, 10240, 27, 1), (1003, 2048, 40, 1),
-                                               (6315, 6912, 15, 1), (33001, 256, 10, 1), (65536, 512, 17, 2), (66000, 256, 31, 2)])
-def test_matches_eight_rows_at_a_time(rows, cols, n, tiles):
+@pytest.mark.parametrize("rows,cols,n,tiles,runs", [(64, 16384, 100, 1, 16), (65, 16384, 40, 1, 16), (527, 12544, 148, 1, 5), (529, 8192, 33, 1, 8), (1866, 10240, 27, 1, 8),
+                                                    (1003, 2048, 40, 1, 1), (6315, 6912, 15, 1, 5), (33001, 256, 10, 1, 1), (65536, 512, 17, 2, 1), (66000, 256, 31, 2, 1)])
+def test_matches_eight_rows_at_a_time(rows, cols, n, tiles, runs):
     """Block sums are integers in both; the scaled blocks are added up in fp32 in another order: 2 K / 32 roundings of 2^-24 of the largest result
     at most.  A captured launch gives the eager one's bits at each replay."""
     import torch
     from densecore_amd import _lib, ops
     path, _, mt = dense_path(Q80, rows, cols // 256, n)
-    assert (path, mt) == (GEMM, tiles)
+    assert (path, mt) == (GEMM, tiles) and gemm_launch(Q80, rows, cols, n)["runs"] == runs
     w = ops.Q4KWeight.synthetic(rows + n, rows, cols, 1, Q80)
     x = torch.randn(n, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
     want = torch.cat([ops.mul_mat(w, x[i:i + 8]) for i in range(0, n, 8)])
@@ -47,7 +47,8 @@ def test_planes_that_cannot_grow_under_capture_leave_k_whole(wtype, rows):
     _lib.check(_lib.lib().mq_shutdown(), "mq_shutdown")  # gives the workspaces back
     _lib.check(_lib.lib().mq_init(torch.cuda.current_device()), "mq_init")
     cols, n, padded = 16384, 100, (rows + 3) // 4 * 4
-    assert wtype == Q80 or (gemm_shape(wtype, padded, cols, 4096)["runs"] == 1 and gemm_shape(wtype, padded, cols, n)["runs"] > 1)
+    assert wtype == Q80 or gemm_shape(wtype, padded, cols, 4096)["runs"] == 1
+    assert gemm_launch(wtype, rows, cols, n)["runs"] > 1
     w, other = (ops.Q4KWeight.synthetic(rows, r, cols, 1, wtype) for r in (rows, 4))
     x = torch.randn(4096, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
     ops.mul_mat(other, x)
