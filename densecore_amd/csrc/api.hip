@@ -1365,7 +1365,8 @@ static bool moe_gemm_estimate(int64_t n_experts, int64_t rowtiles, int64_t rows,
                        0.507f * nb * (wgs > 1.0f ? wgs : 1.0f);
     return gemm < 0.90f * decode;
 }
-// A product by itself (mul_mat_id): from 192 tokens with six routed rows per expert, and from 17 with five where the estimate says so.
+// A product by itself (mul_mat_id): from 192 tokens with six routed rows per expert, and from 17 with five where the estimate says so.  The
+// blocks' line would suit it too: with three to four / four to five rows the GEMM takes 0.82 / 0.77 of the time (820 products), on 5 % over 1.03.
 static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
     if (!moe_gemm_takes(w) || w->n_experts > 4096 || (w->rows & 3) || (w->cols & 3)) return false;
     if (n >= 192) return n * top_k >= 6 * w->n_experts;

@@ -50,8 +50,9 @@ constexpr int kMTilesMid = 4;                  // ... or three or four dozen
 
 // request_a_tiles (pmajor.h) with an address per lane and request, unrolled: the same copies.  Scalar addresses take 1 to 4 % off the
 // wide forms and the pairs (Q6_K 14336 x 4096 at 512 rows 83.4 -> 80.5 us, Q4_K FFN 4096 -> 14336 at 2048 rows 765 -> 759), but
-// the loop around a request costs the forms that have registers to spare: Q5_K 6152 x 4096 at 1000 rows 84.0 with this | 85.6 with
-// scalar addresses, 64-row workgroups of Q4_K and Q6_K 19.3 | 19.8 (Q6_K 4096 x 4096 at 100 rows).  Unrolled scalar requests: 85.4, 20.3.
+// the loop around a request costs the forms that have registers to spare: 64-row workgroups of Q4_K and Q6_K 19.3 with this | 19.8 with scalar
+// addresses (Q6_K 4096 x 4096 at 100 rows; unrolled scalar requests 20.3).  Q5_K's wide forms had gained as much (6152 x 4096 at 1000 rows 84.0 |
+// 85.6), but with loops of their own for five to eight tiles this spills 6, 18, 38 and 61 registers: they take scalar addresses (81.2).
 template <int MT>
 __device__ __forceinline__ void request_a_tiles_by_lane(const uint8_t* __restrict__ src, uint8_t* buf, int copy_words, int wave, int lane) {
     const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)buf;
@@ -258,7 +259,7 @@ __global__ void __launch_bounds__(256, PAIR && MT == kMTilesMid && WT != kWtQ5 ?
                     if (b + 1 < b_end) request_w(b + 1, t);  // the raw tile's registers are free again
                     // The first kFirst of a tile's four operands are read a tile ahead: as many as leave three wavefronts to a SIMD (none of Q5_K's).
                     // With the same in prefill_gemm_resident_kernel, 84 blocks of 31 to 158 rows per expert take 0.982 of the time (16 experts,
-                    // top-4, 2816 x 768, Q6_K down at 180 tokens 60.5 -> 56.2 us; 256 + 1, top-8, 2048 x 512 at 1500 tokens 224 -> 221).
+                    // top-4, 2816 x 768, Q6_K down at 180 tokens 60.5 -> 56.2 us; 256 + 1, top-8, 2048 x 512 at 1500 tokens: gate/up 116 -> 112, down 63.6 -> 63.4).
                     v4i first[2][kFirst + 1];
                     auto read_first = [&](v4i (&f)[kFirst + 1], const uint8_t* at) {
 #pragma unroll
@@ -897,8 +898,8 @@ __global__ void __launch_bounds__(1024) moe_gemm_plan_kernel(const int32_t* __re
 // expert, and places its own pairs in the order of the ids, so a repeated (token, expert) needs no case of its own.  The lists, the
 // plan and the quantizing workgroups are those of build_groups_kernel and moe_gemm_plan_kernel, which took two launches and
 // sixteen workgroups that placed every expert's pairs by bit masks over the tokens.
-// Latency: one read of the ids, LDS counters, two barriers, the scattered stores.  256 + 1 experts, top-8, 2048 x 512: the block at 256 / 1500
-// tokens 135.1 / 228.0 -> 132.6 / 223.6 us (12.2 + 7.5 us by trace in two launches); 64 experts, top-6, at 192 / 256 tokens 66.0 / 64.5 ->
+// Latency: one read of the ids, LDS counters, two barriers, the scattered stores.  256 + 1 experts, top-8, 2048 x 512: at 1500 tokens 10.5 + 6.8
+// -> 12.2 us by trace, the block at 256 135.1 -> 132.6; 64 experts, top-6, at 192 / 256 tokens 66.0 / 64.5 ->
 // 59.7 / 59.5, 16 experts, top-2, 1024 x 256 at 400 / 700 tokens 52.7 / 59.5 -> 43.8 / 44.9.
 __global__ void __launch_bounds__(1024) moe_group_plan_kernel(const int32_t* __restrict__ ids, int n_pairs, int top_k, uint32_t top_k_inverse, int n_experts,
                                                               int32_t* __restrict__ group_expert, int32_t* __restrict__ group_begin,
