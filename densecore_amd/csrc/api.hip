@@ -1419,37 +1419,26 @@ static float moe_gateup_ratio(int type, const MoeShape& m) {
                        0.028f * 2.0f * experts * (float)m.inter * nb * 144e-6f;
     return gemm / decode;
 }
-// Below 192 tokens not every block over the line gains.  Few rows for a gate/up product that loses by itself, and down products that the decode
-// launch gives to several wavefronts a row (which hold off the GEMM by 5 to 18 % up to ten rows per expert and more), stay off it: over 1,820 blocks of that
-// width timed both ways, 916 of which the lines alone take, the GEMM costs over 3 % on 29 instead of 49, at most 1.14 times the time
-// instead of 1.19 (Q6_K, 32 experts, top-2, 3072 x 256 at 47 tokens 39.0 -> 46.3 us), at one block that loses 18 % by it.
-static bool moe_block_loses(int type, const MoeShape& m) {
-    const float ratio = moe_gateup_ratio(type, m);
-    return ratio > 1.0f && (pick_waves(m.inter / kQK, (m.hidden + 15) / 16 * m.n_experts) > 1 || ratio > 0.6f + 0.1f * m.rows() + (float)m.pairs() * (1.0f / 350.0f));
+// Which of a block's products take the GEMM.  Down: within the lines, except where the decode launch gives a row to several wavefronts -- below
+// 192 tokens and 13 rows per expert it is 5 to 18 % ahead there.  Gate and up: where the down product does, unless the estimate says that
+// they lose 12 %; else where they clearly gain, with fewer than 64 pairs too if they walk long rows.  The layer and its two nodes ask the same
+// (nothing tells a node what is beside it), so the layer is their composition bit for bit.  The line at 12 %: a layer of one product
+// each way groups twice, 3.1 us more than the GEMM for both (143 such layers beside each other: 1.05 of its time where the estimate is 1.05 to 1.12, 0.96
+// above, 0.86 above 1.3).  1,820 blocks of 9 to 191 tokens, each product timed both ways, share of the time when the lines were six rows, or five and the
+// estimate, and how many take over 1.03 and 1.08 of it: gate/up node 0.979, 105, 56, at most 1.31 (by the lines alone 0.987, 194, 129, at most 1.55: Q5_K, 16
+// experts, top-4, 3072 x 256 at 18 tokens 17.9 -> 27.1 us), down node 0.896, 62, 29, at most 1.25 (0.898, 100, 59).
+static bool moe_within_lines(const MoeShape& m) {
+    return m.enough() && (m.over_line() || (m.n >= 192 ? m.pairs() >= 6 * m.n_experts : m.down_estimate()));
 }
-static bool moe_layer_takes_gemm(int type, const MoeShape& m) {
-    if (!m.enough()) return false;
-    if (m.n >= 192) return m.over_line() || m.pairs() >= 6 * m.n_experts;
-    return (m.over_line() && !moe_block_loses(type, m)) || m.down_estimate();
-}
-// The down node by itself: the line ends at inter <= 60 rpe^2 (4.1 rows at 1024) and leaves out products of several wavefronts a row: over 1.03 of
-// the time of six rows, or five and the estimate, on 31 of those 1,820 nodes instead of 100.
 static bool moe_down_takes_gemm(const MoeShape& m) {
-    if (!m.enough()) return false;
-    if (m.n >= 192) return m.over_line() || m.pairs() >= 6 * m.n_experts;
-    return (m.over_line() && 60.0f * m.rows() * m.rows() >= (float)m.inter && pick_waves(m.inter / kQK, (m.hidden + 15) / 16 * m.n_experts) == 1) || m.down_estimate();
+    if (!moe_within_lines(m)) return false;
+    return m.n >= 192 || m.rows() >= 13.0f || pick_waves(m.inter / kQK, (m.hidden + 15) / 16 * m.n_experts) == 1 || m.down_estimate();
 }
-// The gate/up node by itself: the block's lines, and below 192 tokens the estimate for its own product, whatever follows it -- ahead of a down
-// stack that the GEMM does not take, Q8_0, nothing makes up for what it loses.  Over those 1,820 nodes the choice takes 0.910 of the decode
-// launches' time (0.920 by the block's rule), over 1.03 of it on 27 (194), at most 1.18 (1.55: Q5_K, 16 experts, top-4, 3072 x 256 at 18
-// tokens 17.9 -> 27.1 us).  From five rows on fewer than 64 pairs take it as well where the decode launch walks long rows (Q4_K, 8 experts,
-// top-2, 1280 x 768 at 27 tokens 0.65 of the time).
 static bool moe_gateup_takes_gemm(int type, const MoeShape& m) {
-    const bool enough = m.enough();
-    if (m.n >= 192) return enough && (m.over_line() || m.pairs() >= 6 * m.n_experts);
-    const bool asked = enough ? m.n < kMoeGemmMinTokens || m.over_line() || m.rows() >= 5.0f
-                              : m.n >= kMoeGemmMinTokens && m.sizes() && m.rows() >= 5.0f && m.gateup_stages() >= 5;
-    return asked && moe_gateup_ratio(type, m) < 0.97f;
+    const bool within = moe_within_lines(m);
+    if (m.n >= 192) return within;
+    if (within) return moe_gateup_ratio(type, m) < (moe_down_takes_gemm(m) ? 1.12f : 0.90f);
+    return m.n >= kMoeGemmMinTokens && m.pairs() < 64 && m.sizes() && m.rows() >= 5.0f && m.gateup_stages() >= 5 && moe_gateup_ratio(type, m) < 0.85f;
 }
 
 // Room for expert-grouped calls of up to n tokens (reserve_ahead): for the decode launches, which take fewer than 192 tokens or six rows per
@@ -2054,15 +2043,19 @@ int decoder_grid(size_t lds_bytes, int* n_workgroups, long long* spin_ticks) {
 // mq_debug_moe_hidden finds them; more stay in its tiles, which its quantizer reads in order.
 constexpr int64_t kMoeRowsInPlaceTokens = 64;
 
-// Decided per product: gate / up (one type) and down each run on the expert-grouped GEMM when their type is one it takes; a layer with
+// Gate / up (one type, which the shared expert has too) and down each run on the expert-grouped GEMM by their own rule; a layer with
 // a Q8_0 down stack (core/src/llm/moe/native.cpp:4611-4620; its activations are Q8_0 as well) keeps its two large
-// products on the matrix cores from 192 tokens on and sends the fp32 hidden rows through the Q8_0 launches.
-static bool moe_gemm_applies(const mq_moe_layer_desc* L, int64_t n) {
+// products on the matrix cores from 192 tokens on and sends the fp32 hidden rows through the Q8_0 launches, which follow either way: 42 us a
+// block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them.
+struct MoeChoice {
+    bool gateup, down;
+};
+static MoeChoice moe_layer_choice(const mq_moe_layer_desc* L, int64_t n) {
     const mq_weight* ge = L->gate_exps;
-    // (a Q8_0 down stack's launches follow either way: 42 us a block at 17 to 48 tokens, up to a quarter more with the GEMM ahead of them)
-    if (n < 192 && !moe_gemm_takes(L->down_exps)) return false;
-    return moe_gemm_takes(ge) && moe_gemm_takes(L->up_exps) &&  // the shared expert has the stacks' types
-           moe_layer_takes_gemm(ge->type, {ge->n_experts, ge->cols, ge->rows, n, L->top_k});
+    const MoeShape m = {ge->n_experts, ge->cols, ge->rows, n, L->top_k};
+    const bool k_quant_down = moe_gemm_takes(L->down_exps);
+    return {moe_gemm_takes(ge) && moe_gemm_takes(L->up_exps) && (k_quant_down || n >= 192) && moe_gateup_takes_gemm(ge->type, m),
+            k_quant_down && moe_down_takes_gemm(m)};
 }
 
 int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float* logits_dev, int64_t n, float* y_dev,
@@ -2129,7 +2122,8 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
     }
     // one arrival counter, kept apart from the quantization counters (last slot of that buffer)
     if (int rc = reserve_counters(4096)) return rc;
-    if (moe_gemm_applies(L, n)) {
+    const MoeChoice gemm = moe_layer_choice(L, n);
+    if (gemm.gateup) {
         // Prefill widths: the three expert products on the matrix-core GEMM in its expert-grouped form, the shared
         // expert as a dense FFN on it; per-(token, slot) rows and the combine as at the other widths.
         // The shared expert rides along as one more group of all tokens (its own weights, its own SiLU form, output slot K).
@@ -2152,7 +2146,7 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         const uint8_t* shd = sh.gate ? sh.down->data : nullptr;
         if (g_gemm_pair && L->gate_exps->type == L->up_exps->type) {
             // gate and up in ONE launch whose epilogue stores silu(gate) * up (the shared expert's rows with its own SiLU form)
-            if (!moe_gemm_takes(L->down_exps)) {  // fp32 rows at their (token, slot) places for the down stack's own kernel
+            if (!gemm.down) {  // fp32 rows at their (token, slot) places for the down stack's own kernel
                 MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
                 MQ_HIP(launch_prefill_gemm_grouped_pair(L->gate_exps->data, L->up_exps->data, L->gate_exps->type, L->gate_exps->expert_bytes, shg, shu, inter,
                                                         L->gate_exps->nb, (const uint8_t*)g.ap.ptr, n, entries, G, plan, true, L->silu_mode,
@@ -2183,8 +2177,8 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
         MQ_HIP(launch_prefill_gemm_grouped(L->up_exps->data, L->up_exps->type, L->up_exps->expert_bytes, shu, inter, L->up_exps->nb,
                                            (const uint8_t*)g.ap.ptr, n, entries, G, plan, false, ubuf, inter, s, mt));
         MQ_HIP(g.ap2.reserve(pmajor_bytes(rows_max, inter / kQK)));
-        if (!moe_gemm_takes(L->down_exps)) {
-            // a down stack of a type the GEMM does not take: the SwiGLU rows leave the quantizer as fp32 at their
+        if (!gemm.down) {
+            // a down stack that does not take the GEMM: the SwiGLU rows leave the quantizer as fp32 at their
             // (token, slot) places as well, and the expert-grouped decode launches take them from there (their own
             // quantizer -- Q8_K, or Q8_0 for Q8_0 experts -- and the same combine)
             MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
@@ -2208,11 +2202,26 @@ int mq_moe_layer_q4k(const mq_moe_layer_desc* L, const float* x_dev, const float
     // few tokens: nearly every (token, slot) pair has an expert of its own, so the pairs are the groups
     if (n <= kDirectPairsMaxTokens) r.direct_ids = ids;
     MQ_HIP(g.mid.reserve(hidden_rows * sizeof(float)));
-    // the hidden rows leave gate/up in Q8_K, unless the token-major down launch quantizes what it reads itself
-    const bool quantize_in_gateup = !token_major_down(L->down_exps, n, slots) && L->down_exps->type != kTypeQ80;
+    // the hidden rows leave gate/up in Q8_K, unless the token-major down launch quantizes what it reads itself or the GEMM takes them in tiles
+    const bool quantize_in_gateup = !token_major_down(L->down_exps, n, slots) && L->down_exps->type != kTypeQ80 && !gemm.down;
     if (int rc = run_moe_gateup(L->gate_exps, L->up_exps, sh, n, K, slots, L->silu_mode, r, (float*)g.mid.ptr, quantize_in_gateup, s))
         return rc;
     g.hidden_rows = hidden_rows;
+    if (gemm.down) {  // (more than eight tokens)
+        const int64_t entries = n * K + (sh.gate ? n : 0), G = E + (sh.gate ? 1 : 0);
+        MQ_HIP(g.plan.reserve(moe_gemm_plan_ints(entries, G) * sizeof(int32_t)));
+        const int mt = g_moe_item_tiles ? g_moe_item_tiles : moe_gemm_item_tiles(entries, G);  // tiles per item: the plan and every launch reading it
+        const int32_t* plan = (const int32_t*)g.plan.ptr;
+        MQ_HIP(g.ap2.reserve(pmajor_bytes(moe_gemm_tiles_max(entries, G) * 16, inter / kQK)));
+        MQ_HIP(g.part.reserve((size_t)n * slots * (size_t)hidden * sizeof(float)));
+        MQ_HIP(launch_moe_group_plan(ids, n, K, E, r.group_expert, r.group_begin, r.n_groups, r.entry_token, r.entry_k, slots, true, sh.gate ? n : 0,
+                                     MQ_SILU_FAST_FMA, (int32_t*)g.plan.ptr, s, mt));
+        MQ_HIP(launch_quantize_q8k_pmajor_grouped((const float*)g.mid.ptr, nullptr, false, 0, inter, inter, entries, G, plan, (uint8_t*)g.ap2.ptr, nullptr, 0, s, true));
+        MQ_HIP(launch_prefill_gemm_grouped(L->down_exps->data, L->down_exps->type, L->down_exps->expert_bytes, sh.gate ? sh.down->data : nullptr, hidden,
+                                           L->down_exps->nb, (const uint8_t*)g.ap2.ptr, 0, entries, G, plan, true, (float*)g.part.ptr, hidden, s, mt));
+        MQ_HIP(launch_moe_combine((const float*)g.part.ptr, n, K, slots, hidden, wts, ids, E, sh.gate ? 1 : 0, L->sh_gate_inp_dev, x_dev, y_dev, s));
+        return MQ_OK;
+    }
     return run_moe_down(L->down_exps, sh, (const float*)g.mid.ptr, quantize_in_gateup, n, K, slots, r, ids, wts, L->sh_gate_inp_dev,
                         x_dev, y_dev, s);
 }
@@ -2495,9 +2504,10 @@ int mq_debug_moe_path(int gate_type, int down_type, int64_t n_experts, int64_t h
     mq_moe_layer_desc layer = {};
     layer.gate_exps = layer.up_exps = &gate, layer.down_exps = &down, layer.top_k = top_k;
     const MoeShape m = {n_experts, hidden, inter, n, top_k};
-    path_out[0] = moe_gemm_applies(&layer, n);
-    path_out[1] = moe_gateup_takes_gemm(gate_type, m);
-    path_out[2] = known(down_type) && moe_down_takes_gemm(m);
+    const MoeChoice c = moe_layer_choice(&layer, n);
+    path_out[0] = c.gateup, path_out[1] = c.down;
+    path_out[2] = moe_gateup_takes_gemm(gate_type, m);
+    path_out[3] = known(down_type) && moe_down_takes_gemm(m);
     return MQ_OK;
 }
 

@@ -228,7 +228,7 @@ int mq_moe_weights_from_logits(const float* logits_dev, int64_t n_experts, int64
  * and more with six rows per expert on average, and from 17 tokens with five rows
  * per expert where an estimate says that it is clearly faster: few experts) run on
  * the int8 matrix-core GEMM in its expert-grouped form, as do
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, by the lines of
+ * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k below, by the rules of
  * mq_moe_layer_q4k. */
 int mq_mul_mat_id_q4k(const mq_weight* w_exps, const float* x_dev, int64_t n, int x_slots, const int32_t* ids_dev,
                       int top_k, float* y_dev, void* stream);
@@ -264,11 +264,11 @@ int mq_moe_down_weighted_q4k(const mq_weight* down_exps, const float* hidden_dev
  * int8 matrix-core GEMM in an expert-grouped form (entries in 16-row tiles per expert), the shared expert as one more
  * group of all tokens; a Q8_0 down stack takes the fp32 hidden rows of that gate/up through its own launches (from 192 tokens); same
  * routing, results within the fp32 tolerance of the other form (the
- * summation order differs), and above 64 tokens mq_debug_moe_hidden has no rows to copy unless the down stack takes them as fp32.
- * Below 192 tokens blocks within these lines stay on the decode launches where an estimate says that they lose: few rows of few experts.
- * mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same lines, below 192 tokens each by what its own product gains.  Where they
- * run on the GEMM if the layer does -- always from 192 tokens on --, the layer is their composition bit for bit, elsewhere within that
- * tolerance. */
+ * summation order differs).  Below 192 tokens each product takes it by itself within these lines: down unless the decode launch gives its rows to
+ * several wavefronts (and r < 13), gate and up unless an estimate says that they lose 12 % -- and with fewer than 64 pairs of long rows where
+ * they clearly gain (r >= 5).  mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k go by the same rules, so the layer is the composition of
+ * its two nodes bit for bit (with a Q8_0 down stack from 192 tokens on).  Above 64 tokens mq_debug_moe_hidden has no rows to copy where both
+ * products run on the GEMM. */
 typedef struct {
     const mq_weight* gate_exps; /* n_experts x [inter][hidden]  */
     const mq_weight* up_exps;

@@ -97,7 +97,7 @@ int mq_debug_gemm_launch(int wtype, int64_t rows, int64_t cols, int64_t n, int* 
 int mq_debug_dense_path(int wtype, int64_t rows, int64_t cols, int64_t n, int pair, int* path_out);
 
 /* Whether the expert products of a MoE block run on the expert-grouped GEMM (1) or on the decode launches (0), for a 256-unit device before
- * mq_init.  path_out: mq_moe_layer_q4k, mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k on such stacks. */
+ * mq_init.  path_out: gate/up and down of mq_moe_layer_q4k, then mq_moe_gateup_swiglu_q4k and mq_moe_down_weighted_q4k on such stacks. */
 int mq_debug_moe_path(int gate_type, int down_type, int64_t n_experts, int64_t hidden, int64_t inter, int64_t n, int top_k, int* path_out);
 
 /* Measurement instrument: while on != 0 every compute and routing launch of the library is replaced by a kernel with

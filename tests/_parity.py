@@ -59,13 +59,13 @@ def dense_path(wtype: int, rows: int, nb: int, n: int, pair: int = 0) -> tuple:
 
 
 def moe_path(gate_type: int, down_type: int, experts: int, hidden: int, inter: int, n: int, top_k: int) -> dict:
-    """Whether the layer and its two nodes run on the expert-grouped GEMM (include/mi355_q4k_debug.h)."""
+    """Whether gate/up and down of the layer, and the two nodes, run on the expert-grouped GEMM (include/mi355_q4k_debug.h)."""
     import ctypes as C
 
     from densecore_amd import _lib
-    out = (C.c_int * 3)()
+    out = (C.c_int * 4)()
     assert _lib.load().mq_debug_moe_path(gate_type, down_type, experts, hidden, inter, n, top_k, out) == 0
-    return dict(zip(("layer", "gateup", "down"), out))
+    return dict(zip(("layer gateup", "layer down", "gateup", "down"), out))
 
 
 def oracle_all_orders(w: np.ndarray, cols: int, q8: np.ndarray):

@@ -60,7 +60,7 @@ def test_layer_with_its_rows_in_place(ops, experts, k, hidden, inter, shared, ea
 # do not decide alone); a Q8_0 down stack; few experts of long rows, where nine tokens take the GEMM already
 BLOCKS = [(64, 6, 512, 512, 12, True, 256, (1, 5, 9, 20, 30, 100)), (16, 8, 512, 256, 14, False, 64, (2, 8, 12, 16, 17, 40)),
           (8, 2, 512, 1024, 13, False, 96, (1, 9, 20, 31, 32, 64)), (32, 4, 512, 512, 8, True, 300, (3, 9, 24, 60, 200)),
-          (8, 8, 2304, 256, 12, False, 40, (1, 8, 9, 16, 24))]
+          (8, 8, 2304, 256, 12, False, 40, (1, 8, 9, 16, 24)), (16, 4, 3072, 256, 12, True, 400, (5, 18, 24, 100)), (8, 2, 1280, 768, 13, False, 200, (9, 25, 27, 31, 64))]
 
 
 @pytest.mark.parametrize("experts,k,hidden,inter,down,shared,eager,widths", BLOCKS)

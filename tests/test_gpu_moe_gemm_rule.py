@@ -59,3 +59,32 @@ def test_layer_is_its_nodes_and_agrees_with_one_token_at_a_time(ops, n, experts,
         near(full[pick], one)
     for m in (G, U, D, *sh):
         m.free()
+
+
+# one product each way: few experts whose gate/up product would lose on the GEMM, few pairs of long rows, a down product of several wavefronts
+# a row; (gate/up, down) on the GEMM
+@pytest.mark.parametrize("n,experts,k,hidden,inter,gemm", [(18, 16, 4, 3072, 256, (0, 1)), (50, 32, 2, 3072, 256, (0, 1)), (17, 8, 6, 4096, 512, (0, 1)), (27, 8, 2, 1280, 768, (1, 0)),
+                                                           (25, 8, 2, 1280, 1024, (1, 0))])
+@pytest.mark.parametrize("gu,dn", [(12, 12), (12, 14), (14, 13)])
+def test_layer_of_one_product_each_way_is_its_nodes(ops, n, experts, k, hidden, inter, gemm, gu, dn):
+    import torch
+    p = moe_path(gu, dn, experts, hidden, inter, n, k)
+    if gu == 12:
+        assert (p["layer gateup"], p["layer down"]) == gemm
+    G, U = (ops.Q4KWeight.synthetic(s, inter, hidden, experts, gu) for s in (1, 2))
+    D = ops.Q4KWeight.synthetic(3, hidden, inter, experts, dn)
+    sh = (ops.Q4KWeight.synthetic(4, inter, hidden, 1, gu), ops.Q4KWeight.synthetic(5, inter, hidden, 1, gu), ops.Q4KWeight.synthetic(6, hidden, inter, 1, dn))
+    gen = torch.Generator(device="cuda").manual_seed(n + experts)
+    x, lg = torch.randn((n, hidden), device="cuda", generator=gen), torch.randn((n, experts), device="cuda", generator=gen)
+    gi = torch.randn(hidden, device="cuda", generator=gen) * hidden ** -0.5
+    y, ids, w = ops.moe_layer(G, U, D, x, lg, k, silu=ops.SILU_FAST)
+    rows = ops.debug_moe_hidden((n, k, inter))
+    h = ops.moe_gateup_swiglu(G, U, x, ids, ops.SILU_FAST)
+    assert torch.equal(rows, h) and torch.equal(y, ops.moe_down_weighted(D, h, ids, w))
+    ys = ops.moe_layer(G, U, D, x, lg, k, shared=(*sh, gi), silu=ops.SILU_FAST)[0]
+    pick = sorted({0, 1, n // 2, n - 1})
+    for shared, full in ((None, y), ((*sh, gi), ys)):
+        one = torch.cat([ops.moe_layer(G, U, D, x[t:t + 1].contiguous(), lg[t:t + 1].contiguous(), k, shared=shared, silu=ops.SILU_FAST)[0] for t in pick])
+        near(full[pick], one)
+    for m in (G, U, D, *sh):
+        m.free()
