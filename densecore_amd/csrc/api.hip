@@ -1372,7 +1372,8 @@ static bool moe_gemm_width(const mq_weight* w, int64_t n, int top_k) {
     if (n >= 192) return n * top_k >= 6 * w->n_experts;
     return n >= kMoeGemmMinTokens && n * top_k >= 5 * w->n_experts && moe_gemm_estimate(w->n_experts, w->rowtiles, w->rows, w->nb, n, top_k);
 }
-// Whether a MoE block runs its expert products on the expert-grouped GEMM (a product whose type the GEMM does not take stays where it is).  By the routed rows per expert rpe:
+// Whether a MoE block runs its expert products on the expert-grouped GEMM (a product whose type the GEMM does not take stays where it
+// is), below 192 tokens by product (moe_gateup_takes_gemm, moe_down_takes_gemm).  By the routed rows per expert rpe:
 // from inter <= 12 rpe^3 on (2.8 rows at 256, 3.5 at 512, 4.4 at 1024), from six, and where the down product's estimate says so.  The line
 // goes through 15,305 blocks (8 to 256 experts, top-2 to 8, 1024 to 4096 x 256 to 1024, every mix of Q4_K, Q5_K and Q6_K, with and without
 // a shared expert, 9 to 400 tokens) timed both ways: the choice takes 1.008 of the faster one's time (1.088 with six rows, or five and the
